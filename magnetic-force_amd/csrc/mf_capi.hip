@@ -44,6 +44,20 @@ Status workspace(mf_ctx *ctx, const std::string &name, size_t bytes, void **out)
   return Status::Ok();
 }
 
+bool workspace_now(mf_ctx *ctx, const std::string &name, size_t bytes, void **out) {
+  const auto it = ctx->ws.find(name);
+  if (it == ctx->ws.end() || it->second.bytes() < bytes) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+      (void)hipGetLastError();
+      return false;
+    }
+  }
+  const bool ok = workspace(ctx, name, bytes, out).ok();
+  if (!ok) (void)hipGetLastError();
+  return ok;
+}
+
 KernelTimer::KernelTimer(mf_ctx *ctx, const char *name) : KernelTimer(ctx, name, ctx->stream) {}
 
 KernelTimer::KernelTimer(mf_ctx *ctx, const char *name, hipStream_t stream)

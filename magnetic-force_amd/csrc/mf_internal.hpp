@@ -145,6 +145,11 @@ namespace mf {
 // Returns a device workspace of at least `bytes` for `name`.
 Status workspace(mf_ctx *ctx, const std::string &name, size_t bytes, void **out);
 
+// The same where the caller has a path that needs no scratch: false (and no
+// error) when the workspace would have to grow and cannot, because the stream
+// is being captured or the allocation fails.
+bool workspace_now(mf_ctx *ctx, const std::string &name, size_t bytes, void **out);
+
 // Records timing events around a kernel family when timing is enabled, on
 // the stream the family is launched on (the context's stream by default).
 class KernelTimer {
