@@ -6,22 +6,32 @@
 //   fitted_force_ofM_kernel :516-605  -> force_allpairs_kernel
 //   cuda_ext_fitted_force_tensor_kernel :432-512 -> hessian_allpairs_kernel
 //
-// Design (one wavefront = 64 lanes x TPT targets):
+// Design (one wavefront = 16 TPT targets):
 //  * Sources live in HBM as 32-byte records {x,y,z,0, mx,my,mz,0}, padded to a
-//    whole tile with far-away zero-moment records.  The source index is
-//    uniform across the wave, so record loads are scalar loads and the pair
-//    math takes source values straight from SGPRs: no LDS traffic and no
-//    barriers in the inner loop.
+//    whole tile with far-away zero-moment records.
+//  * A wave stages 64 records at a time in its own LDS (no barrier: the block
+//    is the wave) and reads them back into vector registers: lane l evaluates
+//    its TPT targets (l mod 16, + 16, ...) against every fourth record (those
+//    of l / 16), so one 24-byte LDS read serves TPT pairs.  A SIMD
+//    issues FP32 vector instructions of two waves at once (2.3 cycles each)
+//    unless both read a scalar register (4.4), and 9 of a field pair's 20 did
+//    while the sources sat in scalar registers.
 //  * Sources are cut into tiles of 64 with a precomputed bounding box.  Each
 //    wave computes the bounding box of its own targets once; a tile whose
 //    box-to-box distance exceeds the smoothing support runs a branch-free
 //    far-field loop (pure dipole, one v_rsq_f32 per pair).  Other tiles run
-//    the mixed loop that also evaluates the smoothed near-field polynomials.
-//  * Per-tile sums are FP32; tile sums are accumulated in FP64, so the
-//    summation error does not grow with N.
-//  * The source range is split into chunks along grid.y to give the 256 CUs
-//    enough waves; chunk partials (FP64) are summed in a fixed order by a
-//    separate reduction kernel, so results are deterministic.
+//    the mixed loop, which reads the smoothed coefficients from a table in LDS.
+//  * Sums of up to four tiles (64 terms a lane) are FP32; they are accumulated
+//    in FP64, so the summation error does not grow with N.
+//  * The source range is split into chunks of whole 16-record groups along
+//    grid.y to give the 256 CUs enough waves; chunk partials (FP64) are summed
+//    in a fixed order by a separate reduction kernel, so results are
+//    deterministic.
+//  Measured per launch, before (scalar sources, closed-form coefficients, chunks
+//  of whole tiles) and now: field 22.6 -> 8.4 us at 512 particles, 65.0 -> 55.9 us
+//  at 8,192, 33.8 -> 29.9 ms at 262,144 (2.3e12 pairs/s; the far loop alone would
+//  reach 2.4e12: a v_rsq_f32 holds its SIMD for 17 of a pair's 66 cycles); force
+//  36.9 -> 10.4 us, 91.9 -> 77.8 us, 49.7 -> 42.3 ms.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -35,8 +45,193 @@ namespace mf {
 
 namespace {
 
-constexpr int kBlock = 256;
 constexpr float kPadCoord = 1.0e18f;  // far-away position of padding records
+
+// ---------------------------------------------------------------------------
+// Near-pair coefficient tables (mf_pair.hpp describes their entries).  The
+// fits are constexpr: at h = 1 they are the constants of the all-pairs kernels
+// (alpha h^5, beta h^3 and the curves times h^4 depend on q alone), which so
+// need no table per h; the FMM builds its tables with h included on the host.
+
+// alpha h^5 and beta h^3 of a near pair at q < 2, in FP64 (the forms of the
+// mf_pair.hpp header; g unexpanded, which is accurate in FP64).
+constexpr void near_coeffs_f64(double q, double &a, double &b) {
+  if (q < 1.0) {
+    a = 0.8 - 0.5 * q;
+    b = -8.0 / 3.0 + q * q * (4.8 - 2.5 * q);
+    return;
+  }
+  const double q3 = q * q * q;
+  const double g = -3.0 * (q3 * (((q / 6.0 - 1.2) * q + 3.0) * q - 8.0 / 3.0) + 1.0 / 15.0);
+  const double w = (2.0 - q) * (2.0 - q) * (2.0 - q);
+  a = (g / q3 - w) / (3.0 * q * q);
+  b = g / (3.0 * q3) - w;
+}
+
+// cos((2 i + 1) pi / 8): the Chebyshev points of a cubic.
+constexpr double kCheb[4] = {0.92387953251128674, 0.38268343236508977, -0.38268343236508977,
+                             -0.92387953251128674};
+
+// Power-basis coefficients c[0..3] of the cubic through (t[i], y[i]), i < 4
+// (Gaussian elimination with partial pivoting on the Vandermonde system).
+constexpr void cubic_through(const double (&t)[4], const double (&y)[4], double (&c)[4]) {
+  double m[4][5] = {};
+  for (int i = 0; i < 4; ++i) {
+    double p = 1.0;
+    for (int j = 0; j < 4; ++j, p *= t[i]) m[i][j] = p;
+    m[i][4] = y[i];
+  }
+  auto mag = [](double v) { return v < 0.0 ? -v : v; };
+  for (int col = 0; col < 4; ++col) {
+    int piv = col;
+    for (int i = col + 1; i < 4; ++i)
+      if (mag(m[i][col]) > mag(m[piv][col])) piv = i;
+    for (int j = 0; j < 5; ++j) {
+      const double x = m[col][j];
+      m[col][j] = m[piv][j];
+      m[piv][j] = x;
+    }
+    for (int i = col + 1; i < 4; ++i) {
+      const double f = m[i][col] / m[col][col];
+      for (int j = col; j < 5; ++j) m[i][j] -= f * m[col][j];
+    }
+  }
+  for (int i = 3; i >= 0; --i) {
+    double s = m[i][4];
+    for (int j = i + 1; j < 4; ++j) s -= m[i][j] * c[j];
+    c[i] = s / m[i][i];
+  }
+}
+
+// Coefficients (ascending powers) of c(t + s) from those of the cubic c(t).
+constexpr void shift_cubic(const double *c, double s, double *out) {
+  out[0] = ((c[3] * s + c[2]) * s + c[1]) * s + c[0];
+  out[1] = (3.0 * c[3] * s + 2.0 * c[2]) * s + c[1];
+  out[2] = 3.0 * c[3] * s + c[2];
+  out[3] = c[3];
+}
+
+// put(entry, cubic of alpha, cubic of beta) for every entry of the field table,
+// alpha times fa and beta times fb.
+template <class Put>
+constexpr void fill_field_table(double fa, double fb, const Put &put) {
+  double t[4] = {};
+  for (int i = 0; i < 4; ++i) t[i] = 0.5 + 0.5 * kCheb[i];
+  double ca[4] = {}, cb[4] = {};
+  for (int k = 0; k < kFieldTabN; ++k) {
+    double ya[4] = {}, yb[4] = {};
+    for (int i = 0; i < 4; ++i) {
+      near_coeffs_f64((k + t[i]) * 2.0 / kFieldTabN, ya[i], yb[i]);
+      ya[i] *= fa;
+      yb[i] *= fb;
+    }
+    cubic_through(t, ya, ca);
+    cubic_through(t, yb, cb);
+    put(k, ca, cb);
+  }
+  double sa[4] = {}, sb[4] = {};  // the last interval's cubics, one interval on
+  shift_cubic(ca, 1.0, sa);
+  shift_cubic(cb, 1.0, sb);
+  put(kFieldTabN, sa, sb);
+}
+
+// Fitted curve table of the reference (Dipole_hessian.kern:53-61), highest
+// power first.  Kept as data: the force must use exactly these curves.
+constexpr double kC1[4][5] = {
+    {9.97813616438174e-09, -2.97897856524718e-08, 2.38918644566813e-09, 4.53199938857366e-08,
+     2.44617454752747e-11},
+    {-2.76473728643294e-09, 2.86975546540539e-08, -9.94582836806651e-08, 1.25129924573675e-07,
+     -2.37010166723652e-08},
+    {-1.09679990621465e-09, 9.77055663264614e-09, -2.54781238661150e-08, 2.65020634884934e-09,
+     5.00787562417835e-08},
+    {3.79927162333632e-10, -6.26368404962679e-09, 3.94760528277489e-08, -1.13580541622200e-07,
+     1.27491333574323e-07}};
+constexpr double kC2[4][5] = {
+    {6.69550479838731e-08, -1.61753307173877e-07, 1.68213714992711e-08, 1.34558143036838e-07,
+     1.10976027980100e-10},
+    {-3.08460139955194e-08, 2.29192245602275e-07, -5.88399621128587e-07, 5.61170054591844e-07,
+     -1.14421132829680e-07},
+    {3.50477408060213e-09, -5.25956271895141e-08, 2.78876509535747e-07, -6.24199554212217e-07,
+     4.91807818904985e-07},
+    {7.33485346367840e-10, -9.58855788627803e-09, 4.37085309763591e-08, -7.48004594092261e-08,
+     2.34161209605651e-08}};
+
+// put(entry, cubic of C1, cubic of -(C2 - 3 C1) / 5) for every entry of the
+// force table, both times scale / (3 mu0 / (4 pi)).
+template <class Put>
+constexpr void fill_hess_table(double scale, const Put &put) {
+  const double f = scale / (3.0 * kMu0 / (4.0 * kPi));
+  constexpr int per_unit = kHessTabN / 4;
+  double t[4] = {};
+  for (int i = 0; i < 4; ++i) t[i] = -0.5 + 0.5 * kCheb[i];
+  double cc[4] = {}, cd[4] = {}, first_c[4] = {}, first_d[4] = {};
+  for (int e = 1; e <= kHessTabN; ++e) {  // entry e: u in (e - 1, e]
+    const int piece = (e - 1) / per_unit;
+    double yc[4] = {}, yd[4] = {};
+    for (int i = 0; i < 4; ++i) {
+      const double q = (e + t[i]) / per_unit;
+      double c1 = 0.0, c2 = 0.0;
+      for (int j = 0; j < 5; ++j) {
+        c1 = c1 * q + kC1[piece][j];
+        c2 = c2 * q + kC2[piece][j];
+      }
+      yc[i] = f * c1;
+      yd[i] = -f * (c2 - 3.0 * c1) / 5.0;
+    }
+    cubic_through(t, yc, cc);
+    cubic_through(t, yd, cd);
+    put(e, cc, cd);
+    if (e == 1)
+      for (int j = 0; j < 4; ++j) {
+        first_c[j] = cc[j];
+        first_d[j] = cd[j];
+      }
+  }
+  double sc[4] = {}, sd[4] = {};
+  shift_cubic(cc, 1.0, sc);  // entry kHessTabN + 1 continues the last one
+  shift_cubic(cd, 1.0, sd);
+  put(kHessTabN + 1, sc, sd);
+  shift_cubic(first_c, -1.0, sc);  // entry 0 (u = 0) continues entry 1
+  shift_cubic(first_d, -1.0, sd);
+  put(0, sc, sd);
+}
+
+// The tables at h = 1 in the split layout (split_near_table).
+template <int N>
+struct UnitTable {
+  float v[2][N][4];
+};
+constexpr UnitTable<kFieldTabEntries> unit_field_table() {
+  UnitTable<kFieldTabEntries> t{};
+  fill_field_table(1.0, 1.0, [&](int e, const double *a, const double *b) {
+    for (int j = 0; j < 4; ++j) {
+      t.v[0][e][j] = static_cast<float>(a[j]);
+      t.v[1][e][j] = static_cast<float>(b[j]);
+    }
+  });
+  return t;
+}
+constexpr UnitTable<kHessTabEntries> unit_hess_table() {
+  UnitTable<kHessTabEntries> t{};
+  fill_hess_table(1.0, [&](int e, const double *a, const double *b) {
+    for (int j = 0; j < 4; ++j) {
+      t.v[0][e][j] = static_cast<float>(a[j]);
+      t.v[1][e][j] = static_cast<float>(b[j]);
+    }
+  });
+  return t;
+}
+static __device__ const UnitTable<kFieldTabEntries> d_field_tab __attribute__((aligned(16))) =
+    unit_field_table();
+static __device__ const UnitTable<kHessTabEntries> d_hess_tab __attribute__((aligned(16))) =
+    unit_hess_table();
+
+void store_entry(float *tab, int e, const double *ca, const double *cb) {
+  for (int j = 0; j < 4; ++j) {
+    tab[8 * e + j] = static_cast<float>(ca[j]);
+    tab[8 * e + 4 + j] = static_cast<float>(cb[j]);
+  }
+}
 
 __device__ __forceinline__ float wave_min(float v) {
 #pragma unroll
@@ -55,56 +250,29 @@ __device__ __forceinline__ float uniform_f(float v) {
 // ---------------------------------------------------------------------------
 // Packing and tile boxes.
 
-__global__ void pack_sources_kernel(int64_t n, int64_t n_pad, const float *__restrict__ x,
-                                    const float *__restrict__ y, const float *__restrict__ z,
-                                    const float *__restrict__ mx, const float *__restrict__ my,
-                                    const float *__restrict__ mz, float scale,
-                                    SrcRec *__restrict__ out) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n_pad) return;
-  SrcRec r;
-  if (i < n) {
-    r.x = x[i];
-    r.y = y[i];
-    r.z = z[i];
-    r.mx = mx ? scale * mx[i] : 0.f;
-    r.my = my ? scale * my[i] : 0.f;
-    r.mz = mz ? scale * mz[i] : 0.f;
-  } else {
-    r.x = kPadCoord;
-    r.y = kPadCoord;
-    r.z = kPadCoord;
-    r.mx = r.my = r.mz = 0.f;
-  }
-  r.w = 0.f;
-  r.mw = 0.f;
-  out[i] = r;
-}
-
-__global__ void pack_moments_kernel(int64_t n, const float *__restrict__ mx,
-                                    const float *__restrict__ my, const float *__restrict__ mz,
-                                    float scale, SrcRec *__restrict__ out) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float4 m = make_float4(scale * mx[i], scale * my[i], scale * mz[i], 0.f);
-  reinterpret_cast<float4 *>(out + i)[1] = m;
-}
-
-// One wave per tile of kTile sources.  Boxes ignore padding records.
-__global__ void tile_box_kernel(int64_t n, int64_t ntiles, const SrcRec *__restrict__ src,
-                                float4 *__restrict__ boxes) {
+// One wave per tile of kTile records: the records (padding included) and the
+// tile's bounding box (padding excluded) in one pass.
+__global__ void pack_tiles_kernel(int64_t n, int64_t ntiles, const float *__restrict__ x,
+                                  const float *__restrict__ y, const float *__restrict__ z,
+                                  const float *__restrict__ mx, const float *__restrict__ my,
+                                  const float *__restrict__ mz, SrcRec *__restrict__ out,
+                                  float4 *__restrict__ boxes) {
   const int lane = threadIdx.x & 63;
   const int64_t tile = static_cast<int64_t>(blockIdx.x) * (blockDim.x / 64) + (threadIdx.x >> 6);
   if (tile >= ntiles) return;
-  const int64_t j = tile * kTile + lane;
+  const int64_t i = tile * kTile + lane;
+  SrcRec r{kPadCoord, kPadCoord, kPadCoord, 0.f, 0.f, 0.f, 0.f, 0.f};
   float lx = INFINITY, ly = INFINITY, lz = INFINITY;
   float hx = -INFINITY, hy = -INFINITY, hz = -INFINITY;
-  if (j < n) {
-    const SrcRec s = src[j];
-    lx = hx = s.x;
-    ly = hy = s.y;
-    lz = hz = s.z;
+  if (i < n) {
+    lx = hx = r.x = x[i];
+    ly = hy = r.y = y[i];
+    lz = hz = r.z = z[i];
+    r.mx = mx ? mx[i] : 0.f;
+    r.my = my ? my[i] : 0.f;
+    r.mz = mz ? mz[i] : 0.f;
   }
+  out[i] = r;
   lx = wave_min(lx);
   ly = wave_min(ly);
   lz = wave_min(lz);
@@ -117,6 +285,15 @@ __global__ void tile_box_kernel(int64_t n, int64_t ntiles, const SrcRec *__restr
   }
 }
 
+__global__ void pack_moments_kernel(int64_t n, const float *__restrict__ mx,
+                                    const float *__restrict__ my, const float *__restrict__ mz,
+                                    float scale, SrcRec *__restrict__ out) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  float4 m = make_float4(scale * mx[i], scale * my[i], scale * mz[i], 0.f);
+  reinterpret_cast<float4 *>(out + i)[1] = m;
+}
+
 // Distance^2 between two axis-aligned boxes (0 when they overlap).
 __device__ __forceinline__ float box_dist2(float tlx, float tly, float tlz, float thx, float thy,
                                            float thz, float4 slo, float4 shi) {
@@ -127,366 +304,478 @@ __device__ __forceinline__ float box_dist2(float tlx, float tly, float tlz, floa
 }
 
 // ---------------------------------------------------------------------------
+// The wave's share of a launch: targets 16 TPT blockIdx.x + 16 k + (lane mod
+// 16), k < TPT; source records [16 sub0, 16 sub1).
+
+constexpr int kSub = 16;    // records per group, the granularity of a chunk
+constexpr int kFlush = 4;   // tiles between FP64 accumulations
+
+struct SourceRange {
+  int64_t sub0, sub1;
+};
+__device__ __forceinline__ SourceRange chunk_range(int64_t nsub, int64_t per) {
+  const int64_t s0 = static_cast<int64_t>(blockIdx.y) * per;
+  return {s0, s0 + per < nsub ? s0 + per : nsub};
+}
+
+// Bounding box of the wave's targets (uniform).
+struct WaveBox {
+  float lx, ly, lz, hx, hy, hz;
+};
+template <int TPT>
+__device__ __forceinline__ WaveBox target_box(const float (&tx)[TPT], const float (&ty)[TPT],
+                                              const float (&tz)[TPT]) {
+  float v[6] = {tx[0], ty[0], tz[0], tx[0], ty[0], tz[0]};
+#pragma unroll
+  for (int k = 1; k < TPT; ++k) {
+    v[0] = fminf(v[0], tx[k]);
+    v[1] = fminf(v[1], ty[k]);
+    v[2] = fminf(v[2], tz[k]);
+    v[3] = fmaxf(v[3], tx[k]);
+    v[4] = fmaxf(v[4], ty[k]);
+    v[5] = fmaxf(v[5], tz[k]);
+  }
+#pragma unroll
+  for (int off = 8; off >= 1; off >>= 1)  // the four groups of 16 lanes hold the same targets
+#pragma unroll
+    for (int a = 0; a < 6; ++a) {
+      const float o = __shfl_xor(v[a], off, 64);
+      v[a] = a < 3 ? fminf(v[a], o) : fmaxf(v[a], o);
+    }
+  return {uniform_f(v[0]), uniform_f(v[1]), uniform_f(v[2]),
+          uniform_f(v[3]), uniform_f(v[4]), uniform_f(v[5])};
+}
+
+// Up to 64 staged records.
+struct Staged {
+  float4 a[kTile];  // x, y, z, mx
+  float2 b[kTile];  // my, mz
+};
+
+// Walks the wave's sources: stages each tile's part of the range and calls
+// body(steps, dist2): `steps` groups of four records are staged (record 4 j + q
+// is lane group q's j-th), dist2 is the distance^2 from the wave's targets to
+// the tile's box.  flush() runs every kFlush tiles and at the end.  The next
+// part's records are loaded before the current one is evaluated.
+template <class Body, class Flush>
+__device__ __forceinline__ void walk_sources(const SrcRec *__restrict__ src,
+                                             const float4 *__restrict__ boxes, SourceRange r,
+                                             const WaveBox &t, Staged &st, int lane,
+                                             const Body &body, const Flush &flush) {
+  const float4 *__restrict__ rec = reinterpret_cast<const float4 *>(src);
+  constexpr int kPer = kTile / kSub;  // groups per tile
+  auto part = [&](int64_t s) {        // groups of s's tile that belong to the range
+    const int64_t e = (s / kPer + 1) * kPer;
+    return static_cast<int>((e < r.sub1 ? e : r.sub1) - s);
+  };
+  // the last record of a short part is read again by the lanes past its end
+  auto load = [&](int64_t s, int cnt, float4 &p, float4 &m) {
+    const int64_t j = s * kSub + min(lane, cnt * kSub - 1);
+    p = rec[2 * j];
+    m = rec[2 * j + 1];
+  };
+  int since = 0;
+  int64_t s = r.sub0;
+  if (s >= r.sub1) return;
+  int cnt = part(s);
+  float4 p, m;
+  load(s, cnt, p, m);
+  while (true) {
+    __builtin_amdgcn_wave_barrier();  // the previous part has been read
+    st.a[lane] = make_float4(p.x, p.y, p.z, m.x);
+    st.b[lane] = make_float2(m.y, m.z);
+    __builtin_amdgcn_wave_barrier();
+    const int64_t tile = s / kPer;
+    const float4 lo = boxes[2 * tile], hi = boxes[2 * tile + 1];
+    const int steps = 4 * cnt;
+    s += cnt;
+    const bool more = s < r.sub1;
+    if (more) {
+      cnt = part(s);
+      load(s, cnt, p, m);
+    }
+    body(steps, uniform_f(box_dist2(t.lx, t.ly, t.lz, t.hx, t.hy, t.hz, lo, hi)));
+    if (++since == kFlush || !more) {
+      flush();
+      since = 0;
+    }
+    if (!more) break;
+  }
+}
+
+// A unit table into the wave's LDS.
+template <int N>
+__device__ __forceinline__ void load_table(const UnitTable<N> &src, float4 (&dst)[2 * N], int lane) {
+  const float4 *__restrict__ t = reinterpret_cast<const float4 *>(&src);
+  for (int i = lane; i < 2 * N; i += 64) dst[i] = t[i];
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Sum over the four lane groups (the same targets against a quarter of the
+// records each).
+__device__ __forceinline__ double group_sum(double v) {
+  v += __shfl_xor(v, 16, 64);
+  v += __shfl_xor(v, 32, 64);
+  return v;
+}
+
+// ---------------------------------------------------------------------------
 // Field: partial[chunk][c][i] = c * sum_{j in chunk} (3 alpha d (d.m) - beta m)_c
 
 template <int TPT>
-__global__ __launch_bounds__(kBlock) void field_allpairs_kernel(
-    const float4 *__restrict__ tpos, int tstride, int64_t nt, const SrcRec *__restrict__ src,
-    const float4 *__restrict__ boxes, int64_t ntiles, int64_t tiles_per_chunk, FieldConsts fc,
-    int64_t nt_ld, double *__restrict__ partial) {
-  const int lane = threadIdx.x & 63;
-  const int64_t wave = static_cast<int64_t>(blockIdx.x) * (kBlock / 64) + (threadIdx.x >> 6);
-  const int64_t tbase = wave * 64 * TPT;
-  if (tbase >= nt) return;  // whole wave idle (uniform)
-
+__global__ __launch_bounds__(64) void field_allpairs_kernel(
+    Points tgt, int64_t nt, const SrcRec *__restrict__ src, const float4 *__restrict__ boxes,
+    int64_t nsub, int64_t per, FieldConsts fc, int64_t nt_ld, double *__restrict__ partial) {
+  __shared__ Staged st;
+  __shared__ float4 s_tab[2 * kFieldTabEntries];
+  const int lane = threadIdx.x, c = lane & 15, q = lane >> 4;
+  const int64_t tbase = static_cast<int64_t>(blockIdx.x) * (16 * TPT);
   float tx[TPT], ty[TPT], tz[TPT];
-  float lx = INFINITY, ly = INFINITY, lz = INFINITY, hx = -INFINITY, hy = -INFINITY,
-        hz = -INFINITY;
 #pragma unroll
   for (int k = 0; k < TPT; ++k) {
-    int64_t i = tbase + k * 64 + lane;
-    const bool valid = i < nt;
-    i = valid ? i : nt - 1;
-    const float4 p = tpos[i * tstride];
-    tx[k] = p.x;
-    ty[k] = p.y;
-    tz[k] = p.z;
-    if (valid) {
-      lx = fminf(lx, p.x);
-      ly = fminf(ly, p.y);
-      lz = fminf(lz, p.z);
-      hx = fmaxf(hx, p.x);
-      hy = fmaxf(hy, p.y);
-      hz = fmaxf(hz, p.z);
-    }
+    const int64_t i = min(tbase + 16 * k + c, nt - 1) * tgt.stride;
+    tx[k] = tgt.x[i];
+    ty[k] = tgt.y[i];
+    tz[k] = tgt.z[i];
   }
-  lx = uniform_f(wave_min(lx));
-  ly = uniform_f(wave_min(ly));
-  lz = uniform_f(wave_min(lz));
-  hx = uniform_f(wave_max(hx));
-  hy = uniform_f(wave_max(hy));
-  hz = uniform_f(wave_max(hz));
-
+  bool have_tab = false;  // read on the first mixed tile
   double acc[TPT][3];
+  float a1[TPT][3], a2[TPT][3];
 #pragma unroll
-  for (int k = 0; k < TPT; ++k) acc[k][0] = acc[k][1] = acc[k][2] = 0.0;
-
-  const int64_t chunk = blockIdx.y;
-  const int64_t t0 = chunk * tiles_per_chunk;
-  const int64_t t1 = t0 + tiles_per_chunk < ntiles ? t0 + tiles_per_chunk : ntiles;
-
-  for (int64_t tile = t0; tile < t1; ++tile) {
-    const float4 slo = boxes[2 * tile];
-    const float4 shi = boxes[2 * tile + 1];
-    const float dist2 = uniform_f(box_dist2(lx, ly, lz, hx, hy, hz, slo, shi));
-    float a1[TPT][3], a2[TPT][3];
+  for (int k = 0; k < TPT; ++k)
 #pragma unroll
-    for (int k = 0; k < TPT; ++k) a1[k][0] = a1[k][1] = a1[k][2] = a2[k][0] = a2[k][1] = a2[k][2] = 0.f;
-    const SrcRec *__restrict__ s = src + tile * kTile;
+    for (int a = 0; a < 3; ++a) {
+      acc[k][a] = 0.0;
+      a1[k][a] = a2[k][a] = 0.f;
+    }
+  auto body = [&](int steps, float dist2) {
     if (dist2 >= fc.near2) {
       // far tile: every pair has q >= 2 (pure dipole)
-#pragma unroll 8
-      for (int j = 0; j < kTile; ++j) {
-        const float sx = s[j].x, sy = s[j].y, sz = s[j].z;
-        const float mx = s[j].mx, my = s[j].my, mz = s[j].mz;
+#pragma unroll 1
+      for (int j = 0; j < steps; ++j) {
+        const float4 u = st.a[4 * j + q];
+        const float2 v = st.b[4 * j + q];
 #pragma unroll
         for (int k = 0; k < TPT; ++k) {
-          const float dx = tx[k] - sx, dy = ty[k] - sy, dz = tz[k] - sz;
+          const float dx = tx[k] - u.x, dy = ty[k] - u.y, dz = tz[k] - u.z;
           const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
           const float ir = __builtin_amdgcn_rsqf(r2);
           const float ir2 = ir * ir;
           const float ir3 = ir2 * ir;
-          const float dm = fmaf(dx, mx, fmaf(dy, my, dz * mz));
+          const float dm = fmaf(dx, u.w, fmaf(dy, v.x, dz * v.y));
           const float s1 = dm * (ir3 * ir2);
           a1[k][0] = fmaf(dx, s1, a1[k][0]);
           a1[k][1] = fmaf(dy, s1, a1[k][1]);
           a1[k][2] = fmaf(dz, s1, a1[k][2]);
-          a2[k][0] = fmaf(mx, ir3, a2[k][0]);
-          a2[k][1] = fmaf(my, ir3, a2[k][1]);
-          a2[k][2] = fmaf(mz, ir3, a2[k][2]);
+          a2[k][0] = fmaf(u.w, ir3, a2[k][0]);
+          a2[k][1] = fmaf(v.x, ir3, a2[k][1]);
+          a2[k][2] = fmaf(v.y, ir3, a2[k][2]);
         }
       }
     } else {
       // mixed tile: smoothed near field where q < 2
-#pragma unroll 2
-      for (int j = 0; j < kTile; ++j) {
-        const float sx = s[j].x, sy = s[j].y, sz = s[j].z;
-        const float mx = s[j].mx, my = s[j].my, mz = s[j].mz;
+      if (!have_tab) {
+        load_table(d_field_tab, s_tab, lane);
+        have_tab = true;
+      }
+#pragma unroll 1
+      for (int j = 0; j < steps; ++j) {
+        const float4 u = st.a[4 * j + q];
+        const float2 v = st.b[4 * j + q];
 #pragma unroll
         for (int k = 0; k < TPT; ++k) {
-          const float dx = tx[k] - sx, dy = ty[k] - sy, dz = tz[k] - sz;
+          const float dx = tx[k] - u.x, dy = ty[k] - u.y, dz = tz[k] - u.z;
           const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
           const float ir = __builtin_amdgcn_rsqf(r2);
           const float ir2 = ir * ir;
           float beta = ir2 * ir;
           float alpha = beta * ir2;
-          if (r2 < fc.near2) field_near_coeffs(fc, r2, ir, alpha, beta);
-          const float dm = fmaf(dx, mx, fmaf(dy, my, dz * mz));
+          if (r2 < fc.near2) {
+            field_near_coeffs_tab(s_tab, fc.tab_scale, r2, ir, alpha, beta);
+            alpha *= fc.inv_h5;
+            beta *= fc.inv_h3;
+          }
+          const float dm = fmaf(dx, u.w, fmaf(dy, v.x, dz * v.y));
           const float s1 = dm * alpha;
           a1[k][0] = fmaf(dx, s1, a1[k][0]);
           a1[k][1] = fmaf(dy, s1, a1[k][1]);
           a1[k][2] = fmaf(dz, s1, a1[k][2]);
-          a2[k][0] = fmaf(mx, beta, a2[k][0]);
-          a2[k][1] = fmaf(my, beta, a2[k][1]);
-          a2[k][2] = fmaf(mz, beta, a2[k][2]);
+          a2[k][0] = fmaf(u.w, beta, a2[k][0]);
+          a2[k][1] = fmaf(v.x, beta, a2[k][1]);
+          a2[k][2] = fmaf(v.y, beta, a2[k][2]);
         }
       }
     }
+  };
+  auto flush = [&]() {
 #pragma unroll
     for (int k = 0; k < TPT; ++k)
 #pragma unroll
-      for (int c = 0; c < 3; ++c)
-        acc[k][c] += 3.0 * static_cast<double>(a1[k][c]) - static_cast<double>(a2[k][c]);
-  }
+      for (int a = 0; a < 3; ++a) {
+        acc[k][a] += 3.0 * static_cast<double>(a1[k][a]) - static_cast<double>(a2[k][a]);
+        a1[k][a] = a2[k][a] = 0.f;
+      }
+  };
+  walk_sources(src, boxes, chunk_range(nsub, per), target_box<TPT>(tx, ty, tz), st, lane, body,
+               flush);
 
   const double cfac = 1.0 / (4.0 * kPi);
-  double *out = partial + chunk * 3 * nt_ld;
+  double *out = partial + static_cast<int64_t>(blockIdx.y) * 3 * nt_ld;
+  const int64_t i = tbase + lane;  // lane group k stores targets 16 k .. 16 k + 15
 #pragma unroll
-  for (int k = 0; k < TPT; ++k) {
-    const int64_t i = tbase + k * 64 + lane;
-    if (i < nt) {
-      out[i] = acc[k][0] * cfac;
-      out[nt_ld + i] = acc[k][1] * cfac;
-      out[2 * nt_ld + i] = acc[k][2] * cfac;
+  for (int a = 0; a < 3; ++a) {
+    double v = 0.0;
+#pragma unroll
+    for (int k = 0; k < TPT; ++k) {
+      const double sum = group_sum(acc[k][a]);
+      v = q == k ? sum : v;
     }
+    if (q < TPT && i < nt) out[a * nt_ld + i] = v * cfac;
   }
 }
 
 // ---------------------------------------------------------------------------
 // Force: targets are the sources themselves (same records), target moment n.
 //   F = s sum_j [ d (P (m.n) + R (d.m)(d.n)) + m P (d.n) + n P (d.m) ]
-// with s = 3 mu0/(4 pi), accumulated as A_d (3), A_m (3), A_n (1).
+// with s = 3 mu0/(4 pi), accumulated as A_d (3), A_m (3), A_n (1).  With n5 = -5 n
+// and R / -5 = P / r^2 (far) the pair takes one multiply less; the m-sums then
+// hold P (d.n5).
 
 template <int TPT>
-__global__ __launch_bounds__(kBlock) void force_allpairs_kernel(
+__global__ __launch_bounds__(64) void force_allpairs_kernel(
     const SrcRec *__restrict__ tgt, int64_t nt, const SrcRec *__restrict__ src,
-    const float4 *__restrict__ boxes, int64_t ntiles, int64_t tiles_per_chunk, HessConsts hc,
-    int64_t nt_ld, double *__restrict__ partial) {
-  __shared__ float4 s_tab[4 * 3];
-  if (threadIdx.x < 12) {
-    const float *row = &hc.curve[threadIdx.x / 3][(threadIdx.x % 3) * 4];
-    s_tab[threadIdx.x] = make_float4(row[0], row[1], row[2], row[3]);
-  }
-  __syncthreads();
-  const float *tab = reinterpret_cast<const float *>(s_tab);
-
-  const int lane = threadIdx.x & 63;
-  const int64_t wave = static_cast<int64_t>(blockIdx.x) * (kBlock / 64) + (threadIdx.x >> 6);
-  const int64_t tbase = wave * 64 * TPT;
-  if (tbase >= nt) return;
-
-  float tx[TPT], ty[TPT], tz[TPT], nx[TPT], ny[TPT], nz[TPT];
-  float lx = INFINITY, ly = INFINITY, lz = INFINITY, hx = -INFINITY, hy = -INFINITY,
-        hz = -INFINITY;
+    const float4 *__restrict__ boxes, int64_t nsub, int64_t per, HessConsts hc, int64_t nt_ld,
+    double *__restrict__ partial) {
+  __shared__ float4 s_tab[2 * kHessTabEntries];
+  __shared__ Staged st;
+  const int lane = threadIdx.x, c = lane & 15, q = lane >> 4;
+  bool have_tab = false;  // read on the first mixed tile
+  const int64_t tbase = static_cast<int64_t>(blockIdx.x) * (16 * TPT);
+  float tx[TPT], ty[TPT], tz[TPT], nx[TPT], ny[TPT], nz[TPT], nx5[TPT], ny5[TPT], nz5[TPT];
 #pragma unroll
   for (int k = 0; k < TPT; ++k) {
-    int64_t i = tbase + k * 64 + lane;
-    const bool valid = i < nt;
-    i = valid ? i : nt - 1;
-    const SrcRec t = tgt[i];
+    const SrcRec t = tgt[min(tbase + 16 * k + c, nt - 1)];
     tx[k] = t.x;
     ty[k] = t.y;
     tz[k] = t.z;
     nx[k] = t.mx;
     ny[k] = t.my;
     nz[k] = t.mz;
-    if (valid) {
-      lx = fminf(lx, t.x);
-      ly = fminf(ly, t.y);
-      lz = fminf(lz, t.z);
-      hx = fmaxf(hx, t.x);
-      hy = fmaxf(hy, t.y);
-      hz = fmaxf(hz, t.z);
+    nx5[k] = -5.f * nx[k];
+    ny5[k] = -5.f * ny[k];
+    nz5[k] = -5.f * nz[k];
+  }
+  double acc[TPT][3];
+  float ad[TPT][3], am[TPT][3], an[TPT];
+#pragma unroll
+  for (int k = 0; k < TPT; ++k) {
+    an[k] = 0.f;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      acc[k][a] = 0.0;
+      ad[k][a] = am[k][a] = 0.f;
     }
   }
-  lx = uniform_f(wave_min(lx));
-  ly = uniform_f(wave_min(ly));
-  lz = uniform_f(wave_min(lz));
-  hx = uniform_f(wave_max(hx));
-  hy = uniform_f(wave_max(hy));
-  hz = uniform_f(wave_max(hz));
-
-  double acc[TPT][4];
-#pragma unroll
-  for (int k = 0; k < TPT; ++k) acc[k][0] = acc[k][1] = acc[k][2] = acc[k][3] = 0.0;
-  double accm[TPT][3];
-#pragma unroll
-  for (int k = 0; k < TPT; ++k) accm[k][0] = accm[k][1] = accm[k][2] = 0.0;
-
-  const int64_t chunk = blockIdx.y;
-  const int64_t t0 = chunk * tiles_per_chunk;
-  const int64_t t1 = t0 + tiles_per_chunk < ntiles ? t0 + tiles_per_chunk : ntiles;
-
-  for (int64_t tile = t0; tile < t1; ++tile) {
-    const float4 slo = boxes[2 * tile];
-    const float4 shi = boxes[2 * tile + 1];
-    const float dist2 = uniform_f(box_dist2(lx, ly, lz, hx, hy, hz, slo, shi));
-    float ad[TPT][3], am[TPT][3], an[TPT];
-#pragma unroll
-    for (int k = 0; k < TPT; ++k) {
-      ad[k][0] = ad[k][1] = ad[k][2] = 0.f;
-      am[k][0] = am[k][1] = am[k][2] = 0.f;
-      an[k] = 0.f;
-    }
-    const SrcRec *__restrict__ s = src + tile * kTile;
+  auto body = [&](int steps, float dist2) {
     if (dist2 > hc.near2) {
-#pragma unroll 4
-      for (int j = 0; j < kTile; ++j) {
-        const float sx = s[j].x, sy = s[j].y, sz = s[j].z;
-        const float mx = s[j].mx, my = s[j].my, mz = s[j].mz;
+#pragma unroll 1
+      for (int j = 0; j < steps; ++j) {
+        const float4 u = st.a[4 * j + q];
+        const float2 v = st.b[4 * j + q];
 #pragma unroll
         for (int k = 0; k < TPT; ++k) {
-          const float dx = tx[k] - sx, dy = ty[k] - sy, dz = tz[k] - sz;
+          const float dx = tx[k] - u.x, dy = ty[k] - u.y, dz = tz[k] - u.z;
           const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
           const float ir = __builtin_amdgcn_rsqf(r2);
           const float ir2 = ir * ir;
-          const float P = ir2 * ir2 * ir;            // r^-5
-          const float dm = fmaf(dx, mx, fmaf(dy, my, dz * mz));
-          const float dn = fmaf(dx, nx[k], fmaf(dy, ny[k], dz * nz[k]));
-          const float mn = fmaf(mx, nx[k], fmaf(my, ny[k], mz * nz[k]));
-          // e = P mn + R dm dn, R = -5 P ir2
-          const float e = P * fmaf(-5.f * ir2, dm * dn, mn);
-          const float f = P * dn;
+          const float P = ir2 * ir2 * ir;  // r^-5
+          const float dm = fmaf(dx, u.w, fmaf(dy, v.x, dz * v.y));
+          const float dn5 = fmaf(dx, nx5[k], fmaf(dy, ny5[k], dz * nz5[k]));
+          const float mn = fmaf(u.w, nx[k], fmaf(v.x, ny[k], v.y * nz[k]));
+          const float e = P * fmaf(dm * ir2, dn5, mn);  // P mn + R dm dn, R = -5 P ir2
+          const float f5 = P * dn5;
           ad[k][0] = fmaf(dx, e, ad[k][0]);
           ad[k][1] = fmaf(dy, e, ad[k][1]);
           ad[k][2] = fmaf(dz, e, ad[k][2]);
-          am[k][0] = fmaf(mx, f, am[k][0]);
-          am[k][1] = fmaf(my, f, am[k][1]);
-          am[k][2] = fmaf(mz, f, am[k][2]);
+          am[k][0] = fmaf(u.w, f5, am[k][0]);
+          am[k][1] = fmaf(v.x, f5, am[k][1]);
+          am[k][2] = fmaf(v.y, f5, am[k][2]);
           an[k] = fmaf(P, dm, an[k]);
         }
       }
     } else {
-#pragma unroll 2
-      for (int j = 0; j < kTile; ++j) {
-        const float sx = s[j].x, sy = s[j].y, sz = s[j].z;
-        const float mx = s[j].mx, my = s[j].my, mz = s[j].mz;
+      if (!have_tab) {
+        load_table(d_hess_tab, s_tab, lane);
+        have_tab = true;
+      }
+#pragma unroll 1
+      for (int j = 0; j < steps; ++j) {
+        const float4 u = st.a[4 * j + q];
+        const float2 v = st.b[4 * j + q];
 #pragma unroll
         for (int k = 0; k < TPT; ++k) {
-          const float dx = tx[k] - sx, dy = ty[k] - sy, dz = tz[k] - sz;
+          const float dx = tx[k] - u.x, dy = ty[k] - u.y, dz = tz[k] - u.z;
           const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-          const float ir = __builtin_amdgcn_rsqf(r2);
+          // the clamp keeps a pair at d = 0 finite
+          const float ir = __builtin_amdgcn_fmed3f(__builtin_amdgcn_rsqf(r2), 0.f, 1e12f);
           const float ir2 = ir * ir;
-          float P = ir2 * ir2 * ir;
-          float R = -5.f * P * ir2;
-          if (!(r2 > hc.near2)) hess_near_coeffs(tab, hc.inv_h, r2, ir, P, R);
-          const float dm = fmaf(dx, mx, fmaf(dy, my, dz * mz));
-          const float dn = fmaf(dx, nx[k], fmaf(dy, ny[k], dz * nz[k]));
-          const float mn = fmaf(mx, nx[k], fmaf(my, ny[k], mz * nz[k]));
-          const float e = fmaf(R, dm * dn, P * mn);
-          const float f = P * dn;
+          float c1 = ir2 * ir2, dq = c1;  // far curves
+          if (!(r2 > hc.near2)) {
+            hess_near_curves_tab(s_tab, hc.tab_scale, r2, ir, c1, dq);
+            const float w = r2 > 0.f ? hc.inv_h4 : 0.f;  // nothing at d = 0
+            c1 *= w;
+            dq *= w;
+          }
+          const float P = c1 * ir;
+          const float dm = fmaf(dx, u.w, fmaf(dy, v.x, dz * v.y));
+          const float dn5 = fmaf(dx, nx5[k], fmaf(dy, ny5[k], dz * nz5[k]));
+          const float mn = fmaf(u.w, nx[k], fmaf(v.x, ny[k], v.y * nz[k]));
+          const float e = fmaf(dq * (ir2 * ir), dm * dn5, P * mn);
+          const float f5 = P * dn5;
           ad[k][0] = fmaf(dx, e, ad[k][0]);
           ad[k][1] = fmaf(dy, e, ad[k][1]);
           ad[k][2] = fmaf(dz, e, ad[k][2]);
-          am[k][0] = fmaf(mx, f, am[k][0]);
-          am[k][1] = fmaf(my, f, am[k][1]);
-          am[k][2] = fmaf(mz, f, am[k][2]);
+          am[k][0] = fmaf(u.w, f5, am[k][0]);
+          am[k][1] = fmaf(v.x, f5, am[k][1]);
+          am[k][2] = fmaf(v.y, f5, am[k][2]);
           an[k] = fmaf(P, dm, an[k]);
         }
       }
     }
+  };
+  auto flush = [&]() {
 #pragma unroll
     for (int k = 0; k < TPT; ++k) {
+      const double n3[3] = {nx[k], ny[k], nz[k]};
+      const double s = static_cast<double>(an[k]);
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        acc[k][c] += static_cast<double>(ad[k][c]);
-        accm[k][c] += static_cast<double>(am[k][c]);
+      for (int a = 0; a < 3; ++a) {
+        // the m-sums hold -5 times their terms
+        acc[k][a] += (static_cast<double>(ad[k][a]) - 0.2 * static_cast<double>(am[k][a])) + n3[a] * s;
+        ad[k][a] = am[k][a] = 0.f;
       }
-      acc[k][3] += static_cast<double>(an[k]);
+      an[k] = 0.f;
     }
-  }
+  };
+  walk_sources(src, boxes, chunk_range(nsub, per), target_box<TPT>(tx, ty, tz), st, lane, body,
+               flush);
 
   const double sfac = 3.0 * kMu0 / (4.0 * kPi);
-  double *out = partial + chunk * 3 * nt_ld;
+  double *out = partial + static_cast<int64_t>(blockIdx.y) * 3 * nt_ld;
+  const int64_t i = tbase + lane;
 #pragma unroll
-  for (int k = 0; k < TPT; ++k) {
-    const int64_t i = tbase + k * 64 + lane;
-    if (i < nt) {
-      out[i] = sfac * (acc[k][0] + accm[k][0] + static_cast<double>(nx[k]) * acc[k][3]);
-      out[nt_ld + i] = sfac * (acc[k][1] + accm[k][1] + static_cast<double>(ny[k]) * acc[k][3]);
-      out[2 * nt_ld + i] = sfac * (acc[k][2] + accm[k][2] + static_cast<double>(nz[k]) * acc[k][3]);
+  for (int a = 0; a < 3; ++a) {
+    double v = 0.0;
+#pragma unroll
+    for (int k = 0; k < TPT; ++k) {
+      const double sum = group_sum(acc[k][a]);
+      v = q == k ? sum : v;
     }
+    if (q < TPT && i < nt) out[a * nt_ld + i] = v * sfac;
   }
 }
 
 // ---------------------------------------------------------------------------
-// Force tensor (6 components).  One target per lane; mixed loop only (this is
-// the external-source product, not on the solve path).
-
 // Force-tensor field at separate targets (the external tensor T_ext of
-// eval_hext), tiled like the field kernel: one target per lane, sources in
-// 64-record tiles through scalar loads; a tile whose box lies beyond 4h of the
-// wave's targets runs the branch-free dipole form.  Chunks of source tiles
-// along grid.y write FP64 partials [chunk][6][nt_ld] (xx yy zz xy xz yz).
-__global__ __launch_bounds__(kBlock) void hessian_allpairs_kernel(
-    const float4 *__restrict__ tpos, int64_t nt, const SrcRec *__restrict__ src,
-    const float4 *__restrict__ boxes, int64_t ntiles, int64_t tiles_per_chunk, HessConsts hc,
-    int64_t nt_ld, double *__restrict__ partial) {
-  __shared__ float4 s_tab[12];
-  if (threadIdx.x < 12) {
-    const float *row = &hc.curve[threadIdx.x / 3][(threadIdx.x % 3) * 4];
-    s_tab[threadIdx.x] = make_float4(row[0], row[1], row[2], row[3]);
+// eval_hext), walked like the field: partials [chunk][6][nt_ld] (xx yy zz xy
+// xz yz).
+template <int TPT>
+__global__ __launch_bounds__(64) void hessian_allpairs_kernel(
+    Points tgt, int64_t nt, const SrcRec *__restrict__ src, const float4 *__restrict__ boxes,
+    int64_t nsub, int64_t per, HessConsts hc, int64_t nt_ld, double *__restrict__ partial) {
+  __shared__ float4 s_tab[2 * kHessTabEntries];
+  __shared__ Staged st;
+  const int lane = threadIdx.x, c = lane & 15, q = lane >> 4;
+  bool have_tab = false;
+  const int64_t tbase = static_cast<int64_t>(blockIdx.x) * (16 * TPT);
+  float tx[TPT], ty[TPT], tz[TPT];
+#pragma unroll
+  for (int k = 0; k < TPT; ++k) {
+    const int64_t i = min(tbase + 16 * k + c, nt - 1) * tgt.stride;
+    tx[k] = tgt.x[i];
+    ty[k] = tgt.y[i];
+    tz[k] = tgt.z[i];
   }
-  __syncthreads();
-  const float *tab = reinterpret_cast<const float *>(s_tab);
-  const int lane = threadIdx.x & 63;
-  const int64_t wave = static_cast<int64_t>(blockIdx.x) * (kBlock / 64) + (threadIdx.x >> 6);
-  int64_t i = wave * 64 + lane;
-  if (wave * 64 >= nt) return;  // whole wave idle (uniform)
-  const bool valid = i < nt;
-  i = valid ? i : nt - 1;
-  const float4 t = tpos[i];
-  float lx = valid ? t.x : INFINITY, ly = valid ? t.y : INFINITY, lz = valid ? t.z : INFINITY;
-  float hx = valid ? t.x : -INFINITY, hy = valid ? t.y : -INFINITY, hz = valid ? t.z : -INFINITY;
-  lx = uniform_f(wave_min(lx));
-  ly = uniform_f(wave_min(ly));
-  lz = uniform_f(wave_min(lz));
-  hx = uniform_f(wave_max(hx));
-  hy = uniform_f(wave_max(hy));
-  hz = uniform_f(wave_max(hz));
-  double acc[6] = {0, 0, 0, 0, 0, 0};
-  const int64_t chunk = blockIdx.y;
-  const int64_t t0 = chunk * tiles_per_chunk;
-  const int64_t t1 = t0 + tiles_per_chunk < ntiles ? t0 + tiles_per_chunk : ntiles;
-  for (int64_t tile = t0; tile < t1; ++tile) {
-    const float4 slo = boxes[2 * tile];
-    const float4 shi = boxes[2 * tile + 1];
-    const float dist2 = uniform_f(box_dist2(lx, ly, lz, hx, hy, hz, slo, shi));
-    float a[6] = {0, 0, 0, 0, 0, 0};
-    const SrcRec *__restrict__ s = src + tile * kTile;
-    auto pair = [&](int j, bool near) {
-      const float dx = t.x - s[j].x, dy = t.y - s[j].y, dz = t.z - s[j].z;
-      const float mx = s[j].mx, my = s[j].my, mz = s[j].mz;
-      const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-      const float ir = __builtin_amdgcn_rsqf(r2);
-      const float ir2 = ir * ir;
-      float P = ir2 * ir2 * ir;
-      float R = -5.f * P * ir2;
-      if (near && !(r2 > hc.near2)) hess_near_coeffs(tab, hc.inv_h, r2, ir, P, R);
-      const float dm = fmaf(dx, mx, fmaf(dy, my, dz * mz));
-      const float Rdm = R * dm;
-      const float Pdm = P * dm;
-      a[0] = fmaf(2.f * P * dx, mx, fmaf(Rdm * dx, dx, a[0] + Pdm));
-      a[1] = fmaf(2.f * P * dy, my, fmaf(Rdm * dy, dy, a[1] + Pdm));
-      a[2] = fmaf(2.f * P * dz, mz, fmaf(Rdm * dz, dz, a[2] + Pdm));
-      a[3] = fmaf(P, fmaf(dx, my, mx * dy), fmaf(Rdm * dx, dy, a[3]));
-      a[4] = fmaf(P, fmaf(dx, mz, mx * dz), fmaf(Rdm * dx, dz, a[4]));
-      a[5] = fmaf(P, fmaf(dy, mz, my * dz), fmaf(Rdm * dy, dz, a[5]));
-    };
-    if (dist2 > hc.near2) {
-#pragma unroll 4
-      for (int j = 0; j < kTile; ++j) pair(j, false);
-    } else {
-#pragma unroll 2
-      for (int j = 0; j < kTile; ++j) pair(j, true);
+  double acc[TPT][6];
+  float s[TPT][6];
+#pragma unroll
+  for (int k = 0; k < TPT; ++k)
+#pragma unroll
+    for (int a = 0; a < 6; ++a) {
+      acc[k][a] = 0.0;
+      s[k][a] = 0.f;
     }
+  auto pair = [&](int k, const float4 &u, const float2 &v, bool near) {
+    const float dx = tx[k] - u.x, dy = ty[k] - u.y, dz = tz[k] - u.z;
+    const float mx = u.w, my = v.x, mz = v.y;
+    const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+    const float ir = near ? __builtin_amdgcn_fmed3f(__builtin_amdgcn_rsqf(r2), 0.f, 1e12f)
+                          : __builtin_amdgcn_rsqf(r2);
+    const float ir2 = ir * ir;
+    float c1 = ir2 * ir2, dq = c1;
+    if (near && !(r2 > hc.near2)) {
+      hess_near_curves_tab(s_tab, hc.tab_scale, r2, ir, c1, dq);
+      const float w = r2 > 0.f ? hc.inv_h4 : 0.f;  // nothing at d = 0
+      c1 *= w;
+      dq *= w;
+    }
+    const float P = c1 * ir;
+    const float dm = fmaf(dx, mx, fmaf(dy, my, dz * mz));
+    // T_ab = d_a (P m_b + (R/2) dm d_b) + (a <-> b) + delta_ab P dm
+    const float h = (-2.5f * dq) * (ir2 * ir) * dm;
+    const float gx = fmaf(P, mx, h * dx), gy = fmaf(P, my, h * dy), gz = fmaf(P, mz, h * dz);
+    s[k][0] = fmaf(dx + dx, gx, fmaf(P, dm, s[k][0]));
+    s[k][1] = fmaf(dy + dy, gy, fmaf(P, dm, s[k][1]));
+    s[k][2] = fmaf(dz + dz, gz, fmaf(P, dm, s[k][2]));
+    s[k][3] = fmaf(dx, gy, fmaf(dy, gx, s[k][3]));
+    s[k][4] = fmaf(dx, gz, fmaf(dz, gx, s[k][4]));
+    s[k][5] = fmaf(dy, gz, fmaf(dz, gy, s[k][5]));
+  };
+  auto body = [&](int steps, float dist2) {
+    if (dist2 > hc.near2) {
+#pragma unroll 2
+      for (int j = 0; j < steps; ++j) {
+        const float4 u = st.a[4 * j + q];
+        const float2 v = st.b[4 * j + q];
 #pragma unroll
-    for (int c = 0; c < 6; ++c) acc[c] += static_cast<double>(a[c]);
-  }
-  if (valid) {
-    double *out = partial + chunk * 6 * nt_ld;
+        for (int k = 0; k < TPT; ++k) pair(k, u, v, false);
+      }
+    } else {
+      if (!have_tab) {
+        load_table(d_hess_tab, s_tab, lane);
+        have_tab = true;
+      }
+#pragma unroll 1
+      for (int j = 0; j < steps; ++j) {
+        const float4 u = st.a[4 * j + q];
+        const float2 v = st.b[4 * j + q];
 #pragma unroll
-    for (int c = 0; c < 6; ++c) out[c * nt_ld + i] = acc[c];
+        for (int k = 0; k < TPT; ++k) pair(k, u, v, true);
+      }
+    }
+  };
+  auto flush = [&]() {
+#pragma unroll
+    for (int k = 0; k < TPT; ++k)
+#pragma unroll
+      for (int a = 0; a < 6; ++a) {
+        acc[k][a] += static_cast<double>(s[k][a]);
+        s[k][a] = 0.f;
+      }
+  };
+  walk_sources(src, boxes, chunk_range(nsub, per), target_box<TPT>(tx, ty, tz), st, lane, body,
+               flush);
+  double *out = partial + static_cast<int64_t>(blockIdx.y) * 6 * nt_ld;
+  const int64_t i = tbase + lane;
+#pragma unroll
+  for (int a = 0; a < 6; ++a) {
+    double v = 0.0;
+#pragma unroll
+    for (int k = 0; k < TPT; ++k) {
+      const double sum = group_sum(acc[k][a]);
+      v = q == k ? sum : v;
+    }
+    if (q < TPT && i < nt) out[a * nt_ld + i] = v;
   }
 }
 
@@ -497,61 +786,108 @@ struct TensorOut {
   int sym[9];
 };
 
-__global__ void reduce_hessian_kernel(int64_t n, int64_t nt_ld, int nchunk,
-                                      const double *__restrict__ partial, TensorOut out) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double s[6] = {0, 0, 0, 0, 0, 0};
-  for (int c = 0; c < nchunk; ++c) {
-    const double *p = partial + static_cast<int64_t>(c) * 6 * nt_ld;
+// ---------------------------------------------------------------------------
+// Chunk reductions (fixed order => deterministic).  A block takes 256 / W
+// targets; its W waves-of-targets add every W-th chunk each, and the sums meet
+// in LDS.  With one thread per target (W = 1, the previous form) 8,192 targets
+// were 32 blocks walking 64 chunks each: 16.6 us, 5.4 us with W = 4.
+
+template <int W, int NC>
+__device__ __forceinline__ bool reduce_chunks(int64_t n, int64_t nt_ld, int nchunk,
+                                              const double *__restrict__ partial, int64_t &i,
+                                              double (&s)[NC]) {
+  constexpr int T = 256 / W;  // targets per block
+  const int t = threadIdx.x % T, w = threadIdx.x / T;
+  i = static_cast<int64_t>(blockIdx.x) * T + t;
 #pragma unroll
-    for (int k = 0; k < 6; ++k) s[k] += p[k * nt_ld + i];
+  for (int a = 0; a < NC; ++a) s[a] = 0.0;
+  if (i < n)
+    for (int c = w; c < nchunk; c += W) {
+      const double *p = partial + static_cast<int64_t>(c) * NC * nt_ld + i;
+#pragma unroll
+      for (int a = 0; a < NC; ++a) s[a] += p[a * nt_ld];
+    }
+  if constexpr (W > 1) {
+    __shared__ double sh[W][NC][T];
+#pragma unroll
+    for (int a = 0; a < NC; ++a) sh[w][a][t] = s[a];
+    __syncthreads();
+    if (w == 0)
+#pragma unroll
+      for (int a = 0; a < NC; ++a) {
+#pragma unroll
+        for (int k = 1; k < W; ++k) s[a] += sh[k][a][t];
+      }
   }
+  return w == 0 && i < n;
+}
+
+template <int W>
+__global__ __launch_bounds__(256) void reduce_hessian_kernel(int64_t n, int64_t nt_ld, int nchunk,
+                                                             const double *__restrict__ partial,
+                                                             TensorOut out) {
+  int64_t i;
+  double s[6];
+  if (!reduce_chunks<W, 6>(n, nt_ld, nchunk, partial, i, s)) return;
   const double sfac = 3.0 * kMu0 / (4.0 * kPi);
 #pragma unroll
   for (int k = 0; k < 9; ++k)
     if (out.p[k]) out.p[k][i] = static_cast<float>(sfac * s[out.sym[k]]);
 }
 
-// ---------------------------------------------------------------------------
-// Chunk reductions (fixed order => deterministic).
+template <int W>
+__global__ __launch_bounds__(256) void reduce_field_kernel(int64_t n, int64_t nt_ld, int nchunk,
+                                                           const double *__restrict__ partial,
+                                                           float hc0, float hc1, float hc2,
+                                                           float *__restrict__ ox,
+                                                           float *__restrict__ oy,
+                                                           float *__restrict__ oz) {
+  int64_t i;
+  double s[3];
+  if (!reduce_chunks<W, 3>(n, nt_ld, nchunk, partial, i, s)) return;
+  ox[i] = static_cast<float>(s[0] + hc0);
+  oy[i] = static_cast<float>(s[1] + hc1);
+  oz[i] = static_cast<float>(s[2] + hc2);
+}
 
-__global__ void reduce_field_kernel(int64_t n, int64_t nt_ld, int nchunk,
-                                    const double *__restrict__ partial, float hc0, float hc1,
-                                    float hc2, float *__restrict__ ox, float *__restrict__ oy,
-                                    float *__restrict__ oz) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-  for (int c = 0; c < nchunk; ++c) {
-    const double *p = partial + static_cast<int64_t>(c) * 3 * nt_ld;
-    s0 += p[i];
-    s1 += p[nt_ld + i];
-    s2 += p[2 * nt_ld + i];
+// The reduction of a conjugate-gradient product: ap = p - g with g the FP32
+// rounding of the sum, and the block's part of p . ap.
+template <int W>
+__global__ __launch_bounds__(256) void reduce_ap_kernel(int64_t n, int64_t nt_ld, int nchunk,
+                                                        const double *__restrict__ partial,
+                                                        ApOut o) {
+  int64_t i;
+  double s[3];
+  double dot = 0.0;
+  if (reduce_chunks<W, 3>(n, nt_ld, nchunk, partial, i, s)) {
+    const float px = o.p[0][i], py = o.p[1][i], pz = o.p[2][i];
+    const float ax = px - static_cast<float>(s[0]), ay = py - static_cast<float>(s[1]),
+                az = pz - static_cast<float>(s[2]);
+    o.ap[0][i] = ax;
+    o.ap[1][i] = ay;
+    o.ap[2][i] = az;
+    dot = static_cast<double>(px) * ax + static_cast<double>(py) * ay + static_cast<double>(pz) * az;
   }
-  ox[i] = static_cast<float>(s0 + hc0);
-  oy[i] = static_cast<float>(s1 + hc1);
-  oz[i] = static_cast<float>(s2 + hc2);
+  __shared__ double sh[4];
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) dot += __shfl_xor(dot, off, 64);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = dot;
+  __syncthreads();
+  if (threadIdx.x == 0) o.dots[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
 }
 
 // F_i = sum_chunks partial + Text_i n_i  (Text given as 9 SoA arrays, may be null).
 struct Text9 {
   const float *p[9];
 };
-__global__ void reduce_force_kernel(int64_t n, int64_t nt_ld, int nchunk,
-                                    const double *__restrict__ partial,
-                                    const SrcRec *__restrict__ tgt, Text9 text, int has_text,
-                                    float *__restrict__ fx, float *__restrict__ fy,
-                                    float *__restrict__ fz) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double s[3] = {0.0, 0.0, 0.0};
-  for (int c = 0; c < nchunk; ++c) {
-    const double *p = partial + static_cast<int64_t>(c) * 3 * nt_ld;
-    s[0] += p[i];
-    s[1] += p[nt_ld + i];
-    s[2] += p[2 * nt_ld + i];
-  }
+template <int W>
+__global__ __launch_bounds__(256) void reduce_force_kernel(
+    int64_t n, int64_t nt_ld, int nchunk, const double *__restrict__ partial,
+    const SrcRec *__restrict__ tgt, Text9 text, int has_text, float *__restrict__ fx,
+    float *__restrict__ fy, float *__restrict__ fz) {
+  int64_t i;
+  double s[3];
+  if (!reduce_chunks<W, 3>(n, nt_ld, nchunk, partial, i, s)) return;
   if (has_text) {
     // Text rows: dHextdx = (p0,p1,p2), dHextdy = (p3,p4,p5), dHextdz = (p6,p7,p8),
     // glm column a holds (d/dx_a H_x, H_y, H_z); the tensor is symmetric for a
@@ -578,171 +914,22 @@ __global__ void reduce_force_kernel(int64_t n, int64_t nt_ld, int nchunk,
 FieldConsts make_field_consts(double h) {
   FieldConsts fc{};
   fc.h = static_cast<float>(h);
-  fc.inv_h = static_cast<float>(1.0 / h);
   fc.near2 = static_cast<float>(4.0 * h * h);
   fc.inv_h3 = static_cast<float>(1.0 / (h * h * h));
   fc.inv_h5 = static_cast<float>(1.0 / (h * h * h * h * h));
-  // g(q) = -3 (q^6/6 - 6 q^5/5 + 3 q^4 - 8 q^3/3 + 1/15) re-expanded exactly
-  // about q = 1.5 (ascending powers of t = q - 1.5).
-  const double g[7] = {1843.0 / 640.0, 27.0 / 32.0, -63.0 / 32.0, 5.0 / 4.0,
-                       9.0 / 8.0,      -9.0 / 10.0, -1.0 / 2.0};
-  for (int k = 0; k < 7; ++k) fc.g[k] = static_cast<float>(g[k]);
   fc.tab_scale = static_cast<float>(kFieldTabN / (2.0 * h));
   return fc;
 }
 
-namespace {
-// alpha h^5 and beta h^3 of a near pair at q < 2, in FP64 (the forms of the
-// mf_pair.hpp header; g unexpanded, which is accurate in FP64).
-void near_coeffs_f64(double q, double &a, double &b) {
-  if (q < 1.0) {
-    a = 0.8 - 0.5 * q;
-    b = -8.0 / 3.0 + q * q * (4.8 - 2.5 * q);
-    return;
-  }
-  const double q3 = q * q * q;
-  const double g = -3.0 * (q3 * (((q / 6.0 - 1.2) * q + 3.0) * q - 8.0 / 3.0) + 1.0 / 15.0);
-  const double w = (2.0 - q) * (2.0 - q) * (2.0 - q);
-  a = (g / q3 - w) / (3.0 * q * q);
-  b = g / (3.0 * q3) - w;
-}
-
-// Power-basis coefficients c[0..3] of the cubic through (t[i], y[i]), i < 4
-// (Gaussian elimination with partial pivoting on the Vandermonde system).
-void cubic_through(const double (&t)[4], const double (&y)[4], double (&c)[4]) {
-  double m[4][5];
-  for (int i = 0; i < 4; ++i) {
-    double p = 1.0;
-    for (int j = 0; j < 4; ++j, p *= t[i]) m[i][j] = p;
-    m[i][4] = y[i];
-  }
-  for (int col = 0; col < 4; ++col) {
-    int piv = col;
-    for (int i = col + 1; i < 4; ++i)
-      if (std::fabs(m[i][col]) > std::fabs(m[piv][col])) piv = i;
-    for (int j = 0; j < 5; ++j) std::swap(m[col][j], m[piv][j]);
-    for (int i = col + 1; i < 4; ++i) {
-      const double f = m[i][col] / m[col][col];
-      for (int j = col; j < 5; ++j) m[i][j] -= f * m[col][j];
-    }
-  }
-  for (int i = 3; i >= 0; --i) {
-    double s = m[i][4];
-    for (int j = i + 1; j < 4; ++j) s -= m[i][j] * c[j];
-    c[i] = s / m[i][i];
-  }
-}
-}  // namespace
-
-// Coefficients (ascending powers) of c(t + s) from those of the cubic c(t).
-static void shift_cubic(const double *c, double s, double *out) {
-  out[0] = ((c[3] * s + c[2]) * s + c[1]) * s + c[0];
-  out[1] = (3.0 * c[3] * s + 2.0 * c[2]) * s + c[1];
-  out[2] = 3.0 * c[3] * s + c[2];
-  out[3] = c[3];
-}
-
-static void store_entry(float *tab, int e, const double *ca, const double *cb) {
-  for (int j = 0; j < 4; ++j) {
-    tab[8 * e + j] = static_cast<float>(ca[j]);
-    tab[8 * e + 4 + j] = static_cast<float>(cb[j]);
-  }
-}
-
 void make_field_table(double h, float *tab) {
   const double ih3 = 1.0 / (h * h * h), ih5 = ih3 / (h * h);
-  double t[4];
-  for (int i = 0; i < 4; ++i) t[i] = 0.5 + 0.5 * std::cos((2 * i + 1) * kPi / 8.0);
-  double ca[4], cb[4];
-  for (int k = 0; k < kFieldTabN; ++k) {
-    double ya[4], yb[4];
-    for (int i = 0; i < 4; ++i) {
-      near_coeffs_f64((k + t[i]) * 2.0 / kFieldTabN, ya[i], yb[i]);
-      ya[i] *= ih5;
-      yb[i] *= ih3;
-    }
-    cubic_through(t, ya, ca);
-    cubic_through(t, yb, cb);
-    store_entry(tab, k, ca, cb);
-  }
-  double sa[4], sb[4];  // the last interval's cubics, one interval on
-  shift_cubic(ca, 1.0, sa);
-  shift_cubic(cb, 1.0, sb);
-  store_entry(tab, kFieldTabN, sa, sb);
-}
-
-// Fitted curve table of the reference (Dipole_hessian.kern:53-61), highest
-// power first.  Kept as data: the force must use exactly these curves.
-static const double kC1[4][5] = {
-    {9.97813616438174e-09, -2.97897856524718e-08, 2.38918644566813e-09, 4.53199938857366e-08,
-     2.44617454752747e-11},
-    {-2.76473728643294e-09, 2.86975546540539e-08, -9.94582836806651e-08, 1.25129924573675e-07,
-     -2.37010166723652e-08},
-    {-1.09679990621465e-09, 9.77055663264614e-09, -2.54781238661150e-08, 2.65020634884934e-09,
-     5.00787562417835e-08},
-    {3.79927162333632e-10, -6.26368404962679e-09, 3.94760528277489e-08, -1.13580541622200e-07,
-     1.27491333574323e-07}};
-static const double kC2[4][5] = {
-    {6.69550479838731e-08, -1.61753307173877e-07, 1.68213714992711e-08, 1.34558143036838e-07,
-     1.10976027980100e-10},
-    {-3.08460139955194e-08, 2.29192245602275e-07, -5.88399621128587e-07, 5.61170054591844e-07,
-     -1.14421132829680e-07},
-    {3.50477408060213e-09, -5.25956271895141e-08, 2.78876509535747e-07, -6.24199554212217e-07,
-     4.91807818904985e-07},
-    {7.33485346367840e-10, -9.58855788627803e-09, 4.37085309763591e-08, -7.48004594092261e-08,
-     2.34161209605651e-08}};
-
-// Taylor shift of a quartic given highest-power-first to ascending powers
-// about q0 (exact up to FP64 rounding: binomial re-expansion).
-static void shift_quartic(const double *desc, double q0, double *asc_out) {
-  double a[5];
-  for (int j = 0; j < 5; ++j) a[j] = desc[4 - j];
-  static const double binom[5][5] = {
-      {1, 0, 0, 0, 0}, {1, 1, 0, 0, 0}, {1, 2, 1, 0, 0}, {1, 3, 3, 1, 0}, {1, 4, 6, 4, 1}};
-  for (int k = 0; k < 5; ++k) {
-    double s = 0.0;
-    for (int j = k; j < 5; ++j) s += a[j] * binom[j][k] * std::pow(q0, j - k);
-    asc_out[k] = s;
-  }
+  fill_field_table(ih5, ih3, [&](int e, const double *a, const double *b) { store_entry(tab, e, a, b); });
 }
 
 void make_hess_table(double h, float *tab) {
-  const double scale = 1.0 / (3.0 * kMu0 / (4.0 * kPi) * h * h * h * h);
-  constexpr int per_unit = kHessTabN / 4;
-  double t[4];
-  for (int i = 0; i < 4; ++i) t[i] = -0.5 + 0.5 * std::cos((2 * i + 1) * kPi / 8.0);
-  double first_c[4], first_d[4];
-  for (int e = 1; e <= kHessTabN; ++e) {  // entry e: u in (e - 1, e]
-    const int piece = (e - 1) / per_unit;
-    double yc[4], yd[4], cc[4], cd[4];
-    for (int i = 0; i < 4; ++i) {
-      const double q = (e + t[i]) / per_unit;
-      double c1 = 0.0, c2 = 0.0;
-      for (int j = 0; j < 5; ++j) {
-        c1 = c1 * q + kC1[piece][j];
-        c2 = c2 * q + kC2[piece][j];
-      }
-      yc[i] = scale * c1;
-      yd[i] = -scale * (c2 - 3.0 * c1) / 5.0;
-    }
-    cubic_through(t, yc, cc);
-    cubic_through(t, yd, cd);
-    store_entry(tab, e, cc, cd);
-    if (e == 1) {
-      std::copy(cc, cc + 4, first_c);
-      std::copy(cd, cd + 4, first_d);
-    }
-    if (e == kHessTabN) {  // entry kHessTabN + 1 continues this one
-      double sc[4], sd[4];
-      shift_cubic(cc, 1.0, sc);
-      shift_cubic(cd, 1.0, sd);
-      store_entry(tab, kHessTabN + 1, sc, sd);
-    }
-  }
-  double sc[4], sd[4];  // entry 0 (u = 0) continues entry 1
-  shift_cubic(first_c, -1.0, sc);
-  shift_cubic(first_d, -1.0, sd);
-  store_entry(tab, 0, sc, sd);
+  fill_hess_table(1.0 / (h * h * h * h), [&](int e, const double *a, const double *b) {
+    store_entry(tab, e, a, b);
+  });
 }
 
 void split_near_table(const float *tab, int entries, float *out) {
@@ -753,41 +940,24 @@ void split_near_table(const float *tab, int entries, float *out) {
     }
 }
 
-const double (*reference_c1_table())[5] { return kC1; }
-const double (*reference_c2_table())[5] { return kC2; }
 
 HessConsts make_hess_consts(double h) {
   HessConsts hc{};
   hc.h = static_cast<float>(h);
-  hc.inv_h = static_cast<float>(1.0 / h);
   hc.near2 = static_cast<float>(16.0 * h * h);
+  hc.inv_h4 = static_cast<float>(1.0 / (h * h * h * h));
   hc.tab_scale = static_cast<float>(kHessTabN / (4.0 * h));
-  const double s = 3.0 * kMu0 / (4.0 * kPi);
-  const double scale = 1.0 / (s * h * h * h * h);
-  for (int k = 0; k < 4; ++k) {
-    double d[5];
-    for (int j = 0; j < 5; ++j) d[j] = kC2[k][j] - 3.0 * kC1[k][j];
-    double c1s[5], ds[5];
-    shift_quartic(kC1[k], k + 0.5, c1s);
-    shift_quartic(d, k + 0.5, ds);
-    for (int j = 0; j < 5; ++j) {
-      hc.curve[k][j] = static_cast<float>(scale * c1s[j]);
-      hc.curve[k][5 + j] = static_cast<float>(scale * ds[j]);
-    }
-    hc.curve[k][10] = hc.curve[k][11] = 0.f;
-  }
   return hc;
 }
 
 int64_t padded_sources(int64_t n) { return ((n + kTile - 1) / kTile) * kTile; }
 
-Status pack_sources(mf_ctx *ctx, int64_t n, const float *x, const float *y, const float *z,
-                    const float *mx, const float *my, const float *mz, float scale,
-                    SrcRec *out) {
-  const int64_t np = padded_sources(n);
-  if (np == 0) return Status::Ok();
-  hipLaunchKernelGGL(pack_sources_kernel, dim3(grid_for(np, 256)), dim3(256), 0, ctx->stream, n,
-                     np, x, y, z, mx, my, mz, scale, out);
+Status pack_tiles(mf_ctx *ctx, int64_t n, const float *x, const float *y, const float *z,
+                  const float *mx, const float *my, const float *mz, SrcRec *out, float4 *boxes) {
+  const int64_t ntiles = padded_sources(n) / kTile;
+  if (ntiles == 0) return Status::Ok();
+  hipLaunchKernelGGL(pack_tiles_kernel, dim3(grid_for(ntiles, 4)), dim3(256), 0, ctx->stream, n,
+                     ntiles, x, y, z, mx, my, mz, out, boxes);
   MF_LAUNCH_CHECK();
   return Status::Ok();
 }
@@ -801,114 +971,147 @@ Status pack_moments(mf_ctx *ctx, int64_t n, const float *mx, const float *my, co
   return Status::Ok();
 }
 
-Status tile_boxes(mf_ctx *ctx, int64_t n, const SrcRec *src, float4 *boxes) {
-  const int64_t ntiles = padded_sources(n) / kTile;
-  if (ntiles == 0) return Status::Ok();
-  hipLaunchKernelGGL(tile_box_kernel, dim3(grid_for(ntiles, 4)), dim3(256), 0, ctx->stream, n,
-                     ntiles, src, boxes);
-  MF_LAUNCH_CHECK();
-  return Status::Ok();
-}
-
 namespace {
+// Targets per lane: 64 targets a wave amortize a staged record over four pairs
+// a lane; the tensor's twelve sums a target leave room for two.
 constexpr int kFieldTPT = 2;
 constexpr int kForceTPT = 2;
+constexpr int kHessTPT = 2;
 
-// Splits the source tiles so that the launch has >= ~8 waves per SIMD.
-int64_t choose_chunks(int64_t target_waves, int64_t ntiles, int num_cu) {
-  const int64_t want = static_cast<int64_t>(num_cu) * 4 * 8;
-  int64_t nchunk = (want + target_waves - 1) / std::max<int64_t>(target_waves, 1);
-  nchunk = std::max<int64_t>(1, std::min<int64_t>(nchunk, 64));
-  nchunk = std::min<int64_t>(nchunk, std::max<int64_t>(ntiles, 1));
-  return nchunk;
-}
-}  // namespace
-
-namespace {
-struct FieldSplit {
-  int64_t ntiles, nchunk, per;
+// Launch shape: target waves along grid.x, chunks of whole 16-record groups
+// along grid.y.  One fill of the chip (four waves per SIMD) comes first, down
+// to two groups a chunk: at 1,859 particles 58 chunks of 32 records take 18.9 us
+// a field product, 117 of 16 take 27.3.  Beyond that, equal waves end a launch
+// together and the last, partly filled round is lost, so up to 16 fills pay
+// (100,000 particles: 5.83 ms with one, 4.87 with four, 4.33 with 16), but each
+// chunk costs its partials: not below 32 groups a chunk (8,000 particles: 53 us
+// with 17 chunks of 480 records, 64 with 125 of 64).
+constexpr int64_t kFillWaves = 16;  // waves per CU of one fill
+constexpr int64_t kFills = 16, kGroupsMin = 2, kGroupsFull = 32;
+struct Split {
+  int64_t nsub, per, nchunk;
   unsigned gx;
 };
-
-// Launch shape of the field kernel: source chunks along grid.y, at most
-// max_chunks of them.
-FieldSplit field_split(mf_ctx *ctx, int64_t nt, int64_t ns, int64_t max_chunks) {
-  FieldSplit f{};
-  f.ntiles = padded_sources(ns) / kTile;
-  const int64_t waves = (nt + 64 * kFieldTPT - 1) / (64 * kFieldTPT);
-  f.gx = static_cast<unsigned>((waves + 3) / 4);
-  int64_t nchunk = std::min(choose_chunks(waves, f.ntiles, ctx->num_cu), std::max<int64_t>(max_chunks, 1));
-  f.per = f.ntiles > 0 ? (f.ntiles + nchunk - 1) / nchunk : 0;
-  f.nchunk = f.per > 0 ? (f.ntiles + f.per - 1) / f.per : 1;
+Split split_sources(const mf_ctx *ctx, int64_t nt, int64_t ns, int tpt, int64_t max_chunks) {
+  Split f{};
+  f.nsub = (ns + kSub - 1) / kSub;  // a tile's all-padding groups are skipped
+  f.gx = static_cast<unsigned>((nt + 16 * tpt - 1) / (16 * tpt));
+  const int64_t fill = static_cast<int64_t>(ctx->num_cu) * kFillWaves;
+  const int64_t one = std::min((fill + f.gx - 1) / f.gx, f.nsub / kGroupsMin);
+  const int64_t many = std::min((fill * kFills + f.gx - 1) / f.gx, f.nsub / kGroupsFull);
+  const int64_t nchunk = std::max<int64_t>(std::min(std::max(one, many), max_chunks), 1);
+  f.per = std::max<int64_t>((f.nsub + nchunk - 1) / nchunk, 1);
+  f.nchunk = std::max<int64_t>((f.nsub + f.per - 1) / f.per, 1);
   return f;
 }
+constexpr int64_t kMaxChunks = 128;
 
 __global__ void zero_f64_kernel(int64_t n, double *__restrict__ a) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < n) a[i] = 0.0;
 }
+
+// Waves of a reduction block that share a target: four where one thread per
+// target would leave CUs without a wave, one beyond.
+constexpr int64_t kReduceWide = 65536;
+inline bool reduce_wide(int64_t n) { return n < kReduceWide; }
+inline dim3 reduce_grid(int64_t n) { return dim3(grid_for(n, reduce_wide(n) ? 64 : 256)); }
 }  // namespace
+
+#define MF_REDUCE(kernel, n, ...)                                                               \
+  do {                                                                                          \
+    if (reduce_wide(n))                                                                         \
+      hipLaunchKernelGGL(kernel<4>, reduce_grid(n), dim3(256), 0, ctx->stream, __VA_ARGS__);    \
+    else                                                                                        \
+      hipLaunchKernelGGL(kernel<1>, reduce_grid(n), dim3(256), 0, ctx->stream, __VA_ARGS__);    \
+    MF_LAUNCH_CHECK();                                                                          \
+  } while (0)
 
 int64_t field_partial_doubles(int64_t nt, int64_t nchunk) { return 3 * nt * nchunk; }
 
-Status field_allpairs_launch_ws(mf_ctx *ctx, const float4 *tpos, int tstride, int64_t nt,
-                                const SrcRec *src, const float4 *boxes, int64_t ns,
-                                const FieldConsts &fc, const float *hconst, float *ox, float *oy,
-                                float *oz, double *partial, int64_t partial_cap) {
-  if (nt == 0) return Status::Ok();
-  MF_ARG(partial_cap >= field_partial_doubles(nt, 1), "field partial buffer too small");
-  const FieldSplit f = field_split(ctx, nt, ns, partial_cap / field_partial_doubles(nt, 1));
-  if (f.ntiles == 0) {
+namespace {
+// The chunk sums of the field into `partial`; returns the chunk count.
+Status field_chunks(mf_ctx *ctx, const Points &tgt, int64_t nt, const SrcRec *src,
+                    const float4 *boxes, const FieldConsts &fc, const Split &f, double *partial) {
+  if (f.nsub == 0) {
     // a fill kernel, not hipMemsetAsync: callers may capture this in a graph
     hipLaunchKernelGGL(zero_f64_kernel, dim3(grid_for(3 * nt, 256)), dim3(256), 0, ctx->stream,
                        3 * nt, partial);
     MF_LAUNCH_CHECK();
-  } else {
-    KernelTimer timer(ctx, "field");
-    hipLaunchKernelGGL(field_allpairs_kernel<kFieldTPT>, dim3(f.gx, static_cast<unsigned>(f.nchunk)),
-                       dim3(kBlock), 0, ctx->stream, tpos, tstride, nt, src, boxes, f.ntiles,
-                       f.per, fc, nt, partial);
-    MF_LAUNCH_CHECK();
+    return Status::Ok();
   }
-  const float h0 = hconst ? hconst[0] : 0.f, h1 = hconst ? hconst[1] : 0.f,
-              h2 = hconst ? hconst[2] : 0.f;
-  hipLaunchKernelGGL(reduce_field_kernel, dim3(grid_for(nt, 256)), dim3(256), 0, ctx->stream, nt,
-                     nt, static_cast<int>(f.nchunk), partial, h0, h1, h2, ox, oy, oz);
+  KernelTimer timer(ctx, "field");
+  hipLaunchKernelGGL(field_allpairs_kernel<kFieldTPT>, dim3(f.gx, static_cast<unsigned>(f.nchunk)),
+                     dim3(64), 0, ctx->stream, tgt, nt, src, boxes, f.nsub, f.per, fc, nt, partial);
   MF_LAUNCH_CHECK();
   return Status::Ok();
 }
+}  // namespace
 
-Status field_allpairs_launch(mf_ctx *ctx, const float4 *tpos, int tstride, int64_t nt,
-                             const SrcRec *src, const float4 *boxes, int64_t ns,
-                             const FieldConsts &fc, const float *hconst, float *ox, float *oy,
-                             float *oz) {
+Status field_allpairs_launch_ws(mf_ctx *ctx, const Points &tgt, int64_t nt, const SrcRec *src,
+                                const float4 *boxes, int64_t ns, const FieldConsts &fc,
+                                const float *hconst, float *ox, float *oy, float *oz,
+                                double *partial, int64_t partial_cap) {
   if (nt == 0) return Status::Ok();
-  const FieldSplit f = field_split(ctx, nt, ns, 64);
-  const int64_t cap = field_partial_doubles(nt, f.nchunk);
+  MF_ARG(partial_cap >= field_partial_doubles(nt, 1), "field partial buffer too small");
+  const int64_t fit = partial_cap / field_partial_doubles(nt, 1);
+  const Split f = split_sources(ctx, nt, ns, kFieldTPT, std::min(fit, kMaxChunks));
+  MF_TRY(field_chunks(ctx, tgt, nt, src, boxes, fc, f, partial));
+  const float h0 = hconst ? hconst[0] : 0.f, h1 = hconst ? hconst[1] : 0.f,
+              h2 = hconst ? hconst[2] : 0.f;
+  MF_REDUCE(reduce_field_kernel, nt, nt, nt, static_cast<int>(f.nchunk), partial, h0, h1, h2, ox,
+            oy, oz);
+  return Status::Ok();
+}
+
+namespace {
+Status field_workspace(mf_ctx *ctx, int64_t nt, int64_t ns, double **partial, int64_t *cap) {
+  const Split f = split_sources(ctx, nt, ns, kFieldTPT, kMaxChunks);
+  *cap = field_partial_doubles(nt, f.nchunk);
   void *pw = nullptr;
-  MF_TRY(workspace(ctx, "field_partial", sizeof(double) * cap, &pw));
-  return field_allpairs_launch_ws(ctx, tpos, tstride, nt, src, boxes, ns, fc, hconst, ox, oy, oz,
-                                  static_cast<double *>(pw), cap);
+  MF_TRY(workspace(ctx, "field_partial", sizeof(double) * *cap, &pw));
+  *partial = static_cast<double *>(pw);
+  return Status::Ok();
+}
+}  // namespace
+
+Status field_allpairs_launch(mf_ctx *ctx, const Points &tgt, int64_t nt, const SrcRec *src,
+                             const float4 *boxes, int64_t ns, const FieldConsts &fc,
+                             const float *hconst, float *ox, float *oy, float *oz) {
+  if (nt == 0) return Status::Ok();
+  double *partial = nullptr;
+  int64_t cap = 0;
+  MF_TRY(field_workspace(ctx, nt, ns, &partial, &cap));
+  return field_allpairs_launch_ws(ctx, tgt, nt, src, boxes, ns, fc, hconst, ox, oy, oz, partial,
+                                  cap);
+}
+
+int field_ap_blocks(int64_t n) { return static_cast<int>(reduce_grid(n).x); }
+
+Status field_allpairs_ap(mf_ctx *ctx, const SrcRec *rec, const float4 *boxes, int64_t n,
+                         const FieldConsts &fc, const ApOut &out) {
+  double *partial = nullptr;
+  int64_t cap = 0;
+  MF_TRY(field_workspace(ctx, n, n, &partial, &cap));
+  const Split f = split_sources(ctx, n, n, kFieldTPT, kMaxChunks);
+  MF_TRY(field_chunks(ctx, record_points(rec), n, rec, boxes, fc, f, partial));
+  MF_REDUCE(reduce_ap_kernel, n, n, n, static_cast<int>(f.nchunk), partial, out);
+  return Status::Ok();
 }
 
 Status force_allpairs_launch(mf_ctx *ctx, const SrcRec *rec, const float4 *boxes, int64_t n,
                              const HessConsts &hc, const float *const *text9, float *fx,
                              float *fy, float *fz) {
   if (n == 0) return Status::Ok();
-  const int64_t ntiles = padded_sources(n) / kTile;
-  const int64_t waves = (n + 64 * kForceTPT - 1) / (64 * kForceTPT);
-  const unsigned gx = static_cast<unsigned>((waves + 3) / 4);
-  int64_t nchunk = choose_chunks(waves, ntiles, ctx->num_cu);
-  const int64_t per = (ntiles + nchunk - 1) / nchunk;
-  nchunk = (ntiles + per - 1) / per;
+  const Split f = split_sources(ctx, n, n, kForceTPT, kMaxChunks);
   void *pw = nullptr;
-  MF_TRY(workspace(ctx, "force_partial", sizeof(double) * 3 * n * nchunk, &pw));
+  MF_TRY(workspace(ctx, "force_partial", sizeof(double) * 3 * n * f.nchunk, &pw));
   double *partial = static_cast<double *>(pw);
   {
     KernelTimer timer(ctx, "force");
-    hipLaunchKernelGGL(force_allpairs_kernel<kForceTPT>, dim3(gx, static_cast<unsigned>(nchunk)),
-                       dim3(kBlock), 0, ctx->stream, rec, n, rec, boxes, ntiles, per, hc, n,
-                       partial);
+    hipLaunchKernelGGL(force_allpairs_kernel<kForceTPT>,
+                       dim3(f.gx, static_cast<unsigned>(f.nchunk)), dim3(64), 0, ctx->stream, rec,
+                       n, rec, boxes, f.nsub, f.per, hc, n, partial);
     MF_LAUNCH_CHECK();
   }
   Text9 t{};
@@ -920,34 +1123,28 @@ Status force_allpairs_launch(mf_ctx *ctx, const SrcRec *rec, const float4 *boxes
       t.p[k] = text9[k];
     }
   }
-  hipLaunchKernelGGL(reduce_force_kernel, dim3(grid_for(n, 256)), dim3(256), 0, ctx->stream, n, n,
-                     static_cast<int>(nchunk), partial, rec, t, has_text, fx, fy, fz);
-  MF_LAUNCH_CHECK();
+  MF_REDUCE(reduce_force_kernel, n, n, n, static_cast<int>(f.nchunk), partial, rec, t, has_text, fx,
+            fy, fz);
   return Status::Ok();
 }
 
-Status hessian_allpairs_launch(mf_ctx *ctx, const float4 *tpos, int64_t nt, const SrcRec *src,
+Status hessian_allpairs_launch(mf_ctx *ctx, const Points &tgt, int64_t nt, const SrcRec *src,
                                const float4 *boxes, int64_t ns, const HessConsts &hc,
                                float *const dst[9], const int sym[9]) {
   if (nt == 0) return Status::Ok();
-  const int64_t ntiles = padded_sources(ns) / kTile;
-  const int64_t waves = (nt + 63) / 64;
-  const unsigned gx = static_cast<unsigned>((waves + 3) / 4);
-  int64_t nchunk = choose_chunks(waves, ntiles, ctx->num_cu);
-  const int64_t per = ntiles > 0 ? (ntiles + nchunk - 1) / nchunk : 0;
-  nchunk = per > 0 ? (ntiles + per - 1) / per : 1;
+  const Split f = split_sources(ctx, nt, ns, kHessTPT, kMaxChunks);
   void *pw = nullptr;
-  MF_TRY(workspace(ctx, "hessian_partial", sizeof(double) * 6 * nt * nchunk, &pw));
+  MF_TRY(workspace(ctx, "hessian_partial", sizeof(double) * 6 * nt * f.nchunk, &pw));
   double *partial = static_cast<double *>(pw);
-  if (ntiles == 0) {
+  if (f.nsub == 0) {
     hipLaunchKernelGGL(zero_f64_kernel, dim3(grid_for(6 * nt, 256)), dim3(256), 0, ctx->stream,
                        6 * nt, partial);
     MF_LAUNCH_CHECK();
   } else {
     KernelTimer timer(ctx, "hessian");
-    hipLaunchKernelGGL(hessian_allpairs_kernel, dim3(gx, static_cast<unsigned>(nchunk)),
-                       dim3(kBlock), 0, ctx->stream, tpos, nt, src, boxes, ntiles, per, hc, nt,
-                       partial);
+    hipLaunchKernelGGL(hessian_allpairs_kernel<kHessTPT>,
+                       dim3(f.gx, static_cast<unsigned>(f.nchunk)), dim3(64), 0, ctx->stream, tgt,
+                       nt, src, boxes, f.nsub, f.per, hc, nt, partial);
     MF_LAUNCH_CHECK();
   }
   TensorOut out{};
@@ -955,11 +1152,10 @@ Status hessian_allpairs_launch(mf_ctx *ctx, const float4 *tpos, int64_t nt, cons
     out.p[k] = dst[k];
     out.sym[k] = sym[k];
   }
-  hipLaunchKernelGGL(reduce_hessian_kernel, dim3(grid_for(nt, 256)), dim3(256), 0, ctx->stream,
-                     nt, nt, static_cast<int>(nchunk), partial, out);
-  MF_LAUNCH_CHECK();
+  MF_REDUCE(reduce_hessian_kernel, nt, nt, nt, static_cast<int>(f.nchunk), partial, out);
   return Status::Ok();
 }
+#undef MF_REDUCE
 
 }  // namespace mf
 

@@ -18,29 +18,47 @@ constexpr int kTile = 64;  // sources per tile (bounding-box granularity)
 
 int64_t padded_sources(int64_t n);
 
-// Packs SoA positions and scale * moments (moments may be null => 0) into
-// n_pad = padded_sources(n) records; padding records are far away, zero moment.
-Status pack_sources(mf_ctx *ctx, int64_t n, const float *x, const float *y, const float *z,
-                    const float *mx, const float *my, const float *mz, float scale, SrcRec *out);
+// Target positions: element i at x[i * stride], y[i * stride], z[i * stride].
+struct Points {
+  const float *x, *y, *z;
+  int stride;
+};
+inline Points record_points(const SrcRec *rec) {
+  return {&rec->x, &rec->y, &rec->z, static_cast<int>(sizeof(SrcRec) / sizeof(float))};
+}
+
+// Packs SoA positions and moments (moments may be null => 0) into
+// padded_sources(n) records (padding records are far away, zero moment) and
+// writes the bounding box (lo, hi float4 pairs) of every tile of kTile records.
+Status pack_tiles(mf_ctx *ctx, int64_t n, const float *x, const float *y, const float *z,
+                  const float *mx, const float *my, const float *mz, SrcRec *out, float4 *boxes);
 // Rewrites only the moments of the first n records.
 Status pack_moments(mf_ctx *ctx, int64_t n, const float *mx, const float *my, const float *mz,
                     float scale, SrcRec *out);
-// Bounding box (lo, hi float4 pairs) of every tile of kTile records.
-Status tile_boxes(mf_ctx *ctx, int64_t n, const SrcRec *src, float4 *boxes);
 
-// out = hconst + G m over targets tpos[i * tstride] (float4 views).
-Status field_allpairs_launch(mf_ctx *ctx, const float4 *tpos, int tstride, int64_t nt,
-                             const SrcRec *src, const float4 *boxes, int64_t ns,
-                             const FieldConsts &fc, const float *hconst, float *ox, float *oy,
-                             float *oz);
+// out = hconst + G m over the targets.
+Status field_allpairs_launch(mf_ctx *ctx, const Points &tgt, int64_t nt, const SrcRec *src,
+                             const float4 *boxes, int64_t ns, const FieldConsts &fc,
+                             const float *hconst, float *ox, float *oy, float *oz);
 // The same with the chunk partials in caller memory (partial_cap doubles, at
 // least field_partial_doubles(nt, 1)); the source chunk count is cut to fit.
 // Allocates nothing.
-Status field_allpairs_launch_ws(mf_ctx *ctx, const float4 *tpos, int tstride, int64_t nt,
-                                const SrcRec *src, const float4 *boxes, int64_t ns,
-                                const FieldConsts &fc, const float *hconst, float *ox, float *oy,
-                                float *oz, double *partial, int64_t partial_cap);
+Status field_allpairs_launch_ws(mf_ctx *ctx, const Points &tgt, int64_t nt, const SrcRec *src,
+                                const float4 *boxes, int64_t ns, const FieldConsts &fc,
+                                const float *hconst, float *ox, float *oy, float *oz,
+                                double *partial, int64_t partial_cap);
 int64_t field_partial_doubles(int64_t nt, int64_t nchunk);
+// The product of a conjugate-gradient step on one record set (its moments
+// packed): ap = p - G m, and dots[b] (b < field_ap_blocks(n)) the parts of
+// p . ap.
+struct ApOut {
+  const float *p[3];
+  float *ap[3];
+  double *dots;
+};
+int field_ap_blocks(int64_t n);
+Status field_allpairs_ap(mf_ctx *ctx, const SrcRec *rec, const float4 *boxes, int64_t n,
+                         const FieldConsts &fc, const ApOut &out);
 // F_i = (sum_j B(x_i - x_j)[m_j] + Text_i) m_i over one record set.
 Status force_allpairs_launch(mf_ctx *ctx, const SrcRec *rec, const float4 *boxes, int64_t n,
                              const HessConsts &hc, const float *const *text9, float *fx,
@@ -48,7 +66,7 @@ Status force_allpairs_launch(mf_ctx *ctx, const SrcRec *rec, const float4 *boxes
 // Force tensor at separate targets: dst[k] (null = skipped) receives the
 // symmetric component sym[k] (0..5 = xx yy zz xy xz yz).  boxes: tile boxes
 // of the source records.
-Status hessian_allpairs_launch(mf_ctx *ctx, const float4 *tpos, int64_t nt, const SrcRec *src,
+Status hessian_allpairs_launch(mf_ctx *ctx, const Points &tgt, int64_t nt, const SrcRec *src,
                                const float4 *boxes, int64_t ns, const HessConsts &hc,
                                float *const dst[9], const int sym[9]);
 
@@ -66,8 +84,5 @@ Status force_subset_f64(mf_ctx *ctx, int64_t n, const double *x, const double *y
                         const double *z, const double *mx, const double *my, const double *mz,
                         double h, int64_t nt, const int64_t *idx, double *fx, double *fy,
                         double *fz);
-
-const double (*reference_c1_table())[5];
-const double (*reference_c2_table())[5];
 
 }  // namespace mf

@@ -130,8 +130,8 @@ Status plan_set_positions(mf_plan *plan, int64_t n, const float *x, const float 
   MF_HIP(hipStreamSynchronize(ctx->stream));
   MF_TRY(plan->rec.reserve(sizeof(SrcRec) * static_cast<size_t>(np > 0 ? np : 1)));
   MF_TRY(plan->boxes.reserve(sizeof(float4) * 2 * static_cast<size_t>(np / kTile + 1)));
-  MF_TRY(pack_sources(ctx, n, x, y, z, nullptr, nullptr, nullptr, 0.f, plan->rec.as<SrcRec>()));
-  MF_TRY(tile_boxes(ctx, n, plan->rec.as<SrcRec>(), plan->boxes.as<float4>()));
+  MF_TRY(pack_tiles(ctx, n, x, y, z, nullptr, nullptr, nullptr, plan->rec.as<SrcRec>(),
+                    plan->boxes.as<float4>()));
   if (plan->opts.mode == MF_MODE_FMM) MF_TRY(fmm_build(plan));
   plan->ready = true;
   return Status::Ok();
@@ -163,8 +163,8 @@ Status plan_apply_G(mf_plan *plan, float scale, const float *px, const float *py
   mf_ctx *ctx = plan->ctx;
   SrcRec *rec = plan->rec.as<SrcRec>();
   MF_TRY(pack_moments(ctx, plan->n, px, py, pz, scale, rec));
-  return field_allpairs_launch(ctx, reinterpret_cast<const float4 *>(rec), 2, plan->n, rec,
-                               plan->boxes.as<float4>(), plan->n, plan->fc, hconst, ox, oy, oz);
+  return field_allpairs_launch(ctx, record_points(rec), plan->n, rec, plan->boxes.as<float4>(),
+                               plan->n, plan->fc, hconst, ox, oy, oz);
 }
 
 Status plan_force(mf_plan *plan, const float *mx, const float *my, const float *mz,
@@ -238,6 +238,10 @@ const char *mf_status_string(int status) {
 
 const char *mf_last_error(void) { return mf::t_last_error.c_str(); }
 
+// doubles of pinned staging per context: two sets of 64 Gram-Schmidt
+// coefficients and a norm (GMRES) is the largest read-back
+static constexpr int kHostScalars = 192;
+
 int mf_ctx_create(int device, mf_ctx **out) {
   if (!out) return mf::finish(nullptr, Status::Err(MF_ERR_INVALID_ARG, "out is null"));
   *out = nullptr;
@@ -264,8 +268,13 @@ int mf_ctx_create(int device, mf_ctx **out) {
     if (err == hipSuccess) err = hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming);
     if (err == hipSuccess) err = hipEventCreateWithFlags(&ctx->ev_join, hipEventDisableTiming);
     if (err == hipSuccess)
-      err = hipHostMalloc(reinterpret_cast<void **>(&ctx->host_scalars), sizeof(double) * 128);
+      err = hipHostMalloc(reinterpret_cast<void **>(&ctx->host_scalars),
+                          sizeof(double) * kHostScalars);
+    if (err == hipSuccess)
+      err = hipHostGetDevicePointer(reinterpret_cast<void **>(&ctx->host_scalars_dev),
+                                    ctx->host_scalars, 0);
     if (err != hipSuccess) {
+      if (ctx->host_scalars) (void)hipHostFree(ctx->host_scalars);
       if (ctx->ev_join) (void)hipEventDestroy(ctx->ev_join);
       if (ctx->ev_fork) (void)hipEventDestroy(ctx->ev_fork);
       if (ctx->aux_stream) (void)hipStreamDestroy(ctx->aux_stream);
@@ -390,18 +399,9 @@ int mf_field_allpairs(mf_ctx *ctx, int64_t n_t, const float *tx, const float *ty
     mf::SrcRec *src = static_cast<mf::SrcRec *>(p);
     MF_TRY(mf::workspace(ctx, "ext_boxes", sizeof(float4) * 2 * static_cast<size_t>(np / mf::kTile + 1), &p));
     float4 *boxes = static_cast<float4 *>(p);
-    // pack_sources writes whole tiles: size the target records to the padded count
-    MF_TRY(mf::workspace(ctx, "ext_tgt",
-                         sizeof(mf::SrcRec) * static_cast<size_t>(mf::padded_sources(n_t) + 1), &p));
-    mf::SrcRec *tgt = static_cast<mf::SrcRec *>(p);
-    MF_TRY(mf::pack_sources(ctx, n_s, sx, sy, sz, mx, my, mz, 1.f, src));
-    MF_TRY(mf::tile_boxes(ctx, n_s, src, boxes));
-    if (n_t > 0) {
-      // exact copy of the targets (no padding needed: pack n_t of them)
-      MF_TRY(mf::pack_sources(ctx, n_t, tx, ty, tz, nullptr, nullptr, nullptr, 0.f, tgt));
-    }
-    return mf::field_allpairs_launch(ctx, reinterpret_cast<const float4 *>(tgt), 2, n_t, src,
-                                     boxes, n_s, mf::make_field_consts(h), hconst, ox, oy, oz);
+    MF_TRY(mf::pack_tiles(ctx, n_s, sx, sy, sz, mx, my, mz, src, boxes));
+    return mf::field_allpairs_launch(ctx, mf::Points{tx, ty, tz, 1}, n_t, src, boxes, n_s,
+                                     mf::make_field_consts(h), hconst, ox, oy, oz);
   };
   return mf::finish(ctx, run());
 }
@@ -442,26 +442,15 @@ int hessian_entry(mf_ctx *ctx, int64_t n_t, const float *tx, const float *ty, co
     mf::SrcRec *src = static_cast<mf::SrcRec *>(p);
     MF_TRY(mf::workspace(ctx, "ext_boxes", sizeof(float4) * 2 * static_cast<size_t>(np / mf::kTile + 1), &p));
     float4 *boxes = static_cast<float4 *>(p);
-    MF_TRY(mf::workspace(ctx, "ext_tgt",
-                         sizeof(mf::SrcRec) * static_cast<size_t>(mf::padded_sources(n_t) + 1), &p));
-    mf::SrcRec *tgt = static_cast<mf::SrcRec *>(p);
-    MF_TRY(mf::pack_sources(ctx, n_s, sx, sy, sz, mx, my, mz, 1.f, src));
-    MF_TRY(mf::tile_boxes(ctx, n_s, src, boxes));
-    if (n_t > 0) MF_TRY(mf::pack_sources(ctx, n_t, tx, ty, tz, nullptr, nullptr, nullptr, 0.f, tgt));
-    // the kernel reads the records' position halves with a stride of two float4
-    MF_TRY(mf::workspace(ctx, "ext_tpos", sizeof(float4) * static_cast<size_t>(n_t + 1), &p));
-    float4 *tpos = static_cast<float4 *>(p);
-    if (n_t > 0)
-      MF_HIP(hipMemcpy2DAsync(tpos, sizeof(float4), tgt, sizeof(mf::SrcRec), sizeof(float4), n_t,
-                              hipMemcpyDeviceToDevice, ctx->stream));
+    MF_TRY(mf::pack_tiles(ctx, n_s, sx, sy, sz, mx, my, mz, src, boxes));
     float *d[9];
     int sy9[9];
     for (int k = 0; k < 9; ++k) {
       d[k] = sym[k] < 0 ? nullptr : dst[k];
       sy9[k] = sym[k] < 0 ? 0 : sym[k];
     }
-    return mf::hessian_allpairs_launch(ctx, tpos, n_t, src, boxes, n_s, mf::make_hess_consts(h), d,
-                                       sy9);
+    return mf::hessian_allpairs_launch(ctx, mf::Points{tx, ty, tz, 1}, n_t, src, boxes, n_s,
+                                       mf::make_hess_consts(h), d, sy9);
   };
   return mf::finish(ctx, run());
 }
@@ -504,8 +493,7 @@ int mf_force_allpairs(mf_ctx *ctx, int64_t n, const float *x, const float *y, co
     mf::SrcRec *src = static_cast<mf::SrcRec *>(p);
     MF_TRY(mf::workspace(ctx, "ext_boxes", sizeof(float4) * 2 * static_cast<size_t>(np / mf::kTile + 1), &p));
     float4 *boxes = static_cast<float4 *>(p);
-    MF_TRY(mf::pack_sources(ctx, n, x, y, z, mx, my, mz, 1.f, src));
-    MF_TRY(mf::tile_boxes(ctx, n, src, boxes));
+    MF_TRY(mf::pack_tiles(ctx, n, x, y, z, mx, my, mz, src, boxes));
     return mf::force_allpairs_launch(ctx, src, boxes, n, mf::make_hess_consts(h), text9, fx, fy,
                                      fz);
   };

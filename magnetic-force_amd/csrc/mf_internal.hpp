@@ -135,8 +135,10 @@ struct mf_ctx {
   std::map<std::string, mf::DeviceBuffer> ws;
   // Long-lived per-context objects (operator tables), keyed by name.
   std::map<std::string, std::shared_ptr<void>> cache;
-  // Pinned host staging for scalar read-backs.
+  // Pinned host staging for scalar read-backs, and its device address (kernels
+  // store the scalars the host decides on there).
   double *host_scalars = nullptr;
+  double *host_scalars_dev = nullptr;
   int num_cu = 256;
 };
 

@@ -116,14 +116,10 @@ extern "C" int mf_field_allpairs_noalloc(mf_ctx *ctx, int64_t n_t, const float *
     const int64_t cap = static_cast<int64_t>((kScratchBytes - need.partial) / sizeof(double));
     mf::SrcRec *src = reinterpret_cast<mf::SrcRec *>(base + need.src);
     float4 *boxes = reinterpret_cast<float4 *>(base + need.boxes);
-    mf::SrcRec *tgt = reinterpret_cast<mf::SrcRec *>(base + need.tgt);
     double *partial = reinterpret_cast<double *>(base + need.partial);
-    MF_TRY(mf::pack_sources(ctx, n_s, sx, sy, sz, mx, my, mz, 1.f, src));
-    MF_TRY(mf::tile_boxes(ctx, n_s, src, boxes));
-    MF_TRY(mf::pack_sources(ctx, n_t, tx, ty, tz, nullptr, nullptr, nullptr, 0.f, tgt));
-    return mf::field_allpairs_launch_ws(ctx, reinterpret_cast<const float4 *>(tgt), 2, n_t, src,
-                                        boxes, n_s, mf::make_field_consts(h), hconst, ox, oy, oz,
-                                        partial, cap);
+    MF_TRY(mf::pack_tiles(ctx, n_s, sx, sy, sz, mx, my, mz, src, boxes));
+    return mf::field_allpairs_launch_ws(ctx, mf::Points{tx, ty, tz, 1}, n_t, src, boxes, n_s,
+                                        mf::make_field_consts(h), hconst, ox, oy, oz, partial, cap);
   };
   return mf::finish(ctx, run());
 }
