@@ -22,7 +22,9 @@
 namespace mf {
 namespace {
 
-enum { S_RR = 0, S_PAP = 1, S_ALPHA = 2, S_BETA = 3, S_BB = 4, S_TMP = 5, S_COUNT = 8 };
+// Device scalars of a CG solve: the residual norms r.r of the even and the odd
+// iterations (an iteration reads one and writes the other), and b.b.
+enum { S_RR0 = 0, S_RR1 = 1, S_BB = 2, S_COUNT = 8 };
 
 __device__ __forceinline__ double block_sum(double v, double *sh) {
 #pragma unroll
@@ -42,6 +44,30 @@ struct CV3 {
   const float *x, *y, *z;
 };
 
+// block_sum, known to every thread of the block.
+__device__ __forceinline__ double block_sum_all(double v, double *sh) {
+  const double s = block_sum(v, sh);
+  __syncthreads();
+  if (threadIdx.x == 0) sh[0] = s;
+  __syncthreads();
+  const double r = sh[0];
+  __syncthreads();  // sh may be reused
+  return r;
+}
+
+// Sum of nb partials (the same value in every block that adds them up).
+__device__ __forceinline__ double sum_of(const double *__restrict__ partials, int nb, double *sh) {
+  double acc = 0.0;
+  for (int i = threadIdx.x; i < nb; i += kRedBlock) acc += partials[i];
+  return block_sum_all(acc, sh);
+}
+
+// FP32 product over the components, one rounding before the FP64 sum (as
+// vec_dot's).
+__device__ __forceinline__ double dot3f(float ax, float ay, float az, float bx, float by, float bz) {
+  return static_cast<double>(fmaf(az, bz, fmaf(ay, by, ax * bx)));
+}
+
 // r = b - x + g (g = G(kappa x)); p = r
 __global__ void cg_init_kernel(int64_t n, CV3 b, CV3 x, CV3 g, V3 r, V3 p) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -56,6 +82,65 @@ __global__ void cg_init_kernel(int64_t n, CV3 b, CV3 x, CV3 g, V3 r, V3 p) {
     p.x[i] = rx;
     p.y[i] = ry;
     p.z[i] = rz;
+  }
+}
+
+// The moments of an all-pairs plan's records, scale * p, written as p is.
+struct RecOut {
+  SrcRec *rec;  // null: the product packs the moments itself
+  float scale;
+  __device__ __forceinline__ void put(int64_t i, float x, float y, float z) const {
+    if (rec) reinterpret_cast<float4 *>(rec + i)[1] = make_float4(scale * x, scale * y, scale * z, 0.f);
+  }
+};
+
+// Start of a CG solve in one pass: r = b - x + g (g null: x = 0 is written and
+// r = b), p = r, the records' moments, and the block's parts of r.r and b.b.
+__global__ __launch_bounds__(kRedBlock) void cg_start_kernel(int64_t n, CV3 b, V3 x, CV3 g, V3 r,
+                                                             V3 p, RecOut rec,
+                                                             double *__restrict__ partials) {
+  __shared__ double sh[kRedBlock / 64];
+  double rr = 0.0, bb = 0.0;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kRedBlock + threadIdx.x; i < n;
+       i += static_cast<int64_t>(gridDim.x) * kRedBlock) {
+    const float bx = b.x[i], by = b.y[i], bz = b.z[i];
+    float rx = bx, ry = by, rz = bz;
+    if (g.x) {
+      rx = bx - x.x[i] + g.x[i];
+      ry = by - x.y[i] + g.y[i];
+      rz = bz - x.z[i] + g.z[i];
+    } else {
+      x.x[i] = 0.f;
+      x.y[i] = 0.f;
+      x.z[i] = 0.f;
+    }
+    r.x[i] = rx;
+    r.y[i] = ry;
+    r.z[i] = rz;
+    p.x[i] = rx;
+    p.y[i] = ry;
+    p.z[i] = rz;
+    rec.put(i, rx, ry, rz);
+    rr += dot3f(rx, ry, rz, rx, ry, rz);
+    bb += dot3f(bx, by, bz, bx, by, bz);
+  }
+  const double s = block_sum_all(rr, sh);
+  if (threadIdx.x == 0) partials[blockIdx.x] = s;
+  const double t = block_sum(bb, sh);
+  if (threadIdx.x == 0) partials[gridDim.x + blockIdx.x] = t;
+}
+
+// host (pinned, read after a stream synchronization): r.r and b.b
+__global__ __launch_bounds__(kRedBlock) void cg_start_sum_kernel(const double *__restrict__ partials,
+                                                                 int nb, double *__restrict__ sc,
+                                                                 double *__restrict__ host) {
+  __shared__ double sh[kRedBlock / 64];
+  const double rr = sum_of(partials, nb, sh), bb = sum_of(partials + nb, nb, sh);
+  if (threadIdx.x == 0) {
+    sc[S_RR0] = rr;
+    sc[S_BB] = bb;
+    host[0] = rr;
+    host[1] = bb;
   }
 }
 
@@ -78,25 +163,16 @@ __global__ __launch_bounds__(kRedBlock) void cg_ap_kernel(int64_t n, CV3 p, CV3 
   if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
 
-__global__ __launch_bounds__(kRedBlock) void cg_alpha_kernel(const double *__restrict__ partials,
-                                                             int nb, double *__restrict__ sc) {
-  __shared__ double sh[kRedBlock / 64];
-  double acc = 0.0;
-  for (int i = threadIdx.x; i < nb; i += kRedBlock) acc += partials[i];
-  const double pap = block_sum(acc, sh);
-  if (threadIdx.x == 0) {
-    sc[S_PAP] = pap;
-    sc[S_ALPHA] = (pap != 0.0) ? sc[S_RR] / pap : 0.0;
-  }
-}
-
-// x += alpha p ; r -= alpha Ap ; partial r.r
-__global__ __launch_bounds__(kRedBlock) void cg_xr_kernel(int64_t n,
-                                                          const double *__restrict__ sc, CV3 p,
-                                                          CV3 ap, V3 x, V3 r,
+// alpha = r.r / p.Ap, x += alpha p ; r -= alpha Ap ; partial r.r.  Every block
+// adds up the parts of p.Ap itself (a few KB from L2): a launch for the one
+// scalar took 4.6 us.
+__global__ __launch_bounds__(kRedBlock) void cg_xr_kernel(int64_t n, const double *__restrict__ rr,
+                                                          const double *__restrict__ dots, int ndots,
+                                                          CV3 p, CV3 ap, V3 x, V3 r,
                                                           double *__restrict__ partials) {
   __shared__ double sh[kRedBlock / 64];
-  const float alpha = static_cast<float>(sc[S_ALPHA]);
+  const double pap = sum_of(dots, ndots, sh);
+  const float alpha = static_cast<float>(pap != 0.0 ? *rr / pap : 0.0);
   double acc = 0.0;
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * kRedBlock + threadIdx.x; i < n;
        i += static_cast<int64_t>(gridDim.x) * kRedBlock) {
@@ -116,26 +192,31 @@ __global__ __launch_bounds__(kRedBlock) void cg_xr_kernel(int64_t n,
   if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
 
-__global__ __launch_bounds__(kRedBlock) void cg_beta_kernel(const double *__restrict__ partials,
-                                                            int nb, double *__restrict__ sc) {
+// beta = new r.r / old r.r, p = r + beta p (and the records' moments); the new
+// r.r goes to rr_new and to the host.
+__global__ __launch_bounds__(kRedBlock) void cg_p_kernel(int64_t n, const double *__restrict__ rr_old,
+                                                         double *__restrict__ rr_new,
+                                                         double *__restrict__ host,
+                                                         const double *__restrict__ partials, int nb,
+                                                         CV3 r, V3 p, RecOut rec) {
   __shared__ double sh[kRedBlock / 64];
-  double acc = 0.0;
-  for (int i = threadIdx.x; i < nb; i += kRedBlock) acc += partials[i];
-  const double rr = block_sum(acc, sh);
-  if (threadIdx.x == 0) {
-    sc[S_BETA] = (sc[S_RR] != 0.0) ? rr / sc[S_RR] : 0.0;
-    sc[S_RR] = rr;
+  const double rr = sum_of(partials, nb, sh);
+  const double old = *rr_old;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    *rr_new = rr;
+    *host = rr;
   }
-}
-
-// p = r + beta p
-__global__ void cg_p_kernel(int64_t n, const double *__restrict__ sc, CV3 r, V3 p) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float beta = static_cast<float>(sc[S_BETA]);
-  p.x[i] = fmaf(beta, p.x[i], r.x[i]);
-  p.y[i] = fmaf(beta, p.y[i], r.y[i]);
-  p.z[i] = fmaf(beta, p.z[i], r.z[i]);
+  const float beta = static_cast<float>(old != 0.0 ? rr / old : 0.0);
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kRedBlock + threadIdx.x; i < n;
+       i += static_cast<int64_t>(gridDim.x) * kRedBlock) {
+    const float px = fmaf(beta, p.x[i], r.x[i]);
+    const float py = fmaf(beta, p.y[i], r.y[i]);
+    const float pz = fmaf(beta, p.z[i], r.z[i]);
+    p.x[i] = px;
+    p.y[i] = py;
+    p.z[i] = pz;
+    rec.put(i, px, py, pz);
+  }
 }
 
 // ---- GMRES helpers --------------------------------------------------------
@@ -183,6 +264,13 @@ __global__ void combine_kernel(int64_t n3, int nk, const float *__restrict__ V,
 __global__ void scale_kernel(int64_t n3, float s, const float *a, float *out) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < n3) out[i] = s * a[i];
+}
+
+// a *= 1 / sqrt(norm2) (left alone when that is zero)
+__global__ void normalize_kernel(int64_t n3, const double *__restrict__ norm2, float *a) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  const double s = sqrt(*norm2);
+  if (i < n3 && s > 0.0) a[i] = static_cast<float>(1.0 / s) * a[i];
 }
 
 // x (SoA, three arrays) += sum_k y[k] V_k
@@ -338,45 +426,66 @@ Status solve_cg(mf_plan *plan, double kappa, CV3 b, V3 x, const mf_solve_opts &o
                 mf_solve_stats *st) {
   mf_ctx *ctx = plan->ctx;
   const int64_t n = plan->n;
+  // An all-pairs product writes Ap and the parts of p.Ap in its own reduction,
+  // and reads moments that the CG kernels pack as they write p: four launches
+  // an iteration.  An FMM product leaves G p, and packs its sorted records.
+  const bool pairs = plan->opts.mode != MF_MODE_FMM;
   Work w{};
   MF_TRY(get_work(ctx, n, w));
   const int nb = red_blocks(n);
-  MF_TRY(vec_dot_device(ctx, n, b.x, b.y, b.z, b.x, b.y, b.z, w.sc + S_BB));
-  MF_TRY(residual(plan, kappa, b, x, w, true, o.zero_start != 0));
-  if (!o.zero_start) st->matvecs += 1;
-  MF_TRY(vec_dot_device(ctx, n, w.r, w.r + n, w.r + 2 * n, w.r, w.r + n, w.r + 2 * n, w.sc + S_RR));
-  double bb = 0.0, rr = 0.0;
-  MF_TRY(read_scalar(ctx, w.sc + S_BB, &bb));
-  MF_TRY(read_scalar(ctx, w.sc + S_RR, &rr));
-  const double bn = std::sqrt(bb);
+  const int ndots = pairs ? field_ap_blocks(n) : nb;
+  void *pd = nullptr;
+  MF_TRY(workspace(ctx, "cg_dots", sizeof(double) * static_cast<size_t>(ndots), &pd));
+  double *dots = static_cast<double *>(pd);
+  double *host = ctx->host_scalars, *host_dev = ctx->host_scalars_dev;
+  const RecOut rec{pairs ? plan->rec.as<SrcRec>() : nullptr, static_cast<float>(kappa)};
+  const V3 r = v3(w.r, n), p = v3(w.p, n), ap = v3(w.ap, n);
+  const CV3 rc = cv3(w.r, n), pc = cv3(w.p, n), apc = cv3(w.ap, n);
+  CV3 g{nullptr, nullptr, nullptr};
+  if (!o.zero_start) {
+    MF_TRY(plan_apply_G(plan, static_cast<float>(kappa), x.x, x.y, x.z, nullptr, w.g, w.g + n,
+                        w.g + 2 * n));
+    st->matvecs += 1;
+    g = cv3(w.g, n);
+  }
+  hipLaunchKernelGGL(cg_start_kernel, dim3(nb), dim3(kRedBlock), 0, ctx->stream, n, b, x, g, r, p,
+                     rec, w.partials);
+  MF_LAUNCH_CHECK();
+  hipLaunchKernelGGL(cg_start_sum_kernel, dim3(1), dim3(kRedBlock), 0, ctx->stream, w.partials, nb,
+                     w.sc, host_dev);
+  MF_LAUNCH_CHECK();
+  MF_HIP(hipStreamSynchronize(ctx->stream));
+  double rr = host[0];
+  const double bn = std::sqrt(host[1]);
   const double tol = o.rtol * (bn > 0.0 ? bn : 1.0);
   M2LOverrideGuard guard(plan);
   bool relaxed = false;
   int it = 0;
   while (std::sqrt(rr) > tol && st->matvecs < o.maxit) {
     if (!relaxed) relaxed = relax_products(plan, o, std::sqrt(rr) / (bn > 0.0 ? bn : 1.0));
-    float *g = w.g;
-    MF_TRY(plan_apply_G(plan, static_cast<float>(kappa), w.p, w.p + n, w.p + 2 * n, nullptr, g,
-                        g + n, g + 2 * n));
+    if (pairs) {
+      MF_TRY(field_allpairs_ap(ctx, plan->rec.as<SrcRec>(), plan->boxes.as<float4>(), n, plan->fc,
+                               ApOut{{pc.x, pc.y, pc.z}, {ap.x, ap.y, ap.z}, dots}));
+    } else {
+      MF_TRY(plan_apply_G(plan, static_cast<float>(kappa), w.p, w.p + n, w.p + 2 * n, nullptr, w.g,
+                          w.g + n, w.g + 2 * n));
+      hipLaunchKernelGGL(cg_ap_kernel, dim3(nb), dim3(kRedBlock), 0, ctx->stream, n, pc,
+                         cv3(w.g, n), ap, dots);
+      MF_LAUNCH_CHECK();
+    }
     st->matvecs += 1;
     if (relaxed) st->relaxed_matvecs += 1;
-    hipLaunchKernelGGL(cg_ap_kernel, dim3(nb), dim3(kRedBlock), 0, ctx->stream, n, cv3(w.p, n),
-                       cv3(g, n), v3(w.ap, n), w.partials);
+    const double *rr_old = w.sc + (it & 1 ? S_RR1 : S_RR0);
+    hipLaunchKernelGGL(cg_xr_kernel, dim3(nb), dim3(kRedBlock), 0, ctx->stream, n, rr_old,
+                       static_cast<const double *>(dots), ndots, pc, apc, x, r, w.partials);
     MF_LAUNCH_CHECK();
-    hipLaunchKernelGGL(cg_alpha_kernel, dim3(1), dim3(kRedBlock), 0, ctx->stream, w.partials, nb,
-                       w.sc);
-    MF_LAUNCH_CHECK();
-    hipLaunchKernelGGL(cg_xr_kernel, dim3(nb), dim3(kRedBlock), 0, ctx->stream, n, w.sc,
-                       cv3(w.p, n), cv3(w.ap, n), x, v3(w.r, n), w.partials);
-    MF_LAUNCH_CHECK();
-    hipLaunchKernelGGL(cg_beta_kernel, dim3(1), dim3(kRedBlock), 0, ctx->stream, w.partials, nb,
-                       w.sc);
-    MF_LAUNCH_CHECK();
-    hipLaunchKernelGGL(cg_p_kernel, dim3(grid_for(n, 256)), dim3(256), 0, ctx->stream, n, w.sc,
-                       cv3(w.r, n), v3(w.p, n));
+    hipLaunchKernelGGL(cg_p_kernel, dim3(nb), dim3(kRedBlock), 0, ctx->stream, n, rr_old,
+                       w.sc + (it & 1 ? S_RR0 : S_RR1), host_dev,
+                       static_cast<const double *>(w.partials), nb, rc, p, rec);
     MF_LAUNCH_CHECK();
     ++it;
-    MF_TRY(read_scalar(ctx, w.sc + S_RR, &rr));
+    MF_HIP(hipStreamSynchronize(ctx->stream));
+    rr = host[0];
     if (!std::isfinite(rr)) return Status::Err(MF_ERR_NOT_CONVERGED, "CG residual is not finite");
   }
   st->iterations = it;
@@ -397,9 +506,11 @@ Status solve_gmres(mf_plan *plan, double kappa, CV3 b, V3 x, const mf_solve_opts
   void *pv = nullptr;
   MF_TRY(workspace(ctx, "gmres_basis", sizeof(float) * static_cast<size_t>(m + 1) * n3, &pv));
   float *V = static_cast<float *>(pv);
+  // device coefficients: two Gram-Schmidt passes, |w|^2 after them, and the
+  // solution of the least-squares problem
   void *pc = nullptr;
-  MF_TRY(workspace(ctx, "gmres_coef", sizeof(double) * 2 * 64, &pc));
-  double *dcoef = static_cast<double *>(pc);
+  MF_TRY(workspace(ctx, "gmres_coef", sizeof(double) * 4 * 64, &pc));
+  double *dcoef = static_cast<double *>(pc), *dnorm = dcoef + 128, *dy = dcoef + 192;
   const int nb = red_blocks(n3);
 
   double bb = 0.0;
@@ -407,21 +518,17 @@ Status solve_gmres(mf_plan *plan, double kappa, CV3 b, V3 x, const mf_solve_opts
   const double bn = std::sqrt(bb) > 0.0 ? std::sqrt(bb) : 1.0;
   const double tol = o.rtol * bn;
   std::vector<double> H((m + 1) * m), cs(m), sn(m), gvec(m + 1), y(m), hcol(m + 1);
-  std::vector<double> hostbuf(64);
   double resid = 0.0;
   int total_it = 0;
 
-  auto multidot = [&](const float *wv, int nk, double *out_host) -> Status {
+  // out[k] = V_k . wv, k < nk
+  auto multidot = [&](const float *wv, int nk, double *out) -> Status {
     hipLaunchKernelGGL(multidot_kernel, dim3(nb), dim3(kRedBlock), 0, ctx->stream, n, nk, V, wv,
                        w.partials);
     MF_LAUNCH_CHECK();
     hipLaunchKernelGGL(multisum_kernel, dim3(nk), dim3(kRedBlock), 0, ctx->stream, w.partials, nb,
-                       dcoef);
+                       out);
     MF_LAUNCH_CHECK();
-    MF_HIP(hipMemcpyAsync(ctx->host_scalars, dcoef, sizeof(double) * nk, hipMemcpyDeviceToHost,
-                          ctx->stream));
-    MF_HIP(hipStreamSynchronize(ctx->stream));
-    for (int k = 0; k < nk; ++k) out_host[k] = ctx->host_scalars[k];
     return Status::Ok();
   };
 
@@ -450,24 +557,25 @@ Status solve_gmres(mf_plan *plan, double kappa, CV3 b, V3 x, const mf_solve_opts
       st->matvecs += 1;
       MF_TRY(vec_axpby<float>(ctx, n, 1.f, vj, vj + n, vj + 2 * n, -1.f, w.g, w.g + n, w.g + 2 * n, wv,
                        wv + n, wv + 2 * n));
-      std::fill(hcol.begin(), hcol.end(), 0.0);
+      // the coefficients of both passes and the norm stay on the device (the
+      // scaling by 1 / |w| too); the host reads all of them in one wait
       for (int pass = 0; pass < 2; ++pass) {
-        MF_TRY(multidot(wv, j + 1, hostbuf.data()));
-        for (int k = 0; k <= j; ++k) hcol[k] += hostbuf[k];
-        MF_HIP(hipMemcpyAsync(dcoef, hostbuf.data(), sizeof(double) * (j + 1),
-                              hipMemcpyHostToDevice, ctx->stream));
+        double *c = dcoef + 64 * pass;
+        MF_TRY(multidot(wv, j + 1, c));
         hipLaunchKernelGGL(combine_kernel, dim3(grid_for(n3, 256)), dim3(256), 0, ctx->stream, n3,
-                           j + 1, V, dcoef, -1.f, wv);
+                           j + 1, V, static_cast<const double *>(c), -1.f, wv);
         MF_LAUNCH_CHECK();
       }
-      double ww = 0.0;
-      MF_TRY(vec_dot(ctx, n, wv, wv + n, wv + 2 * n, wv, wv + n, wv + 2 * n, &ww));
-      hcol[j + 1] = std::sqrt(ww);
-      if (hcol[j + 1] > 0.0) {
-        hipLaunchKernelGGL(scale_kernel, dim3(grid_for(n3, 256)), dim3(256), 0, ctx->stream, n3,
-                           static_cast<float>(1.0 / hcol[j + 1]), wv, wv);
-        MF_LAUNCH_CHECK();
-      }
+      MF_TRY(vec_dot_device(ctx, n, wv, wv + n, wv + 2 * n, wv, wv + n, wv + 2 * n, dnorm));
+      hipLaunchKernelGGL(normalize_kernel, dim3(grid_for(n3, 256)), dim3(256), 0, ctx->stream, n3,
+                         static_cast<const double *>(dnorm), wv);
+      MF_LAUNCH_CHECK();
+      MF_HIP(hipMemcpyAsync(ctx->host_scalars, dcoef, sizeof(double) * 129, hipMemcpyDeviceToHost,
+                            ctx->stream));
+      MF_HIP(hipStreamSynchronize(ctx->stream));
+      std::fill(hcol.begin(), hcol.end(), 0.0);
+      for (int k = 0; k <= j; ++k) hcol[k] = ctx->host_scalars[k] + ctx->host_scalars[64 + k];
+      hcol[j + 1] = std::sqrt(ctx->host_scalars[128]);
       for (int k = 0; k < j; ++k) {
         const double t = cs[k] * hcol[k] + sn[k] * hcol[k + 1];
         hcol[k + 1] = -sn[k] * hcol[k] + cs[k] * hcol[k + 1];
@@ -493,9 +601,9 @@ Status solve_gmres(mf_plan *plan, double kappa, CV3 b, V3 x, const mf_solve_opts
       for (int l = k + 1; l < j; ++l) s -= H[k * m + l] * y[l];
       y[k] = H[k * m + k] != 0.0 ? s / H[k * m + k] : 0.0;
     }
-    MF_HIP(hipMemcpyAsync(dcoef, y.data(), sizeof(double) * j, hipMemcpyHostToDevice, ctx->stream));
+    MF_HIP(hipMemcpyAsync(dy, y.data(), sizeof(double) * j, hipMemcpyHostToDevice, ctx->stream));
     hipLaunchKernelGGL(gmres_update_kernel, dim3(grid_for(n, 256)), dim3(256), 0, ctx->stream, n,
-                       j, V, dcoef, x);
+                       j, V, dy, x);
     MF_LAUNCH_CHECK();
     if (std::fabs(gvec[j]) <= tol && j < m) {
       // converged inside the cycle; the loop head recomputes the true residual
