@@ -1449,60 +1449,70 @@ __global__ __launch_bounds__(64) void l2p_field_kernel(
   }
 }
 
-// Near-field source loops over one contiguous source range, taking every
-// STRIDE-th source from j0.  With STRIDE = 1 the source index is uniform
-// over the wave and the records come through scalar loads.
-template <int STRIDE>
-__device__ __forceinline__ void field_range_far(const SrcRec *__restrict__ rec, int j0, int j1,
-                                                float tx, float ty, float tz, float &a1x,
-                                                float &a1y, float &a1z, float &a2x, float &a2y,
-                                                float &a2z) {
-#pragma unroll 2
-  for (int j = j0; j < j1; j += STRIDE) {
-    const float sx = rec[j].x, sy = rec[j].y, sz = rec[j].z;
-    const float mx = rec[j].mx, my = rec[j].my, mz = rec[j].mz;
-    const float dx = tx - sx, dy = ty - sy, dz = tz - sz;
-    const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-    const float ir = __builtin_amdgcn_rsqf(r2);
-    const float ir2 = ir * ir;
-    const float ir3 = ir2 * ir;
-    const float dm = fmaf(dx, mx, fmaf(dy, my, dz * mz));
-    const float s1 = dm * (ir3 * ir2);
-    a1x = fmaf(dx, s1, a1x);
-    a1y = fmaf(dy, s1, a1y);
-    a1z = fmaf(dz, s1, a1z);
-    a2x = fmaf(mx, ir3, a2x);
-    a2y = fmaf(my, ir3, a2y);
-    a2z = fmaf(mz, ir3, a2z);
+// Near-field source loops over one contiguous source range: the source index
+// is uniform over the wave and the records come through scalar loads.  Sources
+// go in blocks of kNearBlock: all distances, then all reciprocal square roots
+// in one run at raised wave priority, then the sums.  v_rsq_f32 holds its SIMD
+// for about 16 cycles where an FMA takes 2.3; one run per block, started at
+// once, leaves the other waves' plain VALU work in longer stretches.  8.4M particles
+// (full chunks, one wave a leaf), blocks of 2 / 4 / 8: field 17.1 / 16.6 / 22.6 ms,
+// force 52.8 / 52.2 / 58.9 (eight need 117 VGPRs); without the priority 16.7 and
+// 52.9.
+constexpr int kNearBlock = 4;
+
+template <int U>
+__device__ __forceinline__ void rsq_block(const float (&r2)[U], float (&ir)[U]) {
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+  for (int k = 0; k < U; ++k) ir[k] = __builtin_amdgcn_rsqf(r2[k]);
+  __builtin_amdgcn_s_setprio(0);
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// MIXED: the block may hold pairs inside the smoothing support.
+template <int U, bool MIXED>
+__device__ __forceinline__ void field_block(const SrcRec *__restrict__ rec, float tx, float ty,
+                                            float tz, const FieldConsts &fc, const float4 *tab,
+                                            float (&a1)[3], float (&a2)[3]) {
+  float dx[U], dy[U], dz[U], r2[U], ir[U];
+#pragma unroll
+  for (int k = 0; k < U; ++k) {
+    dx[k] = tx - rec[k].x;
+    dy[k] = ty - rec[k].y;
+    dz[k] = tz - rec[k].z;
+    r2[k] = fmaf(dx[k], dx[k], fmaf(dy[k], dy[k], dz[k] * dz[k]));
+  }
+  rsq_block<U>(r2, ir);
+#pragma unroll
+  for (int k = 0; k < U; ++k) {
+    const float mx = rec[k].mx, my = rec[k].my, mz = rec[k].mz;
+    const float ir2 = ir[k] * ir[k];
+    float beta = ir2 * ir[k];
+    float alpha = beta * ir2;
+    if constexpr (MIXED)
+      if (r2[k] < fc.near2) field_near_coeffs_tab(tab, fc.tab_scale, r2[k], ir[k], alpha, beta);
+    const float dm = fmaf(dx[k], mx, fmaf(dy[k], my, dz[k] * mz));
+    const float s1 = dm * alpha;
+    a1[0] = fmaf(dx[k], s1, a1[0]);
+    a1[1] = fmaf(dy[k], s1, a1[1]);
+    a1[2] = fmaf(dz[k], s1, a1[2]);
+    a2[0] = fmaf(mx, beta, a2[0]);
+    a2[1] = fmaf(my, beta, a2[1]);
+    a2[2] = fmaf(mz, beta, a2[2]);
   }
 }
 
-template <int STRIDE>
-__device__ __forceinline__ void field_range_mixed(const SrcRec *__restrict__ rec, int j0, int j1,
-                                                  float tx, float ty, float tz,
-                                                  const FieldConsts &fc, const float4 *tab,
-                                                  float &a1x, float &a1y, float &a1z, float &a2x,
-                                                  float &a2y, float &a2z) {
-#pragma unroll 2
-  for (int j = j0; j < j1; j += STRIDE) {
-    const float sx = rec[j].x, sy = rec[j].y, sz = rec[j].z;
-    const float mx = rec[j].mx, my = rec[j].my, mz = rec[j].mz;
-    const float dx = tx - sx, dy = ty - sy, dz = tz - sz;
-    const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-    const float ir = __builtin_amdgcn_rsqf(r2);
-    const float ir2 = ir * ir;
-    float beta = ir2 * ir;
-    float alpha = beta * ir2;
-    if (r2 < fc.near2) field_near_coeffs_tab(tab, fc.tab_scale, r2, ir, alpha, beta);
-    const float dm = fmaf(dx, mx, fmaf(dy, my, dz * mz));
-    const float s1 = dm * alpha;
-    a1x = fmaf(dx, s1, a1x);
-    a1y = fmaf(dy, s1, a1y);
-    a1z = fmaf(dz, s1, a1z);
-    a2x = fmaf(mx, beta, a2x);
-    a2y = fmaf(my, beta, a2y);
-    a2z = fmaf(mz, beta, a2z);
-  }
+template <bool MIXED>
+__device__ __forceinline__ void field_range(const SrcRec *__restrict__ rec, int j0, int j1,
+                                            float tx, float ty, float tz, const FieldConsts &fc,
+                                            const float4 *tab, float (&a1)[3], float (&a2)[3]) {
+  int j = j0;
+#pragma unroll 1
+  for (; j + kNearBlock <= j1; j += kNearBlock)
+    field_block<kNearBlock, MIXED>(rec + j, tx, ty, tz, fc, tab, a1, a2);
+#pragma unroll 1
+  for (; j < j1; ++j) field_block<1, MIXED>(rec + j, tx, ty, tz, fc, tab, a1, a2);
 }
 
 // Targets [tb, te) of a leaf of cnt particles taken by the full-chunk path.
@@ -1695,65 +1705,81 @@ __global__ __launch_bounds__(64) void l2p_force_kernel(
   }
 }
 
-// Force near-field sums over one contiguous source range, every STRIDE-th
-// source from j0.  NEAR: the range may hold pairs within 4h (fitted curves
+// Force near-field sums v over a block of sources, and over one contiguous
+// source range.  NEAR: the range may hold pairs within 4h (fitted curves
 // below q = 4); otherwise every pair takes the far form, with no test.
 // The pair in the form with the far field's -5 folded away: with n5 = -5 n
 // and Rq = R / -5 (far: P ir^2; near: the table's second curve),
 //   e = Rq (d.m)(d.n5) + P (m.n) = R (d.m)(d.n) + P (m.n),
-// and the m-sums collect P (d.n5) = -5 P (d.n): the caller scales them by
-// -1/5.  One multiply per pair fewer than R = -5 P ir^2.
-template <int STRIDE, bool NEAR>
-__device__ __forceinline__ void force_range(const SrcRec *__restrict__ rec, int j0, int j1,
-                                            float tx, float ty, float tz, float nx, float ny,
-                                            float nz, float nx5, float ny5, float nz5,
-                                            const HessConsts &hc, const float4 *tab, float &dx0,
-                                            float &dy0, float &dz0, float &mx0, float &my0,
-                                            float &mz0, float &n0) {
-#pragma unroll 2
-  for (int j = j0; j < j1; j += STRIDE) {
-    const float sx = rec[j].x, sy = rec[j].y, sz = rec[j].z;
-    const float mx = rec[j].mx, my = rec[j].my, mz = rec[j].mz;
-    const float dx = tx - sx, dy = ty - sy, dz = tz - sz;
-    const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-    const float ir = __builtin_amdgcn_rsqf(r2);
-    const float dm = fmaf(dx, mx, fmaf(dy, my, dz * mz));
-    const float dn5 = fmaf(dx, nx5, fmaf(dy, ny5, dz * nz5));
-    const float mn = fmaf(mx, nx, fmaf(my, ny, mz * nz));
+// and the m-sums v[3 .. 5] collect P (d.n5) = -5 P (d.n): the caller scales
+// them by -1/5.  One multiply per pair fewer than R = -5 P ir^2.
+struct ForceTarget {
+  float x, y, z, nx, ny, nz, nx5, ny5, nz5;
+};
+template <int U, bool NEAR>
+__device__ __forceinline__ void force_block(const SrcRec *__restrict__ rec, const ForceTarget &t,
+                                            const HessConsts &hc, const float4 *tab,
+                                            float (&v)[7]) {
+  float dx[U], dy[U], dz[U], r2[U], ir[U];
+#pragma unroll
+  for (int k = 0; k < U; ++k) {
+    dx[k] = t.x - rec[k].x;
+    dy[k] = t.y - rec[k].y;
+    dz[k] = t.z - rec[k].z;
+    r2[k] = fmaf(dx[k], dx[k], fmaf(dy[k], dy[k], dz[k] * dz[k]));
+  }
+  rsq_block<U>(r2, ir);
+#pragma unroll
+  for (int k = 0; k < U; ++k) {
+    const float mx = rec[k].mx, my = rec[k].my, mz = rec[k].mz;
+    const float dm = fmaf(dx[k], mx, fmaf(dy[k], my, dz[k] * mz));
+    const float dn5 = fmaf(dx[k], t.nx5, fmaf(dy[k], t.ny5, dz[k] * t.nz5));
+    const float mn = fmaf(mx, t.nx, fmaf(my, t.ny, mz * t.nz));
     float Pc, e;
     if constexpr (NEAR) {
       // Both curves default to their far form r^-4 (P = r^-5, R / -5 = r^-7)
       // and the table replaces them within 4h; one scaling serves both.
       // The clamp keeps a pair at d = 0 finite (its terms vanish with d).
-      const float irc = __builtin_amdgcn_fmed3f(ir, 0.f, 1e12f);
+      const float irc = __builtin_amdgcn_fmed3f(ir[k], 0.f, 1e12f);
       const float ir2 = irc * irc;
       float c1 = ir2 * ir2, dq = c1;
-      if (!(r2 > hc.near2)) hess_near_curves_tab(tab, hc.tab_scale, r2, irc, c1, dq);
+      if (!(r2[k] > hc.near2)) hess_near_curves_tab(tab, hc.tab_scale, r2[k], irc, c1, dq);
       Pc = c1 * irc;
       e = fmaf(dq * (ir2 * irc), dm * dn5, Pc * mn);
     } else {
-      const float ir2 = ir * ir;
-      Pc = ir2 * ir2 * ir;
+      const float ir2 = ir[k] * ir[k];
+      Pc = ir2 * ir2 * ir[k];
       e = Pc * fmaf(dm * ir2, dn5, mn);  // R / -5 = P ir^2 factored out
     }
     const float f5 = Pc * dn5;
-    dx0 = fmaf(dx, e, dx0);
-    dy0 = fmaf(dy, e, dy0);
-    dz0 = fmaf(dz, e, dz0);
-    mx0 = fmaf(mx, f5, mx0);
-    my0 = fmaf(my, f5, my0);
-    mz0 = fmaf(mz, f5, mz0);
-    n0 = fmaf(Pc, dm, n0);
+    v[0] = fmaf(dx[k], e, v[0]);
+    v[1] = fmaf(dy[k], e, v[1]);
+    v[2] = fmaf(dz[k], e, v[2]);
+    v[3] = fmaf(mx, f5, v[3]);
+    v[4] = fmaf(my, f5, v[4]);
+    v[5] = fmaf(mz, f5, v[5]);
+    v[6] = fmaf(Pc, dm, v[6]);
   }
+}
+
+template <bool NEAR>
+__device__ __forceinline__ void force_range(const SrcRec *__restrict__ rec, int j0, int j1,
+                                            const ForceTarget &t, const HessConsts &hc,
+                                            const float4 *tab, float (&v)[7]) {
+  int j = j0;
+#pragma unroll 1
+  for (; j + kNearBlock <= j1; j += kNearBlock)
+    force_block<kNearBlock, NEAR>(rec + j, t, hc, tab, v);
+#pragma unroll 1
+  for (; j < j1; ++j) force_block<1, NEAR>(rec + j, t, hc, tab, v);
 }
 
 // ---------------------------------------------------------------------------
 // P2P: the near field of every leaf, in one launch per product over two leaf
 // lists.
-//  * Full chunks (near_*_full): one wave per leaf, one target per lane,
-//    every lane walking all sources (scalar loads), over the leaf's chunks
-//    of 64 targets -- and over its remainder too when that holds more than
-//    32.
+//  * Full chunks (near_*_full): one target per lane, every lane walking all
+//    sources (scalar loads), over the leaf's chunks of 64 targets -- and over
+//    its remainder too when that holds more than 32.
 //  * Remainders (near_*_remainder): the at most 32 targets left after a
 //    leaf's full chunks (a sparse leaf, or the tail of a leaf of 65..96
 //    particles).  One wave per leaf, lanes over sources: the leaf's near
@@ -1769,6 +1795,12 @@ __device__ __forceinline__ void force_range(const SrcRec *__restrict__ rec, int 
 // chunks' work instead of trailing a launch of their own.  Ranges of the
 // leaf's mixed slots (nr.x, first) may hold pairs inside the smoothing
 // support.
+//
+// A workgroup of W waves takes a leaf: each wave an equal part of the leaf's
+// mixed and of its far stream, the waves' FP64 sums added in wave order
+// (combine_waves).  W = 1 where the leaves alone fill the chip; with few leaves
+// the one-wave form is a handful of waves per SIMD waiting for their scalar
+// loads (near_waves holds the rule and its measurements).
 
 // Workgroup -> position in one of two leaf lists (remainders first, then
 // full chunks), each XCD (round-robin dispatch over 8) walking a contiguous
@@ -1819,40 +1851,100 @@ struct ForceOut {
   }
 };
 
+// Per-lane sums of the workgroup's waves into wave 0, in wave order.  xch: LDS
+// of (W - 1) NC 64 doubles; every wave calls it.
+template <int W, int NC>
+__device__ __forceinline__ void combine_waves(double (&v)[NC], double *xch, int wave, int lane) {
+  if constexpr (W > 1) {
+    if (wave > 0) {
+#pragma unroll
+      for (int a = 0; a < NC; ++a) xch[((wave - 1) * NC + a) * 64 + lane] = v[a];
+    }
+    __syncthreads();
+    if (wave == 0) {
+#pragma unroll
+      for (int k = 0; k < W - 1; ++k)
+#pragma unroll
+        for (int a = 0; a < NC; ++a) v[a] += xch[(k * NC + a) * 64 + lane];
+    }
+    __syncthreads();  // xch is written again by the next pass
+  }
+}
+
+// Calls piece(j0, j1) for the records of positions [i0, i1) of the leaf's near
+// stream (range_prefix), one contiguous run at a time, all values uniform.
+template <class Piece>
+__device__ __forceinline__ void stream_pieces(const int *pre, const int *beg, int nrange, int i0,
+                                              int i1, const Piece &piece) {
+  if (i0 >= i1) return;
+  int r = __builtin_amdgcn_readfirstlane(range_of(pre, nrange, i0));
+  for (int i = i0; i < i1; ++r) {
+    const int p0 = __builtin_amdgcn_readfirstlane(pre[r]);
+    const int e = min(__builtin_amdgcn_readfirstlane(pre[r + 1]), i1);
+    const int b = __builtin_amdgcn_readfirstlane(beg[r]) - p0;
+    piece(b + i, b + e);
+    i = max(i, e);
+  }
+}
+
+// Wave w's part of positions [lo, hi).
+template <int W>
+__device__ __forceinline__ void wave_part(int lo, int hi, int w, int &i0, int &i1) {
+  const int len = hi - lo;
+  i0 = lo + static_cast<int>(static_cast<int64_t>(len) * w / W);
+  i1 = lo + static_cast<int>(static_cast<int64_t>(len) * (w + 1) / W);
+}
+
+template <int W>
 __device__ __forceinline__ void near_field_full(const SrcRec *__restrict__ rec,
                                                 const int32_t *__restrict__ perm, int s0, int cnt,
                                                 const int2 *__restrict__ rg, int2 nrb,
+                                                const int *pre, const int *beg, double *xch,
                                                 const FieldConsts &fc, const float4 *s_ftab,
-                                                int lane, const FieldOut &out) {
+                                                int wave, int lane, const FieldOut &out) {
   int tb, te;
   p2p_target_span<64>(cnt, tb, te);
   for (int t0 = tb; t0 < te; t0 += 64) {
     const int t = t0 + lane;
     const SrcRec me = rec[s0 + (t < te ? t : te - 1)];
     const float tx = me.x, ty = me.y, tz = me.z;
-    double acc0 = 0.0, acc1 = 0.0, acc2 = 0.0;
-    for (int r = 0; r < nrb.x + nrb.y; ++r) {
-      const int2 q = rg[r];
-      float a1x = 0.f, a1y = 0.f, a1z = 0.f, a2x = 0.f, a2y = 0.f, a2z = 0.f;
-      if (r < nrb.x)
-        field_range_mixed<1>(rec, q.x, q.y, tx, ty, tz, fc, s_ftab, a1x, a1y, a1z, a2x, a2y, a2z);
+    double acc[3] = {0.0, 0.0, 0.0};
+    auto piece = [&](int j0, int j1, bool mixed) {
+      float a1[3] = {0.f, 0.f, 0.f}, a2[3] = {0.f, 0.f, 0.f};
+      if (mixed)
+        field_range<true>(rec, j0, j1, tx, ty, tz, fc, s_ftab, a1, a2);
       else
-        field_range_far<1>(rec, q.x, q.y, tx, ty, tz, a1x, a1y, a1z, a2x, a2y, a2z);
-      acc0 += 3.0 * static_cast<double>(a1x) - static_cast<double>(a2x);
-      acc1 += 3.0 * static_cast<double>(a1y) - static_cast<double>(a2y);
-      acc2 += 3.0 * static_cast<double>(a1z) - static_cast<double>(a2z);
+        field_range<false>(rec, j0, j1, tx, ty, tz, fc, s_ftab, a1, a2);
+#pragma unroll
+      for (int a = 0; a < 3; ++a)
+        acc[a] += 3.0 * static_cast<double>(a1[a]) - static_cast<double>(a2[a]);
+    };
+    const int nrange = nrb.x + nrb.y;
+    if constexpr (W == 1) {
+      for (int r = 0; r < nrange; ++r) {
+        const int2 q = rg[r];
+        piece(q.x, q.y, r < nrb.x);
+      }
+    } else {
+      const int tm = pre[nrb.x], tot = pre[nrange];
+      int i0, i1;
+      wave_part<W>(0, tm, wave, i0, i1);
+      stream_pieces(pre, beg, nrange, i0, i1, [&](int j0, int j1) { piece(j0, j1, true); });
+      wave_part<W>(tm, tot, wave, i0, i1);
+      stream_pieces(pre, beg, nrange, i0, i1, [&](int j0, int j1) { piece(j0, j1, false); });
     }
-    if (t < te) out.put(perm[s0 + t], acc0, acc1, acc2);
+    combine_waves<W>(acc, xch, wave, lane);
+    if (wave == 0 && t < te) out.put(perm[s0 + t], acc[0], acc[1], acc[2]);
   }
 }
 
-template <int R>
+template <int R, int W>
 __device__ __forceinline__ void near_field_remainder(const SrcRec *__restrict__ rec,
                                                      const int32_t *__restrict__ perm, int s0,
                                                      int cnt, const int *s_pre, const int *s_beg,
-                                                     int nrange, int nmix, const FieldConsts &fc,
-                                                     const float4 *s_ftab, int lane,
-                                                     const FieldOut &out) {
+                                                     int nrange, int nmix, double *xch,
+                                                     const FieldConsts &fc, const float4 *s_ftab,
+                                                     int wave, int lane, const FieldOut &out) {
   int tb, te;
   remainder_span(cnt, tb, te);
   for (int t0 = tb; t0 < te; t0 += R) {
@@ -1867,8 +1959,10 @@ __device__ __forceinline__ void near_field_remainder(const SrcRec *__restrict__ 
       gx[t] = gy[t] = gz[t] = 0.f;
     }
     LaneStream st{reinterpret_cast<const float4 *>(rec), s_pre, s_beg, s_pre[nrange], nmix};
-    st.start(lane, nrange);
-    for (int i0 = lane; i0 < st.total; i0 += 64 * kLaneBlock) {
+    // the waves take blocks of 64 kLaneBlock positions in turn
+    const int first = wave * 64 * kLaneBlock + lane;
+    st.start(first, nrange);
+    for (int i0 = first; i0 < st.total; i0 += W * 64 * kLaneBlock) {
       st.fetch(i0);
 #pragma unroll
       for (int k = 0; k < kLaneBlock; ++k) {
@@ -1895,97 +1989,113 @@ __device__ __forceinline__ void near_field_remainder(const SrcRec *__restrict__ 
         }
       }
     }
+    // lane t keeps target t0 + t
+    double g[3] = {0.0, 0.0, 0.0};
 #pragma unroll
     for (int t = 0; t < R; ++t) {
       if (t < nt) {
         const double sx = wave_sum(static_cast<double>(gx[t]));
         const double sy = wave_sum(static_cast<double>(gy[t]));
         const double sz = wave_sum(static_cast<double>(gz[t]));
-        if (lane == 0) out.put(perm[s0 + t0 + t], sx, sy, sz);
+        g[0] = lane == t ? sx : g[0];
+        g[1] = lane == t ? sy : g[1];
+        g[2] = lane == t ? sz : g[2];
       }
     }
+    combine_waves<W>(g, xch, wave, lane);
+    if (wave == 0 && lane < nt) out.put(perm[s0 + t0 + lane], g[0], g[1], g[2]);
   }
 }
 
 // P2P, field: out[perm] (+)= sum over each leaf's near ranges; accumulate = 0
 // writes H_const + near (trees without a far field).  full / remain: the two
 // leaf lists (see above).
-template <int T>
-__global__ __launch_bounds__(64) void p2p_field_kernel(
+template <int W>
+__global__ __launch_bounds__(64 * W) void p2p_field_kernel(
     const int32_t *__restrict__ full, int nfull, const int32_t *__restrict__ remain, int nrem,
     const int32_t *__restrict__ start, const int32_t *__restrict__ count,
     const SrcRec *__restrict__ rec, const int32_t *__restrict__ perm,
     const int2 *__restrict__ rng, const int2 *__restrict__ nr, int nslot, FieldConsts fc,
     const float4 *__restrict__ ftab, FieldOut out, SysMask mask) {
-  static_assert(T == 64, "one wave per leaf");
   bool rem;
   const int li = xcd_two_lists(nrem, nfull, rem);
   if (li < 0) return;
   const int b = rem ? remain[li] : full[li];
   if (sys_skip(mask, b)) return;  // uniform over the workgroup, before the barrier
-  const int lane = threadIdx.x;
-  // near-pair coefficients from the table (2 KB of LDS); the remainder's
-  // stream offsets
+  const int lane = threadIdx.x & 63;
+  const int wave = W > 1 ? __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)) : 0;
+  // near-pair coefficients from the table (2 KB of LDS); the stream's offsets
+  // (remainders, and the waves' parts); the waves' sums
   __shared__ float4 s_ftab[2 * kFieldTabEntries];
   __shared__ int s_pre[kNearF + 1], s_beg[kNearF];
-  for (int i = lane; i < 2 * kFieldTabEntries; i += 64) s_ftab[i] = ftab[i];
+  __shared__ double xch[(W > 1 ? W - 1 : 1) * (W > 1 ? 3 * 64 : 1)];
+  for (int i = threadIdx.x; i < 2 * kFieldTabEntries; i += 64 * W) s_ftab[i] = ftab[i];
   const int2 nrb = nr[b];
   const int2 *__restrict__ rg = rng + static_cast<int64_t>(b) * nslot;
-  if (rem) range_prefix(s_pre, s_beg, rg, nrb.x + nrb.y, lane);
+  if ((rem || W > 1) && wave == 0) range_prefix(s_pre, s_beg, rg, nrb.x + nrb.y, lane);
   __syncthreads();
   if (rem)
-    near_field_remainder<4>(rec, perm, start[b], count[b], s_pre, s_beg, nrb.x + nrb.y, nrb.x, fc,
-                            s_ftab, lane, out);
+    near_field_remainder<4, W>(rec, perm, start[b], count[b], s_pre, s_beg, nrb.x + nrb.y, nrb.x,
+                               xch, fc, s_ftab, wave, lane, out);
   else
-    near_field_full(rec, perm, start[b], count[b], rg, nrb, fc, s_ftab, lane, out);
+    near_field_full<W>(rec, perm, start[b], count[b], rg, nrb, s_pre, s_beg, xch, fc, s_ftab, wave,
+                       lane, out);
 }
 
+template <int W>
 __device__ __forceinline__ void near_force_full(const SrcRec *__restrict__ rec,
                                                 const int32_t *__restrict__ perm, int s0, int cnt,
                                                 const int2 *__restrict__ rg, int2 nrb,
-                                                const HessConsts &hc, const float4 *tab, int lane,
-                                                const ForceOut &out) {
+                                                const int *pre, const int *beg, double *xch,
+                                                const HessConsts &hc, const float4 *tab, int wave,
+                                                int lane, const ForceOut &out) {
   int tb, te;
   p2p_target_span<64>(cnt, tb, te);
   const int nrange = nrb.x + nrb.y;
   for (int t0 = tb; t0 < te; t0 += 64) {
     const int t = t0 + lane;
     const SrcRec me = rec[s0 + (t < te ? t : te - 1)];
-    const float tx = me.x, ty = me.y, tz = me.z, nx = me.mx, ny = me.my, nz = me.mz;
-    const float nx5 = -5.f * nx, ny5 = -5.f * ny, nz5 = -5.f * nz;
-    double ad0 = 0.0, ad1 = 0.0, ad2 = 0.0, am0 = 0.0, am1 = 0.0, am2 = 0.0, an = 0.0;
-    for (int r = 0; r < nrange; ++r) {
-      const int2 q = rg[r];
-      float dx0 = 0.f, dy0 = 0.f, dz0 = 0.f, mx0 = 0.f, my0 = 0.f, mz0 = 0.f, n0 = 0.f;
-      if (r < nrb.x)
-        force_range<1, true>(rec, q.x, q.y, tx, ty, tz, nx, ny, nz, nx5, ny5, nz5, hc, tab, dx0,
-                             dy0, dz0, mx0, my0, mz0, n0);
+    const float nx = me.mx, ny = me.my, nz = me.mz;
+    const ForceTarget tgt{me.x, me.y, me.z, nx, ny, nz, -5.f * nx, -5.f * ny, -5.f * nz};
+    // the m-sums (acc[3 .. 5]) hold -5 times their terms (force_range)
+    double acc[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    auto piece = [&](int j0, int j1, bool near) {
+      float v[7] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      if (near)
+        force_range<true>(rec, j0, j1, tgt, hc, tab, v);
       else
-        force_range<1, false>(rec, q.x, q.y, tx, ty, tz, nx, ny, nz, nx5, ny5, nz5, hc, tab, dx0,
-                              dy0, dz0, mx0, my0, mz0, n0);
-      ad0 += dx0;
-      ad1 += dy0;
-      ad2 += dz0;
-      am0 += mx0;
-      am1 += my0;
-      am2 += mz0;
-      an += n0;
+        force_range<false>(rec, j0, j1, tgt, hc, tab, v);
+#pragma unroll
+      for (int a = 0; a < 7; ++a) acc[a] += v[a];
+    };
+    if constexpr (W == 1) {
+      for (int r = 0; r < nrange; ++r) {
+        const int2 q = rg[r];
+        piece(q.x, q.y, r < nrb.x);
+      }
+    } else {
+      const int tm = pre[nrb.x], tot = pre[nrange];
+      int i0, i1;
+      wave_part<W>(0, tm, wave, i0, i1);
+      stream_pieces(pre, beg, nrange, i0, i1, [&](int j0, int j1) { piece(j0, j1, true); });
+      wave_part<W>(tm, tot, wave, i0, i1);
+      stream_pieces(pre, beg, nrange, i0, i1, [&](int j0, int j1) { piece(j0, j1, false); });
     }
-    // the m-sums hold -5 times their terms (force_range)
-    if (t < te)
-      out.put(perm[s0 + t], ad0 - 0.2 * am0 + static_cast<double>(nx) * an,
-              ad1 - 0.2 * am1 + static_cast<double>(ny) * an,
-              ad2 - 0.2 * am2 + static_cast<double>(nz) * an);
+    double f[3] = {acc[0] - 0.2 * acc[3] + static_cast<double>(nx) * acc[6],
+                   acc[1] - 0.2 * acc[4] + static_cast<double>(ny) * acc[6],
+                   acc[2] - 0.2 * acc[5] + static_cast<double>(nz) * acc[6]};
+    combine_waves<W>(f, xch, wave, lane);
+    if (wave == 0 && t < te) out.put(perm[s0 + t], f[0], f[1], f[2]);
   }
 }
 
-template <int R>
+template <int R, int W>
 __device__ __forceinline__ void near_force_remainder(const SrcRec *__restrict__ rec,
                                                      const int32_t *__restrict__ perm, int s0,
                                                      int cnt, const int *s_pre, const int *s_beg,
-                                                     int nrange, int nmix, const HessConsts &hc,
-                                                     const float4 *tab, int lane,
-                                                     const ForceOut &out) {
+                                                     int nrange, int nmix, double *xch,
+                                                     const HessConsts &hc, const float4 *tab,
+                                                     int wave, int lane, const ForceOut &out) {
   int tb, te;
   remainder_span(cnt, tb, te);
   for (int t0 = tb; t0 < te; t0 += R) {
@@ -2004,8 +2114,10 @@ __device__ __forceinline__ void near_force_remainder(const SrcRec *__restrict__ 
       ax[t] = ay[t] = az[t] = an[t] = 0.f;
     }
     LaneStream st{reinterpret_cast<const float4 *>(rec), s_pre, s_beg, s_pre[nrange], nmix};
-    st.start(lane, nrange);
-    for (int i0 = lane; i0 < st.total; i0 += 64 * kLaneBlock) {
+    // the waves take blocks of 64 kLaneBlock positions in turn
+    const int first = wave * 64 * kLaneBlock + lane;
+    st.start(first, nrange);
+    for (int i0 = first; i0 < st.total; i0 += W * 64 * kLaneBlock) {
       st.fetch(i0);
 #pragma unroll
       for (int k = 0; k < kLaneBlock; ++k) {
@@ -2038,6 +2150,8 @@ __device__ __forceinline__ void near_force_remainder(const SrcRec *__restrict__ 
         }
       }
     }
+    // lane t keeps target t0 + t
+    double g[3] = {0.0, 0.0, 0.0};
 #pragma unroll
     for (int t = 0; t < R; ++t) {
       if (t < nt) {
@@ -2045,42 +2159,45 @@ __device__ __forceinline__ void near_force_remainder(const SrcRec *__restrict__ 
         const double sy = wave_sum(static_cast<double>(ay[t]));
         const double sz = wave_sum(static_cast<double>(az[t]));
         const double sn = wave_sum(static_cast<double>(an[t]));
-        if (lane == 0)
-          out.put(perm[s0 + t0 + t], sx + static_cast<double>(nx[t]) * sn,
-                  sy + static_cast<double>(ny[t]) * sn, sz + static_cast<double>(nz[t]) * sn);
+        g[0] = lane == t ? sx + static_cast<double>(nx[t]) * sn : g[0];
+        g[1] = lane == t ? sy + static_cast<double>(ny[t]) * sn : g[1];
+        g[2] = lane == t ? sz + static_cast<double>(nz[t]) * sn : g[2];
       }
     }
+    combine_waves<W>(g, xch, wave, lane);
+    if (wave == 0 && lane < nt) out.put(perm[s0 + t0 + lane], g[0], g[1], g[2]);
   }
 }
 
 // P2P, force: F[perm] (+)= (sum over each leaf's near ranges of B[m_j]) . m_i;
 // the two leaf lists as in p2p_field_kernel.
-template <int T>
-__global__ __launch_bounds__(64) void p2p_force_kernel(
+template <int W>
+__global__ __launch_bounds__(64 * W) void p2p_force_kernel(
     const int32_t *__restrict__ full, int nfull, const int32_t *__restrict__ remain, int nrem,
     const int32_t *__restrict__ start, const int32_t *__restrict__ count,
     const SrcRec *__restrict__ rec, const int32_t *__restrict__ perm,
     const int2 *__restrict__ rng, const int2 *__restrict__ nr, int nslot, HessConsts hc,
     const float4 *__restrict__ htab, ForceOut out) {
-  static_assert(T == 64, "one wave per leaf");
   bool rem;
   const int li = xcd_two_lists(nrem, nfull, rem);
   if (li < 0) return;  // uniform over the workgroup, before the barrier
   const int b = rem ? remain[li] : full[li];
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int wave = W > 1 ? __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)) : 0;
   __shared__ float4 s_tab[2 * kHessTabEntries];
   __shared__ int s_pre[kNearH + 1], s_beg[kNearH];
-  for (int i = lane; i < 2 * kHessTabEntries; i += 64) s_tab[i] = htab[i];
-  const float4 *tab = s_tab;
+  __shared__ double xch[(W > 1 ? W - 1 : 1) * (W > 1 ? 3 * 64 : 1)];
+  for (int i = threadIdx.x; i < 2 * kHessTabEntries; i += 64 * W) s_tab[i] = htab[i];
   const int2 nrb = nr[b];
   const int2 *__restrict__ rg = rng + static_cast<int64_t>(b) * nslot;
-  if (rem) range_prefix(s_pre, s_beg, rg, nrb.x + nrb.y, lane);
+  if ((rem || W > 1) && wave == 0) range_prefix(s_pre, s_beg, rg, nrb.x + nrb.y, lane);
   __syncthreads();
   if (rem)
-    near_force_remainder<4>(rec, perm, start[b], count[b], s_pre, s_beg, nrb.x + nrb.y, nrb.x, hc,
-                            tab, lane, out);
+    near_force_remainder<4, W>(rec, perm, start[b], count[b], s_pre, s_beg, nrb.x + nrb.y, nrb.x,
+                               xch, hc, s_tab, wave, lane, out);
   else
-    near_force_full(rec, perm, start[b], count[b], rg, nrb, hc, tab, lane, out);
+    near_force_full<W>(rec, perm, start[b], count[b], rg, nrb, s_pre, s_beg, xch, hc, s_tab, wave,
+                       lane, out);
 }
 
 // Moments into the sorted records: rec[i].m = scale * weight[perm[i]] * m[perm[i]]
@@ -3241,6 +3358,28 @@ Status upward_and_m2l(mf_plan *plan, bool hess, const std::function<Status()> &l
 namespace mf {
 namespace {
 
+// Waves per leaf of the near-field kernels: the smallest power of two that
+// gives the chip kNearFill waves per SIMD (each leaf list entry is a workgroup).
+// Measured, whole solve + force steps with 1 / 2 / 4 / 8 waves a leaf: 600 entries
+// (32,000 particles) 7.30 / 4.80 / 3.39 / 2.86 ms; 2,048 (131,072 particles) 8.00 /
+// 5.75 / 5.00 / 4.78; 19,338 (506,880) 16.2 / 15.1 / 15.3 / 17.2; 43,453
+// (1,153,433) 33.5 / 33.3 / 34.4 / 39.0, where larger workgroups keep the
+// translations beside them off the CUs.
+constexpr int64_t kNearFill = 28;
+inline int near_waves(const mf_ctx *ctx, int nfull, int nrem) {
+  const int64_t want = static_cast<int64_t>(ctx->num_cu) * 4 * kNearFill;
+  int w = 1;
+  while (w < 8 && static_cast<int64_t>(w) * (nfull + nrem) < want) w *= 2;
+  return w;
+}
+#define MF_NEAR_LAUNCH(kernel, waves, ...)                                                      \
+  switch (waves) {                                                                              \
+    case 1: hipLaunchKernelGGL(kernel<1>, dim3(grid), dim3(64), 0, ns, __VA_ARGS__); break;     \
+    case 2: hipLaunchKernelGGL(kernel<2>, dim3(grid), dim3(128), 0, ns, __VA_ARGS__); break;    \
+    case 4: hipLaunchKernelGGL(kernel<4>, dim3(grid), dim3(256), 0, ns, __VA_ARGS__); break;    \
+    default: hipLaunchKernelGGL(kernel<8>, dim3(grid), dim3(512), 0, ns, __VA_ARGS__); break;   \
+  }
+
 template <int P, int KP>
 Status apply_field_impl(mf_plan *plan, float scale, const float *px, const float *py,
                         const float *pz, const float *hconst, float *ox, float *oy, float *oz) {
@@ -3282,11 +3421,11 @@ Status apply_field_impl(mf_plan *plan, float scale, const float *px, const float
         const int nfull = F.leaf_list_n[0], nrem = F.leaf_lists_remainder();
         const int grid = 8 * ((nrem + 7) / 8 + (nfull + 7) / 8);
         if (grid > 0) {
-          hipLaunchKernelGGL((p2p_field_kernel<64>), dim3(grid), dim3(64), 0, ns, lists, nfull,
-                             lists + F.leaf_list_off[1], nrem, F.box_first.as<int32_t>(),
-                             F.box_count.as<int32_t>(), F.rec.as<SrcRec>(), F.perm.as<int32_t>(),
-                             F.rngF.as<int2>(), F.nrF.as<int2>(), kNearF, plan->fc,
-                             F.ftab->buf.as<float4>(), FieldOut{0, h0, h1, h2, ox, oy, oz}, mask);
+          MF_NEAR_LAUNCH(p2p_field_kernel, near_waves(ctx, nfull, nrem), lists, nfull,
+                         lists + F.leaf_list_off[1], nrem, F.box_first.as<int32_t>(),
+                         F.box_count.as<int32_t>(), F.rec.as<SrcRec>(), F.perm.as<int32_t>(),
+                         F.rngF.as<int2>(), F.nrF.as<int2>(), kNearF, plan->fc,
+                         F.ftab->buf.as<float4>(), FieldOut{0, h0, h1, h2, ox, oy, oz}, mask);
           MF_LAUNCH_CHECK();
         }
       }
@@ -3361,11 +3500,11 @@ Status apply_force_impl(mf_plan *plan, const float *mx, const float *my, const f
         const int nfull = F.leaf_list_n[0], nrem = F.leaf_lists_remainder();
         const int grid = 8 * ((nrem + 7) / 8 + (nfull + 7) / 8);
         if (grid > 0) {
-          hipLaunchKernelGGL((p2p_force_kernel<64>), dim3(grid), dim3(64), 0, ns, lists, nfull,
-                             lists + F.leaf_list_off[1], nrem, F.box_first.as<int32_t>(),
-                             F.box_count.as<int32_t>(), F.rec.as<SrcRec>(), F.perm.as<int32_t>(),
-                             F.rngH.as<int2>(), F.nrH.as<int2>(), kNearH, plan->hc,
-                             F.htab->buf.as<float4>(), ForceOut{0, fx, fy, fz});
+          MF_NEAR_LAUNCH(p2p_force_kernel, near_waves(ctx, nfull, nrem), lists, nfull,
+                         lists + F.leaf_list_off[1], nrem, F.box_first.as<int32_t>(),
+                         F.box_count.as<int32_t>(), F.rec.as<SrcRec>(), F.perm.as<int32_t>(),
+                         F.rngH.as<int2>(), F.nrH.as<int2>(), kNearH, plan->hc,
+                         F.htab->buf.as<float4>(), ForceOut{0, fx, fy, fz});
           MF_LAUNCH_CHECK();
         }
       }
