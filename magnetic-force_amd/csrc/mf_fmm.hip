@@ -622,7 +622,44 @@ struct M2LSrc2 {
   const int32_t *src;
   int ld, empty, first_tile;
   const int32_t *order;  // tile order within each XCD's range, or null
+  int parts = 1;            // workgroups per tile, each an equal part of its offsets
+  int64_t part_stride = 0;  // floats between the parts' local expansions
 };
+
+// Workgroup -> (tile, part): each XCD (round-robin dispatch over 8) takes a
+// contiguous range of tiles, a tile's parts one after the other.
+__device__ __forceinline__ int m2l_tile_of(int ntiles, int parts, int &part) {
+  const int per_xcd = (ntiles + 7) / 8, k = static_cast<int>(blockIdx.x / 8);
+  part = parts > 1 ? k % parts : 0;
+  return static_cast<int>(blockIdx.x % 8) * per_xcd + (parts > 1 ? k / parts : k);
+}
+
+// The part's share [lo, hi) of na offsets.
+__device__ __forceinline__ void m2l_part(int na, int parts, int part, int &lo, int &hi) {
+  lo = parts > 1 ? na * part / parts : 0;
+  hi = parts > 1 ? na * (part + 1) / parts : na;
+}
+
+// Lt = the sum of its parts, in part order, for the boxes the M2L writes
+// (list: the class-sorted boxes).  Boxes of converged systems are skipped.
+__global__ void sum_parts_kernel(int64_t nelem, int KP, int parts, int64_t stride,
+                                 const int32_t *__restrict__ boxes, const float *__restrict__ Lp,
+                                 float *__restrict__ Lt, SysMask mask) {
+  const int64_t i = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) * 4;
+  if (i >= nelem) return;
+  const int box = boxes[i / KP];
+  if (sys_skip(mask, box)) return;
+  const int64_t e = static_cast<int64_t>(box) * KP + i % KP;
+  float4 v = *reinterpret_cast<const float4 *>(Lp + e);
+  for (int p = 1; p < parts; ++p) {
+    const float4 w = *reinterpret_cast<const float4 *>(Lp + p * stride + e);
+    v.x += w.x;
+    v.y += w.y;
+    v.z += w.z;
+    v.w += w.w;
+  }
+  *reinterpret_cast<float4 *>(Lt + e) = v;
+}
 
 // Tile order of an M2L launch: each XCD takes a contiguous range of tiles
 // (per = ceil(ntiles / 8)); within it, the tiles with the most non-empty
@@ -670,9 +707,10 @@ void m2l_kernel(const void *__restrict__ Msrc, uint32_t msrc_bytes,
   constexpr int kLds = NPART == 0 ? kTileT * LDF * 4 : NPART * kTileT * LDB * 2;
   __shared__ __attribute__((aligned(16))) unsigned char s_raw[kLds];
   __shared__ int s_tgt[kTileT];
-  const int per_xcd = (ntiles + 7) / 8;
-  int tile_id = static_cast<int>(blockIdx.x % 8) * per_xcd + static_cast<int>(blockIdx.x / 8);
+  int part;
+  int tile_id = m2l_tile_of(ntiles, src2.parts, part);
   if (tile_id >= ntiles) return;  // uniform over the workgroup, before any barrier
+  Lt += part * src2.part_stride;
   if (src2.order) tile_id = src2.order[tile_id];
   if (tile_id >= src2.first_tile) {
     src_slots = src2.src;
@@ -700,8 +738,10 @@ void m2l_kernel(const void *__restrict__ Msrc, uint32_t msrc_bytes,
   const int r16 = lane & 15;
   const int kq = lane >> 4;
   // the tile's non-empty offsets (plan build), walked in slot order
-  const int32_t *__restrict__ tl = tile_list + static_cast<int64_t>(tile_id) * list_ld;
-  const int na = tile_nlist[tile_id];
+  int lo, hi;
+  m2l_part(tile_nlist[tile_id], src2.parts, part, lo, hi);
+  const int32_t *__restrict__ tl = tile_list + static_cast<int64_t>(tile_id) * list_ld + lo;
+  const int na = hi - lo;
   using GA = M2LGather<KP, NPART>;
   // the target box of each of this thread's gather chunks: fixed for the tile,
   // so the source-slot loads of a later offset wait on no LDS read
@@ -1128,9 +1168,10 @@ void m2l_deg_kernel(const void *__restrict__ Msrc, uint32_t msrc_bytes, float *_
   constexpr int NT = 2 * KP, LDB = SPLIT ? KP + 24 : KP + 8;
   __shared__ __attribute__((aligned(16))) uint16_t sB[(SPLIT ? 2 : 1) * kTileT * LDB];
   __shared__ int s_tgt[kTileT];
-  const int per_xcd = (ntiles + 7) / 8;
-  int tile_id = static_cast<int>(blockIdx.x % 8) * per_xcd + static_cast<int>(blockIdx.x / 8);
+  int part;
+  int tile_id = m2l_tile_of(ntiles, src2.parts, part);
   if (tile_id >= ntiles) return;  // uniform over the workgroup, before any barrier
+  Lt += part * src2.part_stride;
   if (src2.order) tile_id = src2.order[tile_id];
   if (tile_id >= src2.first_tile) {
     src_slots = src2.src;
@@ -1147,8 +1188,10 @@ void m2l_deg_kernel(const void *__restrict__ Msrc, uint32_t msrc_bytes, float *_
     if (!__syncthreads_or(live)) return;  // uniform over the workgroup
   }
   const int32_t *__restrict__ smap = slot_table + static_cast<int64_t>(tile.slots) * slot_ld;
-  const int32_t *__restrict__ tl = tile_list + static_cast<int64_t>(tile_id) * list_ld;
-  const int na = tile_nlist[tile_id];
+  int lo, hi;
+  m2l_part(tile_nlist[tile_id], src2.parts, part, lo, hi);
+  const int32_t *__restrict__ tl = tile_list + static_cast<int64_t>(tile_id) * list_ld + lo;
+  const int na = hi - lo;
   const __amdgpu_buffer_rsrc_t msrc_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<void *>(Msrc), 0, static_cast<int>(msrc_bytes), kBufferRsrcWord3);
   // the wave index as a scalar: each wave runs its own loop (no branch joins
@@ -2382,6 +2425,8 @@ struct FmmState {
   DeviceBuffer tilesM, tilesL, tlistM, tnM, tlistL, tnL;
   std::vector<int> tileM_start, tileL_start;  // [level], size D + 2
   DeviceBuffer Mt, Lt;
+  DeviceBuffer Lp;  // the parts' locals [parts][nbox][KP] where the M2L splits its tiles
+  int nm2l = 0;     // boxes at levels >= 2
   DeviceBuffer Mb;  // BF16 parts of Mt [nbox][3][KP], for the BF16-split M2L
   int64_t p2p_field_pairs = 0;  // sum over leaves of targets x near sources
   int64_t p2p_force_pairs = 0;
@@ -2577,6 +2622,18 @@ Status build_field_table(mf_ctx *ctx, double h, bool hess, std::shared_ptr<Field
   ctx->cache[key] = t;
   *out = t;
   return Status::Ok();
+}
+
+// Workgroups per M2L tile: as many equal parts of its offset list as keep the
+// launch within kM2LFill waves per SIMD (KP / 32 waves a workgroup).  A tile's
+// ~500 offsets are a serial chain; 48 tiles of 131,072 particles left 208 CUs
+// idle.  Field launch with 1 / 2 / 4 / 8 / 16 parts: 48 tiles 0.541 / 0.279 / 0.150 /
+// 0.116 / 0.107 ms, 160 tiles at p = 6 in FP32 1.32 / 1.04 / 0.74 / 0.42 / 0.42; 729
+// tiles, which fill the chip, 1.45 / 1.71 / 2.06 ms (the parts' locals and their sum).
+constexpr int kM2LFill = 4, kM2LPartsMax = 16;
+int m2l_parts(const mf_ctx *ctx, int KP, int ntiles) {
+  const int want = ctx->num_cu * 4 * kM2LFill / (KP / 32);
+  return std::max(1, std::min(want / ntiles, kM2LPartsMax));
 }
 
 template <class T>
@@ -2890,6 +2947,7 @@ Status fmm_build_at(mf_plan *plan, double s_leaf) {
   int nm2l = 0;
   for (int l = 2; l <= D; ++l) nm2l += cnt[l];
   F.ntilesF = F.ntilesH = 0;
+  F.nm2l = nm2l;
   if (nm2l > 0) {
     MF_TRY(need<uint64_t>(F.class_keys, nm2l));
     MF_TRY(need<uint64_t>(F.class_keys2, nm2l));
@@ -3066,6 +3124,11 @@ Status fmm_build_at(mf_plan *plan, double s_leaf) {
   }
   MF_TRY(need<float>(F.Mt, static_cast<int64_t>(F.nbox) * F.KP));
   MF_TRY(need<float>(F.Lt, static_cast<int64_t>(F.nbox) * F.KP));
+  {
+    const int parts = std::max(F.ntilesF > 0 ? m2l_parts(ctx, F.KP, F.ntilesF) : 1,
+                               F.ntilesH > 0 ? m2l_parts(ctx, F.KP, F.ntilesH) : 1);
+    if (parts > 1) MF_TRY(need<float>(F.Lp, static_cast<int64_t>(F.nbox) * F.KP * parts));
+  }
   MF_TRY(need<uint16_t>(F.Mb, static_cast<int64_t>(F.nbox) * 3 * F.KP));
   F.counts_valid = false;  // work counts are computed on the first fmm_info
   return Status::Ok();
@@ -3177,18 +3240,26 @@ Status launch_m2l(mf_ctx *ctx, FmmState &F, const FmmTables &tab, int prec, cons
                   const int32_t *tn, SysMask mask, bool fence,
                   M2LSrc2 src2 = M2LSrc2{nullptr, 0, 0, INT_MAX, nullptr}) {
   if (ntiles <= 0) return Status::Ok();
-  const dim3 grid(8 * ((ntiles + 7) / 8)), block(2 * KP);
+  const int parts = m2l_parts(ctx, KP, ntiles);
+  const int64_t stride = static_cast<int64_t>(F.nbox) * KP;
+  float *out = F.Lt.as<float>();
+  if (parts > 1) {
+    src2.parts = parts;
+    src2.part_stride = stride;
+    out = F.Lp.as<float>();
+  }
+  const dim3 grid(8 * ((ntiles + 7) / 8) * parts), block(2 * KP);
   const int npart = prec == MF_M2L_FP32 ? 0 : 3;
   if (!m2l_gather_range_ok(F.nbox, KP, npart))
     return Status::Err(MF_ERR_UNSUPPORTED, "too many boxes for the M2L gather's 32-bit range");
   const uint32_t msrc_bytes = static_cast<uint32_t>(static_cast<int64_t>(F.nbox) * (npart ? 6 * KP : 4 * KP));
 #define MF_M2L_ARGS                                                                           \
-  ctx->stream, msrc, msrc_bytes, F.Lt.as<float>(), tables, tiles, ntiles,                     \
+  ctx->stream, msrc, msrc_bytes, out, tables, tiles, ntiles,                                  \
       F.class_ids2.as<int32_t>(), src, nslot, src_rows, tab.slot_tab.as<int32_t>(),            \
       tab.slot_ld, tlist,                                                                      \
       tn, tab.slot_ld, 0, mask, src2
 #define MF_DEG_LAUNCH                                                                         \
-  ctx->stream, F.Mb.get(), msrc_bytes, F.Lt.as<float>(), tab.Tb.as<uint16_t>(), tiles, ntiles, \
+  ctx->stream, F.Mb.get(), msrc_bytes, out, tab.Tb.as<uint16_t>(), tiles, ntiles,              \
       F.class_ids2.as<int32_t>(), src, nslot, src_rows, tab.slot_tab.as<int32_t>(),            \
       tab.slot_ld, tlist, tn, tab.slot_ld, mask, src2
   switch (prec) {
@@ -3225,6 +3296,13 @@ Status launch_m2l(mf_ctx *ctx, FmmState &F, const FmmTables &tab, int prec, cons
 #undef MF_M2L_ARGS
 #undef MF_DEG_LAUNCH
   MF_LAUNCH_CHECK();
+  if (parts > 1) {
+    const int64_t ne = static_cast<int64_t>(F.nm2l) * KP;
+    hipLaunchKernelGGL(sum_parts_kernel, dim3(grid_for(ne / 4, 256)), dim3(256), 0, ctx->stream, ne,
+                       KP, parts, stride, F.class_ids2.as<int32_t>(),
+                       static_cast<const float *>(F.Lp.as<float>()), F.Lt.as<float>(), mask);
+    MF_LAUNCH_CHECK();
+  }
   return Status::Ok();
 }
 
