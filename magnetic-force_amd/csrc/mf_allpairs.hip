@@ -28,10 +28,11 @@
 //    in a fixed order by a separate reduction kernel, so results are
 //    deterministic.
 //  Measured per launch, before (scalar sources, closed-form coefficients, chunks
-//  of whole tiles) and now: field 22.6 -> 8.4 us at 512 particles, 65.0 -> 55.9 us
-//  at 8,192, 33.8 -> 29.9 ms at 262,144 (2.3e12 pairs/s; the far loop alone would
-//  reach 2.4e12: a v_rsq_f32 holds its SIMD for 17 of a pair's 66 cycles); force
-//  36.9 -> 10.4 us, 91.9 -> 77.8 us, 49.7 -> 42.3 ms.
+//  of whole tiles) and now: field 22.6 -> 8.4 us at 512 particles, 65.0 -> 52.8 us
+//  at 8,192, 33.8 -> 28.3 ms at 262,144 (2.4e12 pairs/s); force 36.9 -> 9.8 us,
+//  91.9 -> 76.2 us, 49.7 -> 40.0 ms; field and tensor of 4,096 records
+//  on 65,520 targets 0.43 -> 0.33 ms.  The VALU bounds the large sizes: a far
+//  field pair is 19 plain instructions at 2.3 cycles and one v_rsq_f32 at 16.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -352,6 +353,43 @@ struct Staged {
   float2 b[kTile];  // my, mz
 };
 
+// Two steps of a tile: the lane's two records, and its TPT targets' distances
+// and inverse distances to each (index g TPT + k).  The reciprocal square roots run
+// together at raised wave priority: v_rsq_f32 holds its SIMD for about 16 cycles
+// where an FMA takes 2.3, and runs that start at once leave the other waves'
+// plain VALU work in longer stretches.  262,144 particles with one step and no
+// priority / one step / two steps / four: field 29.9 / 28.8 / 28.7 / 29.0 ms, force
+// 42.9 / 40.8 / 40.3 / 40.3.
+constexpr int kSteps = 2;
+template <int TPT>
+struct StepPairs {
+  float4 u[kSteps];
+  float2 v[kSteps];
+  float dx[kSteps * TPT], dy[kSteps * TPT], dz[kSteps * TPT], r2[kSteps * TPT], ir[kSteps * TPT];
+  __device__ __forceinline__ StepPairs(const Staged &st, int j, int q, const float (&tx)[TPT],
+                                       const float (&ty)[TPT], const float (&tz)[TPT]) {
+#pragma unroll
+    for (int g = 0; g < kSteps; ++g) {
+      u[g] = st.a[4 * (j + g) + q];
+      v[g] = st.b[4 * (j + g) + q];
+#pragma unroll
+      for (int k = 0; k < TPT; ++k) {
+        const int i = g * TPT + k;
+        dx[i] = tx[k] - u[g].x;
+        dy[i] = ty[k] - u[g].y;
+        dz[i] = tz[k] - u[g].z;
+        r2[i] = fmaf(dx[i], dx[i], fmaf(dy[i], dy[i], dz[i] * dz[i]));
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int i = 0; i < kSteps * TPT; ++i) ir[i] = __builtin_amdgcn_rsqf(r2[i]);
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+};
+
 // Walks the wave's sources: stages each tile's part of the range and calls
 // body(steps, dist2): `steps` groups of four records are staged (record 4 j + q
 // is lane group q's j-th), dist2 is the distance^2 from the wave's targets to
@@ -452,14 +490,14 @@ __global__ __launch_bounds__(64) void field_allpairs_kernel(
     if (dist2 >= fc.near2) {
       // far tile: every pair has q >= 2 (pure dipole)
 #pragma unroll 1
-      for (int j = 0; j < steps; ++j) {
-        const float4 u = st.a[4 * j + q];
-        const float2 v = st.b[4 * j + q];
+      for (int j = 0; j < steps; j += kSteps) {
+        const StepPairs<TPT> sp(st, j, q, tx, ty, tz);
 #pragma unroll
-        for (int k = 0; k < TPT; ++k) {
-          const float dx = tx[k] - u.x, dy = ty[k] - u.y, dz = tz[k] - u.z;
-          const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-          const float ir = __builtin_amdgcn_rsqf(r2);
+        for (int i = 0; i < kSteps * TPT; ++i) {
+          const int k = i % TPT;
+          const float4 u = sp.u[i / TPT];
+          const float2 v = sp.v[i / TPT];
+          const float dx = sp.dx[i], dy = sp.dy[i], dz = sp.dz[i], ir = sp.ir[i];
           const float ir2 = ir * ir;
           const float ir3 = ir2 * ir;
           const float dm = fmaf(dx, u.w, fmaf(dy, v.x, dz * v.y));
@@ -479,14 +517,14 @@ __global__ __launch_bounds__(64) void field_allpairs_kernel(
         have_tab = true;
       }
 #pragma unroll 1
-      for (int j = 0; j < steps; ++j) {
-        const float4 u = st.a[4 * j + q];
-        const float2 v = st.b[4 * j + q];
+      for (int j = 0; j < steps; j += kSteps) {
+        const StepPairs<TPT> sp(st, j, q, tx, ty, tz);
 #pragma unroll
-        for (int k = 0; k < TPT; ++k) {
-          const float dx = tx[k] - u.x, dy = ty[k] - u.y, dz = tz[k] - u.z;
-          const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-          const float ir = __builtin_amdgcn_rsqf(r2);
+        for (int i = 0; i < kSteps * TPT; ++i) {
+          const int k = i % TPT;
+          const float4 u = sp.u[i / TPT];
+          const float2 v = sp.v[i / TPT];
+          const float dx = sp.dx[i], dy = sp.dy[i], dz = sp.dz[i], r2 = sp.r2[i], ir = sp.ir[i];
           const float ir2 = ir * ir;
           float beta = ir2 * ir;
           float alpha = beta * ir2;
@@ -579,14 +617,14 @@ __global__ __launch_bounds__(64) void force_allpairs_kernel(
   auto body = [&](int steps, float dist2) {
     if (dist2 > hc.near2) {
 #pragma unroll 1
-      for (int j = 0; j < steps; ++j) {
-        const float4 u = st.a[4 * j + q];
-        const float2 v = st.b[4 * j + q];
+      for (int j = 0; j < steps; j += kSteps) {
+        const StepPairs<TPT> sp(st, j, q, tx, ty, tz);
 #pragma unroll
-        for (int k = 0; k < TPT; ++k) {
-          const float dx = tx[k] - u.x, dy = ty[k] - u.y, dz = tz[k] - u.z;
-          const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-          const float ir = __builtin_amdgcn_rsqf(r2);
+        for (int i = 0; i < kSteps * TPT; ++i) {
+          const int k = i % TPT;
+          const float4 u = sp.u[i / TPT];
+          const float2 v = sp.v[i / TPT];
+          const float dx = sp.dx[i], dy = sp.dy[i], dz = sp.dz[i], ir = sp.ir[i];
           const float ir2 = ir * ir;
           const float P = ir2 * ir2 * ir;  // r^-5
           const float dm = fmaf(dx, u.w, fmaf(dy, v.x, dz * v.y));
@@ -609,15 +647,16 @@ __global__ __launch_bounds__(64) void force_allpairs_kernel(
         have_tab = true;
       }
 #pragma unroll 1
-      for (int j = 0; j < steps; ++j) {
-        const float4 u = st.a[4 * j + q];
-        const float2 v = st.b[4 * j + q];
+      for (int j = 0; j < steps; j += kSteps) {
+        const StepPairs<TPT> sp(st, j, q, tx, ty, tz);
 #pragma unroll
-        for (int k = 0; k < TPT; ++k) {
-          const float dx = tx[k] - u.x, dy = ty[k] - u.y, dz = tz[k] - u.z;
-          const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+        for (int i = 0; i < kSteps * TPT; ++i) {
+          const int k = i % TPT;
+          const float4 u = sp.u[i / TPT];
+          const float2 v = sp.v[i / TPT];
+          const float dx = sp.dx[i], dy = sp.dy[i], dz = sp.dz[i], r2 = sp.r2[i];
           // the clamp keeps a pair at d = 0 finite
-          const float ir = __builtin_amdgcn_fmed3f(__builtin_amdgcn_rsqf(r2), 0.f, 1e12f);
+          const float ir = __builtin_amdgcn_fmed3f(sp.ir[i], 0.f, 1e12f);
           const float ir2 = ir * ir;
           float c1 = ir2 * ir2, dq = c1;  // far curves
           if (!(r2 > hc.near2)) {
@@ -705,12 +744,11 @@ __global__ __launch_bounds__(64) void hessian_allpairs_kernel(
       acc[k][a] = 0.0;
       s[k][a] = 0.f;
     }
-  auto pair = [&](int k, const float4 &u, const float2 &v, bool near) {
-    const float dx = tx[k] - u.x, dy = ty[k] - u.y, dz = tz[k] - u.z;
-    const float mx = u.w, my = v.x, mz = v.y;
-    const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-    const float ir = near ? __builtin_amdgcn_fmed3f(__builtin_amdgcn_rsqf(r2), 0.f, 1e12f)
-                          : __builtin_amdgcn_rsqf(r2);
+  auto pair = [&](const StepPairs<TPT> &sp, int i, bool near) {
+    const int k = i % TPT;
+    const float dx = sp.dx[i], dy = sp.dy[i], dz = sp.dz[i], r2 = sp.r2[i];
+    const float mx = sp.u[i / TPT].w, my = sp.v[i / TPT].x, mz = sp.v[i / TPT].y;
+    const float ir = near ? __builtin_amdgcn_fmed3f(sp.ir[i], 0.f, 1e12f) : sp.ir[i];
     const float ir2 = ir * ir;
     float c1 = ir2 * ir2, dq = c1;
     if (near && !(r2 > hc.near2)) {
@@ -733,12 +771,11 @@ __global__ __launch_bounds__(64) void hessian_allpairs_kernel(
   };
   auto body = [&](int steps, float dist2) {
     if (dist2 > hc.near2) {
-#pragma unroll 2
-      for (int j = 0; j < steps; ++j) {
-        const float4 u = st.a[4 * j + q];
-        const float2 v = st.b[4 * j + q];
+#pragma unroll 1
+      for (int j = 0; j < steps; j += kSteps) {
+        const StepPairs<TPT> sp(st, j, q, tx, ty, tz);
 #pragma unroll
-        for (int k = 0; k < TPT; ++k) pair(k, u, v, false);
+        for (int i = 0; i < kSteps * TPT; ++i) pair(sp, i, false);
       }
     } else {
       if (!have_tab) {
@@ -746,11 +783,10 @@ __global__ __launch_bounds__(64) void hessian_allpairs_kernel(
         have_tab = true;
       }
 #pragma unroll 1
-      for (int j = 0; j < steps; ++j) {
-        const float4 u = st.a[4 * j + q];
-        const float2 v = st.b[4 * j + q];
+      for (int j = 0; j < steps; j += kSteps) {
+        const StepPairs<TPT> sp(st, j, q, tx, ty, tz);
 #pragma unroll
-        for (int k = 0; k < TPT; ++k) pair(k, u, v, true);
+        for (int i = 0; i < kSteps * TPT; ++i) pair(sp, i, true);
       }
     }
   };
