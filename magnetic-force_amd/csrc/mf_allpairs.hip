@@ -27,12 +27,14 @@
 //    grid.y to give the 256 CUs enough waves; chunk partials (FP64) are summed
 //    in a fixed order by a separate reduction kernel, so results are
 //    deterministic.
-//  Measured per launch, before (scalar sources, closed-form coefficients, chunks
-//  of whole tiles) and now: field 22.6 -> 8.4 us at 512 particles, 65.0 -> 52.8 us
-//  at 8,192, 33.8 -> 28.3 ms at 262,144 (2.4e12 pairs/s); force 36.9 -> 9.8 us,
-//  91.9 -> 76.2 us, 49.7 -> 40.0 ms; field and tensor of 4,096 records
-//  on 65,520 targets 0.43 -> 0.33 ms.  The VALU bounds the large sizes: a far
-//  field pair is 19 plain instructions at 2.3 cycles and one v_rsq_f32 at 16.
+//  * A record set's field and force on itself (4,096 records or more) evaluate
+//    each unordered pair once (field_self_kernel, force_self_kernel below).
+//  Measured per launch, at first (scalar sources, closed-form coefficients, chunks
+//  of whole tiles), directed kernels now, pairs once: field 22.6 / 8.4 us at 512
+//  particles, 65.0 / 52.8 / 41.8 us at 8,192, 33.8 / 28.3 / 22.6 ms at 262,144; force
+//  36.9 / 9.8 us, 91.9 / 76.2 / 57.0 us, 49.7 / 40.0 / 27.8 ms.  Field and tensor of
+//  4,096 records on 65,520 targets 0.43 / 0.33 ms.  The VALU bounds the large sizes: a
+//  directed far field pair is 19 plain instructions at 2.3 cycles and one v_rsq_f32 at 16.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -715,6 +717,391 @@ __global__ __launch_bounds__(64) void force_allpairs_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// One record set against itself, every unordered pair evaluated once.
+//
+// The distance, its inverse root and the radial coefficients of a pair serve
+// both of its particles, and the force on one is minus the force on the other
+// (the pair form of the force is antisymmetric under exchange).  A unit of work
+// is one wave's 64 records (an i-tile, four targets a lane) against one staged
+// j-tile: at step s lane c of each 16-lane row takes record (s + c) mod 16 of its
+// row's sixteen, and the sums for that record move one lane down the row with it
+// (row_ror), so after 16 steps lane c holds the sums of record c over the wave's
+// 64 targets.  64 evaluated pairs then cost 96 (field) and 121 (force) cycles
+// where two directed ones cost 130 and 182.
+//
+// A workgroup is W waves with W consecutive i-tiles (a group) walking the same
+// j-tiles; the j-sums of its waves meet in LDS and leave in FP64, one slot per
+// (group distance d, record): group G takes the j-tiles of groups G, G + 1, ...,
+// G + D modulo an odd number of groups 2 D + 1 (the last one may be empty), so every
+// group pair is met once and every record gets exactly one sum for each d = 1 .. D.
+// The group's own tiles (d = 0) are walked directed, self pairs included.  Chunks of
+// the walk along grid.y, each with its i-sums in a slot of its own, give the
+// chip enough workgroups; the chunk reduction adds the slots in a fixed order.
+
+constexpr int kSelfTPT = 4;      // 64 targets a wave, 64 = kTile
+constexpr int kSelfFlush = 4;    // units between FP64 accumulations
+
+struct SelfWalk {
+  int ntiles;   // tiles of the record set
+  int ngroups;  // odd
+  int first, last;  // the launch's units: j-tiles [first, last) of a group's W (D + 1)
+  int per;          // units per chunk
+  int nchunk;
+};
+
+struct SelfTile {
+  float4 pos[kTile], mom[kTile];
+};
+
+// s_waitcnt vmcnt(0), nothing else waited for (expcnt 7, lgkmcnt 15).
+constexpr int kWaitVm0 = 0x0F70;
+
+// The value of the next lane up in the 16-lane row (cyclic).
+__device__ __forceinline__ float row_next(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x12F, 0xf, 0xf, false));
+}
+
+// Distances and inverse distances of the lane's record (u.xyz) to its targets
+// k0 .. k0 + K - 1; one run of roots at raised priority, as in StepPairs.
+template <int K>
+struct SelfPairs {
+  float dx[K], dy[K], dz[K], r2[K], ir[K];
+  __device__ __forceinline__ SelfPairs(const float4 &u, int k0, const float (&tx)[kSelfTPT],
+                                       const float (&ty)[kSelfTPT], const float (&tz)[kSelfTPT]) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      dx[k] = tx[k0 + k] - u.x;
+      dy[k] = ty[k0 + k] - u.y;
+      dz[k] = tz[k0 + k] - u.z;
+      r2[k] = fmaf(dx[k], dx[k], fmaf(dy[k], dy[k], dz[k] * dz[k]));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int k = 0; k < K; ++k) ir[k] = __builtin_amdgcn_rsqf(r2[k]);
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+};
+
+struct FieldSelf {
+  const FieldConsts &fc;
+  const float4 *tab;
+  float tx[kSelfTPT], ty[kSelfTPT], tz[kSelfTPT], nx[kSelfTPT], ny[kSelfTPT], nz[kSelfTPT];
+  float a1[kSelfTPT][3], a2[kSelfTPT][3];
+  __device__ __forceinline__ FieldSelf(const FieldConsts &consts, const float4 *t)
+      : fc(consts), tab(t) {}
+  __device__ __forceinline__ bool far(float dist2) const { return dist2 >= fc.near2; }
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int k = 0; k < kSelfTPT; ++k)
+#pragma unroll
+      for (int a = 0; a < 3; ++a) a1[k][a] = a2[k][a] = 0.f;
+  }
+  __device__ __forceinline__ void flush(double *acc) {
+#pragma unroll
+    for (int k = 0; k < kSelfTPT; ++k)
+#pragma unroll
+      for (int a = 0; a < 3; ++a)
+        acc[(3 * k + a) * 64] += 3.0 * static_cast<double>(a1[k][a]) - static_cast<double>(a2[k][a]);
+    clear();
+  }
+  template <bool MIXED, bool BOTH>
+  __device__ __forceinline__ void tile(const SelfTile &st, int c, int q, float (&jc)[3]) {
+#pragma unroll 1
+    for (int s = 0; s < 16; ++s) {
+      const int r = 16 * q + ((s + c) & 15);
+      const float4 u = st.pos[r], v = st.mom[r];
+      float b1[3] = {0.f, 0.f, 0.f}, b2[3] = {0.f, 0.f, 0.f};
+      constexpr int K = MIXED ? 1 : kSelfTPT;  // with the table, fewer pairs' registers
+#pragma unroll
+      for (int k0 = 0; k0 < kSelfTPT; k0 += K) {
+        const SelfPairs<K> p(u, k0, tx, ty, tz);
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+          const int k = k0 + i;
+          const float ir2 = p.ir[i] * p.ir[i];
+          float beta = ir2 * p.ir[i];
+          float alpha = beta * ir2;
+          if constexpr (MIXED) {
+            if (p.r2[i] < fc.near2) {
+              field_near_coeffs_tab(tab, fc.tab_scale, p.r2[i], p.ir[i], alpha, beta);
+              alpha *= fc.inv_h5;
+              beta *= fc.inv_h3;
+            }
+          }
+          const float dm = fmaf(p.dx[i], v.x, fmaf(p.dy[i], v.y, p.dz[i] * v.z));
+          const float s1 = dm * alpha;
+          a1[k][0] = fmaf(p.dx[i], s1, a1[k][0]);
+          a1[k][1] = fmaf(p.dy[i], s1, a1[k][1]);
+          a1[k][2] = fmaf(p.dz[i], s1, a1[k][2]);
+          a2[k][0] = fmaf(v.x, beta, a2[k][0]);
+          a2[k][1] = fmaf(v.y, beta, a2[k][1]);
+          a2[k][2] = fmaf(v.z, beta, a2[k][2]);
+          if constexpr (BOTH) {
+            const float dn = fmaf(p.dx[i], nx[k], fmaf(p.dy[i], ny[k], p.dz[i] * nz[k]));
+            const float s2 = dn * alpha;
+            b1[0] = fmaf(p.dx[i], s2, b1[0]);
+            b1[1] = fmaf(p.dy[i], s2, b1[1]);
+            b1[2] = fmaf(p.dz[i], s2, b1[2]);
+            b2[0] = fmaf(nx[k], beta, b2[0]);
+            b2[1] = fmaf(ny[k], beta, b2[1]);
+            b2[2] = fmaf(nz[k], beta, b2[2]);
+          }
+        }
+      }
+      if constexpr (BOTH) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) jc[a] = row_next(jc[a]) + fmaf(3.f, b1[a], -b2[a]);
+      }
+    }
+  }
+};
+
+// The pair force f = d e + m f1 + n g1 on the target is -f on the record:
+// f1 = P (d.n), g1 = P (d.m), e = P (m.n) + R (d.m)(d.n), R = -5 P / r^2 (far).
+struct ForceSelf {
+  const HessConsts &hc;
+  const float4 *tab;
+  float tx[kSelfTPT], ty[kSelfTPT], tz[kSelfTPT], nx[kSelfTPT], ny[kSelfTPT], nz[kSelfTPT];
+  float ad[kSelfTPT][3], am[kSelfTPT][3], an[kSelfTPT];
+  __device__ __forceinline__ ForceSelf(const HessConsts &consts, const float4 *t)
+      : hc(consts), tab(t) {}
+  __device__ __forceinline__ bool far(float dist2) const { return dist2 > hc.near2; }
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int k = 0; k < kSelfTPT; ++k) {
+#pragma unroll
+      for (int a = 0; a < 3; ++a) ad[k][a] = am[k][a] = 0.f;
+      an[k] = 0.f;
+    }
+  }
+  __device__ __forceinline__ void flush(double *acc) {
+#pragma unroll
+    for (int k = 0; k < kSelfTPT; ++k) {
+      float n3[3] = {nx[k], ny[k], nz[k]};
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        // not converted ahead of the walk: 24 registers held through every tile
+        asm volatile("" : "+v"(n3[a]));
+        acc[(3 * k + a) * 64] += (static_cast<double>(ad[k][a]) + static_cast<double>(am[k][a])) +
+                                 static_cast<double>(n3[a]) * static_cast<double>(an[k]);
+      }
+    }
+    clear();
+  }
+  template <bool MIXED, bool BOTH>
+  __device__ __forceinline__ void tile(const SelfTile &st, int c, int q, float (&jc)[3]) {
+#pragma unroll 1
+    for (int s = 0; s < 16; ++s) {
+      const int r = 16 * q + ((s + c) & 15);
+      const float4 u = st.pos[r], v = st.mom[r];
+      float b[3] = {0.f, 0.f, 0.f}, bf = 0.f;
+      constexpr int K = MIXED ? 1 : kSelfTPT;  // with the table, fewer pairs' registers
+#pragma unroll
+      for (int k0 = 0; k0 < kSelfTPT; k0 += K) {
+        const SelfPairs<K> p(u, k0, tx, ty, tz);
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+          const int k = k0 + i;
+          const float dm = fmaf(p.dx[i], v.x, fmaf(p.dy[i], v.y, p.dz[i] * v.z));
+          const float dn = fmaf(p.dx[i], nx[k], fmaf(p.dy[i], ny[k], p.dz[i] * nz[k]));
+          const float mn = fmaf(v.x, nx[k], fmaf(v.y, ny[k], v.z * nz[k]));
+          float P, e;
+          if constexpr (MIXED) {
+            // the clamp keeps a pair at d = 0 finite
+            const float ir = __builtin_amdgcn_fmed3f(p.ir[i], 0.f, 1e12f);
+            const float ir2 = ir * ir;
+            float c1 = ir2 * ir2, dq = c1;  // far curves
+            if (!(p.r2[i] > hc.near2)) {
+              hess_near_curves_tab(tab, hc.tab_scale, p.r2[i], ir, c1, dq);
+              const float w = p.r2[i] > 0.f ? hc.inv_h4 : 0.f;  // nothing at d = 0
+              c1 *= w;
+              dq *= w;
+            }
+            P = c1 * ir;
+            e = fmaf(-5.f * dq * (ir2 * ir), dm * dn, P * mn);
+          } else {
+            const float ir2 = p.ir[i] * p.ir[i];
+            P = ir2 * ir2 * p.ir[i];
+            e = P * fmaf(-5.f * ir2 * dm, dn, mn);
+          }
+          const float f1 = P * dn, g1 = P * dm;
+          ad[k][0] = fmaf(p.dx[i], e, ad[k][0]);
+          ad[k][1] = fmaf(p.dy[i], e, ad[k][1]);
+          ad[k][2] = fmaf(p.dz[i], e, ad[k][2]);
+          am[k][0] = fmaf(v.x, f1, am[k][0]);
+          am[k][1] = fmaf(v.y, f1, am[k][1]);
+          am[k][2] = fmaf(v.z, f1, am[k][2]);
+          an[k] += g1;
+          if constexpr (BOTH) {
+            b[0] = fmaf(nx[k], g1, fmaf(p.dx[i], e, b[0]));
+            b[1] = fmaf(ny[k], g1, fmaf(p.dy[i], e, b[1]));
+            b[2] = fmaf(nz[k], g1, fmaf(p.dz[i], e, b[2]));
+            bf += f1;
+          }
+        }
+      }
+      if constexpr (BOTH) {
+        jc[0] = row_next(jc[0]) - fmaf(v.x, bf, b[0]);
+        jc[1] = row_next(jc[1]) - fmaf(v.y, bf, b[1]);
+        jc[2] = row_next(jc[2]) - fmaf(v.z, bf, b[2]);
+      }
+    }
+  }
+};
+
+template <class Pairs, class Consts, int W, int NTAB>
+__device__ __forceinline__ void self_walk(const SrcRec *__restrict__ rec,
+                                          const float4 *__restrict__ boxes, int64_t n,
+                                          const SelfWalk &w, const Consts &consts,
+                                          const UnitTable<NTAB> &table, double fac,
+                                          double *__restrict__ partial) {
+  __shared__ float4 s_tab[2 * NTAB];
+  __shared__ SelfTile st[2];
+  __shared__ float jp[2][W][3][kTile];
+  __shared__ double s_acc[W][3 * kSelfTPT][64];
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, q = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  {
+    const float4 *__restrict__ t = reinterpret_cast<const float4 *>(&table);
+    for (int i = tid; i < 2 * NTAB; i += 64 * W) s_tab[i] = t[i];
+  }
+  const int group = static_cast<int>(blockIdx.x), chunk = static_cast<int>(blockIdx.y);
+  const int it = group * W + wave;  // the wave's i-tile
+  const bool live = it < w.ntiles;
+  Pairs prs(consts, s_tab);
+  const int64_t last = static_cast<int64_t>(w.ntiles) * kTile - 1;  // padding included
+#pragma unroll
+  for (int k = 0; k < kSelfTPT; ++k) {
+    const int64_t i = static_cast<int64_t>(it) * kTile + 16 * k + c;
+    const SrcRec t = rec[i < last ? i : last];
+    prs.tx[k] = t.x;
+    prs.ty[k] = t.y;
+    prs.tz[k] = t.z;
+    prs.nx[k] = t.mx;
+    prs.ny[k] = t.my;
+    prs.nz[k] = t.mz;
+  }
+  // the i-tile's box is its targets' (padding excluded)
+  const int bt = live ? it : 0;
+  const float4 ilo = boxes[2 * bt], ihi = boxes[2 * bt + 1];
+  // the lane's FP64 sums live in LDS: 24 registers fewer
+  double *acc = &s_acc[wave][0][lane];
+#pragma unroll
+  for (int k = 0; k < 3 * kSelfTPT; ++k) acc[k * 64] = 0.0;
+  prs.clear();
+
+  const int u0 = w.first + chunk * w.per, u1 = min(u0 + w.per, w.last);
+  auto tile_of = [&](int u) {
+    int g = group + u / W;
+    g -= g >= w.ngroups ? w.ngroups : 0;
+    return g * W + u % W;
+  };
+  auto next_unit = [&](int u) {  // the first unit from u on whose j-tile exists
+    while (u < u1 && tile_of(u) >= w.ntiles) ++u;
+    return u;
+  };
+  const float4 *__restrict__ rec4 = reinterpret_cast<const float4 *>(rec);
+  // wave 0 copies the j-tile into LDS, 16 bytes a lane, with no register held
+  auto stage = [&](SelfTile &s, int jt) {
+    const float4 *g = rec4 + 2 * (static_cast<int64_t>(jt) * kTile + lane);
+    __builtin_amdgcn_global_load_lds(
+        reinterpret_cast<const __attribute__((address_space(1))) void *>(
+            reinterpret_cast<uintptr_t>(g)),
+        reinterpret_cast<__attribute__((address_space(3))) void *>(
+            reinterpret_cast<uintptr_t>(&s.pos[0])),
+        16, 0, 0);
+    __builtin_amdgcn_global_load_lds(
+        reinterpret_cast<const __attribute__((address_space(1))) void *>(
+            reinterpret_cast<uintptr_t>(g + 1)),
+        reinterpret_cast<__attribute__((address_space(3))) void *>(
+            reinterpret_cast<uintptr_t>(&s.mom[0])),
+        16, 0, 0);
+  };
+  int u = next_unit(u0), buf = 0, since = 0;
+  if (u < u1 && wave == 0) stage(st[0], tile_of(u));
+  __builtin_amdgcn_s_waitcnt(kWaitVm0);  // the copy has landed
+  __syncthreads();
+  // u, next and buf are uniform over the workgroup: every wave meets every barrier
+  while (u < u1) {
+    const int next = next_unit(u + 1), jt = tile_of(u);
+    const bool both = u >= W;
+    // st[buf ^ 1] was last read before the previous barrier
+    if (wave == 0 && next < u1) stage(st[buf ^ 1], tile_of(next));
+    float jc[3] = {0.f, 0.f, 0.f};
+    if (live) {
+      const float4 lo = boxes[2 * jt], hi = boxes[2 * jt + 1];
+      const bool far = prs.far(uniform_f(box_dist2(ilo.x, ilo.y, ilo.z, ihi.x, ihi.y, ihi.z, lo, hi)));
+      if (both) {
+        if (far)
+          prs.template tile<false, true>(st[buf], c, q, jc);
+        else
+          prs.template tile<true, true>(st[buf], c, q, jc);
+      } else {
+        if (far)
+          prs.template tile<false, false>(st[buf], c, q, jc);
+        else
+          prs.template tile<true, false>(st[buf], c, q, jc);
+      }
+      if (++since == kSelfFlush) {
+        prs.flush(acc);
+        since = 0;
+      }
+    }
+    if (both) {
+#pragma unroll
+      for (int a = 0; a < 3; ++a) jp[buf][wave][a][lane] = row_next(jc[a]);
+    }
+    __builtin_amdgcn_s_waitcnt(kWaitVm0);
+    __syncthreads();
+    if (both && tid < 3 * kTile) {
+      // read again only after the next barrier (two buffers)
+      const int a = tid / kTile;
+      double v = 0.0;
+#pragma unroll
+      for (int k = 0; k < W; ++k) v += static_cast<double>(jp[buf][k][a][lane]);
+      const int64_t j = static_cast<int64_t>(jt) * kTile + lane;
+      const int slot = w.nchunk + u / W - max(w.first / W, 1);
+      if (j < n) partial[(static_cast<int64_t>(slot) * 3 + a) * n + j] = v * fac;
+    }
+    u = next;
+    buf ^= 1;
+  }
+  prs.flush(acc);
+  double *out = partial + static_cast<int64_t>(chunk) * 3 * n;
+  const int64_t i = static_cast<int64_t>(it) * kTile + lane;  // lane group k stores its k-th sixteen
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    double v = 0.0;
+#pragma unroll
+    for (int k = 0; k < kSelfTPT; ++k) {
+      const double sum = group_sum(acc[(3 * k + a) * 64]);
+      v = q == k ? sum : v;
+    }
+    if (i < n) out[a * n + i] = v * fac;
+  }
+}
+
+template <int W>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) void field_self_kernel(const SrcRec *__restrict__ rec,
+                                                            const float4 *__restrict__ boxes,
+                                                            int64_t n, SelfWalk w, FieldConsts fc,
+                                                            double *__restrict__ partial) {
+  self_walk<FieldSelf, FieldConsts, W, kFieldTabEntries>(rec, boxes, n, w, fc, d_field_tab,
+                                                         1.0 / (4.0 * kPi), partial);
+}
+
+template <int W>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) void force_self_kernel(const SrcRec *__restrict__ rec,
+                                                            const float4 *__restrict__ boxes,
+                                                            int64_t n, SelfWalk w, HessConsts hc,
+                                                            double *__restrict__ partial) {
+  self_walk<ForceSelf, HessConsts, W, kHessTabEntries>(rec, boxes, n, w, hc, d_hess_tab,
+                                                       3.0 * kMu0 / (4.0 * kPi), partial);
+}
+
+// ---------------------------------------------------------------------------
 // Force-tensor field at separate targets (the external tensor T_ext of
 // eval_hext), walked like the field: partials [chunk][6][nt_ld] (xx yy zz xy
 // xz yz).
@@ -1122,34 +1509,176 @@ Status field_allpairs_launch(mf_ctx *ctx, const Points &tgt, int64_t nt, const S
                                   cap);
 }
 
+namespace {
+// Walk of the pair-once kernels.  Four waves a workgroup: two write twice the j-sums
+// (262,144 particles: field 24.4 ms, 22.1 with four), eight wait longer for each
+// other (22.6).  Up to sixteen fills of the chip (16 waves per CU) with at least four units a
+// chunk, but one fill in any case: 15,625 particles take 111 us a field product with
+// two to eight units a chunk and 121 with one; 50,000 take 0.88 ms with four fills,
+// 0.86 with sixteen.  Below kSelfMin records the directed kernels end first (2,744: field
+// 20.0 against 20.5 us, force 21.7 against 23.5; 4,096: 24.2 against 22.2, 28.8 against
+// 28.0).
+constexpr int kSelfW = 4;
+constexpr int64_t kSelfMin = 4096;
+constexpr int64_t kSelfUnitsMin = 4;
+// The slots grow with the square of n: beyond kSelfBytes the group distances go in
+// passes, each folded into one slot before the next.
+constexpr int64_t kSelfBytes = int64_t{2} << 30;
+struct SelfSplit {
+  SelfWalk w;     // the walk's constants
+  int dist;       // group distances 0 .. dist - 1
+  int per_pass;   // group distances per pass
+  int64_t slots;  // FP64 slots of 3 n: the folded sums if there are several passes, then a pass's
+};
+int self_chunks(const mf_ctx *ctx, const SelfWalk &w, int units) {
+  const int64_t fill = static_cast<int64_t>(ctx->num_cu) * kFillWaves / kSelfW;
+  const int64_t one = std::min<int64_t>((fill + w.ngroups - 1) / w.ngroups, units);
+  const int64_t many =
+      std::min<int64_t>((fill * kFills + w.ngroups - 1) / w.ngroups, units / kSelfUnitsMin);
+  return static_cast<int>(std::max<int64_t>(std::max(one, many), 1));
+}
+SelfSplit self_split(const mf_ctx *ctx, int64_t n) {
+  SelfSplit f{};
+  f.w.ntiles = static_cast<int>((n + kTile - 1) / kTile);
+  f.w.ngroups = ((f.w.ntiles + kSelfW - 1) / kSelfW) | 1;
+  f.dist = f.w.ngroups / 2 + 1;
+  const int64_t fit = std::max<int64_t>(kSelfBytes / (24 * n), 2);
+  const int chunks = self_chunks(ctx, f.w, kSelfW * f.dist);
+  if (chunks + f.dist - 1 <= fit) {
+    f.per_pass = f.dist;
+    f.slots = chunks + f.dist - 1;
+    return f;
+  }
+  // a pass of d distances takes at most d + self_chunks(d) slots
+  f.per_pass = static_cast<int>(std::max<int64_t>(fit - std::min<int64_t>(chunks, fit / 2), 1));
+  f.slots = 1 + f.per_pass + self_chunks(ctx, f.w, kSelfW * f.per_pass);
+  return f;
+}
+
+// sum[i] (+)= the pass's slots.
+__global__ void fold_slots_kernel(int64_t n3, int slots, int add, const double *__restrict__ p,
+                                  double *__restrict__ sum) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= n3) return;
+  double s = add ? sum[i] : 0.0;
+  for (int k = 0; k < slots; ++k) s += p[k * n3 + i];
+  sum[i] = s;
+}
+
+// The passes: launch(walk, slots) runs one.  On return the first `nchunk` slots of
+// `partial` hold the sums.
+template <class Launch>
+Status self_passes(mf_ctx *ctx, int64_t n, const SelfSplit &f, double *partial, int *nchunk,
+                   const Launch &launch) {
+  const bool one = f.per_pass == f.dist;
+  double *slots = one ? partial : partial + 3 * n;
+  for (int d = 0; d < f.dist; d += f.per_pass) {
+    const int d1 = std::min(d + f.per_pass, f.dist);
+    SelfWalk w = f.w;
+    w.first = kSelfW * d;
+    w.last = kSelfW * d1;
+    w.nchunk = self_chunks(ctx, w, w.last - w.first);
+    w.per = (w.last - w.first + w.nchunk - 1) / w.nchunk;
+    w.nchunk = (w.last - w.first + w.per - 1) / w.per;
+    launch(w, slots);
+    MF_LAUNCH_CHECK();
+    *nchunk = w.nchunk + d1 - std::max(d, 1);
+    if (!one) {
+      hipLaunchKernelGGL(fold_slots_kernel, dim3(grid_for(3 * n, 256)), dim3(256), 0, ctx->stream,
+                         3 * n, *nchunk, d > 0 ? 1 : 0, slots, partial);
+      MF_LAUNCH_CHECK();
+    }
+  }
+  if (!one) *nchunk = 1;
+  return Status::Ok();
+}
+}  // namespace
+
+namespace {
+// The partial sums of the field of a record set on itself.
+Status field_self_chunks(mf_ctx *ctx, const SrcRec *rec, const float4 *boxes, int64_t n,
+                         const FieldConsts &fc, double **partial, int *nchunk) {
+  if (n >= kSelfMin) {
+    const SelfSplit f = self_split(ctx, n);
+    void *pw = nullptr;
+    if (workspace_now(ctx, "field_partial", sizeof(double) * 3 * n * f.slots, &pw)) {
+      *partial = static_cast<double *>(pw);
+      KernelTimer timer(ctx, "field");
+      return self_passes(ctx, n, f, *partial, nchunk, [&](const SelfWalk &w, double *slots) {
+        hipLaunchKernelGGL(field_self_kernel<kSelfW>,
+                           dim3(static_cast<unsigned>(w.ngroups), static_cast<unsigned>(w.nchunk)),
+                           dim3(64 * kSelfW), 0, ctx->stream, rec, boxes, n, w, fc, slots);
+      });
+    }
+  }
+  int64_t cap = 0;
+  MF_TRY(field_workspace(ctx, n, n, partial, &cap));
+  const Split d = split_sources(ctx, n, n, kFieldTPT, kMaxChunks);
+  *nchunk = static_cast<int>(d.nchunk);
+  return field_chunks(ctx, record_points(rec), n, rec, boxes, fc, d, *partial);
+}
+}  // namespace
+
 int field_ap_blocks(int64_t n) { return static_cast<int>(reduce_grid(n).x); }
 
 Status field_allpairs_ap(mf_ctx *ctx, const SrcRec *rec, const float4 *boxes, int64_t n,
                          const FieldConsts &fc, const ApOut &out) {
   double *partial = nullptr;
-  int64_t cap = 0;
-  MF_TRY(field_workspace(ctx, n, n, &partial, &cap));
-  const Split f = split_sources(ctx, n, n, kFieldTPT, kMaxChunks);
-  MF_TRY(field_chunks(ctx, record_points(rec), n, rec, boxes, fc, f, partial));
-  MF_REDUCE(reduce_ap_kernel, n, n, n, static_cast<int>(f.nchunk), partial, out);
+  int nchunk = 0;
+  MF_TRY(field_self_chunks(ctx, rec, boxes, n, fc, &partial, &nchunk));
+  MF_REDUCE(reduce_ap_kernel, n, n, n, nchunk, partial, out);
   return Status::Ok();
 }
+
+Status field_self_launch(mf_ctx *ctx, const SrcRec *rec, const float4 *boxes, int64_t n,
+                         const FieldConsts &fc, const float *hconst, float *ox, float *oy,
+                         float *oz) {
+  if (n == 0) return Status::Ok();
+  double *partial = nullptr;
+  int nchunk = 0;
+  MF_TRY(field_self_chunks(ctx, rec, boxes, n, fc, &partial, &nchunk));
+  const float h0 = hconst ? hconst[0] : 0.f, h1 = hconst ? hconst[1] : 0.f,
+              h2 = hconst ? hconst[2] : 0.f;
+  MF_REDUCE(reduce_field_kernel, n, n, n, nchunk, partial, h0, h1, h2, ox, oy, oz);
+  return Status::Ok();
+}
+
+namespace {
+Status force_self_chunks(mf_ctx *ctx, const SrcRec *rec, const float4 *boxes, int64_t n,
+                         const HessConsts &hc, double **partial, int *nchunk) {
+  void *pw = nullptr;
+  if (n >= kSelfMin) {
+    const SelfSplit f = self_split(ctx, n);
+    if (workspace_now(ctx, "force_partial", sizeof(double) * 3 * n * f.slots, &pw)) {
+      *partial = static_cast<double *>(pw);
+      KernelTimer timer(ctx, "force");
+      return self_passes(ctx, n, f, *partial, nchunk, [&](const SelfWalk &w, double *slots) {
+        hipLaunchKernelGGL(force_self_kernel<kSelfW>,
+                           dim3(static_cast<unsigned>(w.ngroups), static_cast<unsigned>(w.nchunk)),
+                           dim3(64 * kSelfW), 0, ctx->stream, rec, boxes, n, w, hc, slots);
+      });
+    }
+  }
+  const Split d = split_sources(ctx, n, n, kForceTPT, kMaxChunks);
+  MF_TRY(workspace(ctx, "force_partial", sizeof(double) * 3 * n * d.nchunk, &pw));
+  *partial = static_cast<double *>(pw);
+  *nchunk = static_cast<int>(d.nchunk);
+  KernelTimer timer(ctx, "force");
+  hipLaunchKernelGGL(force_allpairs_kernel<kForceTPT>,
+                     dim3(d.gx, static_cast<unsigned>(d.nchunk)), dim3(64), 0, ctx->stream, rec, n,
+                     rec, boxes, d.nsub, d.per, hc, n, *partial);
+  MF_LAUNCH_CHECK();
+  return Status::Ok();
+}
+}  // namespace
 
 Status force_allpairs_launch(mf_ctx *ctx, const SrcRec *rec, const float4 *boxes, int64_t n,
                              const HessConsts &hc, const float *const *text9, float *fx,
                              float *fy, float *fz) {
   if (n == 0) return Status::Ok();
-  const Split f = split_sources(ctx, n, n, kForceTPT, kMaxChunks);
-  void *pw = nullptr;
-  MF_TRY(workspace(ctx, "force_partial", sizeof(double) * 3 * n * f.nchunk, &pw));
-  double *partial = static_cast<double *>(pw);
-  {
-    KernelTimer timer(ctx, "force");
-    hipLaunchKernelGGL(force_allpairs_kernel<kForceTPT>,
-                       dim3(f.gx, static_cast<unsigned>(f.nchunk)), dim3(64), 0, ctx->stream, rec,
-                       n, rec, boxes, f.nsub, f.per, hc, n, partial);
-    MF_LAUNCH_CHECK();
-  }
+  double *partial = nullptr;
+  int nchunk = 0;
+  MF_TRY(force_self_chunks(ctx, rec, boxes, n, hc, &partial, &nchunk));
   Text9 t{};
   int has_text = 0;
   if (text9) {
@@ -1159,7 +1688,7 @@ Status force_allpairs_launch(mf_ctx *ctx, const SrcRec *rec, const float4 *boxes
       t.p[k] = text9[k];
     }
   }
-  MF_REDUCE(reduce_force_kernel, n, n, n, static_cast<int>(f.nchunk), partial, rec, t, has_text, fx,
+  MF_REDUCE(reduce_force_kernel, n, n, n, nchunk, partial, rec, t, has_text, fx,
             fy, fz);
   return Status::Ok();
 }

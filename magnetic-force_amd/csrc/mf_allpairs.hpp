@@ -56,6 +56,10 @@ struct ApOut {
   float *ap[3];
   double *dots;
 };
+// out = hconst + G m of one record set on itself.
+Status field_self_launch(mf_ctx *ctx, const SrcRec *rec, const float4 *boxes, int64_t n,
+                         const FieldConsts &fc, const float *hconst, float *ox, float *oy,
+                         float *oz);
 int field_ap_blocks(int64_t n);
 Status field_allpairs_ap(mf_ctx *ctx, const SrcRec *rec, const float4 *boxes, int64_t n,
                          const FieldConsts &fc, const ApOut &out);

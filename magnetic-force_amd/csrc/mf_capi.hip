@@ -163,8 +163,8 @@ Status plan_apply_G(mf_plan *plan, float scale, const float *px, const float *py
   mf_ctx *ctx = plan->ctx;
   SrcRec *rec = plan->rec.as<SrcRec>();
   MF_TRY(pack_moments(ctx, plan->n, px, py, pz, scale, rec));
-  return field_allpairs_launch(ctx, record_points(rec), plan->n, rec, plan->boxes.as<float4>(),
-                               plan->n, plan->fc, hconst, ox, oy, oz);
+  return field_self_launch(ctx, rec, plan->boxes.as<float4>(), plan->n, plan->fc, hconst, ox, oy,
+                           oz);
 }
 
 Status plan_force(mf_plan *plan, const float *mx, const float *my, const float *mz,
