@@ -41,6 +41,7 @@
 #include <cmath>
 
 #include "mf_allpairs.hpp"
+#include "mf_pair_once.hpp"
 #include "mf_internal.hpp"
 #include "mf_pair.hpp"
 
@@ -48,7 +49,6 @@ namespace mf {
 
 namespace {
 
-constexpr float kPadCoord = 1.0e18f;  // far-away position of padding records
 
 // ---------------------------------------------------------------------------
 // Near-pair coefficient tables (mf_pair.hpp describes their entries).  The
@@ -719,15 +719,8 @@ __global__ __launch_bounds__(64) void force_allpairs_kernel(
 // ---------------------------------------------------------------------------
 // One record set against itself, every unordered pair evaluated once.
 //
-// The distance, its inverse root and the radial coefficients of a pair serve
-// both of its particles, and the force on one is minus the force on the other
-// (the pair form of the force is antisymmetric under exchange).  A unit of work
-// is one wave's 64 records (an i-tile, four targets a lane) against one staged
-// j-tile: at step s lane c of each 16-lane row takes record (s + c) mod 16 of its
-// row's sixteen, and the sums for that record move one lane down the row with it
-// (row_ror), so after 16 steps lane c holds the sums of record c over the wave's
-// 64 targets.  64 evaluated pairs then cost 96 (field) and 121 (force) cycles
-// where two directed ones cost 130 and 182.
+// A unit of work is one wave's 64 records (an i-tile, four targets a lane)
+// against one staged j-tile (mf_pair_once.hpp).
 //
 // A workgroup is W waves with W consecutive i-tiles (a group) walking the same
 // j-tiles; the j-sums of its waves meet in LDS and leave in FP64, one slot per
@@ -747,208 +740,6 @@ struct SelfWalk {
   int first, last;  // the launch's units: j-tiles [first, last) of a group's W (D + 1)
   int per;          // units per chunk
   int nchunk;
-};
-
-struct SelfTile {
-  float4 pos[kTile], mom[kTile];
-};
-
-// s_waitcnt vmcnt(0), nothing else waited for (expcnt 7, lgkmcnt 15).
-constexpr int kWaitVm0 = 0x0F70;
-
-// The value of the next lane up in the 16-lane row (cyclic).
-__device__ __forceinline__ float row_next(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x12F, 0xf, 0xf, false));
-}
-
-// Distances and inverse distances of the lane's record (u.xyz) to its targets
-// k0 .. k0 + K - 1; one run of roots at raised priority, as in StepPairs.
-template <int K>
-struct SelfPairs {
-  float dx[K], dy[K], dz[K], r2[K], ir[K];
-  __device__ __forceinline__ SelfPairs(const float4 &u, int k0, const float (&tx)[kSelfTPT],
-                                       const float (&ty)[kSelfTPT], const float (&tz)[kSelfTPT]) {
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      dx[k] = tx[k0 + k] - u.x;
-      dy[k] = ty[k0 + k] - u.y;
-      dz[k] = tz[k0 + k] - u.z;
-      r2[k] = fmaf(dx[k], dx[k], fmaf(dy[k], dy[k], dz[k] * dz[k]));
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int k = 0; k < K; ++k) ir[k] = __builtin_amdgcn_rsqf(r2[k]);
-    __builtin_amdgcn_s_setprio(0);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-};
-
-struct FieldSelf {
-  const FieldConsts &fc;
-  const float4 *tab;
-  float tx[kSelfTPT], ty[kSelfTPT], tz[kSelfTPT], nx[kSelfTPT], ny[kSelfTPT], nz[kSelfTPT];
-  float a1[kSelfTPT][3], a2[kSelfTPT][3];
-  __device__ __forceinline__ FieldSelf(const FieldConsts &consts, const float4 *t)
-      : fc(consts), tab(t) {}
-  __device__ __forceinline__ bool far(float dist2) const { return dist2 >= fc.near2; }
-  __device__ __forceinline__ void clear() {
-#pragma unroll
-    for (int k = 0; k < kSelfTPT; ++k)
-#pragma unroll
-      for (int a = 0; a < 3; ++a) a1[k][a] = a2[k][a] = 0.f;
-  }
-  __device__ __forceinline__ void flush(double *acc) {
-#pragma unroll
-    for (int k = 0; k < kSelfTPT; ++k)
-#pragma unroll
-      for (int a = 0; a < 3; ++a)
-        acc[(3 * k + a) * 64] += 3.0 * static_cast<double>(a1[k][a]) - static_cast<double>(a2[k][a]);
-    clear();
-  }
-  template <bool MIXED, bool BOTH>
-  __device__ __forceinline__ void tile(const SelfTile &st, int c, int q, float (&jc)[3]) {
-#pragma unroll 1
-    for (int s = 0; s < 16; ++s) {
-      const int r = 16 * q + ((s + c) & 15);
-      const float4 u = st.pos[r], v = st.mom[r];
-      float b1[3] = {0.f, 0.f, 0.f}, b2[3] = {0.f, 0.f, 0.f};
-      constexpr int K = MIXED ? 1 : kSelfTPT;  // with the table, fewer pairs' registers
-#pragma unroll
-      for (int k0 = 0; k0 < kSelfTPT; k0 += K) {
-        const SelfPairs<K> p(u, k0, tx, ty, tz);
-#pragma unroll
-        for (int i = 0; i < K; ++i) {
-          const int k = k0 + i;
-          const float ir2 = p.ir[i] * p.ir[i];
-          float beta = ir2 * p.ir[i];
-          float alpha = beta * ir2;
-          if constexpr (MIXED) {
-            if (p.r2[i] < fc.near2) {
-              field_near_coeffs_tab(tab, fc.tab_scale, p.r2[i], p.ir[i], alpha, beta);
-              alpha *= fc.inv_h5;
-              beta *= fc.inv_h3;
-            }
-          }
-          const float dm = fmaf(p.dx[i], v.x, fmaf(p.dy[i], v.y, p.dz[i] * v.z));
-          const float s1 = dm * alpha;
-          a1[k][0] = fmaf(p.dx[i], s1, a1[k][0]);
-          a1[k][1] = fmaf(p.dy[i], s1, a1[k][1]);
-          a1[k][2] = fmaf(p.dz[i], s1, a1[k][2]);
-          a2[k][0] = fmaf(v.x, beta, a2[k][0]);
-          a2[k][1] = fmaf(v.y, beta, a2[k][1]);
-          a2[k][2] = fmaf(v.z, beta, a2[k][2]);
-          if constexpr (BOTH) {
-            const float dn = fmaf(p.dx[i], nx[k], fmaf(p.dy[i], ny[k], p.dz[i] * nz[k]));
-            const float s2 = dn * alpha;
-            b1[0] = fmaf(p.dx[i], s2, b1[0]);
-            b1[1] = fmaf(p.dy[i], s2, b1[1]);
-            b1[2] = fmaf(p.dz[i], s2, b1[2]);
-            b2[0] = fmaf(nx[k], beta, b2[0]);
-            b2[1] = fmaf(ny[k], beta, b2[1]);
-            b2[2] = fmaf(nz[k], beta, b2[2]);
-          }
-        }
-      }
-      if constexpr (BOTH) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) jc[a] = row_next(jc[a]) + fmaf(3.f, b1[a], -b2[a]);
-      }
-    }
-  }
-};
-
-// The pair force f = d e + m f1 + n g1 on the target is -f on the record:
-// f1 = P (d.n), g1 = P (d.m), e = P (m.n) + R (d.m)(d.n), R = -5 P / r^2 (far).
-struct ForceSelf {
-  const HessConsts &hc;
-  const float4 *tab;
-  float tx[kSelfTPT], ty[kSelfTPT], tz[kSelfTPT], nx[kSelfTPT], ny[kSelfTPT], nz[kSelfTPT];
-  float ad[kSelfTPT][3], am[kSelfTPT][3], an[kSelfTPT];
-  __device__ __forceinline__ ForceSelf(const HessConsts &consts, const float4 *t)
-      : hc(consts), tab(t) {}
-  __device__ __forceinline__ bool far(float dist2) const { return dist2 > hc.near2; }
-  __device__ __forceinline__ void clear() {
-#pragma unroll
-    for (int k = 0; k < kSelfTPT; ++k) {
-#pragma unroll
-      for (int a = 0; a < 3; ++a) ad[k][a] = am[k][a] = 0.f;
-      an[k] = 0.f;
-    }
-  }
-  __device__ __forceinline__ void flush(double *acc) {
-#pragma unroll
-    for (int k = 0; k < kSelfTPT; ++k) {
-      float n3[3] = {nx[k], ny[k], nz[k]};
-#pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        // not converted ahead of the walk: 24 registers held through every tile
-        asm volatile("" : "+v"(n3[a]));
-        acc[(3 * k + a) * 64] += (static_cast<double>(ad[k][a]) + static_cast<double>(am[k][a])) +
-                                 static_cast<double>(n3[a]) * static_cast<double>(an[k]);
-      }
-    }
-    clear();
-  }
-  template <bool MIXED, bool BOTH>
-  __device__ __forceinline__ void tile(const SelfTile &st, int c, int q, float (&jc)[3]) {
-#pragma unroll 1
-    for (int s = 0; s < 16; ++s) {
-      const int r = 16 * q + ((s + c) & 15);
-      const float4 u = st.pos[r], v = st.mom[r];
-      float b[3] = {0.f, 0.f, 0.f}, bf = 0.f;
-      constexpr int K = MIXED ? 1 : kSelfTPT;  // with the table, fewer pairs' registers
-#pragma unroll
-      for (int k0 = 0; k0 < kSelfTPT; k0 += K) {
-        const SelfPairs<K> p(u, k0, tx, ty, tz);
-#pragma unroll
-        for (int i = 0; i < K; ++i) {
-          const int k = k0 + i;
-          const float dm = fmaf(p.dx[i], v.x, fmaf(p.dy[i], v.y, p.dz[i] * v.z));
-          const float dn = fmaf(p.dx[i], nx[k], fmaf(p.dy[i], ny[k], p.dz[i] * nz[k]));
-          const float mn = fmaf(v.x, nx[k], fmaf(v.y, ny[k], v.z * nz[k]));
-          float P, e;
-          if constexpr (MIXED) {
-            // the clamp keeps a pair at d = 0 finite
-            const float ir = __builtin_amdgcn_fmed3f(p.ir[i], 0.f, 1e12f);
-            const float ir2 = ir * ir;
-            float c1 = ir2 * ir2, dq = c1;  // far curves
-            if (!(p.r2[i] > hc.near2)) {
-              hess_near_curves_tab(tab, hc.tab_scale, p.r2[i], ir, c1, dq);
-              const float w = p.r2[i] > 0.f ? hc.inv_h4 : 0.f;  // nothing at d = 0
-              c1 *= w;
-              dq *= w;
-            }
-            P = c1 * ir;
-            e = fmaf(-5.f * dq * (ir2 * ir), dm * dn, P * mn);
-          } else {
-            const float ir2 = p.ir[i] * p.ir[i];
-            P = ir2 * ir2 * p.ir[i];
-            e = P * fmaf(-5.f * ir2 * dm, dn, mn);
-          }
-          const float f1 = P * dn, g1 = P * dm;
-          ad[k][0] = fmaf(p.dx[i], e, ad[k][0]);
-          ad[k][1] = fmaf(p.dy[i], e, ad[k][1]);
-          ad[k][2] = fmaf(p.dz[i], e, ad[k][2]);
-          am[k][0] = fmaf(v.x, f1, am[k][0]);
-          am[k][1] = fmaf(v.y, f1, am[k][1]);
-          am[k][2] = fmaf(v.z, f1, am[k][2]);
-          an[k] += g1;
-          if constexpr (BOTH) {
-            b[0] = fmaf(nx[k], g1, fmaf(p.dx[i], e, b[0]));
-            b[1] = fmaf(ny[k], g1, fmaf(p.dy[i], e, b[1]));
-            b[2] = fmaf(nz[k], g1, fmaf(p.dz[i], e, b[2]));
-            bf += f1;
-          }
-        }
-      }
-      if constexpr (BOTH) {
-        jc[0] = row_next(jc[0]) - fmaf(v.x, bf, b[0]);
-        jc[1] = row_next(jc[1]) - fmaf(v.y, bf, b[1]);
-        jc[2] = row_next(jc[2]) - fmaf(v.z, bf, b[2]);
-      }
-    }
-  }
 };
 
 template <class Pairs, class Consts, int W, int NTAB>
@@ -991,6 +782,13 @@ __device__ __forceinline__ void self_walk(const SrcRec *__restrict__ rec,
 #pragma unroll
   for (int k = 0; k < 3 * kSelfTPT; ++k) acc[k * 64] = 0.0;
   prs.clear();
+  auto flush = [&]() {
+#pragma unroll
+    for (int k = 0; k < kSelfTPT; ++k)
+#pragma unroll
+      for (int a = 0; a < 3; ++a) acc[(3 * k + a) * 64] += prs.sum(k, a);
+    prs.clear();
+  };
 
   const int u0 = w.first + chunk * w.per, u1 = min(u0 + w.per, w.last);
   auto tile_of = [&](int u) {
@@ -1003,25 +801,15 @@ __device__ __forceinline__ void self_walk(const SrcRec *__restrict__ rec,
     return u;
   };
   const float4 *__restrict__ rec4 = reinterpret_cast<const float4 *>(rec);
-  // wave 0 copies the j-tile into LDS, 16 bytes a lane, with no register held
+  // wave 0 copies the j-tile
   auto stage = [&](SelfTile &s, int jt) {
     const float4 *g = rec4 + 2 * (static_cast<int64_t>(jt) * kTile + lane);
-    __builtin_amdgcn_global_load_lds(
-        reinterpret_cast<const __attribute__((address_space(1))) void *>(
-            reinterpret_cast<uintptr_t>(g)),
-        reinterpret_cast<__attribute__((address_space(3))) void *>(
-            reinterpret_cast<uintptr_t>(&s.pos[0])),
-        16, 0, 0);
-    __builtin_amdgcn_global_load_lds(
-        reinterpret_cast<const __attribute__((address_space(1))) void *>(
-            reinterpret_cast<uintptr_t>(g + 1)),
-        reinterpret_cast<__attribute__((address_space(3))) void *>(
-            reinterpret_cast<uintptr_t>(&s.mom[0])),
-        16, 0, 0);
+    copy16_to_lds(g, s.pos);
+    copy16_to_lds(g + 1, s.mom);
   };
   int u = next_unit(u0), buf = 0, since = 0;
   if (u < u1 && wave == 0) stage(st[0], tile_of(u));
-  __builtin_amdgcn_s_waitcnt(kWaitVm0);  // the copy has landed
+  wait_vm<0>();  // the copy has landed
   __syncthreads();
   // u, next and buf are uniform over the workgroup: every wave meets every barrier
   while (u < u1) {
@@ -1045,7 +833,7 @@ __device__ __forceinline__ void self_walk(const SrcRec *__restrict__ rec,
           prs.template tile<true, false>(st[buf], c, q, jc);
       }
       if (++since == kSelfFlush) {
-        prs.flush(acc);
+        flush();
         since = 0;
       }
     }
@@ -1053,7 +841,7 @@ __device__ __forceinline__ void self_walk(const SrcRec *__restrict__ rec,
 #pragma unroll
       for (int a = 0; a < 3; ++a) jp[buf][wave][a][lane] = row_next(jc[a]);
     }
-    __builtin_amdgcn_s_waitcnt(kWaitVm0);
+    wait_vm<0>();
     __syncthreads();
     if (both && tid < 3 * kTile) {
       // read again only after the next barrier (two buffers)
@@ -1068,7 +856,7 @@ __device__ __forceinline__ void self_walk(const SrcRec *__restrict__ rec,
     u = next;
     buf ^= 1;
   }
-  prs.flush(acc);
+  flush();
   double *out = partial + static_cast<int64_t>(chunk) * 3 * n;
   const int64_t i = static_cast<int64_t>(it) * kTile + lane;  // lane group k stores its k-th sixteen
 #pragma unroll
@@ -1088,7 +876,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
                                                             const float4 *__restrict__ boxes,
                                                             int64_t n, SelfWalk w, FieldConsts fc,
                                                             double *__restrict__ partial) {
-  self_walk<FieldSelf, FieldConsts, W, kFieldTabEntries>(rec, boxes, n, w, fc, d_field_tab,
+  self_walk<FieldSelf<kSelfTPT>, FieldConsts, W, kFieldTabEntries>(rec, boxes, n, w, fc, d_field_tab,
                                                          1.0 / (4.0 * kPi), partial);
 }
 
@@ -1097,7 +885,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
                                                             const float4 *__restrict__ boxes,
                                                             int64_t n, SelfWalk w, HessConsts hc,
                                                             double *__restrict__ partial) {
-  self_walk<ForceSelf, HessConsts, W, kHessTabEntries>(rec, boxes, n, w, hc, d_hess_tab,
+  self_walk<ForceSelf<kSelfTPT>, HessConsts, W, kHessTabEntries>(rec, boxes, n, w, hc, d_hess_tab,
                                                        3.0 * kMu0 / (4.0 * kPi), partial);
 }
 

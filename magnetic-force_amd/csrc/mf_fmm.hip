@@ -48,12 +48,16 @@
 #include <set>
 #include <string>
 #include <vector>
+#ifndef ONCE_BYTES
+#define ONCE_BYTES (int64_t{12} << 30)
+#endif
 
 #include "mf_allpairs.hpp"
 #include "mf_expansion.hpp"
 #include "mf_fmm_tables.hpp"
 #include "mf_internal.hpp"
 #include "mf_pair.hpp"
+#include "mf_pair_once.hpp"
 #include "mf_plan.hpp"
 #include "mf_sort.hpp"
 
@@ -1374,93 +1378,7 @@ __device__ __forceinline__ void l2p_hess(const float *__restrict__ Lt, float x, 
 // its sums.  Apart, the near-field kernel needs a third of the registers the
 // solid harmonics of L2P take, and runs at twice the occupancy.
 
-// Near ranges of a leaf: the particle ranges of its near boxes, with boxes of
-// consecutive index merged (leaf b + 1 holds the particles right after leaf
-// b's, so a run of consecutive leaf indices is one contiguous range).  One
-// wave per leaf: the slot entries, keyed (class << 28 | box) with slots
-// [0, nmix) class 0 and [nmix, nslot) class 1, are bitonic-sorted in LDS;
-// runs of consecutive keys are the ranges, emitted in key order (class 0
-// first), so the summation order is fixed.  rng[leaf * nslot + r] =
-// {first, end}; nr[leaf] = {class-0 ranges, class-1 ranges}.  kSortN, the
-// sort size, is a power of two >= nslot (128 for the field's 81 slots, 256
-// for the force's 179).
-template <int kSortN>
-__global__ __launch_bounds__(64) void near_ranges_kernel(int nleaf, const int32_t *__restrict__ list,
-                                                         int nslot, int nmix,
-                                                         const int32_t *__restrict__ first,
-                                                         const int32_t *__restrict__ count,
-                                                         int2 *__restrict__ rng,
-                                                         int2 *__restrict__ nr) {
-  __shared__ int s_key[kSortN];
-  const int b = blockIdx.x;
-  const int lane = threadIdx.x;
-  const int32_t *__restrict__ l = list + static_cast<int64_t>(b) * nslot;
-  for (int k = lane; k < kSortN; k += 64) {
-    int key = 0x7fffffff;
-    if (k < nslot) {
-      const int sb = l[k];
-      if (sb >= 0) key = ((k < nmix ? 0 : 1) << 28) | sb;
-    }
-    s_key[k] = key;
-  }
-  __syncthreads();
-  // bitonic sort, ascending: kSortN / 2 compare-exchanges per step, 2 per lane
-  for (int size = 2; size <= kSortN; size <<= 1)
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      for (int c = lane; c < kSortN / 2; c += 64) {
-        const int i = 2 * c - (c & (stride - 1));
-        const int j = i + stride;
-        const bool up = (i & size) == 0;
-        const int a = s_key[i], d = s_key[j];
-        if ((a > d) == up) {
-          s_key[i] = d;
-          s_key[j] = a;
-        }
-      }
-      __syncthreads();
-    }
-  int2 *__restrict__ out = rng + static_cast<int64_t>(b) * nslot;
-  int pos = 0, n0 = 0;
-  for (int k0 = 0; k0 < kSortN; k0 += 64) {
-    const int k = k0 + lane;
-    const int key = s_key[k];
-    const bool valid = key != 0x7fffffff;
-    const bool is_start = valid && (k == 0 || s_key[k - 1] != key - 1);
-    int j0 = 0, j1 = 0;
-    if (is_start) {
-      int e = k;
-      while (e + 1 < kSortN && s_key[e + 1] == s_key[e] + 1) ++e;
-      const int sb = key & 0x0fffffff, se = s_key[e] & 0x0fffffff;
-      j0 = first[sb];
-      j1 = first[se] + count[se];
-    }
-    const uint64_t mask = __ballot(is_start);
-    const uint64_t cls0 = __ballot(is_start && (key >> 28) == 0);
-    const int before = __popcll(mask & ((1ULL << lane) - 1ULL));
-    if (is_start) out[pos + before] = make_int2(j0, j1);
-    pos += __popcll(mask);
-    n0 += __popcll(cls0);
-  }
-  if (lane == 0) nr[b] = make_int2(n0, pos - n0);
-}
-
-// out += far, per particle in caller order: the far part (L2P, and for the
-// force the external-tensor term) was written in FP64 on the context stream
-// while the near field ran beside it; the sum rounds once, as a single
-// kernel adding FP64 terms would.  Systems that have converged (batch plans)
-// are skipped, as in the other product kernels.
-__global__ void add_far_kernel(int64_t n, const double *__restrict__ far3, float *__restrict__ ox,
-                               float *__restrict__ oy, float *__restrict__ oz,
-                               const int32_t *__restrict__ sys_of, const int32_t *__restrict__ active) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  if (active != nullptr && active[sys_of[i]] == 0) return;
-  ox[i] = static_cast<float>(static_cast<double>(ox[i]) + far3[i]);
-  oy[i] = static_cast<float>(static_cast<double>(oy[i]) + far3[n + i]);
-  oz[i] = static_cast<float>(static_cast<double>(oz[i]) + far3[2 * n + i]);
-}
-
-// L2P, field: far3[.][perm] = far field (FP64; add_far_kernel adds it to
+// L2P, field: far3[.][perm] = far field (FP64; near_gather_kernel adds it to
 // H_const + near).  One wave per leaf.
 template <int P, int KP>
 __global__ __launch_bounds__(64) void l2p_field_kernel(
@@ -1492,113 +1410,6 @@ __global__ __launch_bounds__(64) void l2p_field_kernel(
   }
 }
 
-// Near-field source loops over one contiguous source range: the source index
-// is uniform over the wave and the records come through scalar loads.  Sources
-// go in blocks of kNearBlock: all distances, then all reciprocal square roots
-// in one run at raised wave priority, then the sums.  v_rsq_f32 holds its SIMD
-// for about 16 cycles where an FMA takes 2.3; one run per block, started at
-// once, leaves the other waves' plain VALU work in longer stretches.  8.4M particles
-// (full chunks, one wave a leaf), blocks of 2 / 4 / 8: field 17.1 / 16.6 / 22.6 ms,
-// force 52.8 / 52.2 / 58.9 (eight need 117 VGPRs); without the priority 16.7 and
-// 52.9.
-constexpr int kNearBlock = 4;
-
-template <int U>
-__device__ __forceinline__ void rsq_block(const float (&r2)[U], float (&ir)[U]) {
-  __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-  for (int k = 0; k < U; ++k) ir[k] = __builtin_amdgcn_rsqf(r2[k]);
-  __builtin_amdgcn_s_setprio(0);
-  __builtin_amdgcn_sched_barrier(0);
-}
-
-// MIXED: the block may hold pairs inside the smoothing support.
-template <int U, bool MIXED>
-__device__ __forceinline__ void field_block(const SrcRec *__restrict__ rec, float tx, float ty,
-                                            float tz, const FieldConsts &fc, const float4 *tab,
-                                            float (&a1)[3], float (&a2)[3]) {
-  float dx[U], dy[U], dz[U], r2[U], ir[U];
-#pragma unroll
-  for (int k = 0; k < U; ++k) {
-    dx[k] = tx - rec[k].x;
-    dy[k] = ty - rec[k].y;
-    dz[k] = tz - rec[k].z;
-    r2[k] = fmaf(dx[k], dx[k], fmaf(dy[k], dy[k], dz[k] * dz[k]));
-  }
-  rsq_block<U>(r2, ir);
-#pragma unroll
-  for (int k = 0; k < U; ++k) {
-    const float mx = rec[k].mx, my = rec[k].my, mz = rec[k].mz;
-    const float ir2 = ir[k] * ir[k];
-    float beta = ir2 * ir[k];
-    float alpha = beta * ir2;
-    if constexpr (MIXED)
-      if (r2[k] < fc.near2) field_near_coeffs_tab(tab, fc.tab_scale, r2[k], ir[k], alpha, beta);
-    const float dm = fmaf(dx[k], mx, fmaf(dy[k], my, dz[k] * mz));
-    const float s1 = dm * alpha;
-    a1[0] = fmaf(dx[k], s1, a1[0]);
-    a1[1] = fmaf(dy[k], s1, a1[1]);
-    a1[2] = fmaf(dz[k], s1, a1[2]);
-    a2[0] = fmaf(mx, beta, a2[0]);
-    a2[1] = fmaf(my, beta, a2[1]);
-    a2[2] = fmaf(mz, beta, a2[2]);
-  }
-}
-
-template <bool MIXED>
-__device__ __forceinline__ void field_range(const SrcRec *__restrict__ rec, int j0, int j1,
-                                            float tx, float ty, float tz, const FieldConsts &fc,
-                                            const float4 *tab, float (&a1)[3], float (&a2)[3]) {
-  int j = j0;
-#pragma unroll 1
-  for (; j + kNearBlock <= j1; j += kNearBlock)
-    field_block<kNearBlock, MIXED>(rec + j, tx, ty, tz, fc, tab, a1, a2);
-#pragma unroll 1
-  for (; j < j1; ++j) field_block<1, MIXED>(rec + j, tx, ty, tz, fc, tab, a1, a2);
-}
-
-// Targets [tb, te) of a leaf of cnt particles taken by the full-chunk path.
-template <int T>
-__device__ __forceinline__ void p2p_target_span(int cnt, int &tb, int &te) {
-  const int full = cnt & ~63, r = cnt & 63;
-  if (T == 64) {
-    tb = 0;
-    te = r > 32 ? cnt : full;
-  } else {
-    tb = full;
-    te = r <= 32 ? cnt : full;
-  }
-}
-
-constexpr int kLeafLists = 7;  // leaf shapes: full chunks (64) and remainders (32 .. 1)
-
-// Stream offsets of a leaf's near ranges, concatenated: pre[r] = total
-// length of ranges 0 .. r-1 (pre[nrange] = the stream's length), beg[r] =
-// first record of range r.  One wave.
-__device__ __forceinline__ void range_prefix(int *pre, int *beg, const int2 *__restrict__ rg,
-                                             int nrange, int lane) {
-  int carry = 0;
-  for (int c = 0; c < nrange; c += 64) {
-    const int r = c + lane;
-    int len = 0;
-    if (r < nrange) {
-      const int2 q = rg[r];
-      len = q.y - q.x;
-      beg[r] = q.x;
-    }
-    int incl = len;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int v = __shfl_up(incl, off, 64);
-      if (lane >= off) incl += v;
-    }
-    if (r < nrange) pre[r] = carry + incl - len;
-    carry += __shfl(incl, 63, 64);
-  }
-  if (lane == 0) pre[nrange] = carry;
-}
-
 // The range holding stream position i: the last r with pre[r] <= i (an
 // empty range shares its successor's offset, so "last" skips it).
 __device__ __forceinline__ int range_of(const int *pre, int nrange, int i) {
@@ -1611,84 +1422,27 @@ __device__ __forceinline__ int range_of(const int *pre, int nrange, int i) {
   return lo;
 }
 
-// Sum over the 64 lanes of a wave.
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
+// Leaf lists of the near field: the leaves with a head block and those with a tail
+// (head_count), as two entries per leaf (list 2 = none); a stable sort by list then
+// gives each in leaf (Morton) order.
+constexpr int kLeafLists = 2;
 
-// One lane's share of a leaf's near-source stream, in blocks: block i0
-// holds positions i0, i0 + 64, ..., i0 + 64 (kLaneBlock - 1) (consecutive
-// lanes read consecutive records), and the lane loads all of them before
-// evaluating any, so that kLaneBlock loads are in flight at once.  Two per
-// block and four targets per pass keep the fused kernels at 64 registers
-// or fewer (eight waves per SIMD for the full chunks), measured faster than
-// larger blocks or passes.  The loads
-// are issued without a branch (a load under a branch makes the compiler wait
-// for every outstanding load at its join): a position past the stream's end
-// re-reads the last record and becomes a zero moment 1e18 away, whose pair
-// terms are all exactly zero.
-constexpr int kLaneBlock = 2;
-struct LaneStream {
-  const float4 *__restrict__ rec4;
-  const int *pre;
-  const int *beg;
-  int total, nmix;
-  int lo, nxt, base;
-  float4 pa[kLaneBlock], pb[kLaneBlock];  // records of the block
-  bool mixed[kLaneBlock];  // their ranges may hold pairs inside the smoothing support
-  __device__ __forceinline__ void start(int lane, int nrange) {
-    lo = range_of(pre, nrange, min(lane, total - 1));
-    nxt = pre[lo + 1];
-    base = beg[lo] - pre[lo];
-  }
-  __device__ __forceinline__ void fetch(int i0) {
-#pragma unroll
-    for (int k = 0; k < kLaneBlock; ++k) {
-      const int i = i0 + 64 * k;
-      const int ic = min(i, total - 1);
-      while (nxt <= ic) {
-        ++lo;
-        nxt = pre[lo + 1];
-        base = beg[lo] - pre[lo];
-      }
-      const int64_t j = static_cast<int64_t>(base) + ic;
-      const float4 a = rec4[2 * j], m = rec4[2 * j + 1];
-      const bool live = i < total;
-      const float away = live ? 0.f : 1e18f, w = live ? 1.f : 0.f;
-      pa[k] = make_float4(a.x + away, a.y + away, a.z + away, 0.f);
-      pb[k] = make_float4(m.x * w, m.y * w, m.z * w, 0.f);
-      mixed[k] = live && lo < nmix;
-    }
-  }
-};
+// Particles of a leaf of cnt that belong to its head.
+__device__ __forceinline__ int head_count(int cnt) { return (cnt & 63) > 32 ? cnt : cnt & ~63; }
 
-// Leaf shapes for the near-field kernels.  List 0 holds every leaf with a
-// full chunk of 64 or a remainder of more than 32 (the one-target-per-lane
-// kernels); lists 1..6 hold the leaves whose remainder (cnt mod 64) is
-// 17..32, 9..16, 5..8, 3..4, 2 or 1 (the lanes-over-sources kernels, each
-// list with the pass size that fits it).  A leaf can be in list 0 and in one
-// of the others: they cover disjoint targets.  Two (list, leaf) entries per leaf (list kLeafLists =
-// none); a stable sort by list then gives every list in leaf (Morton) order.
 __global__ void classify_leaves_kernel(int nleaf, const int32_t *__restrict__ count,
                                        uint64_t *__restrict__ key, int32_t *__restrict__ leaf,
                                        int32_t *__restrict__ sizes) {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= nleaf) return;
-  const int c = count[b];
-  const int r = c & 63;
-  const int k0 = (c >= 64 || r > 32) ? 0 : kLeafLists;
-  const int k1 = (r == 0 || r > 32) ? kLeafLists
-                 : r > 16 ? 1 : r > 8 ? 2 : r > 4 ? 3 : r > 2 ? 4 : r > 1 ? 5 : 6;
-  key[2 * b] = static_cast<uint64_t>(k0);
-  key[2 * b + 1] = static_cast<uint64_t>(k1);
-  leaf[2 * b] = b;
-  leaf[2 * b + 1] = b;
-  // one atomic per wave and list instead of one per leaf
+  const int c = count[b], h = head_count(c);
+  const bool has[kLeafLists] = {h > 0, c > h};
 #pragma unroll
   for (int k = 0; k < kLeafLists; ++k) {
-    const uint64_t m = __ballot((k == 0 && k0 == 0) || k1 == k);
+    key[2 * b + k] = static_cast<uint64_t>(has[k] ? k : kLeafLists);
+    leaf[2 * b + k] = b;
+    // one atomic per wave and list instead of one per leaf
+    const uint64_t m = __ballot(has[k]);
     if (m != 0 && (threadIdx.x & 63) == __ffsll(static_cast<long long>(m)) - 1)
       atomicAdd(&sizes[k], __popcll(m));
   }
@@ -1699,7 +1453,7 @@ struct Text9 {
 };
 
 // L2P, force: far3[.][perm] = (far tensor + T_ext) . m (FP64;
-// add_far_kernel adds it to the near force).  One wave per leaf.
+// near_gather_kernel adds it to the near force).  One wave per leaf.
 template <int P, int KP>
 __global__ __launch_bounds__(64) void l2p_force_kernel(
     int nleaf, const int32_t *__restrict__ start, const int32_t *__restrict__ count,
@@ -1748,500 +1502,408 @@ __global__ __launch_bounds__(64) void l2p_force_kernel(
   }
 }
 
-// Force near-field sums v over a block of sources, and over one contiguous
-// source range.  NEAR: the range may hold pairs within 4h (fitted curves
-// below q = 4); otherwise every pair takes the far form, with no test.
-// The pair in the form with the far field's -5 folded away: with n5 = -5 n
-// and Rq = R / -5 (far: P ir^2; near: the table's second curve),
-//   e = Rq (d.m)(d.n5) + P (m.n) = R (d.m)(d.n) + P (m.n),
-// and the m-sums v[3 .. 5] collect P (d.n5) = -5 P (d.n): the caller scales
-// them by -1/5.  One multiply per pair fewer than R = -5 P ir^2.
-struct ForceTarget {
-  float x, y, z, nx, ny, nz, nx5, ny5, nz5;
-};
-template <int U, bool NEAR>
-__device__ __forceinline__ void force_block(const SrcRec *__restrict__ rec, const ForceTarget &t,
-                                            const HessConsts &hc, const float4 *tab,
-                                            float (&v)[7]) {
-  float dx[U], dy[U], dz[U], r2[U], ir[U];
-#pragma unroll
-  for (int k = 0; k < U; ++k) {
-    dx[k] = t.x - rec[k].x;
-    dy[k] = t.y - rec[k].y;
-    dz[k] = t.z - rec[k].z;
-    r2[k] = fmaf(dx[k], dx[k], fmaf(dy[k], dy[k], dz[k] * dz[k]));
-  }
-  rsq_block<U>(r2, ir);
-#pragma unroll
-  for (int k = 0; k < U; ++k) {
-    const float mx = rec[k].mx, my = rec[k].my, mz = rec[k].mz;
-    const float dm = fmaf(dx[k], mx, fmaf(dy[k], my, dz[k] * mz));
-    const float dn5 = fmaf(dx[k], t.nx5, fmaf(dy[k], t.ny5, dz[k] * t.nz5));
-    const float mn = fmaf(mx, t.nx, fmaf(my, t.ny, mz * t.nz));
-    float Pc, e;
-    if constexpr (NEAR) {
-      // Both curves default to their far form r^-4 (P = r^-5, R / -5 = r^-7)
-      // and the table replaces them within 4h; one scaling serves both.
-      // The clamp keeps a pair at d = 0 finite (its terms vanish with d).
-      const float irc = __builtin_amdgcn_fmed3f(ir[k], 0.f, 1e12f);
-      const float ir2 = irc * irc;
-      float c1 = ir2 * ir2, dq = c1;
-      if (!(r2[k] > hc.near2)) hess_near_curves_tab(tab, hc.tab_scale, r2[k], irc, c1, dq);
-      Pc = c1 * irc;
-      e = fmaf(dq * (ir2 * irc), dm * dn5, Pc * mn);
-    } else {
-      const float ir2 = ir[k] * ir[k];
-      Pc = ir2 * ir2 * ir[k];
-      e = Pc * fmaf(dm * ir2, dn5, mn);  // R / -5 = P ir^2 factored out
-    }
-    const float f5 = Pc * dn5;
-    v[0] = fmaf(dx[k], e, v[0]);
-    v[1] = fmaf(dy[k], e, v[1]);
-    v[2] = fmaf(dz[k], e, v[2]);
-    v[3] = fmaf(mx, f5, v[3]);
-    v[4] = fmaf(my, f5, v[4]);
-    v[5] = fmaf(mz, f5, v[5]);
-    v[6] = fmaf(Pc, dm, v[6]);
-  }
-}
-
-template <bool NEAR>
-__device__ __forceinline__ void force_range(const SrcRec *__restrict__ rec, int j0, int j1,
-                                            const ForceTarget &t, const HessConsts &hc,
-                                            const float4 *tab, float (&v)[7]) {
-  int j = j0;
-#pragma unroll 1
-  for (; j + kNearBlock <= j1; j += kNearBlock)
-    force_block<kNearBlock, NEAR>(rec + j, t, hc, tab, v);
-#pragma unroll 1
-  for (; j < j1; ++j) force_block<1, NEAR>(rec + j, t, hc, tab, v);
-}
-
 // ---------------------------------------------------------------------------
-// P2P: the near field of every leaf, in one launch per product over two leaf
-// lists.
-//  * Full chunks (near_*_full): one target per lane, every lane walking all
-//    sources (scalar loads), over the leaf's chunks of 64 targets -- and over
-//    its remainder too when that holds more than 32.
-//  * Remainders (near_*_remainder): the at most 32 targets left after a
-//    leaf's full chunks (a sparse leaf, or the tail of a leaf of 65..96
-//    particles).  One wave per leaf, lanes over sources: the leaf's near
-//    ranges, concatenated, form one stream; lane l takes positions l, l +
-//    64, ... (LaneStream) and evaluates each of its sources against R
-//    remainder targets per pass.  The targets are wave-uniform (scalar
-//    loads; R = 4 keeps them in scalar registers), every lane has work
-//    whatever the remainder's size, and the lanes' partial sums are added
-//    across the wave in FP64.
-// Each XCD takes its share of the remainders before its share of the full
-// chunks (xcd_two_lists): a remainder wave is long (its whole stream, one
-// wave) but there are few, and started first they finish under the full
-// chunks' work instead of trailing a launch of their own.  Ranges of the
-// leaf's mixed slots (nr.x, first) may hold pairs inside the smoothing
-// support.
+// Near field with every unordered pair of leaf blocks evaluated once
+// (mf_pair_once.hpp).
 //
-// A workgroup of W waves takes a leaf: each wave an equal part of the leaf's
-// mixed and of its far stream, the waves' FP64 sums added in wave order
-// (combine_waves).  W = 1 where the leaves alone fill the chip; with few leaves
-// the one-wave form is a handful of waves per SIMD waiting for their scalar
-// loads (near_waves holds the rule and its measurements).
+// A leaf has up to two blocks: the head, its chunks of 64 particles (and a
+// remainder above 32), and the tail, a remainder of at most 32.  A workgroup
+// holds a block's targets in registers, up to 64 a pass, walks the block's own
+// records (directed) and then its stream in tiles of 64; the stream records' sums
+// over the targets go to a buffer with one place per (block, stream position).
+// The stream of a head is the near leaves at lexicographically positive offsets,
+// whole, and the tails of the others and of its own leaf; the stream of a tail is
+// the tails at positive offsets: a pair of a full block and a sparse one has the
+// full one in registers, whose lanes it fills.  near_gather_kernel adds
+// to each particle's own sum what the other blocks left for it, in slot order, so
+// results are deterministic.  W waves share a block: wave w takes every W-th tile.
+//
+// The VALU bounds it: 64 pairs of an interior leaf take 96 (field) and 130 (force) cycles,
+// as the pair loop alone does, for both directions.  Directed kernels (one target a lane,
+// sources through scalar loads; lanes over sources for the tails) took 67 and 99 to 108
+// per direction.  Launches, directed -> pair-once (one box): 131,072 particles field 0.336 ->
+// 0.263 ms, force 0.959 -> 0.747; 1,153,433 in leaves of 1 to 80 2.46 -> 1.76 and 7.36 -> 5.06;
+// 8.4 million 16.6 -> 13.5 and 51.3 -> 39.6.  The places cost 12 bytes a (block, stream
+// record) written and read, 0.87 and 1.7 ms of gather at 8.4 million.  With leaves as
+// blocks, sparse ones in registers met whole streams with 6 targets of 16 lanes: 3.5
+// and 9.5 ms at 1,153,433.
 
-// Workgroup -> position in one of two leaf lists (remainders first, then
-// full chunks), each XCD (round-robin dispatch over 8) walking a contiguous
-// range of each list: neighbouring leaves share most of their near sources,
-// which then hit in that XCD's L2.  Returns -1 for the padding.
-__device__ __forceinline__ int xcd_two_lists(int nrem, int nfull, bool &rem) {
-  const int prem = (nrem + 7) / 8, pfull = (nfull + 7) / 8;
-  const int x = static_cast<int>(blockIdx.x % 8), k = static_cast<int>(blockIdx.x / 8);
-  rem = k < prem;
-  const int pos = rem ? x * prem + k : x * pfull + (k - prem);
-  return pos < (rem ? nrem : nfull) ? pos : -1;
-}
-
-// Remainder targets [tb, te) of a leaf of cnt particles (empty when the
-// full-chunk path takes the remainder).
-__device__ __forceinline__ void remainder_span(int cnt, int &tb, int &te) {
-  tb = cnt & ~63;
-  te = (cnt & 63) <= 32 ? cnt : tb;
-}
-
-struct FieldOut {
-  int accumulate;
-  float hc0, hc1, hc2;
-  float *__restrict__ ox;
-  float *__restrict__ oy;
-  float *__restrict__ oz;
-  __device__ __forceinline__ void put(int o, double g0, double g1, double g2) const {
-    const double cf = 1.0 / (4.0 * kPi);
-    const double b0 = accumulate ? static_cast<double>(ox[o]) : hc0;
-    const double b1 = accumulate ? static_cast<double>(oy[o]) : hc1;
-    const double b2 = accumulate ? static_cast<double>(oz[o]) : hc2;
-    ox[o] = static_cast<float>(b0 + cf * g0);
-    oy[o] = static_cast<float>(b1 + cf * g1);
-    oz[o] = static_cast<float>(b2 + cf * g2);
-  }
+// Block 2 b is the head of leaf b, 2 b + 1 its tail; its stream starts at place 16 off[block].
+// The places are walked in passes: this one has the blocks with lo <= off < hi, and the
+// buffer starts at place 16 lo.
+struct OnceNear {
+  const int32_t *near;  // [nleaf][nslot]
+  const int2 *sym;      // [nslot]: slot of the negative offset, sign of this one
+  const int32_t *pre;   // [2 nleaf][nslot + 1]: stream position of each slot; length
+  const int32_t *off;   // [2 nleaf]
+  const int32_t *heads, *tails;  // leaves that have one
+  int nheads, ntails;
+  int nmix;             // slots [0, nmix) may hold smoothed pairs
+  int lo, hi;
+  int64_t len;          // places of the buffer
+  float *sums;          // [3][len]
 };
 
-struct ForceOut {
-  int accumulate;
-  float *__restrict__ fx;
-  float *__restrict__ fy;
-  float *__restrict__ fz;
-  __device__ __forceinline__ void put(int o, double f0, double f1, double f2) const {
-    const double sfac = 3.0 * kMu0 / (4.0 * kPi);
-    fx[o] = static_cast<float>((accumulate ? static_cast<double>(fx[o]) : 0.0) + sfac * f0);
-    fy[o] = static_cast<float>((accumulate ? static_cast<double>(fy[o]) : 0.0) + sfac * f1);
-    fz[o] = static_cast<float>((accumulate ? static_cast<double>(fz[o]) : 0.0) + sfac * f2);
-  }
-};
+constexpr int kOnceFlush = 8;  // tiles between FP64 accumulations
 
-// Per-lane sums of the workgroup's waves into wave 0, in wave order.  xch: LDS
-// of (W - 1) NC 64 doubles; every wave calls it.
-template <int W, int NC>
-__device__ __forceinline__ void combine_waves(double (&v)[NC], double *xch, int wave, int lane) {
-  if constexpr (W > 1) {
-    if (wave > 0) {
+// The part of near leaf (sign of its offset, cnt) in a block's stream: [first, end).
+__device__ __forceinline__ int2 stream_piece(bool tail, int sign, int cnt) {
+  const int h = head_count(cnt);
+  if (tail) return sign > 0 ? make_int2(h, cnt) : make_int2(0, 0);
+  return sign > 0 ? make_int2(0, cnt) : make_int2(h, cnt);
+}
+
+// Stream positions of one block per wave, its length in units of 16 places and the
+// longest.
+template <int NS>
+__global__ __launch_bounds__(256) void once_stream_kernel(int nleaf, const int32_t *__restrict__ near,
+                                                          const int2 *__restrict__ sym,
+                                                          const int32_t *__restrict__ count,
+                                                          int32_t *__restrict__ pre,
+                                                          int32_t *__restrict__ units,
+                                                          int32_t *__restrict__ longest) {
+  const int id = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (id >= 2 * nleaf) return;
+  const int b = id >> 1, cnt = count[b], h = head_count(cnt);
+  const bool tail = (id & 1) != 0, empty = (tail ? cnt - h : h) == 0;
+  int32_t *__restrict__ out = pre + static_cast<int64_t>(id) * (NS + 1);
+  int carry = 0;
 #pragma unroll
-      for (int a = 0; a < NC; ++a) xch[((wave - 1) * NC + a) * 64 + lane] = v[a];
+  for (int k0 = 0; k0 < NS; k0 += 64) {
+    const int k = k0 + lane;
+    int c = 0;
+    if (k < NS && !empty) {
+      const int nb = near[static_cast<int64_t>(b) * NS + k];
+      if (nb >= 0) {
+        const int2 p = stream_piece(tail, sym[k].y, count[nb]);
+        c = p.y - p.x;
+      }
+    }
+    int incl = c;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += v;
+    }
+    if (k < NS) out[k] = carry + incl - c;
+    carry += __shfl(incl, 63, 64);
+  }
+  if (lane == 0) {
+    out[NS] = carry;
+    units[id] = (carry + 15) / 16;
+    if (carry > 0) atomicMax(longest, (carry + 15) / 16);
+  }
+}
+
+// One pass over a block's stream for its targets [t0, t0 + 16 TPT).
+template <class Pairs, int TPT, int W, int NS>
+__device__ __forceinline__ void once_pass(Pairs &prs, const float4 *__restrict__ rec4, int pad,
+                                          int s0, int cnt, int t0, const int *s_pre,
+                                          const int *s_rec, int tm, SelfTile *st, double *acc,
+                                          int wave, int lane, bool again,
+                                          float *__restrict__ sums, int64_t len) {
+  const int c = lane & 15, q = lane >> 4;
+  // the last pass's lanes past the block's end hold the padding record
+#pragma unroll
+  for (int k = 0; k < TPT; ++k) {
+    const int t = t0 + 16 * k + c;
+    const int64_t i = t < cnt ? s0 + t : pad;
+    const float4 p = rec4[2 * i], m = rec4[2 * i + 1];
+    prs.tx[k] = p.x;
+    prs.ty[k] = p.y;
+    prs.tz[k] = p.z;
+    prs.nx[k] = m.x;
+    prs.ny[k] = m.y;
+    prs.nz[k] = m.z;
+  }
+  prs.clear();
+#pragma unroll
+  for (int a = 0; a < 3; ++a) acc[a * 64] = 0.0;
+  // lane group k keeps the sums of targets 16 k + c
+  auto flush = [&]() {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      double v = 0.0;
+#pragma unroll
+      for (int k = 0; k < TPT; ++k) {
+        double x = prs.sum(k, a);
+        x += __shfl_xor(x, 16, 64);
+        x += __shfl_xor(x, 32, 64);
+        v = q == k ? x : v;
+      }
+      acc[a * 64] += v;
+    }
+    prs.clear();
+  };
+  const int nown = (cnt + 63) / 64, tot = s_pre[NS], ntile = nown + (tot + 63) / 64;
+  auto stage = [&](int tile, SelfTile &to) {
+    int64_t i = pad;
+    if (tile < nown) {
+      const int j = tile * 64 + lane;
+      i = j < cnt ? s0 + j : pad;
+    } else {
+      const int p = (tile - nown) * 64 + lane;
+      if (p < tot) i = s_rec[range_of(s_pre, NS, p)] + p;
+    }
+    copy16_to_lds(rec4 + 2 * i, to.pos);
+    copy16_to_lds(rec4 + 2 * i + 1, to.mom);
+  };
+  int buf = 0, since = 0;
+  bool stored = false;
+  if (wave < ntile) stage(wave, st[0]);
+  for (int tile = wave; tile < ntile; tile += W, buf ^= 1) {
+    // this tile's copy; the last tile's three stores, issued after it, may be under way
+    if (stored)
+      wait_vm<3>();
+    else
+      wait_vm<0>();
+    __builtin_amdgcn_wave_barrier();
+    if (tile + W < ntile) stage(tile + W, st[buf ^ 1]);
+    float jc[3] = {0.f, 0.f, 0.f};
+    if (tile < nown) {
+      prs.template tile<true, false>(st[buf], c, q, jc);
+    } else {
+      const int p0 = (tile - nown) * 64, p = p0 + lane;  // p0 < tot: at least lane 0 stores
+      stored = true;
+      if (p0 < tm)
+        prs.template tile<true, true>(st[buf], c, q, jc);
+      else
+        prs.template tile<false, true>(st[buf], c, q, jc);
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        float v = row_next(jc[a]);
+        if (p < tot) {
+          float *o = sums + a * len + p;
+          if (again) v += *o;  // an earlier pass of this block, by this wave
+          *o = v;
+        }
+      }
+    }
+    if (++since == kOnceFlush) {
+      flush();
+      since = 0;
+    }
+  }
+  if (since) flush();
+}
+
+template <template <int> class Pairs, class Consts, int NTAB, int NS, int W>
+__device__ __forceinline__ void once_leaf(const int32_t *__restrict__ start,
+                                          const int32_t *__restrict__ count,
+                                          const SrcRec *__restrict__ rec, int64_t n,
+                                          const OnceNear &nn, const Consts &consts,
+                                          const float4 *__restrict__ tab,
+                                          double *__restrict__ near3, SysMask mask) {
+  // Each XCD (round-robin dispatch over 8) walks a contiguous range of the heads and
+  // then of the tails, whose streams are short.  A pass of several has a contiguous range
+  // of all blocks, which every XCD has to share.
+  const int ph = (nn.nheads + 7) / 8, pt = (nn.ntails + 7) / 8;
+  const int x = static_cast<int>(blockIdx.x % 8), k8 = static_cast<int>(blockIdx.x / 8);
+  const bool tail = k8 >= ph, one = nn.lo == 0 && nn.hi == INT32_MAX;
+  const int k = tail ? k8 - ph : k8;
+  const int pos = one ? x * (tail ? pt : ph) + k : 8 * k + x;
+  if (pos >= (tail ? nn.ntails : nn.nheads)) return;
+  const int b = tail ? nn.tails[pos] : nn.heads[pos], id = 2 * b + (tail ? 1 : 0);
+  const int all = count[b], h = head_count(all);
+  const int s0 = start[b] + (tail ? h : 0), cnt = tail ? all - h : h;
+  // uniform over the workgroup, before the barrier
+  const int off = nn.off[id];
+  if (off < nn.lo || off >= nn.hi || sys_skip(mask, b)) return;
+  __shared__ float4 s_tab[2 * NTAB];
+  __shared__ int s_pre[NS + 1], s_rec[NS];
+  __shared__ SelfTile st[W][2];
+  __shared__ double s_acc[W][3][64];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = W > 1 ? __builtin_amdgcn_readfirstlane(tid >> 6) : 0;
+  for (int i = tid; i < 2 * NTAB; i += 64 * W) s_tab[i] = tab[i];
+  for (int k = tid; k <= NS; k += 64 * W) {
+    const int p = nn.pre[static_cast<int64_t>(id) * (NS + 1) + k];
+    s_pre[k] = p;
+    if (k < NS) {
+      const int nb = nn.near[static_cast<int64_t>(b) * NS + k];
+      s_rec[k] = nb >= 0 ? start[nb] + stream_piece(tail, nn.sym[k].y, count[nb]).x - p : 0;
+    }
+  }
+  __syncthreads();
+  const int tm = s_pre[nn.nmix];
+  const float4 *__restrict__ rec4 = reinterpret_cast<const float4 *>(rec);
+  float *sums = nn.sums + 16 * static_cast<int64_t>(off - nn.lo);
+  for (int t0 = 0; t0 < cnt; t0 += 64) {
+    const int m = min(cnt - t0, 64);
+    auto pass = [&](auto tpt) {
+      constexpr int T = decltype(tpt)::value;
+      Pairs<T> prs(consts, s_tab);
+      once_pass<Pairs<T>, T, W, NS>(prs, rec4, static_cast<int>(n), s0, cnt, t0, s_pre, s_rec,
+                                       tm, st[wave], &s_acc[wave][0][lane], wave, lane, t0 > 0,
+                                       sums, nn.len);
+    };
+    if (m > 48) pass(std::integral_constant<int, 4>{});
+    else if (m > 32) pass(std::integral_constant<int, 3>{});
+    else if (m > 16) pass(std::integral_constant<int, 2>{});
+    else pass(std::integral_constant<int, 1>{});
+    if (W > 1) __syncthreads();
+    if (wave == 0 && lane < m) {
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        double v = s_acc[0][a][lane];
+#pragma unroll
+        for (int k = 1; k < W; ++k) v += s_acc[k][a][lane];
+        near3[a * n + s0 + t0 + lane] = v;
+      }
+    }
+    if (W > 1) __syncthreads();  // s_acc is written again by the next pass
+  }
+}
+
+template <int W>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) void near_field_once_kernel(
+    const int32_t *__restrict__ start, const int32_t *__restrict__ count,
+    const SrcRec *__restrict__ rec, int64_t n, OnceNear nn, FieldConsts fc,
+    const float4 *__restrict__ tab, double *__restrict__ near3, SysMask mask) {
+  once_leaf<FieldSelf, FieldConsts, kFieldTabEntries, kNearF, W>(start, count, rec, n, nn,
+                                                                 fc, tab, near3, mask);
+}
+
+template <int W>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) void near_force_once_kernel(
+    const int32_t *__restrict__ start, const int32_t *__restrict__ count,
+    const SrcRec *__restrict__ rec, int64_t n, OnceNear nn, HessConsts hc,
+    const float4 *__restrict__ tab, double *__restrict__ near3, SysMask mask) {
+  once_leaf<ForceSelf, HessConsts, kHessTabEntries, kNearH, W>(start, count, rec, n, nn, hc,
+                                                               tab, near3, mask);
+}
+
+// Where the other blocks leave the sums of a leaf's particles: places[leaf][..] =
+// {off of the source block, stream position of the leaf's particle 0}, first the nw
+// blocks that meet the whole leaf, then the nt that meet its tail only, both in slot order;
+// np[leaf] = {nw, nt}.  One thread per slot.
+template <int NS>
+constexpr int kPlaces = (NS - 1) / 2 + NS;  // heads at NS - 1 offsets and their own, tails at half
+template <int NS>
+__global__ __launch_bounds__(256) void near_places_kernel(const int32_t *__restrict__ near,
+                                                          const int2 *__restrict__ sym,
+                                                          const int32_t *__restrict__ count,
+                                                          const int32_t *__restrict__ pre,
+                                                          const int32_t *__restrict__ off,
+                                                          int2 *__restrict__ places,
+                                                          int2 *__restrict__ np) {
+  static_assert(NS <= 256, "one thread per slot");
+  const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int h = head_count(count[b]);
+  __shared__ int s_n[4][2];
+  bool whole = false, found[2] = {false, false};
+  int2 at[2] = {};
+  if (tid < NS) {
+    const int nb = near[static_cast<int64_t>(b) * NS + tid];
+    const int k = sym[tid].x;  // this leaf's slot, seen from the near leaf
+    if (nb >= 0) {
+      whole = sym[k].y > 0;
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const int id = 2 * nb + t;
+        const int32_t *p = pre + static_cast<int64_t>(id) * (NS + 1) + k;
+        found[t] = p[1] > p[0];
+        at[t] = make_int2(off[id], p[0] - (t == 0 && whole ? 0 : h));
+      }
+    }
+  }
+  const uint64_t below = (1ULL << lane) - 1ULL;
+  const uint64_t mw = __ballot(found[0] && whole), m0 = __ballot(found[0] && !whole),
+                 m1 = __ballot(found[1]);
+  if (lane == 0) {
+    s_n[w][0] = __popcll(mw);
+    s_n[w][1] = __popcll(m0) + __popcll(m1);
+  }
+  __syncthreads();
+  int nw = 0, nt = 0, aw = 0, at0 = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    aw = k == w ? nw : aw;
+    at0 = k == w ? nt : at0;
+    nw += s_n[k][0];
+    nt += s_n[k][1];
+  }
+  int2 *__restrict__ out = places + static_cast<int64_t>(b) * kPlaces<NS>;
+  if (found[0]) {
+    if (whole)
+      out[aw + __popcll(mw & below)] = at[0];
+    else
+      out[nw + at0 + __popcll(m0 & below)] = at[0];
+  }
+  if (found[1]) out[nw + at0 + __popcll(m0) + __popcll(m1 & below)] = at[1];
+  if (tid == 0) np[b] = make_int2(nw, nt);
+}
+
+// out[perm] = base + fac (own sum + what the other blocks left) + far, in FP64 up to
+// the one rounding; in a pass before the last one the sums so far go to rest3.  A workgroup takes a leaf: rows of 64, 32 or 16 lanes by the leaf's
+// size, a lane a particle, the 4, 8 or 16 rows each every 4th, 8th or 16th source block.
+template <int NS>
+__global__ __launch_bounds__(256) void near_gather_kernel(
+    const int32_t *__restrict__ start, const int32_t *__restrict__ count,
+    const int32_t *__restrict__ perm, int64_t n, OnceNear nn, const int2 *__restrict__ places,
+    const int2 *__restrict__ np, int pass, int passes, double *__restrict__ rest3,
+    const double *__restrict__ near3, const double *__restrict__ far3, double fac, float b0, float b1, float b2,
+    float *__restrict__ ox, float *__restrict__ oy, float *__restrict__ oz, SysMask mask) {
+  const int b = blockIdx.x;
+  if (sys_skip(mask, b)) return;  // uniform over the workgroup, before the barrier
+  __shared__ int s_at[kPlaces<NS>];
+  __shared__ double sh[3][256];
+  const int tid = threadIdx.x;
+  const int s0 = start[b], cnt = count[b], h = head_count(cnt);
+  const int2 m = np[b];
+  constexpr int kElsewhere = INT32_MIN;  // another pass's
+  for (int k = tid; k < m.x + m.y; k += 256) {
+    const int2 p = places[static_cast<int64_t>(b) * kPlaces<NS> + k];
+    s_at[k] = p.x >= nn.lo && p.x < nn.hi ? 16 * (p.x - nn.lo) + p.y : kElsewhere;
+  }
+  __syncthreads();
+  const int wide = cnt > 32 ? 64 : cnt > 16 ? 32 : 16, rows = 256 / wide;
+  const int c = tid & (wide - 1), row = tid / wide;
+  for (int t0 = 0; t0 < cnt; t0 += wide) {
+    const int t = t0 + c;
+    const bool live = t < cnt;
+    double v[3] = {0.0, 0.0, 0.0};
+    auto add = [&](int k) {
+      if (s_at[k] == kElsewhere) return;
+      const float *p = nn.sums + (s_at[k] + t);
+      v[0] += static_cast<double>(p[0]);
+      v[1] += static_cast<double>(p[nn.len]);
+      v[2] += static_cast<double>(p[2 * nn.len]);
+    };
+    if (live) {
+#pragma unroll 4
+      for (int k = row; k < m.x; k += rows) add(k);
+    }
+    if (live && t >= h) {
+#pragma unroll 4
+      for (int k = row; k < m.y; k += rows) add(m.x + k);
+    }
+#pragma unroll
+    for (int a = 0; a < 3; ++a) sh[a][tid] = v[a];
+    __syncthreads();
+    if (row == 0 && live) {
+      const int o = perm[s0 + t];
+      float *const out[3] = {ox, oy, oz};
+      const float hc[3] = {b0, b1, b2};
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        const int64_t i = a * n + s0 + t;
+        double g = pass > 0 ? rest3[i] : 0.0;
+        for (int k = 0; k < rows; ++k) g += sh[a][k * wide + c];
+        if (pass + 1 < passes) {
+          rest3[i] = g;
+          continue;
+        }
+        g += near3[i];
+        out[a][o] = static_cast<float>(static_cast<double>(hc[a]) + fac * g +
+                                       (far3 ? far3[a * n + o] : 0.0));
+      }
     }
     __syncthreads();
-    if (wave == 0) {
-#pragma unroll
-      for (int k = 0; k < W - 1; ++k)
-#pragma unroll
-        for (int a = 0; a < NC; ++a) v[a] += xch[(k * NC + a) * 64 + lane];
-    }
-    __syncthreads();  // xch is written again by the next pass
   }
 }
 
-// Calls piece(j0, j1) for the records of positions [i0, i1) of the leaf's near
-// stream (range_prefix), one contiguous run at a time, all values uniform.
-template <class Piece>
-__device__ __forceinline__ void stream_pieces(const int *pre, const int *beg, int nrange, int i0,
-                                              int i1, const Piece &piece) {
-  if (i0 >= i1) return;
-  int r = __builtin_amdgcn_readfirstlane(range_of(pre, nrange, i0));
-  for (int i = i0; i < i1; ++r) {
-    const int p0 = __builtin_amdgcn_readfirstlane(pre[r]);
-    const int e = min(__builtin_amdgcn_readfirstlane(pre[r + 1]), i1);
-    const int b = __builtin_amdgcn_readfirstlane(beg[r]) - p0;
-    piece(b + i, b + e);
-    i = max(i, e);
-  }
-}
-
-// Wave w's part of positions [lo, hi).
-template <int W>
-__device__ __forceinline__ void wave_part(int lo, int hi, int w, int &i0, int &i1) {
-  const int len = hi - lo;
-  i0 = lo + static_cast<int>(static_cast<int64_t>(len) * w / W);
-  i1 = lo + static_cast<int>(static_cast<int64_t>(len) * (w + 1) / W);
-}
-
-template <int W>
-__device__ __forceinline__ void near_field_full(const SrcRec *__restrict__ rec,
-                                                const int32_t *__restrict__ perm, int s0, int cnt,
-                                                const int2 *__restrict__ rg, int2 nrb,
-                                                const int *pre, const int *beg, double *xch,
-                                                const FieldConsts &fc, const float4 *s_ftab,
-                                                int wave, int lane, const FieldOut &out) {
-  int tb, te;
-  p2p_target_span<64>(cnt, tb, te);
-  for (int t0 = tb; t0 < te; t0 += 64) {
-    const int t = t0 + lane;
-    const SrcRec me = rec[s0 + (t < te ? t : te - 1)];
-    const float tx = me.x, ty = me.y, tz = me.z;
-    double acc[3] = {0.0, 0.0, 0.0};
-    auto piece = [&](int j0, int j1, bool mixed) {
-      float a1[3] = {0.f, 0.f, 0.f}, a2[3] = {0.f, 0.f, 0.f};
-      if (mixed)
-        field_range<true>(rec, j0, j1, tx, ty, tz, fc, s_ftab, a1, a2);
-      else
-        field_range<false>(rec, j0, j1, tx, ty, tz, fc, s_ftab, a1, a2);
-#pragma unroll
-      for (int a = 0; a < 3; ++a)
-        acc[a] += 3.0 * static_cast<double>(a1[a]) - static_cast<double>(a2[a]);
-    };
-    const int nrange = nrb.x + nrb.y;
-    if constexpr (W == 1) {
-      for (int r = 0; r < nrange; ++r) {
-        const int2 q = rg[r];
-        piece(q.x, q.y, r < nrb.x);
-      }
-    } else {
-      const int tm = pre[nrb.x], tot = pre[nrange];
-      int i0, i1;
-      wave_part<W>(0, tm, wave, i0, i1);
-      stream_pieces(pre, beg, nrange, i0, i1, [&](int j0, int j1) { piece(j0, j1, true); });
-      wave_part<W>(tm, tot, wave, i0, i1);
-      stream_pieces(pre, beg, nrange, i0, i1, [&](int j0, int j1) { piece(j0, j1, false); });
-    }
-    combine_waves<W>(acc, xch, wave, lane);
-    if (wave == 0 && t < te) out.put(perm[s0 + t], acc[0], acc[1], acc[2]);
-  }
-}
-
-template <int R, int W>
-__device__ __forceinline__ void near_field_remainder(const SrcRec *__restrict__ rec,
-                                                     const int32_t *__restrict__ perm, int s0,
-                                                     int cnt, const int *s_pre, const int *s_beg,
-                                                     int nrange, int nmix, double *xch,
-                                                     const FieldConsts &fc, const float4 *s_ftab,
-                                                     int wave, int lane, const FieldOut &out) {
-  int tb, te;
-  remainder_span(cnt, tb, te);
-  for (int t0 = tb; t0 < te; t0 += R) {
-    const int nt = min(R, te - t0);  // uniform
-    float tx[R], ty[R], tz[R], gx[R], gy[R], gz[R];
-#pragma unroll
-    for (int t = 0; t < R; ++t) {
-      const SrcRec me = rec[s0 + t0 + min(t, nt - 1)];
-      tx[t] = me.x;
-      ty[t] = me.y;
-      tz[t] = me.z;
-      gx[t] = gy[t] = gz[t] = 0.f;
-    }
-    LaneStream st{reinterpret_cast<const float4 *>(rec), s_pre, s_beg, s_pre[nrange], nmix};
-    // the waves take blocks of 64 kLaneBlock positions in turn
-    const int first = wave * 64 * kLaneBlock + lane;
-    st.start(first, nrange);
-    for (int i0 = first; i0 < st.total; i0 += W * 64 * kLaneBlock) {
-      st.fetch(i0);
-#pragma unroll
-      for (int k = 0; k < kLaneBlock; ++k) {
-        const float4 pa = st.pa[k], pb = st.pb[k];
-        const bool mixed = st.mixed[k];
-        const float nmx = -pb.x, nmy = -pb.y, nmz = -pb.z;
-#pragma unroll
-        for (int t = 0; t < R; ++t) {
-          if (t < nt) {
-            const float dx = tx[t] - pa.x, dy = ty[t] - pa.y, dz = tz[t] - pa.z;
-            const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-            const float ir = __builtin_amdgcn_rsqf(r2);
-            const float ir2 = ir * ir;
-            float beta = ir2 * ir;
-            float alpha = beta * ir2;
-            if (mixed && r2 < fc.near2)
-              field_near_coeffs_tab(s_ftab, fc.tab_scale, r2, ir, alpha, beta);
-            // g += 3 (d . m) alpha d - beta m
-            const float s1 = 3.f * fmaf(dx, pb.x, fmaf(dy, pb.y, dz * pb.z)) * alpha;
-            gx[t] = fmaf(dx, s1, fmaf(nmx, beta, gx[t]));
-            gy[t] = fmaf(dy, s1, fmaf(nmy, beta, gy[t]));
-            gz[t] = fmaf(dz, s1, fmaf(nmz, beta, gz[t]));
-          }
-        }
-      }
-    }
-    // lane t keeps target t0 + t
-    double g[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-    for (int t = 0; t < R; ++t) {
-      if (t < nt) {
-        const double sx = wave_sum(static_cast<double>(gx[t]));
-        const double sy = wave_sum(static_cast<double>(gy[t]));
-        const double sz = wave_sum(static_cast<double>(gz[t]));
-        g[0] = lane == t ? sx : g[0];
-        g[1] = lane == t ? sy : g[1];
-        g[2] = lane == t ? sz : g[2];
-      }
-    }
-    combine_waves<W>(g, xch, wave, lane);
-    if (wave == 0 && lane < nt) out.put(perm[s0 + t0 + lane], g[0], g[1], g[2]);
-  }
-}
-
-// P2P, field: out[perm] (+)= sum over each leaf's near ranges; accumulate = 0
-// writes H_const + near (trees without a far field).  full / remain: the two
-// leaf lists (see above).
-template <int W>
-__global__ __launch_bounds__(64 * W) void p2p_field_kernel(
-    const int32_t *__restrict__ full, int nfull, const int32_t *__restrict__ remain, int nrem,
-    const int32_t *__restrict__ start, const int32_t *__restrict__ count,
-    const SrcRec *__restrict__ rec, const int32_t *__restrict__ perm,
-    const int2 *__restrict__ rng, const int2 *__restrict__ nr, int nslot, FieldConsts fc,
-    const float4 *__restrict__ ftab, FieldOut out, SysMask mask) {
-  bool rem;
-  const int li = xcd_two_lists(nrem, nfull, rem);
-  if (li < 0) return;
-  const int b = rem ? remain[li] : full[li];
-  if (sys_skip(mask, b)) return;  // uniform over the workgroup, before the barrier
-  const int lane = threadIdx.x & 63;
-  const int wave = W > 1 ? __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)) : 0;
-  // near-pair coefficients from the table (2 KB of LDS); the stream's offsets
-  // (remainders, and the waves' parts); the waves' sums
-  __shared__ float4 s_ftab[2 * kFieldTabEntries];
-  __shared__ int s_pre[kNearF + 1], s_beg[kNearF];
-  __shared__ double xch[(W > 1 ? W - 1 : 1) * (W > 1 ? 3 * 64 : 1)];
-  for (int i = threadIdx.x; i < 2 * kFieldTabEntries; i += 64 * W) s_ftab[i] = ftab[i];
-  const int2 nrb = nr[b];
-  const int2 *__restrict__ rg = rng + static_cast<int64_t>(b) * nslot;
-  if ((rem || W > 1) && wave == 0) range_prefix(s_pre, s_beg, rg, nrb.x + nrb.y, lane);
-  __syncthreads();
-  if (rem)
-    near_field_remainder<4, W>(rec, perm, start[b], count[b], s_pre, s_beg, nrb.x + nrb.y, nrb.x,
-                               xch, fc, s_ftab, wave, lane, out);
-  else
-    near_field_full<W>(rec, perm, start[b], count[b], rg, nrb, s_pre, s_beg, xch, fc, s_ftab, wave,
-                       lane, out);
-}
-
-template <int W>
-__device__ __forceinline__ void near_force_full(const SrcRec *__restrict__ rec,
-                                                const int32_t *__restrict__ perm, int s0, int cnt,
-                                                const int2 *__restrict__ rg, int2 nrb,
-                                                const int *pre, const int *beg, double *xch,
-                                                const HessConsts &hc, const float4 *tab, int wave,
-                                                int lane, const ForceOut &out) {
-  int tb, te;
-  p2p_target_span<64>(cnt, tb, te);
-  const int nrange = nrb.x + nrb.y;
-  for (int t0 = tb; t0 < te; t0 += 64) {
-    const int t = t0 + lane;
-    const SrcRec me = rec[s0 + (t < te ? t : te - 1)];
-    const float nx = me.mx, ny = me.my, nz = me.mz;
-    const ForceTarget tgt{me.x, me.y, me.z, nx, ny, nz, -5.f * nx, -5.f * ny, -5.f * nz};
-    // the m-sums (acc[3 .. 5]) hold -5 times their terms (force_range)
-    double acc[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    auto piece = [&](int j0, int j1, bool near) {
-      float v[7] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      if (near)
-        force_range<true>(rec, j0, j1, tgt, hc, tab, v);
-      else
-        force_range<false>(rec, j0, j1, tgt, hc, tab, v);
-#pragma unroll
-      for (int a = 0; a < 7; ++a) acc[a] += v[a];
-    };
-    if constexpr (W == 1) {
-      for (int r = 0; r < nrange; ++r) {
-        const int2 q = rg[r];
-        piece(q.x, q.y, r < nrb.x);
-      }
-    } else {
-      const int tm = pre[nrb.x], tot = pre[nrange];
-      int i0, i1;
-      wave_part<W>(0, tm, wave, i0, i1);
-      stream_pieces(pre, beg, nrange, i0, i1, [&](int j0, int j1) { piece(j0, j1, true); });
-      wave_part<W>(tm, tot, wave, i0, i1);
-      stream_pieces(pre, beg, nrange, i0, i1, [&](int j0, int j1) { piece(j0, j1, false); });
-    }
-    double f[3] = {acc[0] - 0.2 * acc[3] + static_cast<double>(nx) * acc[6],
-                   acc[1] - 0.2 * acc[4] + static_cast<double>(ny) * acc[6],
-                   acc[2] - 0.2 * acc[5] + static_cast<double>(nz) * acc[6]};
-    combine_waves<W>(f, xch, wave, lane);
-    if (wave == 0 && t < te) out.put(perm[s0 + t], f[0], f[1], f[2]);
-  }
-}
-
-template <int R, int W>
-__device__ __forceinline__ void near_force_remainder(const SrcRec *__restrict__ rec,
-                                                     const int32_t *__restrict__ perm, int s0,
-                                                     int cnt, const int *s_pre, const int *s_beg,
-                                                     int nrange, int nmix, double *xch,
-                                                     const HessConsts &hc, const float4 *tab,
-                                                     int wave, int lane, const ForceOut &out) {
-  int tb, te;
-  remainder_span(cnt, tb, te);
-  for (int t0 = tb; t0 < te; t0 += R) {
-    const int nt = min(R, te - t0);  // uniform
-    float tx[R], ty[R], tz[R], nx[R], ny[R], nz[R];
-    float ax[R], ay[R], az[R], an[R];
-#pragma unroll
-    for (int t = 0; t < R; ++t) {
-      const SrcRec me = rec[s0 + t0 + min(t, nt - 1)];
-      tx[t] = me.x;
-      ty[t] = me.y;
-      tz[t] = me.z;
-      nx[t] = me.mx;
-      ny[t] = me.my;
-      nz[t] = me.mz;
-      ax[t] = ay[t] = az[t] = an[t] = 0.f;
-    }
-    LaneStream st{reinterpret_cast<const float4 *>(rec), s_pre, s_beg, s_pre[nrange], nmix};
-    // the waves take blocks of 64 kLaneBlock positions in turn
-    const int first = wave * 64 * kLaneBlock + lane;
-    st.start(first, nrange);
-    for (int i0 = first; i0 < st.total; i0 += W * 64 * kLaneBlock) {
-      st.fetch(i0);
-#pragma unroll
-      for (int k = 0; k < kLaneBlock; ++k) {
-        const float4 pa = st.pa[k];
-        const float mx = st.pb[k].x, my = st.pb[k].y, mz = st.pb[k].z;
-        const bool mixed = st.mixed[k];
-#pragma unroll
-        for (int t = 0; t < R; ++t) {
-          if (t < nt) {
-            const float dx = tx[t] - pa.x, dy = ty[t] - pa.y, dz = tz[t] - pa.z;
-            const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-            const float ir = __builtin_amdgcn_rsqf(r2);
-            // far curves r^-4 by default, the table's within 4h (force_range)
-            const float irc = __builtin_amdgcn_fmed3f(ir, 0.f, 1e12f);
-            const float ir2 = irc * irc;
-            float c1 = ir2 * ir2, dq = c1;
-            if (mixed && !(r2 > hc.near2)) hess_near_curves_tab(tab, hc.tab_scale, r2, irc, c1, dq);
-            const float Pc = c1 * irc;
-            const float Rc = -5.f * dq * (ir2 * irc);
-            const float dm = fmaf(dx, mx, fmaf(dy, my, dz * mz));
-            const float dn = fmaf(dx, nx[t], fmaf(dy, ny[t], dz * nz[t]));
-            const float mn = fmaf(mx, nx[t], fmaf(my, ny[t], mz * nz[t]));
-            const float e = fmaf(Rc, dm * dn, Pc * mn);
-            const float f = Pc * dn;
-            ax[t] = fmaf(dx, e, fmaf(mx, f, ax[t]));
-            ay[t] = fmaf(dy, e, fmaf(my, f, ay[t]));
-            az[t] = fmaf(dz, e, fmaf(mz, f, az[t]));
-            an[t] = fmaf(Pc, dm, an[t]);
-          }
-        }
-      }
-    }
-    // lane t keeps target t0 + t
-    double g[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-    for (int t = 0; t < R; ++t) {
-      if (t < nt) {
-        const double sx = wave_sum(static_cast<double>(ax[t]));
-        const double sy = wave_sum(static_cast<double>(ay[t]));
-        const double sz = wave_sum(static_cast<double>(az[t]));
-        const double sn = wave_sum(static_cast<double>(an[t]));
-        g[0] = lane == t ? sx + static_cast<double>(nx[t]) * sn : g[0];
-        g[1] = lane == t ? sy + static_cast<double>(ny[t]) * sn : g[1];
-        g[2] = lane == t ? sz + static_cast<double>(nz[t]) * sn : g[2];
-      }
-    }
-    combine_waves<W>(g, xch, wave, lane);
-    if (wave == 0 && lane < nt) out.put(perm[s0 + t0 + lane], g[0], g[1], g[2]);
-  }
-}
-
-// P2P, force: F[perm] (+)= (sum over each leaf's near ranges of B[m_j]) . m_i;
-// the two leaf lists as in p2p_field_kernel.
-template <int W>
-__global__ __launch_bounds__(64 * W) void p2p_force_kernel(
-    const int32_t *__restrict__ full, int nfull, const int32_t *__restrict__ remain, int nrem,
-    const int32_t *__restrict__ start, const int32_t *__restrict__ count,
-    const SrcRec *__restrict__ rec, const int32_t *__restrict__ perm,
-    const int2 *__restrict__ rng, const int2 *__restrict__ nr, int nslot, HessConsts hc,
-    const float4 *__restrict__ htab, ForceOut out) {
-  bool rem;
-  const int li = xcd_two_lists(nrem, nfull, rem);
-  if (li < 0) return;  // uniform over the workgroup, before the barrier
-  const int b = rem ? remain[li] : full[li];
-  const int lane = threadIdx.x & 63;
-  const int wave = W > 1 ? __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)) : 0;
-  __shared__ float4 s_tab[2 * kHessTabEntries];
-  __shared__ int s_pre[kNearH + 1], s_beg[kNearH];
-  __shared__ double xch[(W > 1 ? W - 1 : 1) * (W > 1 ? 3 * 64 : 1)];
-  for (int i = threadIdx.x; i < 2 * kHessTabEntries; i += 64 * W) s_tab[i] = htab[i];
-  const int2 nrb = nr[b];
-  const int2 *__restrict__ rg = rng + static_cast<int64_t>(b) * nslot;
-  if ((rem || W > 1) && wave == 0) range_prefix(s_pre, s_beg, rg, nrb.x + nrb.y, lane);
-  __syncthreads();
-  if (rem)
-    near_force_remainder<4, W>(rec, perm, start[b], count[b], s_pre, s_beg, nrb.x + nrb.y, nrb.x,
-                               xch, hc, s_tab, wave, lane, out);
-  else
-    near_force_full<W>(rec, perm, start[b], count[b], rg, nrb, s_pre, s_beg, xch, hc, s_tab, wave,
-                       lane, out);
-}
+__global__ void set_record_kernel(SrcRec *r, SrcRec v) { *r = v; }
 
 // Moments into the sorted records: rec[i].m = scale * weight[perm[i]] * m[perm[i]]
 // (weight: optional per-particle factor in caller order, e.g. kappa per system).
@@ -2317,6 +1979,19 @@ std::vector<int3> near_offsets_hess() {
   return v;  // 179: 125 with excess2 <= 3, then 54 with excess2 == 4
 }
 
+// Per slot of a symmetric offset set: the slot of the negative offset, and the sign of
+// the first non-zero component.
+std::vector<int2> slot_symmetry(const std::vector<int3> &v) {
+  std::vector<int2> out;
+  for (const int3 &o : v) {
+    const int d = o.x != 0 ? o.x : o.y != 0 ? o.y : o.z;
+    int j = 0;
+    while (v[j].x != -o.x || v[j].y != -o.y || v[j].z != -o.z) ++j;
+    out.push_back(make_int2(j, d > 0 ? 1 : d < 0 ? -1 : 0));
+  }
+  return out;
+}
+
 bool in_near_field(int x, int y, int z) { return x * x + y * y + z * z <= 6; }
 bool in_near_hess(int x, int y, int z) { return excess2(x, y, z) <= 4; }
 
@@ -2365,6 +2040,7 @@ struct FmmTables {
   DeviceBuffer offsH;     // [8][nslotH]
   DeviceBuffer nearF;     // [81] int3
   DeviceBuffer nearH;     // [179] int3
+  DeviceBuffer symF, symH;  // int2 per near slot: slot of the negative offset, sign of this one
   int slot_ld = 0;
 };
 
@@ -2399,17 +2075,15 @@ struct FmmState {
   DeviceBuffer box_sys;      // int32 [nbox] system of each box (batch plans)
   DeviceBuffer nearF, nearH; // leaf lists
   DeviceBuffer cell_grid;    // int32 [8^l]: cell -> box of one level (list building)
-  DeviceBuffer rngF, rngH;   // int2 merged near ranges [nleaf][nslot]
-  DeviceBuffer nrF, nrH;     // int2 range counts per leaf (class 0, class 1)
-  DeviceBuffer leaf_lists;   // int32: the four leaf-shape lists back to back, each in leaf order
+  // near field: stream positions and offsets of the leaf blocks, places per leaf, all
+  // in units of 16 places: their number and the longest stream
+  struct Once {
+    DeviceBuffer pre, off, places, np;
+    int32_t units = 0, longest = 0;
+  } onceF, onceH;
+  DeviceBuffer once_units;
+  DeviceBuffer leaf_lists;   // int32: the leaves with a head, then those with a tail
   int leaf_list_n[kLeafLists] = {};
-  int leaf_list_off[kLeafLists] = {};
-  // lists 1 .. kLeafLists - 1 (the remainders) lie back to back
-  int leaf_lists_remainder() const {
-    int n = 0;
-    for (int k = 1; k < kLeafLists; ++k) n += leaf_list_n[k];
-    return n;
-  }
   DeviceBuffer srcF, srcH;   // M2L source slots [nbox][nslotF], [nleaf][nslotH]
   DeviceBuffer class_ids, class_keys, class_keys2, class_ids2, class_counts;
   DeviceBuffer tilesF, tilesH;
@@ -2596,6 +2270,9 @@ Status build_tables(mf_ctx *ctx, int P, std::shared_ptr<FmmTables> *out) {
   MF_TRY(upload(t->offsH, hoh.data(), hoh.size() * sizeof(int3)));
   MF_TRY(upload(t->nearF, nf.data(), nf.size() * sizeof(int3)));
   MF_TRY(upload(t->nearH, nh.data(), nh.size() * sizeof(int3)));
+  const std::vector<int2> sf = slot_symmetry(nf), sh = slot_symmetry(nh);
+  MF_TRY(upload(t->symF, sf.data(), sf.size() * sizeof(int2)));
+  MF_TRY(upload(t->symH, sh.data(), sh.size() * sizeof(int2)));
   ctx->cache[key] = t;
   *out = t;
   return Status::Ok();
@@ -2654,6 +2331,76 @@ Status read_ints(mf_ctx *ctx, const int32_t *d, int count, std::vector<int32_t> 
 namespace {
 
 // Builds the tree and every list with leaves of side s_leaf (>= 2h).
+// Streams of the leaf blocks; once[field, force] receives, after a synchronize, the last
+// block's offset and units and the longest stream.
+Status build_once(mf_ctx *ctx, FmmState &F, const FmmTables &tab, int nleaf, int64_t n,
+                  int32_t (*once)[3]) {
+  const int64_t nblock = 2 * static_cast<int64_t>(nleaf);
+  MF_TRY(need<int32_t>(F.once_units, nblock + 1));
+  int32_t *units = F.once_units.as<int32_t>(), *longest = units + nblock;
+  const SrcRec pad{kPadCoord, kPadCoord, kPadCoord, 0.f, 0.f, 0.f, 0.f, 0.f};
+  hipLaunchKernelGGL(set_record_kernel, dim3(1), dim3(1), 0, ctx->stream, F.rec.as<SrcRec>() + n, pad);
+  MF_LAUNCH_CHECK();
+  auto build = [&](auto nslot, const DeviceBuffer &near, const DeviceBuffer &sym,
+                   FmmState::Once &o, int32_t *last) -> Status {
+    constexpr int NS = decltype(nslot)::value;
+    MF_TRY(need<int32_t>(o.pre, nblock * (NS + 1)));
+    MF_TRY(need<int32_t>(o.off, nblock));
+    MF_TRY(need<int2>(o.places, static_cast<int64_t>(nleaf) * kPlaces<NS>));
+    MF_TRY(need<int2>(o.np, nleaf));
+    MF_HIP(hipMemsetAsync(longest, 0, sizeof(int32_t), ctx->stream));
+    hipLaunchKernelGGL(once_stream_kernel<NS>, dim3(grid_for(nblock, 4)), dim3(256), 0, ctx->stream,
+                       nleaf, near.as<int32_t>(), sym.as<int2>(), F.box_count.as<int32_t>(),
+                       o.pre.as<int32_t>(), units, longest);
+    MF_LAUNCH_CHECK();
+    MF_TRY(exclusive_scan_i32(ctx, units, o.off.as<int32_t>(), nblock));
+    hipLaunchKernelGGL(near_places_kernel<NS>, dim3(nleaf), dim3(256), 0, ctx->stream,
+                       near.as<int32_t>(), sym.as<int2>(), F.box_count.as<int32_t>(),
+                       o.pre.as<int32_t>(), o.off.as<int32_t>(), o.places.as<int2>(),
+                       o.np.as<int2>());
+    MF_LAUNCH_CHECK();
+    MF_HIP(hipMemcpyAsync(last, o.off.as<int32_t>() + nblock - 1, sizeof(int32_t),
+                          hipMemcpyDeviceToHost, ctx->stream));
+    // the last block's units and the longest stream lie side by side
+    MF_HIP(hipMemcpyAsync(last + 1, units + nblock - 1, 2 * sizeof(int32_t), hipMemcpyDeviceToHost,
+                          ctx->stream));
+    return Status::Ok();
+  };
+  MF_TRY(build(std::integral_constant<int, kNearF>{}, F.nearF, tab.symF, F.onceF, once[0]));
+  return build(std::integral_constant<int, kNearH>{}, F.nearH, tab.symH, F.onceH, once[1]);
+}
+
+// Places of a pass: all, or what kOnceBytes hold; a block belongs to the pass that its stream
+// starts in, so the buffer has room for one more stream.
+constexpr int64_t kOnceBytes = ONCE_BYTES;
+int once_window(const FmmState::Once &o) {
+  constexpr int64_t most = kOnceBytes / (12 * 16);
+  return static_cast<int>(std::max<int64_t>(std::min<int64_t>(o.units, most), 1));
+}
+int once_passes(const FmmState::Once &o) {
+  const int w = once_window(o);
+  return std::max(1, (o.units + w - 1) / w);
+}
+
+// Buffers of a near-field product: nn's, the particles' own sums, and with several
+// passes what the earlier ones left.
+Status once_buffers(mf_ctx *ctx, const FmmState::Once &o, int64_t n, OnceNear &nn, double **near3,
+                    double **rest3) {
+  void *p = nullptr;
+  MF_TRY(workspace(ctx, "fmm_near3", sizeof(double) * 3 * static_cast<size_t>(n), &p));
+  *near3 = static_cast<double *>(p);
+  *rest3 = nullptr;
+  const int passes = once_passes(o);
+  if (passes > 1) {
+    MF_TRY(workspace(ctx, "fmm_rest3", sizeof(double) * 3 * static_cast<size_t>(n), &p));
+    *rest3 = static_cast<double *>(p);
+  }
+  nn.len = 16 * (static_cast<int64_t>(once_window(o)) + (passes > 1 ? o.longest : 0));
+  MF_TRY(workspace(ctx, "fmm_pair_sums", 12 * static_cast<size_t>(nn.len), &p));
+  nn.sums = static_cast<float *>(p);
+  return Status::Ok();
+}
+
 Status fmm_build_at(mf_plan *plan, double s_leaf) {
   mf_ctx *ctx = plan->ctx;
   if (!plan->fmm) plan->fmm.reset(new FmmState());
@@ -2758,7 +2505,7 @@ Status fmm_build_at(mf_plan *plan, double s_leaf) {
   MF_TRY(need<int32_t>(F.perm, n));
   MF_TRY(need<int32_t>(F.flags, n + 1));
   MF_TRY(need<int32_t>(F.scan, n + 1));
-  MF_TRY(need<SrcRec>(F.rec, n));
+  MF_TRY(need<SrcRec>(F.rec, n + 1));  // and the padding record
   hipLaunchKernelGGL(keys_kernel, dim3(grid_for(n, 256)), dim3(256), 0, ctx->stream, n, rec_in,
                      nsys > 1 ? plan->sys_of.as<int32_t>() : static_cast<const int32_t *>(nullptr),
                      F.sys_lo.as<double>(), 1.0 / F.s_leaf, cells, 3 * D, F.keys.as<uint64_t>(),
@@ -2879,21 +2626,8 @@ Status fmm_build_at(mf_plan *plan, double s_leaf) {
                      dim3(256), 0, ctx->stream, nleaf, F.box_keys.as<uint64_t>(), cells, 3 * D,
                      tab.nearH.as<int3>(), kNearH, leaf_grid, F.nearH.as<int32_t>());
   MF_LAUNCH_CHECK();
-  MF_TRY(need<int2>(F.rngF, static_cast<int64_t>(nleaf) * kNearF));
-  MF_TRY(need<int2>(F.rngH, static_cast<int64_t>(nleaf) * kNearH));
-  MF_TRY(need<int2>(F.nrF, nleaf));
-  MF_TRY(need<int2>(F.nrH, nleaf));
-  static_assert(kNearF <= 128 && kNearH <= 256, "near-range sort sizes");
-  hipLaunchKernelGGL(near_ranges_kernel<128>, dim3(nleaf), dim3(64), 0, ctx->stream, nleaf,
-                     F.nearF.as<int32_t>(), kNearF, kNearFMixed, F.box_first.as<int32_t>(),
-                     F.box_count.as<int32_t>(), F.rngF.as<int2>(), F.nrF.as<int2>());
-  MF_LAUNCH_CHECK();
-  hipLaunchKernelGGL(near_ranges_kernel<256>, dim3(nleaf), dim3(64), 0, ctx->stream, nleaf,
-                     F.nearH.as<int32_t>(), kNearH, F.nmixH, F.box_first.as<int32_t>(),
-                     F.box_count.as<int32_t>(), F.rngH.as<int2>(), F.nrH.as<int2>());
-  MF_LAUNCH_CHECK();
   {
-    // leaf shapes of the near-field kernels, each list in leaf order
+    // heads and tails of the near-field kernels, each list in leaf order; their streams
     const int64_t ne = 2 * static_cast<int64_t>(nleaf);
     MF_TRY(need<int32_t>(F.leaf_lists, ne));
     void *pk = nullptr, *pz = nullptr;
@@ -2906,11 +2640,19 @@ Status fmm_build_at(mf_plan *plan, double s_leaf) {
                        ctx->stream, nleaf, F.box_count.as<int32_t>(), k_in, v_in,
                        static_cast<int32_t *>(pz));
     MF_LAUNCH_CHECK();
-    MF_TRY(sort_pairs_u64_i32(ctx, k_in, k_out, v_in, F.leaf_lists.as<int32_t>(), ne, 0, 3));
+    MF_TRY(sort_pairs_u64_i32(ctx, k_in, k_out, v_in, F.leaf_lists.as<int32_t>(), ne, 0, 2));
     MF_HIP(hipMemcpyAsync(F.leaf_list_n, pz, sizeof(int32_t) * kLeafLists, hipMemcpyDeviceToHost, ctx->stream));
+    int32_t once[2][3] = {};
+    MF_TRY(build_once(ctx, F, tab, nleaf, n, once));
     MF_HIP(hipStreamSynchronize(ctx->stream));
-    F.leaf_list_off[0] = 0;
-    for (int k = 1; k < kLeafLists; ++k) F.leaf_list_off[k] = F.leaf_list_off[k - 1] + F.leaf_list_n[k - 1];
+    F.onceF.units = once[0][0] + once[0][1];
+    F.onceF.longest = once[0][2];
+    F.onceH.units = once[1][0] + once[1][1];
+    F.onceH.longest = once[1][2];
+    OnceNear nn{};
+    double *near3 = nullptr, *rest3 = nullptr;
+    MF_TRY(once_buffers(ctx, F.onceF, n, nn, &near3, &rest3));
+    MF_TRY(once_buffers(ctx, F.onceH, n, nn, &near3, &rest3));
   }
   // 5. M2L source slots (levels >= 2) and the class-sorted tile lists
   // one row past the last box of each slot array holds -1 throughout: the
@@ -3436,18 +3178,15 @@ Status upward_and_m2l(mf_plan *plan, bool hess, const std::function<Status()> &l
 namespace mf {
 namespace {
 
-// Waves per leaf of the near-field kernels: the smallest power of two that
-// gives the chip kNearFill waves per SIMD (each leaf list entry is a workgroup).
-// Measured, whole solve + force steps with 1 / 2 / 4 / 8 waves a leaf: 600 entries
-// (32,000 particles) 7.30 / 4.80 / 3.39 / 2.86 ms; 2,048 (131,072 particles) 8.00 /
-// 5.75 / 5.00 / 4.78; 19,338 (506,880) 16.2 / 15.1 / 15.3 / 17.2; 43,453
-// (1,153,433) 33.5 / 33.3 / 34.4 / 39.0, where larger workgroups keep the
-// translations beside them off the CUs.
-constexpr int64_t kNearFill = 28;
-inline int near_waves(const mf_ctx *ctx, int nfull, int nrem) {
-  const int64_t want = static_cast<int64_t>(ctx->num_cu) * 4 * kNearFill;
+// Waves per leaf block: the smallest power of two that gives the chip kOnceFill waves
+// per SIMD (four are resident).  Whole solve + force steps with 4 / 8 / 16 / 32: 131,072
+// particles 4.35 / 4.28 / 4.15 / 4.00 ms, 1,153,433 31.9 / 32.0 / 32.5 / 32.2,
+// products of 253,555 at p = 6 2.90 / 2.90 / 2.59 / 2.47, 96 droplets 20.1 / 20.0 / 20.0 / 20.5.
+constexpr int kOnceFill = 16;
+inline int once_waves(const mf_ctx *ctx, int nblock) {
+  const int64_t want = static_cast<int64_t>(ctx->num_cu) * 4 * kOnceFill;
   int w = 1;
-  while (w < 8 && static_cast<int64_t>(w) * (nfull + nrem) < want) w *= 2;
+  while (w < 8 && static_cast<int64_t>(w) * nblock < want) w *= 2;
   return w;
 }
 #define MF_NEAR_LAUNCH(kernel, waves, ...)                                                      \
@@ -3457,6 +3196,36 @@ inline int near_waves(const mf_ctx *ctx, int nfull, int nrem) {
     case 4: hipLaunchKernelGGL(kernel<4>, dim3(grid), dim3(256), 0, ns, __VA_ARGS__); break;    \
     default: hipLaunchKernelGGL(kernel<8>, dim3(grid), dim3(512), 0, ns, __VA_ARGS__); break;   \
   }
+
+OnceNear once_near(const FmmState &F, const FmmState::Once &o, const DeviceBuffer &near,
+                   const DeviceBuffer &sym, int nmix) {
+  OnceNear nn{};
+  nn.near = near.as<int32_t>();
+  nn.sym = sym.as<int2>();
+  nn.pre = o.pre.as<int32_t>();
+  nn.off = o.off.as<int32_t>();
+  nn.heads = F.leaf_lists.as<int32_t>();
+  nn.tails = nn.heads + F.leaf_list_n[0];
+  nn.nheads = F.leaf_list_n[0];
+  nn.ntails = F.leaf_list_n[1];
+  nn.nmix = nmix;
+  return nn;
+}
+
+// The near field in passes: launch(nn) sums a pass's pairs and gather(nn, pass, passes)
+// adds up the places; the last gather, which writes the result, is the caller's.
+template <class Launch, class Gather>
+Status once_passes_run(const FmmState::Once &o, OnceNear &nn, const Launch &launch,
+                       const Gather &gather) {
+  const int passes = once_passes(o), w = once_window(o);
+  for (int k = 0; k < passes; ++k) {
+    nn.lo = k * w;
+    nn.hi = k + 1 < passes ? nn.lo + w : INT32_MAX;
+    MF_TRY(launch(nn));
+    if (k + 1 < passes) MF_TRY(gather(k, passes));
+  }
+  return Status::Ok();
+}
 
 template <int P, int KP>
 Status apply_field_impl(mf_plan *plan, float scale, const float *px, const float *py,
@@ -3474,17 +3243,27 @@ Status apply_field_impl(mf_plan *plan, float scale, const float *px, const float
   const int use_far = D >= 2 ? 1 : 0;
   SysMask mask{};
   if (plan->active_sys && F.nsys > 1) mask = SysMask{F.box_sys.as<int32_t>(), plan->active_sys};
+  OnceNear nn = once_near(F, F.onceF, F.nearF, F.tab->symF, kNearFMixed);
+  double *near3 = nullptr, *rest3 = nullptr;
+  MF_TRY(once_buffers(ctx, F.onceF, n, nn, &near3, &rest3));
   double *far3 = nullptr;
   if (use_far) {
     void *pf = nullptr;
     MF_TRY(workspace(ctx, "fmm_far3", sizeof(double) * 3 * static_cast<size_t>(n), &pf));
     far3 = static_cast<double *>(pf);
   }
+  auto gather = [&](hipStream_t st, int pass, int passes) -> Status {
+    hipLaunchKernelGGL(near_gather_kernel<kNearF>, dim3(nleaf), dim3(256), 0, st,
+                       F.box_first.as<int32_t>(), F.box_count.as<int32_t>(), F.perm.as<int32_t>(), n,
+                       nn, F.onceF.places.as<int2>(), F.onceF.np.as<int2>(), pass, passes, rest3,
+                       near3, far3, 1.0 / (4.0 * kPi), h0, h1, h2, ox, oy, oz, mask);
+    MF_LAUNCH_CHECK();
+    return Status::Ok();
+  };
   {
     // The near field (VALU) runs on the auxiliary stream, concurrently with
-    // the far-field chain (P2M .. L2L, L2P); it writes H_const + near, the
-    // L2P writes the far field into FP64 scratch, and add_far_kernel sums
-    // them once both are done.
+    // the far-field chain (P2M .. L2L, L2P); the L2P writes the far field
+    // into FP64 scratch, and the last gather sums both once they are done.
     NearOverlap ov(ctx);
     const bool serial = plan->opts.serial_near != 0;
     auto near = [&]() -> Status {
@@ -3494,19 +3273,19 @@ Status apply_field_impl(mf_plan *plan, float scale, const float *px, const float
         ns = ctx->aux_stream;
       }
       KernelTimer timer(ctx, "p2p_field", ns);
-      const int32_t *lists = F.leaf_lists.as<int32_t>();
-      {
-        const int nfull = F.leaf_list_n[0], nrem = F.leaf_lists_remainder();
-        const int grid = 8 * ((nrem + 7) / 8 + (nfull + 7) / 8);
-        if (grid > 0) {
-          MF_NEAR_LAUNCH(p2p_field_kernel, near_waves(ctx, nfull, nrem), lists, nfull,
-                         lists + F.leaf_list_off[1], nrem, F.box_first.as<int32_t>(),
-                         F.box_count.as<int32_t>(), F.rec.as<SrcRec>(), F.perm.as<int32_t>(),
-                         F.rngF.as<int2>(), F.nrF.as<int2>(), kNearF, plan->fc,
-                         F.ftab->buf.as<float4>(), FieldOut{0, h0, h1, h2, ox, oy, oz}, mask);
-          MF_LAUNCH_CHECK();
-        }
-      }
+      const int grid = 8 * ((nn.nheads + 7) / 8 + (nn.ntails + 7) / 8);
+      FieldConsts fc = plan->fc;  // the plan's table holds h
+      fc.inv_h3 = fc.inv_h5 = 1.f;
+      MF_TRY(once_passes_run(
+          F.onceF, nn,
+          [&](const OnceNear &pass) -> Status {
+            MF_NEAR_LAUNCH(near_field_once_kernel, once_waves(ctx, nn.nheads + nn.ntails),
+                           F.box_first.as<int32_t>(), F.box_count.as<int32_t>(),
+                           F.rec.as<SrcRec>(), n, pass, fc, F.ftab->buf.as<float4>(), near3, mask);
+            MF_LAUNCH_CHECK();
+            return Status::Ok();
+          },
+          [&](int k, int passes) { return gather(ns, k, passes); }));
       timer.stop();
       return serial ? Status::Ok() : ov.record();
     };
@@ -3524,14 +3303,7 @@ Status apply_field_impl(mf_plan *plan, float scale, const float *px, const float
     }
     MF_TRY(ov.join());
   }
-  if (use_far) {
-    hipLaunchKernelGGL(add_far_kernel, dim3(grid_for(n, 256)), dim3(256), 0, ctx->stream, n, far3,
-                       ox, oy, oz,
-                       mask.active ? plan->sys_of.as<int32_t>() : static_cast<const int32_t *>(nullptr),
-                       mask.active);
-    MF_LAUNCH_CHECK();
-  }
-  return Status::Ok();
+  return gather(ctx->stream, once_passes(F.onceF) - 1, once_passes(F.onceF));
 }
 
 template <int P, int KP>
@@ -3554,16 +3326,28 @@ Status apply_force_impl(mf_plan *plan, const float *mx, const float *my, const f
       t.p[k] = text9[k];
     }
   }
+  const int nleaf = F.count[F.D];
+  OnceNear nn = once_near(F, F.onceH, F.nearH, F.tab->symH, F.nmixH);
+  double *near3 = nullptr, *rest3 = nullptr;
+  MF_TRY(once_buffers(ctx, F.onceH, n, nn, &near3, &rest3));
   double *far3 = nullptr;
   {
     void *pf = nullptr;
     MF_TRY(workspace(ctx, "fmm_far3", sizeof(double) * 3 * static_cast<size_t>(n), &pf));
     far3 = static_cast<double *>(pf);
   }
+  auto gather = [&](hipStream_t st, int pass, int passes) -> Status {
+    hipLaunchKernelGGL(near_gather_kernel<kNearH>, dim3(nleaf), dim3(256), 0, st,
+                       F.box_first.as<int32_t>(), F.box_count.as<int32_t>(), F.perm.as<int32_t>(), n,
+                       nn, F.onceH.places.as<int2>(), F.onceH.np.as<int2>(), pass, passes, rest3,
+                       near3, far3, 3.0 * kMu0 / (4.0 * kPi), 0.f, 0.f, 0.f, fx, fy, fz, SysMask{});
+    MF_LAUNCH_CHECK();
+    return Status::Ok();
+  };
   {
-    // near force on the auxiliary stream (writes), concurrently with the
-    // far-field chain; the L2P writes the far part and T_ext . m into FP64
-    // scratch, and add_far_kernel sums them once both are done
+    // near force on the auxiliary stream, concurrently with the far-field
+    // chain; the L2P writes the far part and T_ext . m into FP64 scratch, and
+    // the last gather sums both once they are done
     NearOverlap ov(ctx);
     const bool serial = plan->opts.serial_near != 0;
     auto near = [&]() -> Status {
@@ -3573,19 +3357,20 @@ Status apply_force_impl(mf_plan *plan, const float *mx, const float *my, const f
         ns = ctx->aux_stream;
       }
       KernelTimer timer(ctx, "p2p_force", ns);
-      const int32_t *lists = F.leaf_lists.as<int32_t>();
-      {
-        const int nfull = F.leaf_list_n[0], nrem = F.leaf_lists_remainder();
-        const int grid = 8 * ((nrem + 7) / 8 + (nfull + 7) / 8);
-        if (grid > 0) {
-          MF_NEAR_LAUNCH(p2p_force_kernel, near_waves(ctx, nfull, nrem), lists, nfull,
-                         lists + F.leaf_list_off[1], nrem, F.box_first.as<int32_t>(),
-                         F.box_count.as<int32_t>(), F.rec.as<SrcRec>(), F.perm.as<int32_t>(),
-                         F.rngH.as<int2>(), F.nrH.as<int2>(), kNearH, plan->hc,
-                         F.htab->buf.as<float4>(), ForceOut{0, fx, fy, fz});
-          MF_LAUNCH_CHECK();
-        }
-      }
+      const int grid = 8 * ((nn.nheads + 7) / 8 + (nn.ntails + 7) / 8);
+      HessConsts hc = plan->hc;  // the plan's table holds h
+      hc.inv_h4 = 1.f;
+      MF_TRY(once_passes_run(
+          F.onceH, nn,
+          [&](const OnceNear &pass) -> Status {
+            MF_NEAR_LAUNCH(near_force_once_kernel, once_waves(ctx, nn.nheads + nn.ntails),
+                           F.box_first.as<int32_t>(), F.box_count.as<int32_t>(),
+                           F.rec.as<SrcRec>(), n, pass, hc, F.htab->buf.as<float4>(), near3,
+                           SysMask{});
+            MF_LAUNCH_CHECK();
+            return Status::Ok();
+          },
+          [&](int k, int passes) { return gather(ns, k, passes); }));
       timer.stop();
       return serial ? Status::Ok() : ov.record();
     };
@@ -3593,7 +3378,7 @@ Status apply_force_impl(mf_plan *plan, const float *mx, const float *my, const f
     {
       // far part + T_ext . m into FP64 scratch, beside the near field
       KernelTimer timer(ctx, "l2p_force");
-      const int D = F.D, nleaf = F.count[D];
+      const int D = F.D;
       hipLaunchKernelGGL((l2p_force_kernel<P, KP>), dim3(nleaf), dim3(64), 0, ctx->stream, nleaf,
                          F.box_first.as<int32_t>(), F.box_count.as<int32_t>(),
                          F.box_keys.as<uint64_t>(), F.rec.as<SrcRec>(), F.perm.as<int32_t>(),
@@ -3603,11 +3388,7 @@ Status apply_force_impl(mf_plan *plan, const float *mx, const float *my, const f
     }
     MF_TRY(ov.join());
   }
-  hipLaunchKernelGGL(add_far_kernel, dim3(grid_for(n, 256)), dim3(256), 0, ctx->stream, n, far3,
-                     fx, fy, fz, static_cast<const int32_t *>(nullptr),
-                     static_cast<const int32_t *>(nullptr));
-  MF_LAUNCH_CHECK();
-  return Status::Ok();
+  return gather(ctx->stream, once_passes(F.onceH) - 1, once_passes(F.onceH));
 }
 
 }  // namespace
