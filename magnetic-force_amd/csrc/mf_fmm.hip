@@ -361,27 +361,30 @@ __global__ void grid_scatter_kernel(int nbox, const uint64_t *__restrict__ keys,
 
 // M2L source slots of the boxes of one level: src[b * nslot + k] = global
 // index of the source box at offset offs[parity][k] (target - source), or -1.
+// A workgroup of kListThreads per box: with a thread per (box, slot) the division and the
+// key's decoding per slot took longer than the loads (8.4 million particles 698 us, 399 now).
+constexpr int kListThreads = 192;  // 567 and 469 slots in three turns
 __global__ void m2l_list_kernel(int nbox, int box_base, const uint64_t *__restrict__ keys,
                                 int cells, int shift, const int3 *__restrict__ offs, int nslot,
                                 const int32_t *__restrict__ grid, int32_t *__restrict__ src) {
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= static_cast<int64_t>(nbox) * nslot) return;
-  const int b = static_cast<int>(t / nslot), k = static_cast<int>(t % nslot);
+  const int b = blockIdx.x;
   const uint64_t key = keys[b];
   const uint64_t sys_bits = (key >> shift) << shift;
   const I3 c = demorton(key & ((1ULL << shift) - 1ULL));
   const int parity = (c.x & 1) | ((c.y & 1) << 1) | ((c.z & 1) << 2);
-  const int3 o = offs[parity * nslot + k];
-  int r = -1;
-  if (o.x != 0x7fffffff) {
-    const int x = c.x - o.x, y = c.y - o.y, z = c.z - o.z;
-    if (x >= 0 && y >= 0 && z >= 0 && x < cells && y < cells && z < cells) {
-      const int f = grid ? grid[sys_bits | morton(x, y, z)]
-                         : find_key(keys, nbox, sys_bits | morton(x, y, z));
-      r = f >= 0 ? box_base + f : -1;
+  for (int k = threadIdx.x; k < nslot; k += blockDim.x) {
+    const int3 o = offs[parity * nslot + k];
+    int r = -1;
+    if (o.x != 0x7fffffff) {
+      const int x = c.x - o.x, y = c.y - o.y, z = c.z - o.z;
+      if (x >= 0 && y >= 0 && z >= 0 && x < cells && y < cells && z < cells) {
+        const int f = grid ? grid[sys_bits | morton(x, y, z)]
+                           : find_key(keys, nbox, sys_bits | morton(x, y, z));
+        r = f >= 0 ? box_base + f : -1;
+      }
     }
+    src[static_cast<int64_t>(box_base + b) * nslot + k] = r;
   }
-  src[static_cast<int64_t>(box_base + b) * nslot + k] = r;
 }
 
 // Class key (level << 3 | parity) of every box at levels >= 2.
@@ -1215,7 +1218,9 @@ void m2l_deg_kernel(const void *__restrict__ Msrc, uint32_t msrc_bytes, float *_
 
 // Non-empty offsets of every M2L tile: list[tile][0 .. nlist[tile]) = the
 // slots (in order) where at least one target of the tile has a source box.
-// One workgroup per tile; nslot <= 1024.
+// One workgroup per tile; nslot <= 1024, at most kTileT targets.  The targets come
+// through LDS and a thread's loads for its slot do not wait on each other: as a chain of
+// target, slot and flag per target the launch took 32 us whatever the tree's size (7 now).
 __global__ __launch_bounds__(256) void tile_slots_kernel(const M2LTile *__restrict__ tiles,
                                                          const int32_t *__restrict__ sorted_boxes,
                                                          const int32_t *__restrict__ src_slots,
@@ -1224,17 +1229,20 @@ __global__ __launch_bounds__(256) void tile_slots_kernel(const M2LTile *__restri
                                                          int slot_ld, int list_ld,
                                                          int32_t *__restrict__ list,
                                                          int32_t *__restrict__ nlist) {
-  __shared__ int s_flag[1024];
+  __shared__ int s_tgt[kTileT];
   const M2LTile tile = tiles[blockIdx.x];
   const int32_t *__restrict__ smap = slot_table + static_cast<int64_t>(tile.slots) * slot_ld;
-  for (int k = threadIdx.x; k < tile.nslot; k += 256) s_flag[k] = 0;
+  // entries past the tile's last target repeat it
+  for (int j = threadIdx.x; j < kTileT; j += 256)
+    s_tgt[j] = sorted_boxes[tile.first + min(j, tile.count - 1)];
   __syncthreads();
-  for (int j = 0; j < tile.count; ++j) {
-    const int tgt = sorted_boxes[tile.first + j];
-    for (int k = threadIdx.x; k < tile.nslot; k += 256)
-      if (src_slots[static_cast<int64_t>(tgt) * src_ld + k] >= 0) s_flag[k] = 1;
-  }
-  __syncthreads();
+  auto any_source = [&](int k) {
+    int live = -1;  // stays negative while no target has a source
+#pragma unroll 16
+    for (int j = 0; j < kTileT; ++j)
+      live = max(live, src_slots[static_cast<int64_t>(s_tgt[j]) * src_ld + k]);
+    return live >= 0;
+  };
   // Compaction in slot order, 256 slots per pass: a slot's position is the
   // count of flagged slots before it (earlier passes, earlier waves, lower
   // lanes of its own wave).
@@ -1244,7 +1252,7 @@ __global__ __launch_bounds__(256) void tile_slots_kernel(const M2LTile *__restri
   int base = 0;
   for (int k0 = 0; k0 < tile.nslot; k0 += 256) {
     const int k = k0 + static_cast<int>(threadIdx.x);
-    const bool f = k < tile.nslot && s_flag[k] != 0 && smap[k] >= 0;
+    const bool f = k < tile.nslot && smap[k] >= 0 && any_source(k);
     const uint64_t m = __ballot(f);
     if (lane == 0) s_wave[w] = __popcll(m);
     __syncthreads();
@@ -1590,8 +1598,10 @@ __global__ __launch_bounds__(256) void once_stream_kernel(int nleaf, const int32
   }
   if (lane == 0) {
     out[NS] = carry;
-    units[id] = (carry + 15) / 16;
-    if (carry > 0) atomicMax(longest, (carry + 15) / 16);
+    const int u = (carry + 15) / 16;
+    units[id] = u;
+    // most blocks see a longer one: one atomic each cost 1.5 ms at 8.4 million particles
+    if (u > __hip_atomic_load(longest, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(longest, u);
   }
 }
 
@@ -2671,9 +2681,8 @@ Status fmm_build_at(mf_plan *plan, double s_leaf) {
     if (cnt[l] == 0) continue;
     const int32_t *g = nullptr;
     MF_TRY(level_grid(l, &g));
-    hipLaunchKernelGGL(m2l_list_kernel, dim3(grid_for(static_cast<int64_t>(cnt[l]) * tab.nslotF, 256)),
-                       dim3(256), 0, ctx->stream, cnt[l], F.base[l],
-                       F.box_keys.as<uint64_t>() + F.base[l], 1 << l, 3 * l, tab.offsF.as<int3>(),
+    hipLaunchKernelGGL(m2l_list_kernel, dim3(cnt[l]), dim3(kListThreads), 0, ctx->stream, cnt[l],
+                       F.base[l], F.box_keys.as<uint64_t>() + F.base[l], 1 << l, 3 * l, tab.offsF.as<int3>(),
                        tab.nslotF, g, F.srcF.as<int32_t>());
     MF_LAUNCH_CHECK();
   }
@@ -2681,8 +2690,8 @@ Status fmm_build_at(mf_plan *plan, double s_leaf) {
     // leaf level Hessian slots: indexed by leaf (global index == leaf index, base[D] = 0)
     const int32_t *g = nullptr;
     MF_TRY(level_grid(D, &g));
-    hipLaunchKernelGGL(m2l_list_kernel, dim3(grid_for(static_cast<int64_t>(nleaf) * tab.nslotH, 256)),
-                       dim3(256), 0, ctx->stream, nleaf, 0, F.box_keys.as<uint64_t>(), cells, 3 * D,
+    hipLaunchKernelGGL(m2l_list_kernel, dim3(nleaf), dim3(kListThreads), 0, ctx->stream, nleaf, 0,
+                       F.box_keys.as<uint64_t>(), cells, 3 * D,
                        tab.offsH.as<int3>(), tab.nslotH, g, F.srcH.as<int32_t>());
     MF_LAUNCH_CHECK();
   }
