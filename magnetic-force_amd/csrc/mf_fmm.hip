@@ -410,6 +410,36 @@ __global__ void class_key_kernel(int nbox, int box_base, int level,
 // ---------------------------------------------------------------------------
 // Upward pass.
 
+__device__ __forceinline__ uint32_t bf16_bits_rne(float x) {
+  const uint32_t u = __float_as_uint(x);
+  return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
+}
+
+template <int NPART>
+__device__ __forceinline__ void split_bf16(float x, uint32_t (&p)[NPART]) {
+  float r = x;
+#pragma unroll
+  for (int i = 0; i < NPART; ++i) {
+    p[i] = bf16_bits_rne(r);
+    if (i + 1 < NPART) r -= __uint_as_float(p[i] << 16);
+  }
+}
+
+// BF16 parts of rows row .. row + 3 of box's expansion into parts [box][3][KP].
+template <int KP>
+__device__ __forceinline__ void put_parts4(uint16_t *__restrict__ parts, int box, int row, float a,
+                                           float b, float c, float d) {
+  uint32_t p[4][3];
+  split_bf16<3>(a, p[0]);
+  split_bf16<3>(b, p[1]);
+  split_bf16<3>(c, p[2]);
+  split_bf16<3>(d, p[3]);
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+    *reinterpret_cast<uint2 *>(parts + (static_cast<int64_t>(box) * 3 + k) * KP + row) =
+        make_uint2(p[0][k] | (p[1][k] << 16), p[2][k] | (p[3][k] << 16));
+}
+
 // P2M: one wave per leaf; each lane accumulates its particles' dipole
 // multipoles, the wave reduces through LDS.
 template <int P, int KP>
@@ -417,7 +447,8 @@ __global__ __launch_bounds__(64) void p2m_kernel(int nleaf, const int32_t *__res
                                                  const int32_t *__restrict__ count,
                                                  const uint64_t *__restrict__ keys,
                                                  const SrcRec *__restrict__ rec, Frame fr,
-                                                 double s, float *__restrict__ Mt, SysMask mask) {
+                                                 double s, float *__restrict__ Mt,
+                                                 uint16_t *__restrict__ Mb, SysMask mask) {
   constexpr int ND = (P + 1) * (P + 1);
   // The wave's sums go through LDS in two halves of the dofs: a 64 x ND
   // buffer (31 KB at p = 10) would hold P2M to 5 waves per CU.
@@ -430,6 +461,18 @@ __global__ __launch_bounds__(64) void p2m_kernel(int nleaf, const int32_t *__res
   double cx, cy, cz;
   box_centre(fr, keys[b], s, cx, cy, cz);
   const float inv_s = static_cast<float>(1.0 / s);
+  // the expansion itself, or its BF16 parts where only those are read
+  auto put = [&](int d, float v) {
+    if (!Mb) {
+      Mt[static_cast<int64_t>(b) * KP + d] = v;
+      return;
+    }
+    uint32_t p[3];
+    split_bf16<3>(v, p);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      Mb[(static_cast<int64_t>(b) * 3 + k) * KP + d] = static_cast<uint16_t>(p[k]);
+  };
   float acc[ND];
 #pragma unroll
   for (int d = 0; d < ND; ++d) acc[d] = 0.f;
@@ -465,10 +508,10 @@ __global__ __launch_bounds__(64) void p2m_kernel(int nleaf, const int32_t *__res
     if (lane < NH && d < ND) {
       float sum = 0.f;
       for (int l = 0; l < 64; ++l) sum += red[l][lane];
-      Mt[static_cast<int64_t>(b) * KP + d] = sum * inv_s;
+      put(d, sum * inv_s);
     }
   }
-  for (int d = ND + lane; d < KP; d += 64) Mt[static_cast<int64_t>(b) * KP + d] = 0.f;
+  for (int d = ND + lane; d < KP; d += 64) put(d, 0.f);
 }
 
 // ---------------------------------------------------------------------------
@@ -510,7 +553,7 @@ __global__ __launch_bounds__(64) void p2m_kernel(int nleaf, const int32_t *__res
 //    pre-split (from their FP64 values) in fragment order: a lane's eight
 //    consecutive k of one row are one 16-byte load, and a wave's fragment is
 //    1 KB of consecutive memory (whole cache lines).  The multipoles are
-//    pre-split once per product (split_multipoles_kernel).
+//    split by the kernels that make them (put_parts4).
 constexpr int kTileT = 64;
 // Word 3 of a raw buffer resource on gfx950 (32-bit data format, no
 // swizzle): loads past the range return zeros.
@@ -525,21 +568,6 @@ struct M2LTile {
 };
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-
-__device__ __forceinline__ uint32_t bf16_bits_rne(float x) {
-  const uint32_t u = __float_as_uint(x);
-  return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
-}
-
-template <int NPART>
-__device__ __forceinline__ void split_bf16(float x, uint32_t (&p)[NPART]) {
-  float r = x;
-#pragma unroll
-  for (int i = 0; i < NPART; ++i) {
-    p[i] = bf16_bits_rne(r);
-    if (i + 1 < NPART) r -= __uint_as_float(p[i] << 16);
-  }
-}
 
 // Source multipoles of one offset for the tile: the 64 x KP block as 16-byte
 // chunks, FP32 float4 (NPART = 0) or BF16x8 of the pre-split parts (Mb,
@@ -631,6 +659,7 @@ struct M2LSrc2 {
   const int32_t *order;  // tile order within each XCD's range, or null
   int parts = 1;            // workgroups per tile, each an equal part of its offsets
   int64_t part_stride = 0;  // floats between the parts' local expansions
+  uint16_t *split = nullptr;  // octant passes: BF16 parts of the result go here too
 };
 
 // Workgroup -> (tile, part): each XCD (round-robin dispatch over 8) takes a
@@ -648,10 +677,14 @@ __device__ __forceinline__ void m2l_part(int na, int parts, int part, int &lo, i
 }
 
 // Lt = the sum of its parts, in part order, for the boxes the M2L writes
-// (list: the class-sorted boxes).  Boxes of converged systems are skipped.
-__global__ void sum_parts_kernel(int64_t nelem, int KP, int parts, int64_t stride,
+// (list: the class-sorted boxes).  Boxes of converged systems are skipped.  Mb (or
+// null) receives the BF16 parts for the n2 boxes from lo2 on (level 2, whose locals the
+// first L2L reads).
+template <int KP>
+__global__ void sum_parts_kernel(int64_t nelem, int parts, int64_t stride,
                                  const int32_t *__restrict__ boxes, const float *__restrict__ Lp,
-                                 float *__restrict__ Lt, SysMask mask) {
+                                 float *__restrict__ Lt, int lo2, int n2, uint16_t *__restrict__ Mb,
+                                 SysMask mask) {
   const int64_t i = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) * 4;
   if (i >= nelem) return;
   const int box = boxes[i / KP];
@@ -666,6 +699,8 @@ __global__ void sum_parts_kernel(int64_t nelem, int KP, int parts, int64_t strid
     v.w += w.w;
   }
   *reinterpret_cast<float4 *>(Lt + e) = v;
+  if (Mb && box >= lo2 && box < lo2 + n2)
+    put_parts4<KP>(Mb, box, static_cast<int>(i % KP), v.x, v.y, v.z, v.w);
 }
 
 // Tile order of an M2L launch: each XCD takes a contiguous range of tiles
@@ -896,13 +931,14 @@ void m2l_kernel(const void *__restrict__ Msrc, uint32_t msrc_bytes,
     const int tgt = s_tgt[r16 + 16 * cb];
     if (tgt < 0) continue;
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = 32 * wave + 16 * rb + 4 * kq + r;
-        float *o = Lt + static_cast<int64_t>(tgt) * KP + row;
-        *o = accumulate ? *o + acc[rb][cb][r] : acc[rb][cb][r];
-      }
+    for (int rb = 0; rb < 2; ++rb) {
+      const int row = 32 * wave + 16 * rb + 4 * kq;
+      f4 *o = reinterpret_cast<f4 *>(Lt + static_cast<int64_t>(tgt) * KP + row);
+      const f4 v = accumulate ? *o + acc[rb][cb] : acc[rb][cb];
+      *o = v;
+      if constexpr (OCTANT)
+        if (src2.split) put_parts4<KP>(src2.split, tgt, row, v[0], v[1], v[2], v[3]);
+    }
   }
 }
 
@@ -3049,9 +3085,10 @@ Status launch_m2l(mf_ctx *ctx, FmmState &F, const FmmTables &tab, int prec, cons
   MF_LAUNCH_CHECK();
   if (parts > 1) {
     const int64_t ne = static_cast<int64_t>(F.nm2l) * KP;
-    hipLaunchKernelGGL(sum_parts_kernel, dim3(grid_for(ne / 4, 256)), dim3(256), 0, ctx->stream, ne,
-                       KP, parts, stride, F.class_ids2.as<int32_t>(),
-                       static_cast<const float *>(F.Lp.as<float>()), F.Lt.as<float>(), mask);
+    hipLaunchKernelGGL(sum_parts_kernel<KP>, dim3(grid_for(ne / 4, 256)), dim3(256), 0, ctx->stream,
+                       ne, parts, stride, F.class_ids2.as<int32_t>(),
+                       static_cast<const float *>(F.Lp.as<float>()), F.Lt.as<float>(), F.base[2],
+                       F.count[2], npart ? F.Mb.as<uint16_t>() : nullptr, mask);
     MF_LAUNCH_CHECK();
   }
   return Status::Ok();
@@ -3073,18 +3110,20 @@ Status upward_and_m2l(mf_plan *plan, bool hess, const std::function<Status()> &l
   const int nleaf = F.count[D];
   MF_TRY(launch_near());
   if (D < 2) return Status::Ok();
+  const int prec = plan->m2l_precision();
   {
     KernelTimer timer(ctx, "p2m");
     hipLaunchKernelGGL((p2m_kernel<P, KP>), dim3(nleaf), dim3(64), 0, ctx->stream, nleaf,
                        F.box_first.as<int32_t>(), F.box_count.as<int32_t>(),
                        F.box_keys.as<uint64_t>(), F.rec.as<SrcRec>(),
-                       Frame{F.sys_lo.as<double>(), 3 * D}, F.s_leaf, F.Mt.as<float>(), mask);
+                       Frame{F.sys_lo.as<double>(), 3 * D}, F.s_leaf, F.Mt.as<float>(),
+                       prec == MF_M2L_FP32 ? nullptr : F.Mb.as<uint16_t>(), mask);
     MF_LAUNCH_CHECK();
   }
   // M2M and L2L run on the M2L kernel, in the M2L's precision: FP32 MFMA, or
   // the BF16 parts of the octant matrices against BF16 parts of the source
-  // expansions, which are split level by level just before they are read.
-  const int prec = plan->m2l_precision();
+  // expansions, which the kernel that makes an expansion writes with it.  (Split by
+  // launches of their own, five a product at 131,072 particles, a step took 0.25 ms more.)
   const int npart = prec == MF_M2L_FP32 ? 0
                     : prec == MF_M2L_BF16X6 ? 3
                     : prec == MF_M2L_BF16X3 ? 2
@@ -3100,7 +3139,10 @@ Status upward_and_m2l(mf_plan *plan, bool hess, const std::function<Status()> &l
   };
   auto octant_pass = [&](const void *msrc, float *out, const void *tables, const M2LTile *tiles, int nt,
                          const int32_t *boxes, const int32_t *src, int src_ld,
-                         const int32_t *tlist, const int32_t *tn, int accumulate) -> Status {
+                         const int32_t *tlist, const int32_t *tn, int accumulate,
+                         bool split) -> Status {
+    M2LSrc2 src2{nullptr, 0, 0, INT_MAX, nullptr};
+    src2.split = npart && split ? F.Mb.as<uint16_t>() : nullptr;
     const dim3 grid(8 * ((nt + 7) / 8)), block(2 * KP);
     if (!m2l_gather_range_ok(F.nbox, KP, npart))
       return Status::Err(MF_ERR_UNSUPPORTED, "too many boxes for the M2L gather's 32-bit range");
@@ -3109,7 +3151,7 @@ Status upward_and_m2l(mf_plan *plan, bool hess, const std::function<Status()> &l
 #define MF_OCTANT_ARGS                                                                          \
   ctx->stream, msrc, msrc_bytes, out, tables, tiles, nt, boxes, src, src_ld, F.nbox,          \
       tab.slot_tab.as<int32_t>(), tab.slot_ld, tlist, tn, tab.slot_ld, accumulate, mask,       \
-      M2LSrc2{nullptr, 0, 0, INT_MAX, nullptr}
+      src2
     if (npart == 0) hipLaunchKernelGGL((m2l_kernel<KP, 0, true>), grid, block, 0, MF_OCTANT_ARGS);
     else if (npart == 1) hipLaunchKernelGGL((m2l_kernel<KP, 1, true>), grid, block, 0, MF_OCTANT_ARGS);
     else if (npart == 2) hipLaunchKernelGGL((m2l_kernel<KP, 2, true>), grid, block, 0, MF_OCTANT_ARGS);
@@ -3123,7 +3165,6 @@ Status upward_and_m2l(mf_plan *plan, bool hess, const std::function<Status()> &l
     // and apply that octant's matrix.
     KernelTimer timer(ctx, "m2m");
     for (int l = D - 1; l >= 2; --l) {
-      if (npart) MF_TRY(split_level(F.Mt.as<float>(), l + 1));
       const int t0 = F.tileM_start[l], nt = F.tileM_start[l + 1] - t0;
       if (nt <= 0) continue;
       MF_TRY(octant_pass(npart ? F.Mb.get() : F.Mt.get(), F.Mt.as<float>(),
@@ -3131,13 +3172,8 @@ Status upward_and_m2l(mf_plan *plan, bool hess, const std::function<Status()> &l
                          F.tilesM.as<M2LTile>() + t0, nt, F.box_ids.as<int32_t>(),
                          F.child_tab.as<int32_t>(), 8,
                          F.tlistM.as<int32_t>() + static_cast<int64_t>(t0) * tab.slot_ld,
-                         F.tnM.as<int32_t>() + t0, 0));
+                         F.tnM.as<int32_t>() + t0, 0, true));
     }
-  }
-  if (npart) {
-    // levels D .. 3 were split for the M2M; the M2L also reads level 2
-    KernelTimer timer(ctx, "split");
-    MF_TRY(split_level(F.Mt.as<float>(), 2));
   }
   {
     // field M2L launches made at a precision other than the plan's own (the
@@ -3163,18 +3199,21 @@ Status upward_and_m2l(mf_plan *plan, bool hess, const std::function<Status()> &l
   {
     // L2L (accumulating): the children of level l (tiles of one octant class)
     // add their parent's local expansion.  With BF16 parts, the parents'
-    // locals are split into the multipole-part buffer, which the M2L no
-    // longer needs.
+    // locals go to the multipole-part buffer, which the M2L no longer needs:
+    // level 2's here (or with the sum of the M2L's parts), each further level's
+    // with its L2L.
     KernelTimer timer(ctx, "l2l");
+    const int ntiles = hess ? F.ntilesH : F.ntilesF;
+    const bool split2 = ntiles > 0 && m2l_parts(ctx, KP, ntiles) > 1;
     for (int l = 3; l <= D; ++l) {
       const int t0 = F.tileL_start[l], nt = F.tileL_start[l + 1] - t0;
       if (nt <= 0) continue;
-      if (npart) MF_TRY(split_level(F.Lt.as<float>(), l - 1));
+      if (npart && l == 3 && !split2) MF_TRY(split_level(F.Lt.as<float>(), 2));
       MF_TRY(octant_pass(npart ? F.Mb.get() : F.Lt.get(), F.Lt.as<float>(),
                          npart ? tab.W_l2l_b.get() : tab.W_l2l.get(), F.tilesL.as<M2LTile>() + t0,
                          nt, F.class_ids2.as<int32_t>(), F.box_parent.as<int32_t>(), 1,
                          F.tlistL.as<int32_t>() + static_cast<int64_t>(t0) * tab.slot_ld,
-                         F.tnL.as<int32_t>() + t0, 1));
+                         F.tnL.as<int32_t>() + t0, 1, l < D));
     }
   }
   return Status::Ok();
