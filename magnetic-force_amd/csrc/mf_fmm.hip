@@ -676,10 +676,10 @@ __device__ __forceinline__ void m2l_part(int na, int parts, int part, int &lo, i
   hi = parts > 1 ? na * (part + 1) / parts : na;
 }
 
-// Lt = the sum of its parts, in part order, for the boxes the M2L writes
-// (list: the class-sorted boxes).  Boxes of converged systems are skipped.  Mb (or
-// null) receives the BF16 parts for the n2 boxes from lo2 on (level 2, whose locals the
-// first L2L reads).
+// Lt = the sum of its parts, in part order, for the boxes that an M2L or M2M launch
+// writes (list).  Boxes of converged systems are skipped.  Mb (or
+// null) receives the BF16 parts for the n2 boxes from lo2 on (a level's multipoles, or
+// the level-2 locals, which the first L2L reads).
 template <int KP>
 __global__ void sum_parts_kernel(int64_t nelem, int parts, int64_t stride,
                                  const int32_t *__restrict__ boxes, const float *__restrict__ Lp,
@@ -2359,6 +2359,13 @@ int m2l_parts(const mf_ctx *ctx, int KP, int ntiles) {
   return std::max(1, std::min(want / ntiles, kM2LPartsMax));
 }
 
+// Workgroups per M2M tile, each with some of its eight octants, by the same rule: a
+// tile's octants are a chain of gathers and matrix steps, and the few tiles of a level
+// leave most CUs idle.
+int m2m_parts(const mf_ctx *ctx, int KP, int ntiles) {
+  return std::min(m2l_parts(ctx, KP, ntiles), 8);
+}
+
 template <class T>
 Status need(DeviceBuffer &b, int64_t count) {
   return b.reserve(sizeof(T) * static_cast<size_t>(count > 0 ? count : 1));
@@ -2914,7 +2921,13 @@ Status fmm_build_at(mf_plan *plan, double s_leaf) {
   {
     const int parts = std::max(F.ntilesF > 0 ? m2l_parts(ctx, F.KP, F.ntilesF) : 1,
                                F.ntilesH > 0 ? m2l_parts(ctx, F.KP, F.ntilesH) : 1);
-    if (parts > 1) MF_TRY(need<float>(F.Lp, static_cast<int64_t>(F.nbox) * F.KP * parts));
+    int64_t boxes = parts > 1 ? static_cast<int64_t>(F.nbox) * parts : 0;
+    for (int l = 2; l < D; ++l) {
+      const int nt = F.tileM_start[l + 1] - F.tileM_start[l];
+      const int mp = nt > 0 ? m2m_parts(ctx, F.KP, nt) : 1;
+      if (mp > 1) boxes = std::max(boxes, static_cast<int64_t>(cnt[l]) * mp);
+    }
+    if (boxes > 0) MF_TRY(need<float>(F.Lp, boxes * F.KP));
   }
   MF_TRY(need<uint16_t>(F.Mb, static_cast<int64_t>(F.nbox) * 3 * F.KP));
   F.counts_valid = false;  // work counts are computed on the first fmm_info
@@ -3140,10 +3153,12 @@ Status upward_and_m2l(mf_plan *plan, bool hess, const std::function<Status()> &l
   auto octant_pass = [&](const void *msrc, float *out, const void *tables, const M2LTile *tiles, int nt,
                          const int32_t *boxes, const int32_t *src, int src_ld,
                          const int32_t *tlist, const int32_t *tn, int accumulate,
-                         bool split) -> Status {
+                         bool split, int parts, int64_t part_stride) -> Status {
     M2LSrc2 src2{nullptr, 0, 0, INT_MAX, nullptr};
     src2.split = npart && split ? F.Mb.as<uint16_t>() : nullptr;
-    const dim3 grid(8 * ((nt + 7) / 8)), block(2 * KP);
+    src2.parts = parts;
+    src2.part_stride = part_stride;
+    const dim3 grid(8 * ((nt + 7) / 8) * parts), block(2 * KP);
     if (!m2l_gather_range_ok(F.nbox, KP, npart))
       return Status::Err(MF_ERR_UNSUPPORTED, "too many boxes for the M2L gather's 32-bit range");
     const uint32_t msrc_bytes =
@@ -3167,12 +3182,24 @@ Status upward_and_m2l(mf_plan *plan, bool hess, const std::function<Status()> &l
     for (int l = D - 1; l >= 2; --l) {
       const int t0 = F.tileM_start[l], nt = F.tileM_start[l + 1] - t0;
       if (nt <= 0) continue;
-      MF_TRY(octant_pass(npart ? F.Mb.get() : F.Mt.get(), F.Mt.as<float>(),
+      const int parts = m2m_parts(ctx, KP, nt);
+      const int64_t first = static_cast<int64_t>(F.base[l]) * KP,
+                    ne = static_cast<int64_t>(F.count[l]) * KP;
+      // the parts of a level's boxes lie from the buffer's start on
+      float *out = parts > 1 ? F.Lp.as<float>() - first : F.Mt.as<float>();
+      MF_TRY(octant_pass(npart ? F.Mb.get() : F.Mt.get(), out,
                          npart ? tab.W_m2m_b.get() : tab.W_m2m.get(),
                          F.tilesM.as<M2LTile>() + t0, nt, F.box_ids.as<int32_t>(),
                          F.child_tab.as<int32_t>(), 8,
                          F.tlistM.as<int32_t>() + static_cast<int64_t>(t0) * tab.slot_ld,
-                         F.tnM.as<int32_t>() + t0, 0, true));
+                         F.tnM.as<int32_t>() + t0, 0, parts == 1, parts, ne));
+      if (parts > 1) {
+        hipLaunchKernelGGL(sum_parts_kernel<KP>, dim3(grid_for(ne / 4, 256)), dim3(256), 0,
+                           ctx->stream, ne, parts, ne, F.box_ids.as<int32_t>() + F.base[l],
+                           static_cast<const float *>(out), F.Mt.as<float>(), F.base[l], F.count[l],
+                           npart ? F.Mb.as<uint16_t>() : nullptr, mask);
+        MF_LAUNCH_CHECK();
+      }
     }
   }
   {
@@ -3213,7 +3240,7 @@ Status upward_and_m2l(mf_plan *plan, bool hess, const std::function<Status()> &l
                          npart ? tab.W_l2l_b.get() : tab.W_l2l.get(), F.tilesL.as<M2LTile>() + t0,
                          nt, F.class_ids2.as<int32_t>(), F.box_parent.as<int32_t>(), 1,
                          F.tlistL.as<int32_t>() + static_cast<int64_t>(t0) * tab.slot_ld,
-                         F.tnL.as<int32_t>() + t0, 1, l < D));
+                         F.tnL.as<int32_t>() + t0, 1, l < D, 1, 0));
     }
   }
   return Status::Ok();
