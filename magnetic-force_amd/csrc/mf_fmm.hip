@@ -47,6 +47,7 @@
 #include <mutex>
 #include <set>
 #include <string>
+#include <tuple>
 #include <vector>
 #ifndef ONCE_BYTES
 #define ONCE_BYTES (int64_t{12} << 30)
@@ -2057,11 +2058,16 @@ std::vector<int3> m2l_offsets(int beta, bool hess_leaf) {
           if (!near) out.push_back(make_int3(ox, oy, oz));
         }
       }
-  std::sort(out.begin(), out.end(), [](const int3 &a, const int3 &b) {
-    if (a.x != b.x) return a.x < b.x;
-    if (a.y != b.y) return a.y < b.y;
-    return a.z < b.z;
-  });
+  // By the parity of the source box, then in space: a tile's targets are every second box
+  // of each axis, so at the next offset of the same parity most of their sources are the
+  // ones just read, still in L2.  In plain lexicographic order the sources came from two
+  // to four parities in turn and were fetched again: field M2L of 8.4 million particles
+  // 5.34 -> 4.06 ms, force 4.11 -> 3.36.
+  auto key = [](const int3 &o) {
+    return std::make_tuple(o.x & 1, o.y & 1, o.z & 1, o.z, o.y, o.x);
+  };
+  std::sort(out.begin(), out.end(),
+            [&](const int3 &a, const int3 &b) { return key(a) < key(b); });
   return out;
 }
 
