@@ -658,17 +658,23 @@ struct M2LSrc2 {
   const int32_t *src;
   int ld, empty, first_tile;
   const int32_t *order;  // tile order within each XCD's range, or null
-  int parts = 1;            // workgroups per tile, each an equal part of its offsets
-  int64_t part_stride = 0;  // floats between the parts' local expansions
+  // In each XCD's range the tiles from position `whole` on have `parts` workgroups, each
+  // with an equal part of its offsets, whose results go to Lp (part_stride floats
+  // apart); the tiles before them have one.
+  int whole = INT_MAX, parts = 1;
+  float *Lp = nullptr;
+  int64_t part_stride = 0;
   uint16_t *split = nullptr;  // octant passes: BF16 parts of the result go here too
 };
 
-// Workgroup -> (tile, part): each XCD (round-robin dispatch over 8) takes a
+// Workgroup -> tile, part of how many: each XCD (round-robin dispatch over 8) takes a
 // contiguous range of tiles, a tile's parts one after the other.
-__device__ __forceinline__ int m2l_tile_of(int ntiles, int parts, int &part) {
+__device__ __forceinline__ int m2l_tile_of(int ntiles, const M2LSrc2 &s, int &part, int &parts) {
   const int per_xcd = (ntiles + 7) / 8, k = static_cast<int>(blockIdx.x / 8);
-  part = parts > 1 ? k % parts : 0;
-  return static_cast<int>(blockIdx.x % 8) * per_xcd + (parts > 1 ? k / parts : k);
+  const int r = max(k - s.whole, 0);
+  parts = k < s.whole ? 1 : s.parts;
+  part = parts > 1 ? r % parts : 0;
+  return static_cast<int>(blockIdx.x % 8) * per_xcd + (parts > 1 ? s.whole + r / parts : k);
 }
 
 // The part's share [lo, hi) of na offsets.
@@ -677,31 +683,34 @@ __device__ __forceinline__ void m2l_part(int na, int parts, int part, int &lo, i
   hi = parts > 1 ? na * (part + 1) / parts : na;
 }
 
-// Lt = the sum of its parts, in part order, for the boxes that an M2L or M2M launch
-// writes (list).  Boxes of converged systems are skipped.  Mb (or
+// Lt = the sum of its parts, in part order, for the boxes of the tiles that an M2L or
+// M2M launch split; grid.x the tiles, grid.y slices of one.  Boxes of converged systems are skipped.  Mb (or
 // null) receives the BF16 parts for the n2 boxes from lo2 on (a level's multipoles, or
 // the level-2 locals, which the first L2L reads).
 template <int KP>
-__global__ void sum_parts_kernel(int64_t nelem, int parts, int64_t stride,
-                                 const int32_t *__restrict__ boxes, const float *__restrict__ Lp,
-                                 float *__restrict__ Lt, int lo2, int n2, uint16_t *__restrict__ Mb,
-                                 SysMask mask) {
-  const int64_t i = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) * 4;
-  if (i >= nelem) return;
-  const int box = boxes[i / KP];
+__global__ __launch_bounds__(256) void sum_parts_kernel(
+    const M2LTile *__restrict__ tiles, int ntiles, M2LSrc2 s, const int32_t *__restrict__ boxes,
+    float *__restrict__ Lt, int lo2, int n2, uint16_t *__restrict__ Mb, SysMask mask) {
+  const int per_xcd = (ntiles + 7) / 8;
+  const int pos = static_cast<int>(blockIdx.x % 8) * per_xcd + s.whole + static_cast<int>(blockIdx.x / 8);
+  if (pos >= ntiles) return;
+  const M2LTile tile = tiles[s.order ? s.order[pos] : pos];
+  const int i = static_cast<int>(blockIdx.y) * 256 + static_cast<int>(threadIdx.x);
+  if (i >= tile.count * (KP / 4)) return;
+  const int box = boxes[tile.first + i / (KP / 4)], row = 4 * (i % (KP / 4));
   if (sys_skip(mask, box)) return;
-  const int64_t e = static_cast<int64_t>(box) * KP + i % KP;
-  float4 v = *reinterpret_cast<const float4 *>(Lp + e);
-  for (int p = 1; p < parts; ++p) {
-    const float4 w = *reinterpret_cast<const float4 *>(Lp + p * stride + e);
+  const int64_t e = static_cast<int64_t>(box) * KP + row;
+  float4 v = *reinterpret_cast<const float4 *>(s.Lp + e);
+#pragma unroll 4
+  for (int p = 1; p < s.parts; ++p) {
+    const float4 w = *reinterpret_cast<const float4 *>(s.Lp + p * s.part_stride + e);
     v.x += w.x;
     v.y += w.y;
     v.z += w.z;
     v.w += w.w;
   }
   *reinterpret_cast<float4 *>(Lt + e) = v;
-  if (Mb && box >= lo2 && box < lo2 + n2)
-    put_parts4<KP>(Mb, box, static_cast<int>(i % KP), v.x, v.y, v.z, v.w);
+  if (Mb && box >= lo2 && box < lo2 + n2) put_parts4<KP>(Mb, box, row, v.x, v.y, v.z, v.w);
 }
 
 // Tile order of an M2L launch: each XCD takes a contiguous range of tiles
@@ -750,10 +759,10 @@ void m2l_kernel(const void *__restrict__ Msrc, uint32_t msrc_bytes,
   constexpr int kLds = NPART == 0 ? kTileT * LDF * 4 : NPART * kTileT * LDB * 2;
   __shared__ __attribute__((aligned(16))) unsigned char s_raw[kLds];
   __shared__ int s_tgt[kTileT];
-  int part;
-  int tile_id = m2l_tile_of(ntiles, src2.parts, part);
+  int part, parts;
+  int tile_id = m2l_tile_of(ntiles, src2, part, parts);
   if (tile_id >= ntiles) return;  // uniform over the workgroup, before any barrier
-  Lt += part * src2.part_stride;
+  if (parts > 1) Lt = src2.Lp + part * src2.part_stride;
   if (src2.order) tile_id = src2.order[tile_id];
   if (tile_id >= src2.first_tile) {
     src_slots = src2.src;
@@ -782,7 +791,7 @@ void m2l_kernel(const void *__restrict__ Msrc, uint32_t msrc_bytes,
   const int kq = lane >> 4;
   // the tile's non-empty offsets (plan build), walked in slot order
   int lo, hi;
-  m2l_part(tile_nlist[tile_id], src2.parts, part, lo, hi);
+  m2l_part(tile_nlist[tile_id], parts, part, lo, hi);
   const int32_t *__restrict__ tl = tile_list + static_cast<int64_t>(tile_id) * list_ld + lo;
   const int na = hi - lo;
   using GA = M2LGather<KP, NPART>;
@@ -1212,10 +1221,10 @@ void m2l_deg_kernel(const void *__restrict__ Msrc, uint32_t msrc_bytes, float *_
   constexpr int NT = 2 * KP, LDB = SPLIT ? KP + 24 : KP + 8;
   __shared__ __attribute__((aligned(16))) uint16_t sB[(SPLIT ? 2 : 1) * kTileT * LDB];
   __shared__ int s_tgt[kTileT];
-  int part;
-  int tile_id = m2l_tile_of(ntiles, src2.parts, part);
+  int part, parts;
+  int tile_id = m2l_tile_of(ntiles, src2, part, parts);
   if (tile_id >= ntiles) return;  // uniform over the workgroup, before any barrier
-  Lt += part * src2.part_stride;
+  if (parts > 1) Lt = src2.Lp + part * src2.part_stride;
   if (src2.order) tile_id = src2.order[tile_id];
   if (tile_id >= src2.first_tile) {
     src_slots = src2.src;
@@ -1233,7 +1242,7 @@ void m2l_deg_kernel(const void *__restrict__ Msrc, uint32_t msrc_bytes, float *_
   }
   const int32_t *__restrict__ smap = slot_table + static_cast<int64_t>(tile.slots) * slot_ld;
   int lo, hi;
-  m2l_part(tile_nlist[tile_id], src2.parts, part, lo, hi);
+  m2l_part(tile_nlist[tile_id], parts, part, lo, hi);
   const int32_t *__restrict__ tl = tile_list + static_cast<int64_t>(tile_id) * list_ld + lo;
   const int na = hi - lo;
   const __amdgpu_buffer_rsrc_t msrc_rsrc = __builtin_amdgcn_make_buffer_rsrc(
@@ -2152,7 +2161,6 @@ struct FmmState {
   std::vector<int> tileM_start, tileL_start;  // [level], size D + 2
   DeviceBuffer Mt, Lt;
   DeviceBuffer Lp;  // the parts' locals [parts][nbox][KP] where the M2L splits its tiles
-  int nm2l = 0;     // boxes at levels >= 2
   DeviceBuffer Mb;  // BF16 parts of Mt [nbox][3][KP], for the BF16-split M2L
   int64_t p2p_field_pairs = 0;  // sum over leaves of targets x near sources
   int64_t p2p_force_pairs = 0;
@@ -2353,23 +2361,38 @@ Status build_field_table(mf_ctx *ctx, double h, bool hess, std::shared_ptr<Field
   return Status::Ok();
 }
 
-// Workgroups per M2L tile: as many equal parts of its offset list as keep the
-// launch within kM2LFill waves per SIMD (KP / 32 waves a workgroup).  A tile's
-// ~500 offsets are a serial chain; 48 tiles of 131,072 particles left 208 CUs
-// idle.  Field launch with 1 / 2 / 4 / 8 / 16 parts: 48 tiles 0.541 / 0.279 / 0.150 /
-// 0.116 / 0.107 ms, 160 tiles at p = 6 in FP32 1.32 / 1.04 / 0.74 / 0.42 / 0.42; 729
-// tiles, which fill the chip, 1.45 / 1.71 / 2.06 ms (the parts' locals and their sum).
-constexpr int kM2LFill = 4, kM2LPartsMax = 16;
-int m2l_parts(const mf_ctx *ctx, int KP, int ntiles) {
+// Split of an M2L launch's tiles (M2LSrc2).  A tile's ~500 offsets are a serial chain, so
+//  * few tiles get as many parts each as keep the launch within kM2LFill waves per
+//    SIMD (KP / 32 waves a workgroup): the 48 tiles of 131,072 particles left 208 CUs idle.
+//    Field launch with 1 / 2 / 4 / 8 / 16 parts: 48 tiles 0.541 / 0.279 / 0.150 / 0.116 / 0.107 ms,
+//    160 tiles at p = 6 in FP32 1.32 / 1.04 / 0.74 / 0.42 / 0.42;
+//  * where the tiles fill the chip's resident workgroups, the ones left for a last, partly
+//    filled round (the shortest) share it: 1,153,433
+//    particles' 729 tiles over 512 resident workgroups 1.42 -> 1.35 ms, 1.36 with at most
+//    two parts; with every tile in two parts 1.71.
+constexpr int kM2LFill = 4, kM2LPartsMax = 16, kM2LTailMax = 4;
+struct M2LSplit {
+  int whole, parts;
+};
+M2LSplit m2l_split(const mf_ctx *ctx, int KP, int ntiles, int resident) {
+  const int per = (ntiles + 7) / 8;
+  const int slots = std::max(ctx->num_cu / 8 * 4 * resident / (KP / 32), 1);  // per XCD
+  if (per > slots) {
+    const int last = per % slots;
+    const int parts = last > 0 ? std::min(slots / last, kM2LTailMax) : 1;
+    return parts > 1 ? M2LSplit{per - last, parts} : M2LSplit{INT_MAX, 1};
+  }
   const int want = ctx->num_cu * 4 * kM2LFill / (KP / 32);
-  return std::max(1, std::min(want / ntiles, kM2LPartsMax));
+  const int parts = std::max(1, std::min(want / std::max(ntiles, 1), kM2LPartsMax));
+  return parts > 1 ? M2LSplit{0, parts} : M2LSplit{INT_MAX, 1};
 }
 
 // Workgroups per M2M tile, each with some of its eight octants, by the same rule: a
 // tile's octants are a chain of gathers and matrix steps, and the few tiles of a level
 // leave most CUs idle.
 int m2m_parts(const mf_ctx *ctx, int KP, int ntiles) {
-  return std::min(m2l_parts(ctx, KP, ntiles), 8);
+  const int want = ctx->num_cu * 4 * kM2LFill / (KP / 32);
+  return std::max(1, std::min(want / std::max(ntiles, 1), 8));
 }
 
 template <class T>
@@ -2747,7 +2770,6 @@ Status fmm_build_at(mf_plan *plan, double s_leaf) {
   int nm2l = 0;
   for (int l = 2; l <= D; ++l) nm2l += cnt[l];
   F.ntilesF = F.ntilesH = 0;
-  F.nm2l = nm2l;
   if (nm2l > 0) {
     MF_TRY(need<uint64_t>(F.class_keys, nm2l));
     MF_TRY(need<uint64_t>(F.class_keys2, nm2l));
@@ -2925,8 +2947,10 @@ Status fmm_build_at(mf_plan *plan, double s_leaf) {
   MF_TRY(need<float>(F.Mt, static_cast<int64_t>(F.nbox) * F.KP));
   MF_TRY(need<float>(F.Lt, static_cast<int64_t>(F.nbox) * F.KP));
   {
-    const int parts = std::max(F.ntilesF > 0 ? m2l_parts(ctx, F.KP, F.ntilesF) : 1,
-                               F.ntilesH > 0 ? m2l_parts(ctx, F.KP, F.ntilesH) : 1);
+    int parts = 1;  // over the precisions' resident waves
+    for (int r = 2; r <= 4; ++r)
+      for (int nt : {F.ntilesF, F.ntilesH})
+        parts = std::max(parts, m2l_split(ctx, F.KP, nt, r).parts);
     int64_t boxes = parts > 1 ? static_cast<int64_t>(F.nbox) * parts : 0;
     for (int l = 2; l < D; ++l) {
       const int nt = F.tileM_start[l + 1] - F.tileM_start[l];
@@ -3040,21 +3064,27 @@ Status fmm_info(mf_plan *plan, mf_plan_info *info) {
 
 namespace {
 
+// Waves per SIMD that an M2L kernel's registers admit (p = 10).
+int m2l_resident(int prec) {
+  return prec == MF_M2L_BF16X1_CUT ? 4 : prec == MF_M2L_BF16X3 || prec == MF_M2L_BF16X6 ? 2 : 3;
+}
+
 template <int P, int KP>
 Status launch_m2l(mf_ctx *ctx, FmmState &F, const FmmTables &tab, int prec, const M2LTile *tiles,
                   int ntiles, const int32_t *src, int src_rows, int nslot, const int32_t *tlist,
                   const int32_t *tn, SysMask mask, bool fence,
                   M2LSrc2 src2 = M2LSrc2{nullptr, 0, 0, INT_MAX, nullptr}) {
   if (ntiles <= 0) return Status::Ok();
-  const int parts = m2l_parts(ctx, KP, ntiles);
-  const int64_t stride = static_cast<int64_t>(F.nbox) * KP;
+  const M2LSplit split = m2l_split(ctx, KP, ntiles, m2l_resident(prec));
   float *out = F.Lt.as<float>();
-  if (parts > 1) {
-    src2.parts = parts;
-    src2.part_stride = stride;
-    out = F.Lp.as<float>();
+  if (split.parts > 1) {
+    src2.whole = split.whole;
+    src2.parts = split.parts;
+    src2.part_stride = static_cast<int64_t>(F.nbox) * KP;
+    src2.Lp = F.Lp.as<float>();
   }
-  const dim3 grid(8 * ((ntiles + 7) / 8) * parts), block(2 * KP);
+  const int per = (ntiles + 7) / 8, nsplit = std::max(per - split.whole, 0);
+  const dim3 grid(8 * (per - nsplit + nsplit * split.parts)), block(2 * KP);
   const int npart = prec == MF_M2L_FP32 ? 0 : 3;
   if (!m2l_gather_range_ok(F.nbox, KP, npart))
     return Status::Err(MF_ERR_UNSUPPORTED, "too many boxes for the M2L gather's 32-bit range");
@@ -3102,12 +3132,10 @@ Status launch_m2l(mf_ctx *ctx, FmmState &F, const FmmTables &tab, int prec, cons
 #undef MF_M2L_ARGS
 #undef MF_DEG_LAUNCH
   MF_LAUNCH_CHECK();
-  if (parts > 1) {
-    const int64_t ne = static_cast<int64_t>(F.nm2l) * KP;
-    hipLaunchKernelGGL(sum_parts_kernel<KP>, dim3(grid_for(ne / 4, 256)), dim3(256), 0, ctx->stream,
-                       ne, parts, stride, F.class_ids2.as<int32_t>(),
-                       static_cast<const float *>(F.Lp.as<float>()), F.Lt.as<float>(), F.base[2],
-                       F.count[2], npart ? F.Mb.as<uint16_t>() : nullptr, mask);
+  if (split.parts > 1) {
+    hipLaunchKernelGGL(sum_parts_kernel<KP>, dim3(8 * nsplit, kTileT * KP / 1024), dim3(256), 0,
+                       ctx->stream, tiles, ntiles, src2, F.class_ids2.as<int32_t>(), F.Lt.as<float>(), F.base[2],
+                       F.count[2], npart && split.whole == 0 ? F.Mb.as<uint16_t>() : nullptr, mask);
     MF_LAUNCH_CHECK();
   }
   return Status::Ok();
@@ -3159,11 +3187,15 @@ Status upward_and_m2l(mf_plan *plan, bool hess, const std::function<Status()> &l
   auto octant_pass = [&](const void *msrc, float *out, const void *tables, const M2LTile *tiles, int nt,
                          const int32_t *boxes, const int32_t *src, int src_ld,
                          const int32_t *tlist, const int32_t *tn, int accumulate,
-                         bool split, int parts, int64_t part_stride) -> Status {
+                         bool split, int parts, float *lp, int64_t part_stride) -> Status {
     M2LSrc2 src2{nullptr, 0, 0, INT_MAX, nullptr};
     src2.split = npart && split ? F.Mb.as<uint16_t>() : nullptr;
-    src2.parts = parts;
-    src2.part_stride = part_stride;
+    if (parts > 1) {
+      src2.whole = 0;
+      src2.parts = parts;
+      src2.Lp = lp;
+      src2.part_stride = part_stride;
+    }
     const dim3 grid(8 * ((nt + 7) / 8) * parts), block(2 * KP);
     if (!m2l_gather_range_ok(F.nbox, KP, npart))
       return Status::Err(MF_ERR_UNSUPPORTED, "too many boxes for the M2L gather's 32-bit range");
@@ -3192,17 +3224,23 @@ Status upward_and_m2l(mf_plan *plan, bool hess, const std::function<Status()> &l
       const int64_t first = static_cast<int64_t>(F.base[l]) * KP,
                     ne = static_cast<int64_t>(F.count[l]) * KP;
       // the parts of a level's boxes lie from the buffer's start on
-      float *out = parts > 1 ? F.Lp.as<float>() - first : F.Mt.as<float>();
-      MF_TRY(octant_pass(npart ? F.Mb.get() : F.Mt.get(), out,
+      float *lp = parts > 1 ? F.Lp.as<float>() - first : nullptr;
+      MF_TRY(octant_pass(npart ? F.Mb.get() : F.Mt.get(), F.Mt.as<float>(),
                          npart ? tab.W_m2m_b.get() : tab.W_m2m.get(),
                          F.tilesM.as<M2LTile>() + t0, nt, F.box_ids.as<int32_t>(),
                          F.child_tab.as<int32_t>(), 8,
                          F.tlistM.as<int32_t>() + static_cast<int64_t>(t0) * tab.slot_ld,
-                         F.tnM.as<int32_t>() + t0, 0, parts == 1, parts, ne));
+                         F.tnM.as<int32_t>() + t0, 0, parts == 1, parts, lp, ne));
       if (parts > 1) {
-        hipLaunchKernelGGL(sum_parts_kernel<KP>, dim3(grid_for(ne / 4, 256)), dim3(256), 0,
-                           ctx->stream, ne, parts, ne, F.box_ids.as<int32_t>() + F.base[l],
-                           static_cast<const float *>(out), F.Mt.as<float>(), F.base[l], F.count[l],
+        M2LSrc2 parts2{nullptr, 0, 0, INT_MAX, nullptr};
+        parts2.whole = 0;
+        parts2.parts = parts;
+        parts2.Lp = lp;
+        parts2.part_stride = ne;
+        hipLaunchKernelGGL(sum_parts_kernel<KP>, dim3(8 * ((nt + 7) / 8), kTileT * KP / 1024),
+                           dim3(256), 0, ctx->stream, F.tilesM.as<M2LTile>() + t0, nt, parts2,
+                           F.box_ids.as<int32_t>(),
+                           F.Mt.as<float>(), F.base[l], F.count[l],
                            npart ? F.Mb.as<uint16_t>() : nullptr, mask);
         MF_LAUNCH_CHECK();
       }
@@ -3237,7 +3275,7 @@ Status upward_and_m2l(mf_plan *plan, bool hess, const std::function<Status()> &l
     // with its L2L.
     KernelTimer timer(ctx, "l2l");
     const int ntiles = hess ? F.ntilesH : F.ntilesF;
-    const bool split2 = ntiles > 0 && m2l_parts(ctx, KP, ntiles) > 1;
+    const bool split2 = ntiles > 0 && m2l_split(ctx, KP, ntiles, m2l_resident(prec)).whole == 0;
     for (int l = 3; l <= D; ++l) {
       const int t0 = F.tileL_start[l], nt = F.tileL_start[l + 1] - t0;
       if (nt <= 0) continue;
@@ -3246,7 +3284,7 @@ Status upward_and_m2l(mf_plan *plan, bool hess, const std::function<Status()> &l
                          npart ? tab.W_l2l_b.get() : tab.W_l2l.get(), F.tilesL.as<M2LTile>() + t0,
                          nt, F.class_ids2.as<int32_t>(), F.box_parent.as<int32_t>(), 1,
                          F.tlistL.as<int32_t>() + static_cast<int64_t>(t0) * tab.slot_ld,
-                         F.tnL.as<int32_t>() + t0, 1, l < D, 1, 0));
+                         F.tnL.as<int32_t>() + t0, 1, l < D, 1, nullptr, 0));
     }
   }
   return Status::Ok();
