@@ -2139,10 +2139,11 @@ struct FmmState {
   // near field: stream positions and offsets of the leaf blocks, places per leaf, all
   // in units of 16 places: their number and the longest stream
   struct Once {
-    DeviceBuffer pre, off, places, np;
+    DeviceBuffer mem;  // the four arrays below: one allocation
+    int2 *places = nullptr, *np = nullptr;
+    int32_t *pre = nullptr, *off = nullptr;
     int32_t units = 0, longest = 0;
   } onceF, onceH;
-  DeviceBuffer once_units;
   DeviceBuffer leaf_lists;   // int32: the leaves with a head, then those with a tail
   int leaf_list_n[kLeafLists] = {};
   DeviceBuffer srcF, srcH;   // M2L source slots [nbox][nslotF], [nleaf][nslotH]
@@ -2418,30 +2419,34 @@ namespace {
 Status build_once(mf_ctx *ctx, FmmState &F, const FmmTables &tab, int nleaf, int64_t n,
                   int32_t (*once)[3]) {
   const int64_t nblock = 2 * static_cast<int64_t>(nleaf);
-  MF_TRY(need<int32_t>(F.once_units, nblock + 1));
-  int32_t *units = F.once_units.as<int32_t>(), *longest = units + nblock;
+  void *pu = nullptr;
+  MF_TRY(workspace(ctx, "fmm_once_units", sizeof(int32_t) * static_cast<size_t>(nblock + 1), &pu));
+  int32_t *units = static_cast<int32_t *>(pu), *longest = units + nblock;
   const SrcRec pad{kPadCoord, kPadCoord, kPadCoord, 0.f, 0.f, 0.f, 0.f, 0.f};
   hipLaunchKernelGGL(set_record_kernel, dim3(1), dim3(1), 0, ctx->stream, F.rec.as<SrcRec>() + n, pad);
   MF_LAUNCH_CHECK();
   auto build = [&](auto nslot, const DeviceBuffer &near, const DeviceBuffer &sym,
                    FmmState::Once &o, int32_t *last) -> Status {
     constexpr int NS = decltype(nslot)::value;
-    MF_TRY(need<int32_t>(o.pre, nblock * (NS + 1)));
-    MF_TRY(need<int32_t>(o.off, nblock));
-    MF_TRY(need<int2>(o.places, static_cast<int64_t>(nleaf) * kPlaces<NS>));
-    MF_TRY(need<int2>(o.np, nleaf));
+    const int64_t npl = static_cast<int64_t>(nleaf) * kPlaces<NS>, npre = nblock * (NS + 1);
+    MF_TRY(o.mem.reserve(sizeof(int2) * static_cast<size_t>(npl + nleaf) +
+                         sizeof(int32_t) * static_cast<size_t>(npre + nblock)));
+    o.places = o.mem.as<int2>();
+    o.np = o.places + npl;
+    o.pre = reinterpret_cast<int32_t *>(o.np + nleaf);
+    o.off = o.pre + npre;
     MF_HIP(hipMemsetAsync(longest, 0, sizeof(int32_t), ctx->stream));
     hipLaunchKernelGGL(once_stream_kernel<NS>, dim3(grid_for(nblock, 4)), dim3(256), 0, ctx->stream,
                        nleaf, near.as<int32_t>(), sym.as<int2>(), F.box_count.as<int32_t>(),
-                       o.pre.as<int32_t>(), units, longest);
+                       o.pre, units, longest);
     MF_LAUNCH_CHECK();
-    MF_TRY(exclusive_scan_i32(ctx, units, o.off.as<int32_t>(), nblock));
+    MF_TRY(exclusive_scan_i32(ctx, units, o.off, nblock));
     hipLaunchKernelGGL(near_places_kernel<NS>, dim3(nleaf), dim3(256), 0, ctx->stream,
                        near.as<int32_t>(), sym.as<int2>(), F.box_count.as<int32_t>(),
-                       o.pre.as<int32_t>(), o.off.as<int32_t>(), o.places.as<int2>(),
-                       o.np.as<int2>());
+                       o.pre, o.off, o.places,
+                       o.np);
     MF_LAUNCH_CHECK();
-    MF_HIP(hipMemcpyAsync(last, o.off.as<int32_t>() + nblock - 1, sizeof(int32_t),
+    MF_HIP(hipMemcpyAsync(last, o.off + nblock - 1, sizeof(int32_t),
                           hipMemcpyDeviceToHost, ctx->stream));
     // the last block's units and the longest stream lie side by side
     MF_HIP(hipMemcpyAsync(last + 1, units + nblock - 1, 2 * sizeof(int32_t), hipMemcpyDeviceToHost,
@@ -3321,8 +3326,8 @@ OnceNear once_near(const FmmState &F, const FmmState::Once &o, const DeviceBuffe
   OnceNear nn{};
   nn.near = near.as<int32_t>();
   nn.sym = sym.as<int2>();
-  nn.pre = o.pre.as<int32_t>();
-  nn.off = o.off.as<int32_t>();
+  nn.pre = o.pre;
+  nn.off = o.off;
   nn.heads = F.leaf_lists.as<int32_t>();
   nn.tails = nn.heads + F.leaf_list_n[0];
   nn.nheads = F.leaf_list_n[0];
@@ -3374,7 +3379,7 @@ Status apply_field_impl(mf_plan *plan, float scale, const float *px, const float
   auto gather = [&](hipStream_t st, int pass, int passes) -> Status {
     hipLaunchKernelGGL(near_gather_kernel<kNearF>, dim3(nleaf), dim3(256), 0, st,
                        F.box_first.as<int32_t>(), F.box_count.as<int32_t>(), F.perm.as<int32_t>(), n,
-                       nn, F.onceF.places.as<int2>(), F.onceF.np.as<int2>(), pass, passes, rest3,
+                       nn, F.onceF.places, F.onceF.np, pass, passes, rest3,
                        near3, far3, 1.0 / (4.0 * kPi), h0, h1, h2, ox, oy, oz, mask);
     MF_LAUNCH_CHECK();
     return Status::Ok();
@@ -3458,7 +3463,7 @@ Status apply_force_impl(mf_plan *plan, const float *mx, const float *my, const f
   auto gather = [&](hipStream_t st, int pass, int passes) -> Status {
     hipLaunchKernelGGL(near_gather_kernel<kNearH>, dim3(nleaf), dim3(256), 0, st,
                        F.box_first.as<int32_t>(), F.box_count.as<int32_t>(), F.perm.as<int32_t>(), n,
-                       nn, F.onceH.places.as<int2>(), F.onceH.np.as<int2>(), pass, passes, rest3,
+                       nn, F.onceH.places, F.onceH.np, pass, passes, rest3,
                        near3, far3, 3.0 * kMu0 / (4.0 * kPi), 0.f, 0.f, 0.f, fx, fy, fz, SysMask{});
     MF_LAUNCH_CHECK();
     return Status::Ok();
