@@ -49,9 +49,6 @@
 #include <string>
 #include <tuple>
 #include <vector>
-#ifndef ONCE_BYTES
-#define ONCE_BYTES (int64_t{12} << 30)
-#endif
 
 #include "mf_allpairs.hpp"
 #include "mf_expansion.hpp"
@@ -2143,6 +2140,7 @@ struct FmmState {
     int2 *places = nullptr, *np = nullptr;
     int32_t *pre = nullptr, *off = nullptr;
     int32_t units = 0, longest = 0;
+    int32_t window = 0, passes = 1;  // chosen with the buffers; 0: not yet
   } onceF, onceH;
   DeviceBuffer leaf_lists;   // int32: the leaves with a head, then those with a tail
   int leaf_list_n[kLeafLists] = {};
@@ -2413,7 +2411,6 @@ Status read_ints(mf_ctx *ctx, const int32_t *d, int count, std::vector<int32_t> 
 
 namespace {
 
-// Builds the tree and every list with leaves of side s_leaf (>= 2h).
 // Streams of the leaf blocks; once[field, force] receives, after a synchronize, the last
 // block's offset and units and the longest stream.
 Status build_once(mf_ctx *ctx, FmmState &F, const FmmTables &tab, int nleaf, int64_t n,
@@ -2431,6 +2428,7 @@ Status build_once(mf_ctx *ctx, FmmState &F, const FmmTables &tab, int nleaf, int
     const int64_t npl = static_cast<int64_t>(nleaf) * kPlaces<NS>, npre = nblock * (NS + 1);
     MF_TRY(o.mem.reserve(sizeof(int2) * static_cast<size_t>(npl + nleaf) +
                          sizeof(int32_t) * static_cast<size_t>(npre + nblock)));
+    o.window = 0;
     o.places = o.mem.as<int2>();
     o.np = o.places + npl;
     o.pre = reinterpret_cast<int32_t *>(o.np + nleaf);
@@ -2443,8 +2441,7 @@ Status build_once(mf_ctx *ctx, FmmState &F, const FmmTables &tab, int nleaf, int
     MF_TRY(exclusive_scan_i32(ctx, units, o.off, nblock));
     hipLaunchKernelGGL(near_places_kernel<NS>, dim3(nleaf), dim3(256), 0, ctx->stream,
                        near.as<int32_t>(), sym.as<int2>(), F.box_count.as<int32_t>(),
-                       o.pre, o.off, o.places,
-                       o.np);
+                       o.pre, o.off, o.places, o.np);
     MF_LAUNCH_CHECK();
     MF_HIP(hipMemcpyAsync(last, o.off + nblock - 1, sizeof(int32_t),
                           hipMemcpyDeviceToHost, ctx->stream));
@@ -2457,37 +2454,42 @@ Status build_once(mf_ctx *ctx, FmmState &F, const FmmTables &tab, int nleaf, int
   return build(std::integral_constant<int, kNearH>{}, F.nearH, tab.symH, F.onceH, once[1]);
 }
 
-// Places of a pass: all, or what kOnceBytes hold; a block belongs to the pass that its stream
-// starts in, so the buffer has room for one more stream.
-constexpr int64_t kOnceBytes = ONCE_BYTES;
-int once_window(const FmmState::Once &o) {
-  constexpr int64_t most = kOnceBytes / (12 * 16);
-  return static_cast<int>(std::max<int64_t>(std::min<int64_t>(o.units, most), 1));
-}
-int once_passes(const FmmState::Once &o) {
-  const int w = once_window(o);
-  return std::max(1, (o.units + w - 1) / w);
-}
+// A near-field product's passes over its places: window units of 16 places each.  A block
+// belongs to the pass that its stream starts in, so with several passes the buffer has
+// room for one more stream.  A pass takes all places, or what kOnceBytes hold, or where
+// that much cannot be had half as much and so on: each halving costs a launch and a gather,
+// and below kOnceBytesLeast a refusal is an error, as for any other buffer.  The plan build
+// chooses, so that a product asks for what is there.
+constexpr int64_t kOnceBytes = int64_t{12} << 30, kOnceBytesLeast = int64_t{256} << 20;
 
 // Buffers of a near-field product: nn's, the particles' own sums, and with several
 // passes what the earlier ones left.
-Status once_buffers(mf_ctx *ctx, const FmmState::Once &o, int64_t n, OnceNear &nn, double **near3,
+Status once_buffers(mf_ctx *ctx, FmmState::Once &o, int64_t n, OnceNear &nn, double **near3,
                     double **rest3) {
   void *p = nullptr;
   MF_TRY(workspace(ctx, "fmm_near3", sizeof(double) * 3 * static_cast<size_t>(n), &p));
   *near3 = static_cast<double *>(p);
   *rest3 = nullptr;
-  const int passes = once_passes(o);
-  if (passes > 1) {
+  const int64_t all = 12 * 16 * static_cast<int64_t>(o.window > 0 ? o.window : std::max(o.units, 1));
+  for (int64_t most = std::min(all, kOnceBytes);; most /= 2) {
+    const int64_t w = std::max<int64_t>(std::min<int64_t>(o.units, most / (12 * 16)), 1);
+    o.window = static_cast<int>(w);
+    o.passes = static_cast<int>(std::max<int64_t>((o.units + w - 1) / w, 1));
+    nn.len = 16 * (w + (o.passes > 1 ? o.longest : 0));
+    const Status s = workspace(ctx, "fmm_pair_sums", 12 * static_cast<size_t>(nn.len), &p);
+    if (s.ok()) break;
+    if (s.code != MF_ERR_ALLOC || most <= kOnceBytesLeast) return s;
+    (void)hipGetLastError();  // a smaller buffer may be had
+  }
+  nn.sums = static_cast<float *>(p);
+  if (o.passes > 1) {
     MF_TRY(workspace(ctx, "fmm_rest3", sizeof(double) * 3 * static_cast<size_t>(n), &p));
     *rest3 = static_cast<double *>(p);
   }
-  nn.len = 16 * (static_cast<int64_t>(once_window(o)) + (passes > 1 ? o.longest : 0));
-  MF_TRY(workspace(ctx, "fmm_pair_sums", 12 * static_cast<size_t>(nn.len), &p));
-  nn.sums = static_cast<float *>(p);
   return Status::Ok();
 }
 
+// Builds the tree and every list with leaves of side s_leaf (>= 2h).
 Status fmm_build_at(mf_plan *plan, double s_leaf) {
   mf_ctx *ctx = plan->ctx;
   if (!plan->fmm) plan->fmm.reset(new FmmState());
@@ -3341,7 +3343,7 @@ OnceNear once_near(const FmmState &F, const FmmState::Once &o, const DeviceBuffe
 template <class Launch, class Gather>
 Status once_passes_run(const FmmState::Once &o, OnceNear &nn, const Launch &launch,
                        const Gather &gather) {
-  const int passes = once_passes(o), w = once_window(o);
+  const int passes = o.passes, w = o.window;
   for (int k = 0; k < passes; ++k) {
     nn.lo = k * w;
     nn.hi = k + 1 < passes ? nn.lo + w : INT32_MAX;
@@ -3427,7 +3429,7 @@ Status apply_field_impl(mf_plan *plan, float scale, const float *px, const float
     }
     MF_TRY(ov.join());
   }
-  return gather(ctx->stream, once_passes(F.onceF) - 1, once_passes(F.onceF));
+  return gather(ctx->stream, F.onceF.passes - 1, F.onceF.passes);
 }
 
 template <int P, int KP>
@@ -3512,7 +3514,7 @@ Status apply_force_impl(mf_plan *plan, const float *mx, const float *my, const f
     }
     MF_TRY(ov.join());
   }
-  return gather(ctx->stream, once_passes(F.onceH) - 1, once_passes(F.onceH));
+  return gather(ctx->stream, F.onceH.passes - 1, F.onceH.passes);
 }
 
 }  // namespace

@@ -71,3 +71,32 @@ def test_two_passes_vs_fp64(ctx):
     assert rel_err(host(plan.field(m)[:, idx]), host(want)) < TOL
     want = magforce.force_subset_f64(ctx, p64, m64, 2.0, idx)
     assert rel_err(host(plan.force(m)[:, idx]), host(want)) < TOL
+
+
+def test_passes_where_memory_is_short():
+    """737,280 particles where no allocation beyond 320 MiB succeeds: the force's places (about
+    600 MiB) are walked in more passes.  The same FP32 block sums are added in FP64 in
+    another order, so results differ by at most the final rounding."""
+    import magforce
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(8)
+    nx, ny, nz = 96, 96, 80
+    k = torch.arange(nx * ny * nz, device="cuda")
+    pos = torch.stack([k % nx, (k // nx) % ny, k // (nx * ny)]).float()
+    pos += 0.2 * torch.rand(pos.shape, generator=g, device="cuda") - 0.1
+    m = 0.5 * torch.randn(pos.shape, generator=g, device="cuda")
+    refused, out = [], []
+    for limit in (1 << 62, 320 << 20):
+        c = magforce.Context(0)
+        magforce.set_alloc_hook(lambda n: n > limit and (refused.append(n) or True))
+        try:
+            plan = magforce.Plan(c, pos, 2.0, mode=magforce.MODE_FMM)
+            out.append((host(plan.field(m)), host(plan.force(m))))
+            plan.close()
+        finally:
+            magforce.set_alloc_hook(None)
+        c.close()
+    print(f"refused {refused}")
+    assert refused
+    for a, b in zip(*out):
+        assert rel_err(b, a) < 2.0 ** -23
