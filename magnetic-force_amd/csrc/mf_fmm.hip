@@ -1424,19 +1424,18 @@ __device__ __forceinline__ void l2p_hess(const float *__restrict__ Lt, float x, 
 
 // ---------------------------------------------------------------------------
 // Leaf kernels.  The far field (L2P) and the near field (P2P) are separate
-// launches: L2P writes H_const + far field (or the far force + external
-// tensor term) in the caller's particle order, then the near-field kernel adds
-// its sums.  Apart, the near-field kernel needs a third of the registers the
-// solid harmonics of L2P take, and runs at twice the occupancy.
+// launches that run side by side: L2P writes the far field (or the far force +
+// external tensor term) in FP64 in sorted order, the near-field kernels their
+// particles' own sums and places, and near_gather_kernel adds all of them up.
 
-// L2P, field: far3[.][perm] = far field (FP64; near_gather_kernel adds it to
+// L2P, field: far3[.][i] (sorted order) = far field (FP64; near_gather_kernel adds it to
 // H_const + near).  One wave per leaf.
 template <int P, int KP>
 __global__ __launch_bounds__(64) void l2p_field_kernel(
     int nleaf, const int32_t *__restrict__ start, const int32_t *__restrict__ count,
     const uint64_t *__restrict__ keys, const SrcRec *__restrict__ rec,
-    const int32_t *__restrict__ perm, const float *__restrict__ Lt, Frame fr, double s,
-    int64_t n, double *__restrict__ far3, SysMask mask) {
+    const float *__restrict__ Lt, Frame fr, double s, int64_t n, double *__restrict__ far3,
+    SysMask mask) {
   const int b = blockIdx.x;
   if (sys_skip(mask, b)) return;
   const int lane = threadIdx.x;
@@ -1453,10 +1452,10 @@ __global__ __launch_bounds__(64) void l2p_field_kernel(
     l2p_grad<P>(L, static_cast<float>(me.x - cx) * inv_s, static_cast<float>(me.y - cy) * inv_s,
                 static_cast<float>(me.z - cz) * inv_s, gx, gy, gz);
     if (t < cnt) {
-      const int o = perm[s0 + t];
-      far3[o] = far_scale * gx;
-      far3[n + o] = far_scale * gy;
-      far3[2 * n + o] = far_scale * gz;
+      const int64_t i = s0 + t;
+      far3[i] = far_scale * gx;
+      far3[n + i] = far_scale * gy;
+      far3[2 * n + i] = far_scale * gz;
     }
   }
 }
@@ -1503,7 +1502,7 @@ struct Text9 {
   const float *p[9];
 };
 
-// L2P, force: far3[.][perm] = (far tensor + T_ext) . m (FP64;
+// L2P, force: far3[.][i] (sorted order) = (far tensor + T_ext) . m (FP64;
 // near_gather_kernel adds it to the near force).  One wave per leaf.
 template <int P, int KP>
 __global__ __launch_bounds__(64) void l2p_force_kernel(
@@ -1536,8 +1535,9 @@ __global__ __launch_bounds__(64) void l2p_force_kernel(
                         static_cast<double>(Hs[2]) * nz);
     }
     if (t < cnt) {
-      const int o = perm[s0 + t];
+      const int64_t i = s0 + t;
       if (has_text) {
+        const int o = perm[i];
         const double n3[3] = {nx, ny, nz};
         double v[3] = {0.0, 0.0, 0.0};
         for (int r = 0; r < 3; ++r)
@@ -1546,9 +1546,9 @@ __global__ __launch_bounds__(64) void l2p_force_kernel(
         F1 += v[1];
         F2 += v[2];
       }
-      far3[o] = F0;
-      far3[n + o] = F1;
-      far3[2 * n + o] = F2;
+      far3[i] = F0;
+      far3[n + i] = F1;
+      far3[2 * n + i] = F2;
     }
   }
 }
@@ -1888,15 +1888,18 @@ __global__ __launch_bounds__(256) void near_places_kernel(const int32_t *__restr
 }
 
 // out[perm] = base + fac (own sum + what the other blocks left) + far, in FP64 up to
-// the one rounding; in a pass before the last one the sums so far go to rest3.  A workgroup takes a leaf: rows of 64, 32 or 16 lanes by the leaf's
-// size, a lane a particle, the 4, 8 or 16 rows each every 4th, 8th or 16th source block.
-template <int NS>
+// the one rounding; in a pass before the last one the sums so far go to rest3.  A
+// workgroup takes a leaf: rows of 64, 32 or 16 lanes by the leaf's size, a lane a
+// particle, the 4, 8 or 16 rows each every 4th, 8th or 16th source block.  Reading the
+// places bounds it, so the loads of four blocks are under way at a time (ONE: all of the
+// places are this pass's, and no test parts the loads) beside the particle's own sums.
+template <int NS, bool ONE>
 __global__ __launch_bounds__(256) void near_gather_kernel(
     const int32_t *__restrict__ start, const int32_t *__restrict__ count,
     const int32_t *__restrict__ perm, int64_t n, OnceNear nn, const int2 *__restrict__ places,
     const int2 *__restrict__ np, int pass, int passes, double *__restrict__ rest3,
-    const double *__restrict__ near3, const double *__restrict__ far3, double fac, float b0, float b1, float b2,
-    float *__restrict__ ox, float *__restrict__ oy, float *__restrict__ oz, SysMask mask) {
+    const double *__restrict__ near3, const double *__restrict__ far3, double fac, float b0, float b1,
+    float b2, float *__restrict__ ox, float *__restrict__ oy, float *__restrict__ oz, SysMask mask) {
   const int b = blockIdx.x;
   if (sys_skip(mask, b)) return;  // uniform over the workgroup, before the barrier
   __shared__ int s_at[kPlaces<NS>];
@@ -1907,18 +1910,36 @@ __global__ __launch_bounds__(256) void near_gather_kernel(
   constexpr int kElsewhere = INT32_MIN;  // another pass's
   for (int k = tid; k < m.x + m.y; k += 256) {
     const int2 p = places[static_cast<int64_t>(b) * kPlaces<NS> + k];
-    s_at[k] = p.x >= nn.lo && p.x < nn.hi ? 16 * (p.x - nn.lo) + p.y : kElsewhere;
+    s_at[k] = ONE || (p.x >= nn.lo && p.x < nn.hi) ? 16 * (p.x - nn.lo) + p.y : kElsewhere;
   }
-  __syncthreads();
   const int wide = cnt > 32 ? 64 : cnt > 16 ? 32 : 16, rows = 256 / wide;
   const int c = tid & (wide - 1), row = tid / wide;
+  const bool last = ONE || pass + 1 == passes;
   for (int t0 = 0; t0 < cnt; t0 += wide) {
     const int t = t0 + c;
-    const bool live = t < cnt;
+    const bool live = t < cnt, mine = row == 0 && live;
+    const int64_t i = s0 + t;
+    int o = 0;
+    double own[3] = {}, far[3] = {}, rest[3] = {};
+    if (mine) {
+      if (!ONE && pass > 0)
+#pragma unroll
+        for (int a = 0; a < 3; ++a) rest[a] = rest3[a * n + i];
+      if (last) {
+        o = perm[i];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) own[a] = near3[a * n + i];
+        if (far3)
+#pragma unroll
+          for (int a = 0; a < 3; ++a) far[a] = far3[a * n + i];
+      }
+    }
+    __syncthreads();  // the places are there, and sh is free
     double v[3] = {0.0, 0.0, 0.0};
     auto add = [&](int k) {
-      if (s_at[k] == kElsewhere) return;
-      const float *p = nn.sums + (s_at[k] + t);
+      const int at = s_at[k];
+      if (!ONE && at == kElsewhere) return;
+      const float *p = nn.sums + (at + t);
       v[0] += static_cast<double>(p[0]);
       v[1] += static_cast<double>(p[nn.len]);
       v[2] += static_cast<double>(p[2 * nn.len]);
@@ -1934,25 +1955,19 @@ __global__ __launch_bounds__(256) void near_gather_kernel(
 #pragma unroll
     for (int a = 0; a < 3; ++a) sh[a][tid] = v[a];
     __syncthreads();
-    if (row == 0 && live) {
-      const int o = perm[s0 + t];
+    if (mine) {
       float *const out[3] = {ox, oy, oz};
       const float hc[3] = {b0, b1, b2};
 #pragma unroll
       for (int a = 0; a < 3; ++a) {
-        const int64_t i = a * n + s0 + t;
-        double g = pass > 0 ? rest3[i] : 0.0;
+        double g = rest[a];
         for (int k = 0; k < rows; ++k) g += sh[a][k * wide + c];
-        if (pass + 1 < passes) {
-          rest3[i] = g;
-          continue;
-        }
-        g += near3[i];
-        out[a][o] = static_cast<float>(static_cast<double>(hc[a]) + fac * g +
-                                       (far3 ? far3[a * n + o] : 0.0));
+        if (last)
+          out[a][o] = static_cast<float>(static_cast<double>(hc[a]) + fac * (g + own[a]) + far[a]);
+        else
+          rest3[a * n + i] = g;
       }
     }
-    __syncthreads();
   }
 }
 
@@ -3379,7 +3394,8 @@ Status apply_field_impl(mf_plan *plan, float scale, const float *px, const float
     far3 = static_cast<double *>(pf);
   }
   auto gather = [&](hipStream_t st, int pass, int passes) -> Status {
-    hipLaunchKernelGGL(near_gather_kernel<kNearF>, dim3(nleaf), dim3(256), 0, st,
+    const auto kernel = passes == 1 ? near_gather_kernel<kNearF, true> : near_gather_kernel<kNearF, false>;
+    hipLaunchKernelGGL(kernel, dim3(nleaf), dim3(256), 0, st,
                        F.box_first.as<int32_t>(), F.box_count.as<int32_t>(), F.perm.as<int32_t>(), n,
                        nn, F.onceF.places, F.onceF.np, pass, passes, rest3,
                        near3, far3, 1.0 / (4.0 * kPi), h0, h1, h2, ox, oy, oz, mask);
@@ -3422,9 +3438,8 @@ Status apply_field_impl(mf_plan *plan, float scale, const float *px, const float
       KernelTimer timer(ctx, "l2p_field");
       hipLaunchKernelGGL((l2p_field_kernel<P, KP>), dim3(nleaf), dim3(64), 0, ctx->stream, nleaf,
                          F.box_first.as<int32_t>(), F.box_count.as<int32_t>(),
-                         F.box_keys.as<uint64_t>(), F.rec.as<SrcRec>(), F.perm.as<int32_t>(),
-                         F.Lt.as<float>(), Frame{F.sys_lo.as<double>(), 3 * D}, F.s_leaf, n, far3,
-                         mask);
+                         F.box_keys.as<uint64_t>(), F.rec.as<SrcRec>(), F.Lt.as<float>(),
+                         Frame{F.sys_lo.as<double>(), 3 * D}, F.s_leaf, n, far3, mask);
       MF_LAUNCH_CHECK();
     }
     MF_TRY(ov.join());
@@ -3463,7 +3478,8 @@ Status apply_force_impl(mf_plan *plan, const float *mx, const float *my, const f
     far3 = static_cast<double *>(pf);
   }
   auto gather = [&](hipStream_t st, int pass, int passes) -> Status {
-    hipLaunchKernelGGL(near_gather_kernel<kNearH>, dim3(nleaf), dim3(256), 0, st,
+    const auto kernel = passes == 1 ? near_gather_kernel<kNearH, true> : near_gather_kernel<kNearH, false>;
+    hipLaunchKernelGGL(kernel, dim3(nleaf), dim3(256), 0, st,
                        F.box_first.as<int32_t>(), F.box_count.as<int32_t>(), F.perm.as<int32_t>(), n,
                        nn, F.onceH.places, F.onceH.np, pass, passes, rest3,
                        near3, far3, 3.0 * kMu0 / (4.0 * kPi), 0.f, 0.f, 0.f, fx, fy, fz, SysMask{});
