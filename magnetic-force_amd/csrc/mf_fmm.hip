@@ -1474,13 +1474,19 @@ __device__ __forceinline__ int range_of(const int *pre, int nrange, int i) {
 
 // Leaf lists of the near field: the leaves with a head block and those with a tail
 // (head_count), as two entries per leaf (list 2 = none); a stable sort by list then
-// gives each in leaf (Morton) order.
-constexpr int kLeafLists = 2;
+// gives each in leaf (Morton) order.  Where a leaf has kOrderWaves waves (units given:
+// 16-place units of each block's stream), each XCD's part of the leaves goes longest block
+// first: a launch is a few rounds of workgroups then, and long ones started last are its
+// end.  Steps of 131,072 particles 3.95 -> 3.82 ms, field + force products of 65,536 0.56 ->
+// 0.53.  With more leaves the far chain beside it loses what this gains: products of
+// 253,555 at p = 6 in FP32 (6,000 leaves) 2.52 -> 2.60 ms.
+constexpr int kLeafLists = 2, kOrderWaves = 8;
 
 // Particles of a leaf of cnt that belong to its head.
 __device__ __forceinline__ int head_count(int cnt) { return (cnt & 63) > 32 ? cnt : cnt & ~63; }
 
 __global__ void classify_leaves_kernel(int nleaf, const int32_t *__restrict__ count,
+                                       const int32_t *__restrict__ units,
                                        uint64_t *__restrict__ key, int32_t *__restrict__ leaf,
                                        int32_t *__restrict__ sizes) {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1489,7 +1495,15 @@ __global__ void classify_leaves_kernel(int nleaf, const int32_t *__restrict__ co
   const bool has[kLeafLists] = {h > 0, c > h};
 #pragma unroll
   for (int k = 0; k < kLeafLists; ++k) {
-    key[2 * b + k] = static_cast<uint64_t>(has[k] ? k : kLeafLists);
+    uint64_t v = static_cast<uint64_t>(has[k] ? k : kLeafLists);
+    if (units) {
+      // quarters of 16 targets that meet the stream, in steps of 16 (255: 64 targets and
+      // 16,320 records)
+      const int64_t work = static_cast<int64_t>(((k == 0 ? h : c - h) + 15) / 16) * units[2 * b + k];
+      const int64_t part = static_cast<int64_t>(b) * 8 / nleaf;
+      v = v << 11 | static_cast<uint64_t>(part << 8 | 255 - min(work / 16, int64_t{255}));
+    }
+    key[2 * b + k] = v;
     leaf[2 * b + k] = b;
     // one atomic per wave and list instead of one per leaf
     const uint64_t m = __ballot(has[k]);
@@ -2426,14 +2440,27 @@ Status read_ints(mf_ctx *ctx, const int32_t *d, int count, std::vector<int32_t> 
 
 namespace {
 
+// Waves per leaf block: the smallest power of two that gives the chip kOnceFill waves
+// per SIMD (four are resident).  Whole solve + force steps with 4 / 8 / 16 / 32: 131,072
+// particles 4.35 / 4.28 / 4.15 / 4.00 ms, 1,153,433 31.9 / 32.0 / 32.5 / 32.2,
+// products of 253,555 at p = 6 2.90 / 2.90 / 2.59 / 2.47, 96 droplets 20.1 / 20.0 / 20.0 / 20.5.
+constexpr int kOnceFill = 16;
+inline int once_waves(const mf_ctx *ctx, int nblock) {
+  const int64_t want = static_cast<int64_t>(ctx->num_cu) * 4 * kOnceFill;
+  int w = 1;
+  while (w < 8 && static_cast<int64_t>(w) * nblock < want) w *= 2;
+  return w;
+}
+
 // Streams of the leaf blocks; once[field, force] receives, after a synchronize, the last
 // block's offset and units and the longest stream.
 Status build_once(mf_ctx *ctx, FmmState &F, const FmmTables &tab, int nleaf, int64_t n,
-                  int32_t (*once)[3]) {
+                  int32_t (*once)[3], const int32_t **block_units) {
   const int64_t nblock = 2 * static_cast<int64_t>(nleaf);
   void *pu = nullptr;
   MF_TRY(workspace(ctx, "fmm_once_units", sizeof(int32_t) * static_cast<size_t>(nblock + 1), &pu));
   int32_t *units = static_cast<int32_t *>(pu), *longest = units + nblock;
+  *block_units = units;  // the force's, once both are built
   const SrcRec pad{kPadCoord, kPadCoord, kPadCoord, 0.f, 0.f, 0.f, 0.f, 0.f};
   hipLaunchKernelGGL(set_record_kernel, dim3(1), dim3(1), 0, ctx->stream, F.rec.as<SrcRec>() + n, pad);
   MF_LAUNCH_CHECK();
@@ -2731,8 +2758,12 @@ Status fmm_build_at(mf_plan *plan, double s_leaf) {
                      tab.nearH.as<int3>(), kNearH, leaf_grid, F.nearH.as<int32_t>());
   MF_LAUNCH_CHECK();
   {
-    // heads and tails of the near-field kernels, each list in leaf order; their streams
+    // streams of the near-field kernels' blocks, heads and tails
+    int32_t once[2][3] = {};
+    const int32_t *units = nullptr;
+    MF_TRY(build_once(ctx, F, tab, nleaf, n, once, &units));
     const int64_t ne = 2 * static_cast<int64_t>(nleaf);
+    const bool ordered = once_waves(ctx, nleaf) >= kOrderWaves;
     MF_TRY(need<int32_t>(F.leaf_lists, ne));
     void *pk = nullptr, *pz = nullptr;
     MF_TRY(workspace(ctx, "fmm_leaf_keys", (sizeof(uint64_t) * 2 + sizeof(int32_t)) * ne, &pk));
@@ -2741,13 +2772,12 @@ Status fmm_build_at(mf_plan *plan, double s_leaf) {
     int32_t *v_in = reinterpret_cast<int32_t *>(k_out + ne);
     MF_HIP(hipMemsetAsync(pz, 0, sizeof(int32_t) * kLeafLists, ctx->stream));
     hipLaunchKernelGGL(classify_leaves_kernel, dim3(grid_for(nleaf, 256)), dim3(256), 0,
-                       ctx->stream, nleaf, F.box_count.as<int32_t>(), k_in, v_in,
-                       static_cast<int32_t *>(pz));
+                       ctx->stream, nleaf, F.box_count.as<int32_t>(),
+                       ordered ? units : nullptr, k_in, v_in, static_cast<int32_t *>(pz));
     MF_LAUNCH_CHECK();
-    MF_TRY(sort_pairs_u64_i32(ctx, k_in, k_out, v_in, F.leaf_lists.as<int32_t>(), ne, 0, 2));
+    MF_TRY(sort_pairs_u64_i32(ctx, k_in, k_out, v_in, F.leaf_lists.as<int32_t>(), ne, 0,
+                              ordered ? 13 : 2));
     MF_HIP(hipMemcpyAsync(F.leaf_list_n, pz, sizeof(int32_t) * kLeafLists, hipMemcpyDeviceToHost, ctx->stream));
-    int32_t once[2][3] = {};
-    MF_TRY(build_once(ctx, F, tab, nleaf, n, once));
     MF_HIP(hipStreamSynchronize(ctx->stream));
     F.onceF.units = once[0][0] + once[0][1];
     F.onceF.longest = once[0][2];
@@ -3319,17 +3349,6 @@ Status upward_and_m2l(mf_plan *plan, bool hess, const std::function<Status()> &l
 namespace mf {
 namespace {
 
-// Waves per leaf block: the smallest power of two that gives the chip kOnceFill waves
-// per SIMD (four are resident).  Whole solve + force steps with 4 / 8 / 16 / 32: 131,072
-// particles 4.35 / 4.28 / 4.15 / 4.00 ms, 1,153,433 31.9 / 32.0 / 32.5 / 32.2,
-// products of 253,555 at p = 6 2.90 / 2.90 / 2.59 / 2.47, 96 droplets 20.1 / 20.0 / 20.0 / 20.5.
-constexpr int kOnceFill = 16;
-inline int once_waves(const mf_ctx *ctx, int nblock) {
-  const int64_t want = static_cast<int64_t>(ctx->num_cu) * 4 * kOnceFill;
-  int w = 1;
-  while (w < 8 && static_cast<int64_t>(w) * nblock < want) w *= 2;
-  return w;
-}
 #define MF_NEAR_LAUNCH(kernel, waves, ...)                                                      \
   switch (waves) {                                                                              \
     case 1: hipLaunchKernelGGL(kernel<1>, dim3(grid), dim3(64), 0, ns, __VA_ARGS__); break;     \
