@@ -443,6 +443,40 @@ __device__ __forceinline__ void walk_sources(const SrcRec *__restrict__ src,
   }
 }
 
+// The same over a few sources read from the caller's arrays: each wave stages whole tiles
+// and bounds them itself.
+template <class Body, class Flush>
+__device__ __forceinline__ void walk_arrays(const SourceArrays &src, const WaveBox &t, Staged &st,
+                                            int lane, const Body &body, const Flush &flush) {
+  for (int s = 0; s < src.n; s += kTile) {
+    const int cnt = min(src.n - s, kTile), j = s + lane;
+    const bool live = lane < cnt;
+    float p[3] = {kPadCoord, kPadCoord, kPadCoord}, m[3] = {0.f, 0.f, 0.f};
+    if (live) {
+      p[0] = src.x[j];
+      p[1] = src.y[j];
+      p[2] = src.z[j];
+      m[0] = src.mx[j];
+      m[1] = src.my[j];
+      m[2] = src.mz[j];
+    }
+    float4 lo, hi;
+    lo.x = uniform_f(wave_min(live ? p[0] : INFINITY));
+    lo.y = uniform_f(wave_min(live ? p[1] : INFINITY));
+    lo.z = uniform_f(wave_min(live ? p[2] : INFINITY));
+    hi.x = uniform_f(wave_max(live ? p[0] : -INFINITY));
+    hi.y = uniform_f(wave_max(live ? p[1] : -INFINITY));
+    hi.z = uniform_f(wave_max(live ? p[2] : -INFINITY));
+    __builtin_amdgcn_wave_barrier();  // the previous tile has been read
+    st.a[lane] = make_float4(p[0], p[1], p[2], m[0]);
+    st.b[lane] = make_float2(m[1], m[2]);
+    __builtin_amdgcn_wave_barrier();
+    body(4 * ((cnt + kSub - 1) / kSub),
+         uniform_f(box_dist2(t.lx, t.ly, t.lz, t.hx, t.hy, t.hz, lo, hi)));
+    if ((s / kTile + 1) % kFlush == 0 || s + kTile >= src.n) flush();
+  }
+}
+
 // A unit table into the wave's LDS.
 template <int N>
 __device__ __forceinline__ void load_table(const UnitTable<N> &src, float4 (&dst)[2 * N], int lane) {
@@ -462,10 +496,11 @@ __device__ __forceinline__ double group_sum(double v) {
 // ---------------------------------------------------------------------------
 // Field: partial[chunk][c][i] = c * sum_{j in chunk} (3 alpha d (d.m) - beta m)_c
 
-template <int TPT>
-__global__ __launch_bounds__(64) void field_allpairs_kernel(
-    Points tgt, int64_t nt, const SrcRec *__restrict__ src, const float4 *__restrict__ boxes,
-    int64_t nsub, int64_t per, FieldConsts fc, int64_t nt_ld, double *__restrict__ partial) {
+// walk(box, staged, body, flush) takes the wave along its sources, put(a, i, v) receives
+// target i's sum.
+template <int TPT, class Walk, class Put>
+__device__ __forceinline__ void field_wave(const Points &tgt, int64_t nt, const FieldConsts &fc,
+                                           const Walk &walk, const Put &put) {
   __shared__ Staged st;
   __shared__ float4 s_tab[2 * kFieldTabEntries];
   const int lane = threadIdx.x, c = lane & 15, q = lane >> 4;
@@ -556,11 +591,9 @@ __global__ __launch_bounds__(64) void field_allpairs_kernel(
         a1[k][a] = a2[k][a] = 0.f;
       }
   };
-  walk_sources(src, boxes, chunk_range(nsub, per), target_box<TPT>(tx, ty, tz), st, lane, body,
-               flush);
+  walk(target_box<TPT>(tx, ty, tz), st, body, flush);
 
   const double cfac = 1.0 / (4.0 * kPi);
-  double *out = partial + static_cast<int64_t>(blockIdx.y) * 3 * nt_ld;
   const int64_t i = tbase + lane;  // lane group k stores targets 16 k .. 16 k + 15
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
@@ -570,8 +603,36 @@ __global__ __launch_bounds__(64) void field_allpairs_kernel(
       const double sum = group_sum(acc[k][a]);
       v = q == k ? sum : v;
     }
-    if (q < TPT && i < nt) out[a * nt_ld + i] = v * cfac;
+    if (q < TPT && i < nt) put(a, i, v * cfac);
   }
+}
+
+template <int TPT>
+__global__ __launch_bounds__(64) void field_allpairs_kernel(
+    Points tgt, int64_t nt, const SrcRec *__restrict__ src, const float4 *__restrict__ boxes,
+    int64_t nsub, int64_t per, FieldConsts fc, int64_t nt_ld, double *__restrict__ partial) {
+  double *out = partial + static_cast<int64_t>(blockIdx.y) * 3 * nt_ld;
+  field_wave<TPT>(
+      tgt, nt, fc,
+      [&](const WaveBox &box, Staged &st, const auto &body, const auto &flush) {
+        walk_sources(src, boxes, chunk_range(nsub, per), box, st, threadIdx.x, body, flush);
+      },
+      [&](int a, int64_t i, double v) { out[a * nt_ld + i] = v; });
+}
+
+struct FieldOut {
+  float *p[3];
+  float hconst[3];
+};
+template <int TPT>
+__global__ __launch_bounds__(64) void field_few_kernel(Points tgt, int64_t nt, SourceArrays src,
+                                                       FieldConsts fc, FieldOut out) {
+  field_wave<TPT>(
+      tgt, nt, fc,
+      [&](const WaveBox &box, Staged &st, const auto &body, const auto &flush) {
+        walk_arrays(src, box, st, threadIdx.x, body, flush);
+      },
+      [&](int a, int64_t i, double v) { out.p[a][i] = static_cast<float>(v + out.hconst[a]); });
 }
 
 // ---------------------------------------------------------------------------
@@ -893,10 +954,9 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
 // Force-tensor field at separate targets (the external tensor T_ext of
 // eval_hext), walked like the field: partials [chunk][6][nt_ld] (xx yy zz xy
 // xz yz).
-template <int TPT>
-__global__ __launch_bounds__(64) void hessian_allpairs_kernel(
-    Points tgt, int64_t nt, const SrcRec *__restrict__ src, const float4 *__restrict__ boxes,
-    int64_t nsub, int64_t per, HessConsts hc, int64_t nt_ld, double *__restrict__ partial) {
+template <int TPT, class Walk, class Put>
+__device__ __forceinline__ void hessian_wave(const Points &tgt, int64_t nt, const HessConsts &hc,
+                                             const Walk &walk, const Put &put) {
   __shared__ float4 s_tab[2 * kHessTabEntries];
   __shared__ Staged st;
   const int lane = threadIdx.x, c = lane & 15, q = lane >> 4;
@@ -974,20 +1034,35 @@ __global__ __launch_bounds__(64) void hessian_allpairs_kernel(
         s[k][a] = 0.f;
       }
   };
-  walk_sources(src, boxes, chunk_range(nsub, per), target_box<TPT>(tx, ty, tz), st, lane, body,
-               flush);
-  double *out = partial + static_cast<int64_t>(blockIdx.y) * 6 * nt_ld;
+  walk(target_box<TPT>(tx, ty, tz), st, body, flush);
   const int64_t i = tbase + lane;
+  double v[6];
 #pragma unroll
   for (int a = 0; a < 6; ++a) {
-    double v = 0.0;
+    v[a] = 0.0;
 #pragma unroll
     for (int k = 0; k < TPT; ++k) {
       const double sum = group_sum(acc[k][a]);
-      v = q == k ? sum : v;
+      v[a] = q == k ? sum : v[a];
     }
-    if (q < TPT && i < nt) out[a * nt_ld + i] = v;
   }
+  if (q < TPT && i < nt) put(i, v);
+}
+
+template <int TPT>
+__global__ __launch_bounds__(64) void hessian_allpairs_kernel(
+    Points tgt, int64_t nt, const SrcRec *__restrict__ src, const float4 *__restrict__ boxes,
+    int64_t nsub, int64_t per, HessConsts hc, int64_t nt_ld, double *__restrict__ partial) {
+  double *out = partial + static_cast<int64_t>(blockIdx.y) * 6 * nt_ld;
+  hessian_wave<TPT>(
+      tgt, nt, hc,
+      [&](const WaveBox &box, Staged &st, const auto &body, const auto &flush) {
+        walk_sources(src, boxes, chunk_range(nsub, per), box, st, threadIdx.x, body, flush);
+      },
+      [&](int64_t i, const double (&v)[6]) {
+#pragma unroll
+        for (int a = 0; a < 6; ++a) out[a * nt_ld + i] = v[a];
+      });
 }
 
 // Destinations of the six tensor components: out[k] (may be null) receives
@@ -995,7 +1070,29 @@ __global__ __launch_bounds__(64) void hessian_allpairs_kernel(
 struct TensorOut {
   float *p[9];
   int sym[9];
+  __device__ __forceinline__ void put(int64_t i, const double (&s)[6]) const {
+    const double sfac = 3.0 * kMu0 / (4.0 * kPi);
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+      if (!p[k]) continue;
+      double v = s[0];
+#pragma unroll
+      for (int a = 1; a < 6; ++a) v = sym[k] == a ? s[a] : v;  // s stays in registers
+      p[k][i] = static_cast<float>(sfac * v);
+    }
+  }
 };
+
+template <int TPT>
+__global__ __launch_bounds__(64) void hessian_few_kernel(Points tgt, int64_t nt, SourceArrays src,
+                                                         HessConsts hc, TensorOut out) {
+  hessian_wave<TPT>(
+      tgt, nt, hc,
+      [&](const WaveBox &box, Staged &st, const auto &body, const auto &flush) {
+        walk_arrays(src, box, st, threadIdx.x, body, flush);
+      },
+      [&](int64_t i, const double (&v)[6]) { out.put(i, v); });
+}
 
 // ---------------------------------------------------------------------------
 // Chunk reductions (fixed order => deterministic).  A block takes 256 / W
@@ -1040,10 +1137,7 @@ __global__ __launch_bounds__(256) void reduce_hessian_kernel(int64_t n, int64_t 
   int64_t i;
   double s[6];
   if (!reduce_chunks<W, 6>(n, nt_ld, nchunk, partial, i, s)) return;
-  const double sfac = 3.0 * kMu0 / (4.0 * kPi);
-#pragma unroll
-  for (int k = 0; k < 9; ++k)
-    if (out.p[k]) out.p[k][i] = static_cast<float>(sfac * s[out.sym[k]]);
+  out.put(i, s);
 }
 
 template <int W>
@@ -1258,6 +1352,60 @@ Status field_chunks(mf_ctx *ctx, const Points &tgt, int64_t nt, const SrcRec *sr
   return Status::Ok();
 }
 }  // namespace
+
+// Few sources (external magnets): one launch reads the caller's arrays and writes the
+// result, where the general path packs records, writes chunk sums and adds them up: field
+// and tensor calls of 27 sources, general -> few: 4,096 targets 26.4 -> 19.7 us and 32.4 ->
+// 25.7, 1,048,576 42.1 -> 37.8 and 69.4 -> 66.3.  Each wave walks all of the sources, so
+// their number is bounded: at 128 the two paths meet (1,048,576 targets: 85.3 -> 84.1 and 148.4 ->
+// 149.9), at 512 the few lose (4,096: 26.3 -> 27.2 and 32.2 -> 47.0).  A launch may write
+// what another wave has yet to read: outputs that overlap an input take the general path,
+// which reads everything first.
+constexpr int64_t kFewSources = 128;
+bool few_sources(int64_t nt, int64_t ns, const Points &tgt, const SourceArrays &src, float *const *out,
+                 int nout) {
+  if (ns < 1 || ns > kFewSources) return false;
+  auto apart = [](const float *a, int64_t na, const float *b, int64_t nb) {
+    const auto pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
+    return pa + sizeof(float) * na <= pb || pb + sizeof(float) * nb <= pa;
+  };
+  for (int k = 0; k < nout; ++k) {
+    if (!out[k]) continue;
+    for (const float *v : {tgt.x, tgt.y, tgt.z})
+      if (!apart(out[k], nt, v, nt)) return false;
+    for (const float *v : {src.x, src.y, src.z, src.mx, src.my, src.mz})
+      if (!apart(out[k], nt, v, ns)) return false;
+  }
+  return true;
+}
+
+Status field_few_launch(mf_ctx *ctx, const Points &tgt, int64_t nt, const SourceArrays &src,
+                        const FieldConsts &fc, const float *hconst, float *ox, float *oy,
+                        float *oz) {
+  if (nt == 0) return Status::Ok();
+  FieldOut out{{ox, oy, oz}, {}};
+  for (int a = 0; a < 3; ++a) out.hconst[a] = hconst ? hconst[a] : 0.f;
+  KernelTimer timer(ctx, "field");
+  hipLaunchKernelGGL(field_few_kernel<kFieldTPT>, dim3(grid_for(nt, 16 * kFieldTPT)), dim3(64), 0,
+                     ctx->stream, tgt, nt, src, fc, out);
+  MF_LAUNCH_CHECK();
+  return Status::Ok();
+}
+
+Status hessian_few_launch(mf_ctx *ctx, const Points &tgt, int64_t nt, const SourceArrays &src,
+                          const HessConsts &hc, float *const dst[9], const int sym[9]) {
+  if (nt == 0) return Status::Ok();
+  TensorOut out{};
+  for (int k = 0; k < 9; ++k) {
+    out.p[k] = dst[k];
+    out.sym[k] = sym[k];
+  }
+  KernelTimer timer(ctx, "hessian");
+  hipLaunchKernelGGL(hessian_few_kernel<kHessTPT>, dim3(grid_for(nt, 16 * kHessTPT)), dim3(64), 0,
+                     ctx->stream, tgt, nt, src, hc, out);
+  MF_LAUNCH_CHECK();
+  return Status::Ok();
+}
 
 Status field_allpairs_launch_ws(mf_ctx *ctx, const Points &tgt, int64_t nt, const SrcRec *src,
                                 const float4 *boxes, int64_t ns, const FieldConsts &fc,

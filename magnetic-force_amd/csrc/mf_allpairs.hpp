@@ -36,6 +36,20 @@ Status pack_tiles(mf_ctx *ctx, int64_t n, const float *x, const float *y, const 
 Status pack_moments(mf_ctx *ctx, int64_t n, const float *mx, const float *my, const float *mz,
                     float scale, SrcRec *out);
 
+// A few sources, in the caller's arrays.
+struct SourceArrays {
+  const float *x, *y, *z, *mx, *my, *mz;
+  int n;
+};
+// Whether the launches below take these sources: few of them, and no output (nt
+// elements each, null skipped) overlaps an input.
+bool few_sources(int64_t nt, int64_t ns, const Points &tgt, const SourceArrays &src, float *const *out,
+                 int nout);
+Status field_few_launch(mf_ctx *ctx, const Points &tgt, int64_t nt, const SourceArrays &src,
+                        const FieldConsts &fc, const float *hconst, float *ox, float *oy, float *oz);
+Status hessian_few_launch(mf_ctx *ctx, const Points &tgt, int64_t nt, const SourceArrays &src,
+                          const HessConsts &hc, float *const dst[9], const int sym[9]);
+
 // out = hconst + G m over the targets.
 Status field_allpairs_launch(mf_ctx *ctx, const Points &tgt, int64_t nt, const SrcRec *src,
                              const float4 *boxes, int64_t ns, const FieldConsts &fc,

@@ -393,6 +393,11 @@ int mf_field_allpairs(mf_ctx *ctx, int64_t n_t, const float *tx, const float *ty
     MF_ARG(n_t == 0 || (tx && ty && tz && ox && oy && oz), "target/output pointers are null");
     MF_ARG(n_s == 0 || (sx && sy && sz && mx && my && mz), "source pointers are null");
     MF_HIP(hipSetDevice(ctx->device));
+    const mf::Points tgt{tx, ty, tz, 1};
+    const mf::SourceArrays few{sx, sy, sz, mx, my, mz, static_cast<int>(n_s)};
+    float *const out[3] = {ox, oy, oz};
+    if (mf::few_sources(n_t, n_s, tgt, few, out, 3))
+      return mf::field_few_launch(ctx, tgt, n_t, few, mf::make_field_consts(h), hconst, ox, oy, oz);
     const int64_t np = mf::padded_sources(n_s);
     void *p = nullptr;
     MF_TRY(mf::workspace(ctx, "ext_src", sizeof(mf::SrcRec) * static_cast<size_t>(np + 1), &p));
@@ -400,8 +405,8 @@ int mf_field_allpairs(mf_ctx *ctx, int64_t n_t, const float *tx, const float *ty
     MF_TRY(mf::workspace(ctx, "ext_boxes", sizeof(float4) * 2 * static_cast<size_t>(np / mf::kTile + 1), &p));
     float4 *boxes = static_cast<float4 *>(p);
     MF_TRY(mf::pack_tiles(ctx, n_s, sx, sy, sz, mx, my, mz, src, boxes));
-    return mf::field_allpairs_launch(ctx, mf::Points{tx, ty, tz, 1}, n_t, src, boxes, n_s,
-                                     mf::make_field_consts(h), hconst, ox, oy, oz);
+    return mf::field_allpairs_launch(ctx, tgt, n_t, src, boxes, n_s, mf::make_field_consts(h),
+                                     hconst, ox, oy, oz);
   };
   return mf::finish(ctx, run());
 }
@@ -436,6 +441,16 @@ int hessian_entry(mf_ctx *ctx, int64_t n_t, const float *tx, const float *ty, co
     for (int k = 0; k < 9; ++k) MF_ARG(n_t == 0 || sym[k] < 0 || dst[k], "output pointers are null");
     MF_ARG(n_s == 0 || (sx && sy && sz && mx && my && mz), "source pointers are null");
     MF_HIP(hipSetDevice(ctx->device));
+    float *d[9];
+    int sy9[9];
+    for (int k = 0; k < 9; ++k) {
+      d[k] = sym[k] < 0 ? nullptr : dst[k];
+      sy9[k] = sym[k] < 0 ? 0 : sym[k];
+    }
+    const mf::Points tgt{tx, ty, tz, 1};
+    const mf::SourceArrays few{sx, sy, sz, mx, my, mz, static_cast<int>(n_s)};
+    if (mf::few_sources(n_t, n_s, tgt, few, d, 9))
+      return mf::hessian_few_launch(ctx, tgt, n_t, few, mf::make_hess_consts(h), d, sy9);
     const int64_t np = mf::padded_sources(n_s);
     void *p = nullptr;
     MF_TRY(mf::workspace(ctx, "ext_src", sizeof(mf::SrcRec) * static_cast<size_t>(np + 1), &p));
@@ -443,14 +458,8 @@ int hessian_entry(mf_ctx *ctx, int64_t n_t, const float *tx, const float *ty, co
     MF_TRY(mf::workspace(ctx, "ext_boxes", sizeof(float4) * 2 * static_cast<size_t>(np / mf::kTile + 1), &p));
     float4 *boxes = static_cast<float4 *>(p);
     MF_TRY(mf::pack_tiles(ctx, n_s, sx, sy, sz, mx, my, mz, src, boxes));
-    float *d[9];
-    int sy9[9];
-    for (int k = 0; k < 9; ++k) {
-      d[k] = sym[k] < 0 ? nullptr : dst[k];
-      sy9[k] = sym[k] < 0 ? 0 : sym[k];
-    }
-    return mf::hessian_allpairs_launch(ctx, mf::Points{tx, ty, tz, 1}, n_t, src, boxes, n_s,
-                                       mf::make_hess_consts(h), d, sy9);
+    return mf::hessian_allpairs_launch(ctx, tgt, n_t, src, boxes, n_s, mf::make_hess_consts(h), d,
+                                       sy9);
   };
   return mf::finish(ctx, run());
 }

@@ -89,3 +89,36 @@ def test_solve_edges_vs_oracle(ctx, oracle, n, method, warm):
     assert res.stats["converged"] == 1 and res.stats["rel_residual"] <= 1e-6
     want, _, _ = oracle.cg_solve(pos, 2.0, 0.5, b, rtol=1e-12)
     assert rel_err(host(res.x), want) < TOL
+
+
+@pytest.mark.parametrize("ns", [1, 16, 17, 63, 64, 65, 127, 128, 129])
+@pytest.mark.parametrize("nt", [1, 33, 1000])
+def test_few_sources_vs_oracle(ctx, oracle, nt, ns):
+    """Around the largest source count that one launch takes; targets on, near and far from the
+    sources, and outputs that overwrite the targets and the sources, which get the same
+    values as separate ones."""
+    import ctypes
+    import magforce
+    import torch
+    pos = f32(jittered_block(11, 11, 11, seed=nt + ns))
+    t, s, m = pos[:nt], pos[max(nt - ns // 2, 0):][:ns], f32(random_moments(ns, seed=ns))
+    dt, ds, dm = dev(t), dev(s), dev(m)
+    got = magforce.field_allpairs(ctx, dt, ds, dm, 2.0, hconst=[1, 2, 3])
+    assert rel_err(host(got), oracle.field_allpairs(t, s, m, 2.0, hconst=[1, 2, 3])) < TOL
+    want = oracle.hessian_allpairs(t, s, m, 2.0).transpose(0, 2, 1).reshape(nt, 9)
+    nine = host(magforce.hessian_allpairs9(ctx, dt, ds, dm, 2.0))
+    assert rel_err(nine, want) < TOL
+    # one buffer holds targets or sources first, and then the result
+    for over in ("targets", "sources"):
+        buf = torch.zeros((3, max(nt, ns)), device="cuda")
+        first = dt if over == "targets" else ds
+        buf[:, :first.shape[1]] = first
+        row = [buf[k].data_ptr() for k in range(3)]
+        tp = row if over == "targets" else [dt[k].data_ptr() for k in range(3)]
+        sp = row if over == "sources" else [ds[k].data_ptr() for k in range(3)]
+        p = [ctypes.c_void_p(v) for v in (*tp, *sp, *[dm[k].data_ptr() for k in range(3)], *row)]
+        rc = magforce.lib().mf_field_allpairs(ctx.h, nt, *p[:3], ns, *p[3:9], 2.0,
+                                              (ctypes.c_float * 3)(1, 2, 3), *p[9:])
+        torch.cuda.synchronize()
+        assert rc == magforce.MF_OK
+        assert rel_err(host(buf[:, :nt]), host(got)) < 2 * TOL  # each within TOL of the oracle
