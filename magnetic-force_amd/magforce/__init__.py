@@ -194,7 +194,14 @@ def _ptr(t, row=None):
         return None
     if row is None:
         return ctypes.c_void_p(t.data_ptr())
-    return ctypes.c_void_p(t[row].data_ptr())
+    return ctypes.c_void_p(_row_address(t, row))
+
+
+def _row_address(t, row):
+    """t[row].data_ptr() without making the view, which takes about a microsecond each."""
+    if not 0 <= row < t.shape[0]:
+        raise IndexError(f"row {row} of a tensor of {t.shape[0]}")
+    return t.data_ptr() + row * t.stride(0) * t.element_size()
 
 
 def _soa(t, n=None):
@@ -349,7 +356,7 @@ def hessian_allpairs9(ctx: Context, tpos, spos, smom, h: float):
     s = _soa(spos)
     m = _soa(smom, s.shape[1])
     out = torch.empty((9, t.shape[1]), dtype=torch.float32, device=t.device)
-    ptrs = (ctypes.c_void_p * 9)(*[out[k].data_ptr() for k in range(9)])
+    ptrs = (ctypes.c_void_p * 9)(*[_row_address(out, k) for k in range(9)])
     _check(lib().mf_hessian_allpairs9(ctx.h, t.shape[1], _ptr(t, 0), _ptr(t, 1), _ptr(t, 2),
                                       s.shape[1], _ptr(s, 0), _ptr(s, 1), _ptr(s, 2), _ptr(m, 0),
                                       _ptr(m, 1), _ptr(m, 2), float(h), ptrs), ctx.h)
@@ -361,7 +368,7 @@ def _text_ptrs(text):
         return None
     if text.shape[0] != 9:
         raise ValueError("text must have shape (9, n)")
-    return (ctypes.c_void_p * 9)(*[text[k].data_ptr() for k in range(9)])
+    return (ctypes.c_void_p * 9)(*[_row_address(text, k) for k in range(9)])
 
 
 def force_allpairs(ctx: Context, pos, mom, h: float, text=None):
