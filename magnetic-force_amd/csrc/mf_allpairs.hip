@@ -610,7 +610,9 @@ __device__ __forceinline__ void field_wave(const Points &tgt, int64_t nt, const 
 template <int TPT>
 __global__ __launch_bounds__(64) void field_allpairs_kernel(
     Points tgt, int64_t nt, const SrcRec *__restrict__ src, const float4 *__restrict__ boxes,
-    int64_t nsub, int64_t per, FieldConsts fc, int64_t nt_ld, double *__restrict__ partial) {
+    int64_t nsub, int64_t per, FieldConsts fc, int64_t nt_ld, double *__restrict__ partial,
+    Skip skip) {
+  if (skipped(skip)) return;
   double *out = partial + static_cast<int64_t>(blockIdx.y) * 3 * nt_ld;
   field_wave<TPT>(
       tgt, nt, fc,
@@ -936,7 +938,8 @@ template <int W>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) void field_self_kernel(const SrcRec *__restrict__ rec,
                                                             const float4 *__restrict__ boxes,
                                                             int64_t n, SelfWalk w, FieldConsts fc,
-                                                            double *__restrict__ partial) {
+                                                            double *__restrict__ partial, Skip skip) {
+  if (skipped(skip)) return;
   self_walk<FieldSelf<kSelfTPT>, FieldConsts, W, kFieldTabEntries>(rec, boxes, n, w, fc, d_field_tab,
                                                          1.0 / (4.0 * kPi), partial);
 }
@@ -1161,6 +1164,7 @@ template <int W>
 __global__ __launch_bounds__(256) void reduce_ap_kernel(int64_t n, int64_t nt_ld, int nchunk,
                                                         const double *__restrict__ partial,
                                                         ApOut o) {
+  if (skipped(o.skip)) return;
   int64_t i;
   double s[3];
   double dot = 0.0;
@@ -1337,7 +1341,8 @@ int64_t field_partial_doubles(int64_t nt, int64_t nchunk) { return 3 * nt * nchu
 namespace {
 // The chunk sums of the field into `partial`; returns the chunk count.
 Status field_chunks(mf_ctx *ctx, const Points &tgt, int64_t nt, const SrcRec *src,
-                    const float4 *boxes, const FieldConsts &fc, const Split &f, double *partial) {
+                    const float4 *boxes, const FieldConsts &fc, const Split &f, double *partial,
+                    const Skip &skip = {}) {
   if (f.nsub == 0) {
     // a fill kernel, not hipMemsetAsync: callers may capture this in a graph
     hipLaunchKernelGGL(zero_f64_kernel, dim3(grid_for(3 * nt, 256)), dim3(256), 0, ctx->stream,
@@ -1347,7 +1352,8 @@ Status field_chunks(mf_ctx *ctx, const Points &tgt, int64_t nt, const SrcRec *sr
   }
   KernelTimer timer(ctx, "field");
   hipLaunchKernelGGL(field_allpairs_kernel<kFieldTPT>, dim3(f.gx, static_cast<unsigned>(f.nchunk)),
-                     dim3(64), 0, ctx->stream, tgt, nt, src, boxes, f.nsub, f.per, fc, nt, partial);
+                     dim3(64), 0, ctx->stream, tgt, nt, src, boxes, f.nsub, f.per, fc, nt, partial,
+                     skip);
   MF_LAUNCH_CHECK();
   return Status::Ok();
 }
@@ -1533,7 +1539,8 @@ Status self_passes(mf_ctx *ctx, int64_t n, const SelfSplit &f, double *partial, 
 namespace {
 // The partial sums of the field of a record set on itself.
 Status field_self_chunks(mf_ctx *ctx, const SrcRec *rec, const float4 *boxes, int64_t n,
-                         const FieldConsts &fc, double **partial, int *nchunk) {
+                         const FieldConsts &fc, double **partial, int *nchunk,
+                         const Skip &skip = {}) {
   if (n >= kSelfMin) {
     const SelfSplit f = self_split(ctx, n);
     void *pw = nullptr;
@@ -1543,7 +1550,7 @@ Status field_self_chunks(mf_ctx *ctx, const SrcRec *rec, const float4 *boxes, in
       return self_passes(ctx, n, f, *partial, nchunk, [&](const SelfWalk &w, double *slots) {
         hipLaunchKernelGGL(field_self_kernel<kSelfW>,
                            dim3(static_cast<unsigned>(w.ngroups), static_cast<unsigned>(w.nchunk)),
-                           dim3(64 * kSelfW), 0, ctx->stream, rec, boxes, n, w, fc, slots);
+                           dim3(64 * kSelfW), 0, ctx->stream, rec, boxes, n, w, fc, slots, skip);
       });
     }
   }
@@ -1551,7 +1558,7 @@ Status field_self_chunks(mf_ctx *ctx, const SrcRec *rec, const float4 *boxes, in
   MF_TRY(field_workspace(ctx, n, n, partial, &cap));
   const Split d = split_sources(ctx, n, n, kFieldTPT, kMaxChunks);
   *nchunk = static_cast<int>(d.nchunk);
-  return field_chunks(ctx, record_points(rec), n, rec, boxes, fc, d, *partial);
+  return field_chunks(ctx, record_points(rec), n, rec, boxes, fc, d, *partial, skip);
 }
 }  // namespace
 
@@ -1561,7 +1568,7 @@ Status field_allpairs_ap(mf_ctx *ctx, const SrcRec *rec, const float4 *boxes, in
                          const FieldConsts &fc, const ApOut &out) {
   double *partial = nullptr;
   int nchunk = 0;
-  MF_TRY(field_self_chunks(ctx, rec, boxes, n, fc, &partial, &nchunk));
+  MF_TRY(field_self_chunks(ctx, rec, boxes, n, fc, &partial, &nchunk, out.skip));
   MF_REDUCE(reduce_ap_kernel, n, n, n, nchunk, partial, out);
   return Status::Ok();
 }

@@ -62,6 +62,15 @@ Status field_allpairs_launch_ws(mf_ctx *ctx, const Points &tgt, int64_t nt, cons
                                 const float *hconst, float *ox, float *oy, float *oz,
                                 double *partial, int64_t partial_cap);
 int64_t field_partial_doubles(int64_t nt, int64_t nchunk);
+// A product whose use the host has not decided yet when it is launched: its kernels end at
+// once where *rr < below (a solve that has converged).
+struct Skip {
+  const double *rr = nullptr;  // null: never
+  double below = 0.0;
+};
+#ifdef __HIPCC__
+__device__ __forceinline__ bool skipped(const Skip &s) { return s.rr && *s.rr < s.below; }
+#endif
 // The product of a conjugate-gradient step on one record set (its moments
 // packed): ap = p - G m, and dots[b] (b < field_ap_blocks(n)) the parts of
 // p . ap.
@@ -69,6 +78,7 @@ struct ApOut {
   const float *p[3];
   float *ap[3];
   double *dots;
+  Skip skip;
 };
 // out = hconst + G m of one record set on itself.
 Status field_self_launch(mf_ctx *ctx, const SrcRec *rec, const float4 *boxes, int64_t n,

@@ -13,6 +13,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 #include "mf_internal.hpp"
@@ -204,7 +205,8 @@ __global__ __launch_bounds__(kRedBlock) void cg_p_kernel(int64_t n, const double
   const double old = *rr_old;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     *rr_new = rr;
-    *host = rr;
+    // the host may be waiting for it (wait_scalar)
+    __hip_atomic_store(host, rr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
   const float beta = static_cast<float>(old != 0.0 ? rr / old : 0.0);
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * kRedBlock + threadIdx.x; i < n;
@@ -422,6 +424,39 @@ bool relax_products(mf_plan *plan, const mf_solve_opts &o, double rel_residual) 
   return true;
 }
 
+// Particles up to which an all-pairs solve launches the next iteration's product before
+// it knows the residual: the product of 50,000 takes 0.9 ms, of which a host round trip of
+// about 8 us is nothing.
+constexpr int64_t kAheadMax = 32768;
+
+// A scalar that a kernel will store to pinned memory: pending(), then the launch, then
+// wait_scalar() as the host needs it.
+constexpr uint64_t kPending = 0x7ff4dead00c0ffeeULL;  // a NaN that arithmetic does not make
+void pending(mf_ctx *ctx) {
+  __atomic_store_n(reinterpret_cast<uint64_t *>(ctx->host_scalars), kPending, __ATOMIC_RELEASE);
+}
+Status wait_scalar(mf_ctx *ctx, double *out) {
+  const uint64_t *p = reinterpret_cast<const uint64_t *>(ctx->host_scalars);
+  uint64_t v = __atomic_load_n(p, __ATOMIC_ACQUIRE);
+  for (int spin = 1; v == kPending; ++spin) {
+    if (spin % 2048 == 0) {
+      // a stream that has ended, or failed, ends the wait
+      const hipError_t e = hipStreamQuery(ctx->stream);
+      if (e == hipErrorNotReady) {
+        (void)hipGetLastError();
+      } else {
+        MF_HIP(e);
+        v = __atomic_load_n(p, __ATOMIC_ACQUIRE);
+        break;
+      }
+    }
+    __builtin_ia32_pause();
+    v = __atomic_load_n(p, __ATOMIC_ACQUIRE);
+  }
+  std::memcpy(out, &v, sizeof(v));
+  return Status::Ok();
+}
+
 Status solve_cg(mf_plan *plan, double kappa, CV3 b, V3 x, const mf_solve_opts &o,
                 mf_solve_stats *st) {
   mf_ctx *ctx = plan->ctx;
@@ -461,11 +496,20 @@ Status solve_cg(mf_plan *plan, double kappa, CV3 b, V3 x, const mf_solve_opts &o
   M2LOverrideGuard guard(plan);
   bool relaxed = false;
   int it = 0;
-  while (std::sqrt(rr) > tol && st->matvecs < o.maxit) {
+  // An all-pairs product only writes scratch, so the next one is launched before the
+  // residual is known, and the host's round trip (8 us) passes under it.  Its kernels end at
+  // once where the residual is clearly below the tolerance (in doubt they run, unused).  Step
+  // of 512 particles 0.217 -> 0.201 ms, of 8,192 with magnets 0.544 -> 0.511.
+  const bool ahead = pairs && n <= kAheadMax && !ctx->timing;
+  bool issued = false, lost = false;
+  auto product = [&](const Skip &skip) -> Status {
+    return field_allpairs_ap(ctx, plan->rec.as<SrcRec>(), plan->boxes.as<float4>(), n, plan->fc,
+                             ApOut{{pc.x, pc.y, pc.z}, {ap.x, ap.y, ap.z}, dots, skip});
+  };
+  while (!lost && std::sqrt(rr) > tol && st->matvecs < o.maxit) {
     if (!relaxed) relaxed = relax_products(plan, o, std::sqrt(rr) / (bn > 0.0 ? bn : 1.0));
     if (pairs) {
-      MF_TRY(field_allpairs_ap(ctx, plan->rec.as<SrcRec>(), plan->boxes.as<float4>(), n, plan->fc,
-                               ApOut{{pc.x, pc.y, pc.z}, {ap.x, ap.y, ap.z}, dots}));
+      if (!issued) MF_TRY(product(Skip{}));
     } else {
       MF_TRY(plan_apply_G(plan, static_cast<float>(kappa), w.p, w.p + n, w.p + 2 * n, nullptr, w.g,
                           w.g + n, w.g + 2 * n));
@@ -479,15 +523,24 @@ Status solve_cg(mf_plan *plan, double kappa, CV3 b, V3 x, const mf_solve_opts &o
     hipLaunchKernelGGL(cg_xr_kernel, dim3(nb), dim3(kRedBlock), 0, ctx->stream, n, rr_old,
                        static_cast<const double *>(dots), ndots, pc, apc, x, r, w.partials);
     MF_LAUNCH_CHECK();
-    hipLaunchKernelGGL(cg_p_kernel, dim3(nb), dim3(kRedBlock), 0, ctx->stream, n, rr_old,
-                       w.sc + (it & 1 ? S_RR0 : S_RR1), host_dev,
-                       static_cast<const double *>(w.partials), nb, rc, p, rec);
+    if (ahead) pending(ctx);
+    double *rr_new = w.sc + (it & 1 ? S_RR0 : S_RR1);
+    hipLaunchKernelGGL(cg_p_kernel, dim3(nb), dim3(kRedBlock), 0, ctx->stream, n, rr_old, rr_new,
+                       host_dev, static_cast<const double *>(w.partials), nb, rc, p, rec);
     MF_LAUNCH_CHECK();
     ++it;
-    MF_HIP(hipStreamSynchronize(ctx->stream));
-    rr = host[0];
-    if (!std::isfinite(rr)) return Status::Err(MF_ERR_NOT_CONVERGED, "CG residual is not finite");
+    if (ahead) {
+      issued = st->matvecs < o.maxit;
+      if (issued) MF_TRY(product(Skip{rr_new, 0.999 * tol * tol}));
+      MF_TRY(wait_scalar(ctx, &rr));
+    } else {
+      MF_HIP(hipStreamSynchronize(ctx->stream));
+      rr = host[0];
+    }
+    lost = !std::isfinite(rr);
   }
+  if (ahead) MF_HIP(hipStreamSynchronize(ctx->stream));
+  if (lost) return Status::Err(MF_ERR_NOT_CONVERGED, "CG residual is not finite");
   st->iterations = it;
   st->rel_residual = std::sqrt(rr) / (bn > 0.0 ? bn : 1.0);
   st->converged = std::sqrt(rr) <= tol;

@@ -122,3 +122,31 @@ def test_few_sources_vs_oracle(ctx, oracle, nt, ns):
         torch.cuda.synchronize()
         assert rc == magforce.MF_OK
         assert rel_err(host(buf[:, :nt]), host(got)) < 2 * TOL  # each within TOL of the oracle
+
+
+@pytest.mark.parametrize("n", [1, 65, 700, 4096, 4999])
+@pytest.mark.parametrize("maxit", [1, 3, 100])
+def test_product_launched_ahead(oracle, n, maxit):
+    """A CG solve launches the next product before it knows the residual, and with kernel
+    timing on it waits first: the same solution, counts and residual bit for bit, from
+    solves that converge and that maxit stops, one after the other on one context."""
+    import magforce
+    pos = f32(jittered_block(18, 18, 18, seed=n))[:n]
+    b = f32(random_moments(n, seed=n + 5))
+    out = []
+    for timing in (False, True, False):
+        c = magforce.Context(0)
+        plan = magforce.Plan(c, dev(pos), 2.0)
+        c.enable_timing(timing)
+        res = [plan.solve(0.5, dev(b), rtol=rtol, maxit=maxit) for rtol in (1e-6, 1e-3)]
+        out.append([(host(r.x), {k: r.stats[k] for k in ("matvecs", "iterations", "rel_residual",
+                                                         "converged")}) for r in res])
+        plan.close()
+        c.close()
+    for other in out[1:]:
+        for (x, st), (y, su) in zip(out[0], other):
+            assert np.array_equal(x, y) and st == su, (st, su)
+    assert all(st["matvecs"] <= maxit for _, st in out[0])
+    if maxit == 100:
+        want, _, _ = oracle.cg_solve(pos, 2.0, 0.5, b, rtol=1e-12)
+        assert rel_err(out[0][0][0], want) < TOL
