@@ -2,9 +2,11 @@
 //
 // Replaces the reference's naive kernels (magnetic_solver/magnetic_force.cu):
 //   cuda_Apply_G            :8-110    -> field_allpairs_kernel
-//   cuda_ext_field_kernel   :120-237  -> field_allpairs_kernel (separate sources)
+//   cuda_ext_field_kernel   :120-237  -> field_allpairs_kernel (separate sources),
+//                                        field_few_kernel (a few of them)
 //   fitted_force_ofM_kernel :516-605  -> force_allpairs_kernel
-//   cuda_ext_fitted_force_tensor_kernel :432-512 -> hessian_allpairs_kernel
+//   cuda_ext_fitted_force_tensor_kernel :432-512 -> hessian_allpairs_kernel,
+//                                        hessian_few_kernel
 //
 // Design (one wavefront = 16 TPT targets):
 //  * Sources live in HBM as 32-byte records {x,y,z,0, mx,my,mz,0}, padded to a
@@ -48,7 +50,6 @@
 namespace mf {
 
 namespace {
-
 
 // ---------------------------------------------------------------------------
 // Near-pair coefficient tables (mf_pair.hpp describes their entries).  The

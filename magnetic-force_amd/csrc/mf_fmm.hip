@@ -28,10 +28,10 @@
 //    offset list; per offset it gathers the 64 source multipoles into LDS and
 //    multiplies by the offset's matrix, accumulating the 64 local expansions
 //    in registers.
-//  * Leaf pass: L2P (one wave per leaf, local expansion through scalar loads)
-//    writes H_const + far field in the caller's particle order; the near-field
-//    kernel then adds the sums over the leaf's near boxes, whose particle
-//    ranges are merged into contiguous runs at plan build.
+//  * Leaf pass: L2P (one wave per leaf, local expansion through scalar loads) writes the
+//    far field in FP64; beside it the near-field kernels evaluate each unordered pair of
+//    near leaf blocks once, and a gather adds far field, own sums and what the other
+//    blocks left for a particle.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
