@@ -641,9 +641,9 @@ __global__ __launch_bounds__(64) void field_few_kernel(Points tgt, int64_t nt, S
 // ---------------------------------------------------------------------------
 // Force: targets are the sources themselves (same records), target moment n.
 //   F = s sum_j [ d (P (m.n) + R (d.m)(d.n)) + m P (d.n) + n P (d.m) ]
-// with s = 3 mu0/(4 pi), accumulated as A_d (3), A_m (3), A_n (1).  With n5 = -5 n
-// and R / -5 = P / r^2 (far) the pair takes one multiply less; the m-sums then
-// hold P (d.n5).
+// with s = 3 mu0/(4 pi), accumulated as A_d (3), A_m (3), A_n (1); R = -5 P / r^2
+// (far).  -5 goes to the pair, not to n: rounding -5 n once per target would weigh on all of
+// its pairs.
 
 template <int TPT>
 __global__ __launch_bounds__(64) void force_allpairs_kernel(
@@ -655,7 +655,7 @@ __global__ __launch_bounds__(64) void force_allpairs_kernel(
   const int lane = threadIdx.x, c = lane & 15, q = lane >> 4;
   bool have_tab = false;  // read on the first mixed tile
   const int64_t tbase = static_cast<int64_t>(blockIdx.x) * (16 * TPT);
-  float tx[TPT], ty[TPT], tz[TPT], nx[TPT], ny[TPT], nz[TPT], nx5[TPT], ny5[TPT], nz5[TPT];
+  float tx[TPT], ty[TPT], tz[TPT], nx[TPT], ny[TPT], nz[TPT];
 #pragma unroll
   for (int k = 0; k < TPT; ++k) {
     const SrcRec t = tgt[min(tbase + 16 * k + c, nt - 1)];
@@ -665,9 +665,6 @@ __global__ __launch_bounds__(64) void force_allpairs_kernel(
     nx[k] = t.mx;
     ny[k] = t.my;
     nz[k] = t.mz;
-    nx5[k] = -5.f * nx[k];
-    ny5[k] = -5.f * ny[k];
-    nz5[k] = -5.f * nz[k];
   }
   double acc[TPT][3];
   float ad[TPT][3], am[TPT][3], an[TPT];
@@ -694,16 +691,16 @@ __global__ __launch_bounds__(64) void force_allpairs_kernel(
           const float ir2 = ir * ir;
           const float P = ir2 * ir2 * ir;  // r^-5
           const float dm = fmaf(dx, u.w, fmaf(dy, v.x, dz * v.y));
-          const float dn5 = fmaf(dx, nx5[k], fmaf(dy, ny5[k], dz * nz5[k]));
+          const float dn = fmaf(dx, nx[k], fmaf(dy, ny[k], dz * nz[k]));
           const float mn = fmaf(u.w, nx[k], fmaf(v.x, ny[k], v.y * nz[k]));
-          const float e = P * fmaf(dm * ir2, dn5, mn);  // P mn + R dm dn, R = -5 P ir2
-          const float f5 = P * dn5;
+          const float e = P * fmaf(-5.f * ir2 * dm, dn, mn);  // P mn + R dm dn
+          const float f1 = P * dn;
           ad[k][0] = fmaf(dx, e, ad[k][0]);
           ad[k][1] = fmaf(dy, e, ad[k][1]);
           ad[k][2] = fmaf(dz, e, ad[k][2]);
-          am[k][0] = fmaf(u.w, f5, am[k][0]);
-          am[k][1] = fmaf(v.x, f5, am[k][1]);
-          am[k][2] = fmaf(v.y, f5, am[k][2]);
+          am[k][0] = fmaf(u.w, f1, am[k][0]);
+          am[k][1] = fmaf(v.x, f1, am[k][1]);
+          am[k][2] = fmaf(v.y, f1, am[k][2]);
           an[k] = fmaf(P, dm, an[k]);
         }
       }
@@ -733,16 +730,16 @@ __global__ __launch_bounds__(64) void force_allpairs_kernel(
           }
           const float P = c1 * ir;
           const float dm = fmaf(dx, u.w, fmaf(dy, v.x, dz * v.y));
-          const float dn5 = fmaf(dx, nx5[k], fmaf(dy, ny5[k], dz * nz5[k]));
+          const float dn = fmaf(dx, nx[k], fmaf(dy, ny[k], dz * nz[k]));
           const float mn = fmaf(u.w, nx[k], fmaf(v.x, ny[k], v.y * nz[k]));
-          const float e = fmaf(dq * (ir2 * ir), dm * dn5, P * mn);
-          const float f5 = P * dn5;
+          const float e = fmaf(-5.f * dq * (ir2 * ir), dm * dn, P * mn);
+          const float f1 = P * dn;
           ad[k][0] = fmaf(dx, e, ad[k][0]);
           ad[k][1] = fmaf(dy, e, ad[k][1]);
           ad[k][2] = fmaf(dz, e, ad[k][2]);
-          am[k][0] = fmaf(u.w, f5, am[k][0]);
-          am[k][1] = fmaf(v.x, f5, am[k][1]);
-          am[k][2] = fmaf(v.y, f5, am[k][2]);
+          am[k][0] = fmaf(u.w, f1, am[k][0]);
+          am[k][1] = fmaf(v.x, f1, am[k][1]);
+          am[k][2] = fmaf(v.y, f1, am[k][2]);
           an[k] = fmaf(P, dm, an[k]);
         }
       }
@@ -755,8 +752,7 @@ __global__ __launch_bounds__(64) void force_allpairs_kernel(
       const double s = static_cast<double>(an[k]);
 #pragma unroll
       for (int a = 0; a < 3; ++a) {
-        // the m-sums hold -5 times their terms
-        acc[k][a] += (static_cast<double>(ad[k][a]) - 0.2 * static_cast<double>(am[k][a])) + n3[a] * s;
+        acc[k][a] += (static_cast<double>(ad[k][a]) + static_cast<double>(am[k][a])) + n3[a] * s;
         ad[k][a] = am[k][a] = 0.f;
       }
       an[k] = 0.f;
