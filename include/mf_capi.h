@@ -310,7 +310,9 @@ int mf_plan_create_batch(mf_ctx *ctx, int nsys, const int64_t *offsets, const fl
  * a system stops updating once ||r_s|| <= rtol ||b_s||.  kappa: host, nsys.
  * opts: method must be MF_SOLVE_CG (rtol, maxit, zero_start honoured).
  * stats->rel_residual is the largest per-system relative residual;
- * sys_rel_residual (host, nsys, may be NULL) receives each system's. */
+ * sys_rel_residual (host, nsys, may be NULL) receives each system's.  A system
+ * whose residual is NaN (NaN in its b or x, say) is left where it is while the
+ * others are solved; rel_residual is then NaN and converged 0. */
 int mf_plan_solve_batch(mf_plan *plan, const double *kappa, const float *bx, const float *by,
                         const float *bz, float *xx, float *xy, float *xz,
                         const mf_solve_opts *opts, mf_solve_stats *stats,

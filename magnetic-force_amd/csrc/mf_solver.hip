@@ -1014,12 +1014,15 @@ __global__ __launch_bounds__(kRedBlock) void bcg_xr_kernel(const int64_t *__rest
 }
 
 // r.r from the partials, beta, activity and the largest relative residual
-// (one block).
+// (one block).  A system whose residual is NaN is frozen and does not stop the
+// others; maxratio[0] is the largest residual of the others, maxratio[1] whether
+// there is such a system (fmax alone would drop it).
 __global__ __launch_bounds__(kRedBlock) void bcg_beta_kernel(int nsys,
                                                              const int32_t *__restrict__ seg_first,
                                                              double rtol, int first, SegState st) {
   __shared__ double sh[kRedBlock];
   double mx = 0.0;
+  int lost = 0;
   for (int s = threadIdx.x; s < nsys; s += kRedBlock) {
     const double bn = st.bb[s] > 0.0 ? sqrt(st.bb[s]) : 1.0;
     const double rrn = system_sum(seg_first, st.partial, s);
@@ -1035,14 +1038,18 @@ __global__ __launch_bounds__(kRedBlock) void bcg_beta_kernel(int nsys,
     const double ratio = sqrt(st.rr[s]) / bn;
     st.active[s] = (st.active[s] || first) && ratio > rtol ? 1 : 0;
     mx = fmax(mx, ratio);
+    lost |= ratio != ratio;
   }
   sh[threadIdx.x] = mx;
-  __syncthreads();
+  lost = __syncthreads_or(lost);  // also orders the writes above
   for (int o = kRedBlock / 2; o > 0; o >>= 1) {
     if (threadIdx.x < o) sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + o]);
     __syncthreads();
   }
-  if (threadIdx.x == 0) st.maxratio[0] = sh[0];
+  if (threadIdx.x == 0) {
+    st.maxratio[0] = sh[0];
+    st.maxratio[1] = lost ? 1.0 : 0.0;
+  }
 }
 
 __global__ void bcg_p_kernel(int64_t n, const int32_t *__restrict__ sys_of,
@@ -1277,9 +1284,10 @@ Status solve_batch(mf_plan *plan, const double *kappa, const float *bx, const fl
     mx = ctx->host_scalars[0];
     if (!std::isfinite(mx)) return Status::Err(MF_ERR_NOT_CONVERGED, "CG residual is not finite");
   }
+  const bool lost = ctx->host_scalars[1] != 0.0;  // a system's residual is NaN
   st->iterations = it;
-  st->rel_residual = mx;
-  st->converged = mx <= rtol;
+  st->rel_residual = lost ? std::nan("") : mx;
+  st->converged = mx <= rtol && !lost;
   if (sys_rel_residual) {
     std::vector<double> rr(nsys), bb(nsys);
     MF_HIP(hipMemcpyAsync(rr.data(), S.rr, sizeof(double) * nsys, hipMemcpyDeviceToHost, ctx->stream));
