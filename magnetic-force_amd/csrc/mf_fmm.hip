@@ -2501,33 +2501,44 @@ Status build_once(mf_ctx *ctx, FmmState &F, const FmmTables &tab, int nleaf, int
 // room for one more stream.  A pass takes all places, or what kOnceBytes hold, or where
 // that much cannot be had half as much and so on: each halving costs a launch and a gather,
 // and below kOnceBytesLeast a refusal is an error, as for any other buffer.  The plan build
-// chooses, so that a product asks for what is there.
+// chooses, once it has every other buffer of the plan and its products, so that a product
+// asks for what is there.
 constexpr int64_t kOnceBytes = int64_t{12} << 30, kOnceBytesLeast = int64_t{256} << 20;
 
 // Buffers of a near-field product: nn's, the particles' own sums, and with several
-// passes what the earlier ones left.
+// passes what the earlier ones left.  A pass takes at most `cap` bytes of places; with
+// `taken`, it receives the bytes that were chosen.
 Status once_buffers(mf_ctx *ctx, FmmState::Once &o, int64_t n, OnceNear &nn, double **near3,
-                    double **rest3) {
+                    double **rest3, int64_t cap = kOnceBytes, int64_t *taken = nullptr) {
   void *p = nullptr;
   MF_TRY(workspace(ctx, "fmm_near3", sizeof(double) * 3 * static_cast<size_t>(n), &p));
   *near3 = static_cast<double *>(p);
   *rest3 = nullptr;
   const int64_t all = 12 * 16 * static_cast<int64_t>(o.window > 0 ? o.window : std::max(o.units, 1));
-  for (int64_t most = std::min(all, kOnceBytes);; most /= 2) {
+  for (int64_t most = std::min(all, cap);; most /= 2) {
+    if (taken) *taken = most;
     const int64_t w = std::max<int64_t>(std::min<int64_t>(o.units, most / (12 * 16)), 1);
     o.window = static_cast<int>(w);
     o.passes = static_cast<int>(std::max<int64_t>((o.units + w - 1) / w, 1));
     nn.len = 16 * (w + (o.passes > 1 ? o.longest : 0));
+    if (o.passes > 1) {
+      MF_TRY(workspace(ctx, "fmm_rest3", sizeof(double) * 3 * static_cast<size_t>(n), &p));
+      *rest3 = static_cast<double *>(p);
+    }
     const Status s = workspace(ctx, "fmm_pair_sums", 12 * static_cast<size_t>(nn.len), &p);
     if (s.ok()) break;
     if (s.code != MF_ERR_ALLOC || most <= kOnceBytesLeast) return s;
     (void)hipGetLastError();  // a smaller buffer may be had
   }
   nn.sums = static_cast<float *>(p);
-  if (o.passes > 1) {
-    MF_TRY(workspace(ctx, "fmm_rest3", sizeof(double) * 3 * static_cast<size_t>(n), &p));
-    *rest3 = static_cast<double *>(p);
-  }
+  return Status::Ok();
+}
+
+// The far part of a product, [3][n] in sorted order.
+Status far_buffer(mf_ctx *ctx, int64_t n, double **far3) {
+  void *p = nullptr;
+  MF_TRY(workspace(ctx, "fmm_far3", sizeof(double) * 3 * static_cast<size_t>(n), &p));
+  *far3 = static_cast<double *>(p);
   return Status::Ok();
 }
 
@@ -2795,10 +2806,6 @@ Status fmm_build_at(mf_plan *plan, double s_leaf, int *wider = nullptr) {
     F.onceF.longest = once[0][2];
     F.onceH.units = once[1][0] + once[1][1];
     F.onceH.longest = once[1][2];
-    OnceNear nn{};
-    double *near3 = nullptr, *rest3 = nullptr;
-    MF_TRY(once_buffers(ctx, F.onceF, n, nn, &near3, &rest3));
-    MF_TRY(once_buffers(ctx, F.onceH, n, nn, &near3, &rest3));
   }
   // 5. M2L source slots (levels >= 2) and the class-sorted tile lists
   // one row past the last box of each slot array holds -1 throughout: the
@@ -3024,6 +3031,16 @@ Status fmm_build_at(mf_plan *plan, double s_leaf, int *wider = nullptr) {
     if (boxes > 0) MF_TRY(need<float>(F.Lp, boxes * F.KP));
   }
   MF_TRY(need<uint16_t>(F.Mb, static_cast<int64_t>(F.nbox) * 3 * F.KP));
+  {
+    // Last: the places take what memory the rest leaves.  The force's near set holds the
+    // field's, so a buffer with the force's window has room for as large a one of the field's.
+    OnceNear nn{};
+    double *near3 = nullptr, *rest3 = nullptr, *far3 = nullptr;
+    int64_t taken = 0;
+    MF_TRY(far_buffer(ctx, n, &far3));
+    MF_TRY(once_buffers(ctx, F.onceH, n, nn, &near3, &rest3, kOnceBytes, &taken));
+    MF_TRY(once_buffers(ctx, F.onceF, n, nn, &near3, &rest3, taken));
+  }
   F.counts_valid = false;  // work counts are computed on the first fmm_info
   return Status::Ok();
 }
@@ -3414,11 +3431,7 @@ Status apply_field_impl(mf_plan *plan, float scale, const float *px, const float
   double *near3 = nullptr, *rest3 = nullptr;
   MF_TRY(once_buffers(ctx, F.onceF, n, nn, &near3, &rest3));
   double *far3 = nullptr;
-  if (use_far) {
-    void *pf = nullptr;
-    MF_TRY(workspace(ctx, "fmm_far3", sizeof(double) * 3 * static_cast<size_t>(n), &pf));
-    far3 = static_cast<double *>(pf);
-  }
+  if (use_far) MF_TRY(far_buffer(ctx, n, &far3));
   auto gather = [&](hipStream_t st, int pass, int passes) -> Status {
     const auto kernel = passes == 1 ? near_gather_kernel<kNearF, true> : near_gather_kernel<kNearF, false>;
     hipLaunchKernelGGL(kernel, dim3(nleaf), dim3(256), 0, st,
@@ -3498,11 +3511,7 @@ Status apply_force_impl(mf_plan *plan, const float *mx, const float *my, const f
   double *near3 = nullptr, *rest3 = nullptr;
   MF_TRY(once_buffers(ctx, F.onceH, n, nn, &near3, &rest3));
   double *far3 = nullptr;
-  {
-    void *pf = nullptr;
-    MF_TRY(workspace(ctx, "fmm_far3", sizeof(double) * 3 * static_cast<size_t>(n), &pf));
-    far3 = static_cast<double *>(pf);
-  }
+  MF_TRY(far_buffer(ctx, n, &far3));
   auto gather = [&](hipStream_t st, int pass, int passes) -> Status {
     const auto kernel = passes == 1 ? near_gather_kernel<kNearH, true> : near_gather_kernel<kNearH, false>;
     hipLaunchKernelGGL(kernel, dim3(nleaf), dim3(256), 0, st,
