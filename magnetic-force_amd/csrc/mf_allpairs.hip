@@ -1461,8 +1461,9 @@ constexpr int kSelfW = 4;
 constexpr int64_t kSelfMin = 4096;
 constexpr int64_t kSelfUnitsMin = 4;
 // The slots grow with the square of n: beyond kSelfBytes the group distances go in
-// passes, each folded into one slot before the next.
-constexpr int64_t kSelfBytes = int64_t{2} << 30;
+// passes, each folded into one slot before the next.  Where that much cannot be had, half
+// as much and so on (self_slots); below kSelfBytesLeast the directed kernels take over.
+constexpr int64_t kSelfBytes = int64_t{2} << 30, kSelfBytesLeast = int64_t{128} << 20;
 struct SelfSplit {
   SelfWalk w;     // the walk's constants
   int dist;       // group distances 0 .. dist - 1
@@ -1476,12 +1477,12 @@ int self_chunks(const mf_ctx *ctx, const SelfWalk &w, int units) {
       std::min<int64_t>((fill * kFills + w.ngroups - 1) / w.ngroups, units / kSelfUnitsMin);
   return static_cast<int>(std::max<int64_t>(std::max(one, many), 1));
 }
-SelfSplit self_split(const mf_ctx *ctx, int64_t n) {
+SelfSplit self_split(const mf_ctx *ctx, int64_t n, int64_t bytes) {
   SelfSplit f{};
   f.w.ntiles = static_cast<int>((n + kTile - 1) / kTile);
   f.w.ngroups = ((f.w.ntiles + kSelfW - 1) / kSelfW) | 1;
   f.dist = f.w.ngroups / 2 + 1;
-  const int64_t fit = std::max<int64_t>(kSelfBytes / (24 * n), 2);
+  const int64_t fit = std::max<int64_t>(bytes / (24 * n), 2);
   const int chunks = self_chunks(ctx, f.w, kSelfW * f.dist);
   if (chunks + f.dist - 1 <= fit) {
     f.per_pass = f.dist;
@@ -1492,6 +1493,25 @@ SelfSplit self_split(const mf_ctx *ctx, int64_t n) {
   f.per_pass = static_cast<int>(std::max<int64_t>(fit - std::min<int64_t>(chunks, fit / 2), 1));
   f.slots = 1 + f.per_pass + self_chunks(ctx, f.w, kSelfW * f.per_pass);
   return f;
+}
+
+// Split and slots of a product (kind 0 field, 1 force); false: none can be had now.  What
+// was refused is remembered (mf_ctx::self_bytes), so that later products do not ask for it.
+bool self_slots(mf_ctx *ctx, int kind, const char *name, int64_t n, SelfSplit *f, double **slots) {
+  int64_t &may = ctx->self_bytes[kind];
+  while (true) {
+    const int64_t bytes = std::min(kSelfBytes, may);
+    *f = self_split(ctx, n, bytes);
+    const int64_t need = 24 * n * f->slots;
+    if (f->per_pass < f->dist && bytes < kSelfBytesLeast) return false;
+    void *pw = nullptr;
+    if (workspace_now(ctx, name, static_cast<size_t>(need), &pw)) {
+      *slots = static_cast<double *>(pw);
+      return true;
+    }
+    if (stream_capturing(ctx)) return false;
+    may = std::min(bytes, need) / 2;
+  }
 }
 
 // sum[i] (+)= the pass's slots.
@@ -1538,18 +1558,14 @@ namespace {
 Status field_self_chunks(mf_ctx *ctx, const SrcRec *rec, const float4 *boxes, int64_t n,
                          const FieldConsts &fc, double **partial, int *nchunk,
                          const Skip &skip = {}) {
-  if (n >= kSelfMin) {
-    const SelfSplit f = self_split(ctx, n);
-    void *pw = nullptr;
-    if (workspace_now(ctx, "field_partial", sizeof(double) * 3 * n * f.slots, &pw)) {
-      *partial = static_cast<double *>(pw);
-      KernelTimer timer(ctx, "field");
-      return self_passes(ctx, n, f, *partial, nchunk, [&](const SelfWalk &w, double *slots) {
-        hipLaunchKernelGGL(field_self_kernel<kSelfW>,
-                           dim3(static_cast<unsigned>(w.ngroups), static_cast<unsigned>(w.nchunk)),
-                           dim3(64 * kSelfW), 0, ctx->stream, rec, boxes, n, w, fc, slots, skip);
-      });
-    }
+  SelfSplit f;
+  if (n >= kSelfMin && self_slots(ctx, 0, "field_partial", n, &f, partial)) {
+    KernelTimer timer(ctx, "field");
+    return self_passes(ctx, n, f, *partial, nchunk, [&](const SelfWalk &w, double *slots) {
+      hipLaunchKernelGGL(field_self_kernel<kSelfW>,
+                         dim3(static_cast<unsigned>(w.ngroups), static_cast<unsigned>(w.nchunk)),
+                         dim3(64 * kSelfW), 0, ctx->stream, rec, boxes, n, w, fc, slots, skip);
+    });
   }
   int64_t cap = 0;
   MF_TRY(field_workspace(ctx, n, n, partial, &cap));
@@ -1586,20 +1602,17 @@ Status field_self_launch(mf_ctx *ctx, const SrcRec *rec, const float4 *boxes, in
 namespace {
 Status force_self_chunks(mf_ctx *ctx, const SrcRec *rec, const float4 *boxes, int64_t n,
                          const HessConsts &hc, double **partial, int *nchunk) {
-  void *pw = nullptr;
-  if (n >= kSelfMin) {
-    const SelfSplit f = self_split(ctx, n);
-    if (workspace_now(ctx, "force_partial", sizeof(double) * 3 * n * f.slots, &pw)) {
-      *partial = static_cast<double *>(pw);
-      KernelTimer timer(ctx, "force");
-      return self_passes(ctx, n, f, *partial, nchunk, [&](const SelfWalk &w, double *slots) {
-        hipLaunchKernelGGL(force_self_kernel<kSelfW>,
-                           dim3(static_cast<unsigned>(w.ngroups), static_cast<unsigned>(w.nchunk)),
-                           dim3(64 * kSelfW), 0, ctx->stream, rec, boxes, n, w, hc, slots);
-      });
-    }
+  SelfSplit f;
+  if (n >= kSelfMin && self_slots(ctx, 1, "force_partial", n, &f, partial)) {
+    KernelTimer timer(ctx, "force");
+    return self_passes(ctx, n, f, *partial, nchunk, [&](const SelfWalk &w, double *slots) {
+      hipLaunchKernelGGL(force_self_kernel<kSelfW>,
+                         dim3(static_cast<unsigned>(w.ngroups), static_cast<unsigned>(w.nchunk)),
+                         dim3(64 * kSelfW), 0, ctx->stream, rec, boxes, n, w, hc, slots);
+    });
   }
   const Split d = split_sources(ctx, n, n, kForceTPT, kMaxChunks);
+  void *pw = nullptr;
   MF_TRY(workspace(ctx, "force_partial", sizeof(double) * 3 * n * d.nchunk, &pw));
   *partial = static_cast<double *>(pw);
   *nchunk = static_cast<int>(d.nchunk);

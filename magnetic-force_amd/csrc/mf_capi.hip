@@ -44,15 +44,16 @@ Status workspace(mf_ctx *ctx, const std::string &name, size_t bytes, void **out)
   return Status::Ok();
 }
 
+bool stream_capturing(mf_ctx *ctx) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx->stream, &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
 bool workspace_now(mf_ctx *ctx, const std::string &name, size_t bytes, void **out) {
   const auto it = ctx->ws.find(name);
-  if (it == ctx->ws.end() || it->second.bytes() < bytes) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
-      (void)hipGetLastError();
-      return false;
-    }
-  }
+  if ((it == ctx->ws.end() || it->second.bytes() < bytes) && stream_capturing(ctx)) return false;
   const bool ok = workspace(ctx, name, bytes, out).ok();
   if (!ok) (void)hipGetLastError();
   return ok;
@@ -126,6 +127,7 @@ Status plan_set_positions(mf_plan *plan, int64_t n, const float *x, const float 
   plan->ready = false;
   plan->n = n;
   plan->pos64_valid = false;
+  ctx->self_bytes[0] = ctx->self_bytes[1] = INT64_MAX;
   const int64_t np = padded_sources(n);
   MF_HIP(hipStreamSynchronize(ctx->stream));
   MF_TRY(plan->rec.reserve(sizeof(SrcRec) * static_cast<size_t>(np > 0 ? np : 1)));

@@ -140,6 +140,9 @@ struct mf_ctx {
   double *host_scalars = nullptr;
   double *host_scalars_dev = nullptr;
   int num_cu = 256;
+  // Bytes that the slots of an all-pairs product of a set on itself (field, force) may
+  // take: less than was last refused, until positions are set again.
+  int64_t self_bytes[2] = {INT64_MAX, INT64_MAX};
 };
 
 namespace mf {
@@ -151,6 +154,7 @@ Status workspace(mf_ctx *ctx, const std::string &name, size_t bytes, void **out)
 // error) when the workspace would have to grow and cannot, because the stream
 // is being captured or the allocation fails.
 bool workspace_now(mf_ctx *ctx, const std::string &name, size_t bytes, void **out);
+bool stream_capturing(mf_ctx *ctx);
 
 // Records timing events around a kernel family when timing is enabled, on
 // the stream the family is launched on (the context's stream by default).
