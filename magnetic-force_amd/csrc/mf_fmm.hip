@@ -126,8 +126,9 @@ __device__ inline int find_key(const uint64_t *__restrict__ keys, int count, uin
 // Products of a batch plan inside its batched solve skip the boxes of
 // systems that have converged: box_sys[box] is the box's system, active[s]
 // (device, written by the solver) whether system s still iterates.  active ==
-// nullptr: every box runs.  The skipped boxes keep their last outputs, which
-// the solver no longer reads.
+// nullptr: every box runs.  The leaf kernels skip boxes, which keep their last outputs;
+// the translations skip whole tiles, and rewrite a converged box in a tile with live
+// ones.  Neither is read: no box takes anything from another system's.
 struct SysMask {
   const int32_t *box_sys = nullptr;
   const int32_t *active = nullptr;
@@ -681,9 +682,10 @@ __device__ __forceinline__ void m2l_part(int na, int parts, int part, int &lo, i
 }
 
 // Lt = the sum of its parts, in part order, for the boxes of the tiles that an M2L or
-// M2M launch split; grid.x the tiles, grid.y slices of one.  Boxes of converged systems are skipped.  Mb (or
-// null) receives the BF16 parts for the n2 boxes from lo2 on (a level's multipoles, or
-// the level-2 locals, which the first L2L reads).
+// M2M launch split; grid.x the tiles, grid.y slices of one.  A tile is skipped where the
+// launch skipped it: all of its boxes belong to converged systems.  Mb (or null) receives
+// the BF16 parts for the n2 boxes from lo2 on (a level's multipoles, or the level-2
+// locals, which the first L2L reads).
 template <int KP>
 __global__ __launch_bounds__(256) void sum_parts_kernel(
     const M2LTile *__restrict__ tiles, int ntiles, M2LSrc2 s, const int32_t *__restrict__ boxes,
@@ -692,10 +694,15 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(
   const int pos = static_cast<int>(blockIdx.x % 8) * per_xcd + s.whole + static_cast<int>(blockIdx.x / 8);
   if (pos >= ntiles) return;
   const M2LTile tile = tiles[s.order ? s.order[pos] : pos];
+  if (mask.active) {
+    int live = 0;
+    for (int j = threadIdx.x; j < tile.count; j += 256)
+      live |= mask.active[mask.box_sys[boxes[tile.first + j]]];
+    if (!__syncthreads_or(live)) return;  // uniform over the workgroup
+  }
   const int i = static_cast<int>(blockIdx.y) * 256 + static_cast<int>(threadIdx.x);
   if (i >= tile.count * (KP / 4)) return;
   const int box = boxes[tile.first + i / (KP / 4)], row = 4 * (i % (KP / 4));
-  if (sys_skip(mask, box)) return;
   const int64_t e = static_cast<int64_t>(box) * KP + row;
   float4 v = *reinterpret_cast<const float4 *>(s.Lp + e);
 #pragma unroll 4
