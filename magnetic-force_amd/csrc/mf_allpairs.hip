@@ -115,6 +115,28 @@ constexpr void shift_cubic(const double *c, double s, double *out) {
   out[3] = c[3];
 }
 
+// v_rsq_f32 is low by 7.4e-9 in the mean over all significands, and with it the r and the
+// q of a table lookup: the tables hold the curves at q (1 + kRsqLow).
+constexpr double kRsqLow = 7.4e-9;
+
+// The FP32 coefficients of a cubic over t in [0, 1] (dir = 1) or (-1, 0] (dir = -1).  What
+// the rounding of one coefficient takes off is given to the later ones, as their best fit
+// to it over the interval: of an error d of the constant term a quarter remains in the
+// mean square and a sixteenth in the mean.  Errors of neighbouring pairs, whose distances
+// read the same entries, do not average out: with the coefficients simply rounded a field
+// of equal moments on a jittered lattice at h = 2 was 3.4e-8 too large.
+constexpr void round_cubic(const double *c, int dir, float *out) {
+  out[0] = static_cast<float>(c[0]);
+  const double e0 = c[0] - static_cast<double>(out[0]);
+  const double c1 = c[1] + dir * 7.5 * e0;
+  out[1] = static_cast<float>(c1);
+  const double e1 = c1 - static_cast<double>(out[1]);
+  const double c2 = c[2] - 15.0 * e0 + dir * 3.0 * e1;
+  out[2] = static_cast<float>(c2);
+  const double e2 = c2 - static_cast<double>(out[2]);
+  out[3] = static_cast<float>(c[3] + dir * 8.75 * e0 - 2.1 * e1 + dir * (7.0 / 6.0) * e2);
+}
+
 // put(entry, cubic of alpha, cubic of beta) for every entry of the field table,
 // alpha times fa and beta times fb.
 template <class Put>
@@ -125,7 +147,7 @@ constexpr void fill_field_table(double fa, double fb, const Put &put) {
   for (int k = 0; k < kFieldTabN; ++k) {
     double ya[4] = {}, yb[4] = {};
     for (int i = 0; i < 4; ++i) {
-      near_coeffs_f64((k + t[i]) * 2.0 / kFieldTabN, ya[i], yb[i]);
+      near_coeffs_f64((k + t[i]) * (2.0 / kFieldTabN) * (1.0 + kRsqLow), ya[i], yb[i]);
       ya[i] *= fa;
       yb[i] *= fb;
     }
@@ -160,8 +182,8 @@ constexpr double kC2[4][5] = {
     {7.33485346367840e-10, -9.58855788627803e-09, 4.37085309763591e-08, -7.48004594092261e-08,
      2.34161209605651e-08}};
 
-// put(entry, cubic of C1, cubic of -(C2 - 3 C1) / 5) for every entry of the
-// force table, both times scale / (3 mu0 / (4 pi)).
+// put(entry, cubic of C1, cubic of C2 - 3 C1) for every entry of the force table,
+// both times scale / (3 mu0 / (4 pi)).
 template <class Put>
 constexpr void fill_hess_table(double scale, const Put &put) {
   const double f = scale / (3.0 * kMu0 / (4.0 * kPi));
@@ -173,14 +195,14 @@ constexpr void fill_hess_table(double scale, const Put &put) {
     const int piece = (e - 1) / per_unit;
     double yc[4] = {}, yd[4] = {};
     for (int i = 0; i < 4; ++i) {
-      const double q = (e + t[i]) / per_unit;
+      const double q = (e + t[i]) / per_unit * (1.0 + kRsqLow);
       double c1 = 0.0, c2 = 0.0;
       for (int j = 0; j < 5; ++j) {
         c1 = c1 * q + kC1[piece][j];
         c2 = c2 * q + kC2[piece][j];
       }
       yc[i] = f * c1;
-      yd[i] = -f * (c2 - 3.0 * c1) / 5.0;
+      yd[i] = f * (c2 - 3.0 * c1);
     }
     cubic_through(t, yc, cc);
     cubic_through(t, yd, cd);
@@ -208,20 +230,16 @@ struct UnitTable {
 constexpr UnitTable<kFieldTabEntries> unit_field_table() {
   UnitTable<kFieldTabEntries> t{};
   fill_field_table(1.0, 1.0, [&](int e, const double *a, const double *b) {
-    for (int j = 0; j < 4; ++j) {
-      t.v[0][e][j] = static_cast<float>(a[j]);
-      t.v[1][e][j] = static_cast<float>(b[j]);
-    }
+    round_cubic(a, 1, t.v[0][e]);
+    round_cubic(b, 1, t.v[1][e]);
   });
   return t;
 }
 constexpr UnitTable<kHessTabEntries> unit_hess_table() {
   UnitTable<kHessTabEntries> t{};
   fill_hess_table(1.0, [&](int e, const double *a, const double *b) {
-    for (int j = 0; j < 4; ++j) {
-      t.v[0][e][j] = static_cast<float>(a[j]);
-      t.v[1][e][j] = static_cast<float>(b[j]);
-    }
+    round_cubic(a, -1, t.v[0][e]);
+    round_cubic(b, -1, t.v[1][e]);
   });
   return t;
 }
@@ -230,11 +248,11 @@ static __device__ const UnitTable<kFieldTabEntries> d_field_tab __attribute__((a
 static __device__ const UnitTable<kHessTabEntries> d_hess_tab __attribute__((aligned(16))) =
     unit_hess_table();
 
-void store_entry(float *tab, int e, const double *ca, const double *cb) {
-  for (int j = 0; j < 4; ++j) {
-    tab[8 * e + j] = static_cast<float>(ca[j]);
-    tab[8 * e + 4 + j] = static_cast<float>(cb[j]);
-  }
+constexpr float kFieldTabMid = 0.5f, kHessTabMid = -0.5f;  // middle of an entry's t
+
+void store_entry(float *tab, int e, int dir, const double *ca, const double *cb) {
+  round_cubic(ca, dir, tab + 8 * e);
+  round_cubic(cb, dir, tab + 8 * e + 4);
 }
 
 __device__ __forceinline__ float wave_min(float v) {
@@ -478,12 +496,22 @@ __device__ __forceinline__ void walk_arrays(const SourceArrays &src, const WaveB
   }
 }
 
-// A unit table into the wave's LDS.
-template <int N>
-__device__ __forceinline__ void load_table(const UnitTable<N> &src, float4 (&dst)[2 * N], int lane) {
+// A unit table into LDS, its curves times consts.tab_a and tab_b, by `threads`.  Roundings
+// of the constants would weigh on all near pairs alike, so the factors are FP32 values and
+// what these leave, and the curves are moved by what tab_scale is off: u = (entry + t) is
+// high by tab_high of itself, the mean over the entry (at t = `mid`) taken for all of it.
+template <int N, class Consts>
+__device__ __forceinline__ void load_table(const UnitTable<N> &src, const Consts &consts, float mid,
+                                           float4 (&dst)[2 * N], int tid, int threads) {
   const float4 *__restrict__ t = reinterpret_cast<const float4 *>(&src);
-  for (int i = lane; i < 2 * N; i += 64) dst[i] = t[i];
-  __builtin_amdgcn_wave_barrier();
+  for (int i = tid; i < 2 * N; i += threads) {
+    const float4 c = t[i];
+    const float2 f = i < N ? consts.tab_a : consts.tab_b;
+    const float u = static_cast<float>(i < N ? i : i - N) + mid;
+    const float moved = -consts.tab_high * u * c.y * f.x;
+    dst[i] = make_float4(fmaf(c.x, f.x, fmaf(c.x, f.y, moved)), fmaf(c.y, f.x, c.y * f.y),
+                         fmaf(c.z, f.x, c.z * f.y), fmaf(c.w, f.x, c.w * f.y));
+  }
 }
 
 // Sum over the four lane groups (the same targets against a quarter of the
@@ -551,7 +579,8 @@ __device__ __forceinline__ void field_wave(const Points &tgt, int64_t nt, const 
     } else {
       // mixed tile: smoothed near field where q < 2
       if (!have_tab) {
-        load_table(d_field_tab, s_tab, lane);
+        load_table(d_field_tab, fc, kFieldTabMid, s_tab, lane, 64);
+        __builtin_amdgcn_wave_barrier();
         have_tab = true;
       }
 #pragma unroll 1
@@ -566,11 +595,7 @@ __device__ __forceinline__ void field_wave(const Points &tgt, int64_t nt, const 
           const float ir2 = ir * ir;
           float beta = ir2 * ir;
           float alpha = beta * ir2;
-          if (r2 < fc.near2) {
-            field_near_coeffs_tab(s_tab, fc.tab_scale, r2, ir, alpha, beta);
-            alpha *= fc.inv_h5;
-            beta *= fc.inv_h3;
-          }
+          if (r2 < fc.near2) field_near_coeffs_tab(s_tab, fc.tab_scale, r2, ir, alpha, beta);
           const float dm = fmaf(dx, u.w, fmaf(dy, v.x, dz * v.y));
           const float s1 = dm * alpha;
           a1[k][0] = fmaf(dx, s1, a1[k][0]);
@@ -706,7 +731,8 @@ __global__ __launch_bounds__(64) void force_allpairs_kernel(
       }
     } else {
       if (!have_tab) {
-        load_table(d_hess_tab, s_tab, lane);
+        load_table(d_hess_tab, hc, kHessTabMid, s_tab, lane, 64);
+        __builtin_amdgcn_wave_barrier();
         have_tab = true;
       }
 #pragma unroll 1
@@ -721,18 +747,18 @@ __global__ __launch_bounds__(64) void force_allpairs_kernel(
           // the clamp keeps a pair at d = 0 finite
           const float ir = __builtin_amdgcn_fmed3f(sp.ir[i], 0.f, 1e12f);
           const float ir2 = ir * ir;
-          float c1 = ir2 * ir2, dq = c1;  // far curves
+          float c1 = ir2 * ir2, dq = -5.f * c1;  // far curves
           if (!(r2 > hc.near2)) {
             hess_near_curves_tab(s_tab, hc.tab_scale, r2, ir, c1, dq);
-            const float w = r2 > 0.f ? hc.inv_h4 : 0.f;  // nothing at d = 0
-            c1 *= w;
-            dq *= w;
+            const bool apart = r2 > 0.f;  // nothing at d = 0
+            c1 = apart ? c1 : 0.f;
+            dq = apart ? dq : 0.f;
           }
           const float P = c1 * ir;
           const float dm = fmaf(dx, u.w, fmaf(dy, v.x, dz * v.y));
           const float dn = fmaf(dx, nx[k], fmaf(dy, ny[k], dz * nz[k]));
           const float mn = fmaf(u.w, nx[k], fmaf(v.x, ny[k], v.y * nz[k]));
-          const float e = fmaf(-5.f * dq * (ir2 * ir), dm * dn, P * mn);
+          const float e = fmaf(dq * (ir2 * ir), dm * dn, P * mn);
           const float f1 = P * dn;
           ad[k][0] = fmaf(dx, e, ad[k][0]);
           ad[k][1] = fmaf(dy, e, ad[k][1]);
@@ -806,7 +832,7 @@ template <class Pairs, class Consts, int W, int NTAB>
 __device__ __forceinline__ void self_walk(const SrcRec *__restrict__ rec,
                                           const float4 *__restrict__ boxes, int64_t n,
                                           const SelfWalk &w, const Consts &consts,
-                                          const UnitTable<NTAB> &table, double fac,
+                                          const UnitTable<NTAB> &table, float mid, double fac,
                                           double *__restrict__ partial) {
   __shared__ float4 s_tab[2 * NTAB];
   __shared__ SelfTile st[2];
@@ -814,10 +840,7 @@ __device__ __forceinline__ void self_walk(const SrcRec *__restrict__ rec,
   __shared__ double s_acc[W][3 * kSelfTPT][64];
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, q = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  {
-    const float4 *__restrict__ t = reinterpret_cast<const float4 *>(&table);
-    for (int i = tid; i < 2 * NTAB; i += 64 * W) s_tab[i] = t[i];
-  }
+  load_table(table, consts, mid, s_tab, tid, 64 * W);
   const int group = static_cast<int>(blockIdx.x), chunk = static_cast<int>(blockIdx.y);
   const int it = group * W + wave;  // the wave's i-tile
   const bool live = it < w.ntiles;
@@ -937,8 +960,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
                                                             int64_t n, SelfWalk w, FieldConsts fc,
                                                             double *__restrict__ partial, Skip skip) {
   if (skipped(skip)) return;
-  self_walk<FieldSelf<kSelfTPT>, FieldConsts, W, kFieldTabEntries>(rec, boxes, n, w, fc, d_field_tab,
-                                                         1.0 / (4.0 * kPi), partial);
+  self_walk<FieldSelf<kSelfTPT>, FieldConsts, W, kFieldTabEntries>(
+      rec, boxes, n, w, fc, d_field_tab, kFieldTabMid, 1.0 / (4.0 * kPi), partial);
 }
 
 template <int W>
@@ -946,8 +969,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
                                                             const float4 *__restrict__ boxes,
                                                             int64_t n, SelfWalk w, HessConsts hc,
                                                             double *__restrict__ partial) {
-  self_walk<ForceSelf<kSelfTPT>, HessConsts, W, kHessTabEntries>(rec, boxes, n, w, hc, d_hess_tab,
-                                                       3.0 * kMu0 / (4.0 * kPi), partial);
+  self_walk<ForceSelf<kSelfTPT>, HessConsts, W, kHessTabEntries>(
+      rec, boxes, n, w, hc, d_hess_tab, kHessTabMid, 3.0 * kMu0 / (4.0 * kPi), partial);
 }
 
 // ---------------------------------------------------------------------------
@@ -985,17 +1008,17 @@ __device__ __forceinline__ void hessian_wave(const Points &tgt, int64_t nt, cons
     const float mx = sp.u[i / TPT].w, my = sp.v[i / TPT].x, mz = sp.v[i / TPT].y;
     const float ir = near ? __builtin_amdgcn_fmed3f(sp.ir[i], 0.f, 1e12f) : sp.ir[i];
     const float ir2 = ir * ir;
-    float c1 = ir2 * ir2, dq = c1;
+    float c1 = ir2 * ir2, hq = -2.5f * c1;  // hq: half of R's curve
     if (near && !(r2 > hc.near2)) {
-      hess_near_curves_tab(s_tab, hc.tab_scale, r2, ir, c1, dq);
-      const float w = r2 > 0.f ? hc.inv_h4 : 0.f;  // nothing at d = 0
-      c1 *= w;
-      dq *= w;
+      hess_near_curves_tab(s_tab, hc.tab_scale, r2, ir, c1, hq);
+      const bool apart = r2 > 0.f;  // nothing at d = 0
+      c1 = apart ? c1 : 0.f;
+      hq = apart ? 0.5f * hq : 0.f;
     }
     const float P = c1 * ir;
     const float dm = fmaf(dx, mx, fmaf(dy, my, dz * mz));
     // T_ab = d_a (P m_b + (R/2) dm d_b) + (a <-> b) + delta_ab P dm
-    const float h = (-2.5f * dq) * (ir2 * ir) * dm;
+    const float h = hq * (ir2 * ir) * dm;
     const float gx = fmaf(P, mx, h * dx), gy = fmaf(P, my, h * dy), gz = fmaf(P, mz, h * dz);
     s[k][0] = fmaf(dx + dx, gx, fmaf(P, dm, s[k][0]));
     s[k][1] = fmaf(dy + dy, gy, fmaf(P, dm, s[k][1]));
@@ -1014,7 +1037,8 @@ __device__ __forceinline__ void hessian_wave(const Points &tgt, int64_t nt, cons
       }
     } else {
       if (!have_tab) {
-        load_table(d_hess_tab, s_tab, lane);
+        load_table(d_hess_tab, hc, kHessTabMid, s_tab, lane, 64);
+        __builtin_amdgcn_wave_barrier();
         have_tab = true;
       }
 #pragma unroll 1
@@ -1217,24 +1241,31 @@ __global__ __launch_bounds__(256) void reduce_force_kernel(
 // ---------------------------------------------------------------------------
 // Host side.
 
+// v as its FP32 value and what that leaves.
+static float2 two_floats(double v) {
+  const float hi = static_cast<float>(v);
+  return {hi, std::isfinite(hi) ? static_cast<float>(v - static_cast<double>(hi)) : 0.f};
+}
+
 FieldConsts make_field_consts(double h) {
   FieldConsts fc{};
   fc.h = static_cast<float>(h);
   fc.near2 = static_cast<float>(4.0 * h * h);
-  fc.inv_h3 = static_cast<float>(1.0 / (h * h * h));
-  fc.inv_h5 = static_cast<float>(1.0 / (h * h * h * h * h));
   fc.tab_scale = static_cast<float>(kFieldTabN / (2.0 * h));
+  fc.tab_high = static_cast<float>(fc.tab_scale * (2.0 * h) / kFieldTabN - 1.0);
+  fc.tab_a = two_floats(1.0 / (h * h * h * h * h));
+  fc.tab_b = two_floats(1.0 / (h * h * h));
   return fc;
 }
 
 void make_field_table(double h, float *tab) {
   const double ih3 = 1.0 / (h * h * h), ih5 = ih3 / (h * h);
-  fill_field_table(ih5, ih3, [&](int e, const double *a, const double *b) { store_entry(tab, e, a, b); });
+  fill_field_table(ih5, ih3, [&](int e, const double *a, const double *b) { store_entry(tab, e, 1, a, b); });
 }
 
 void make_hess_table(double h, float *tab) {
   fill_hess_table(1.0 / (h * h * h * h), [&](int e, const double *a, const double *b) {
-    store_entry(tab, e, a, b);
+    store_entry(tab, e, -1, a, b);
   });
 }
 
@@ -1251,8 +1282,9 @@ HessConsts make_hess_consts(double h) {
   HessConsts hc{};
   hc.h = static_cast<float>(h);
   hc.near2 = static_cast<float>(16.0 * h * h);
-  hc.inv_h4 = static_cast<float>(1.0 / (h * h * h * h));
   hc.tab_scale = static_cast<float>(kHessTabN / (4.0 * h));
+  hc.tab_high = static_cast<float>(hc.tab_scale * (4.0 * h) / kHessTabN - 1.0);
+  hc.tab_a = hc.tab_b = two_floats(1.0 / (h * h * h * h));
   return hc;
 }
 
@@ -1679,11 +1711,15 @@ Status hessian_allpairs_launch(mf_ctx *ctx, const Points &tgt, int64_t nt, const
 
 // Internal: the near-pair coefficient tables, for the CPU tests (not part of
 // mf_capi.h).  kind 0 = field (kFieldTabEntries x 8 floats), 1 = force
-// (kHessTabEntries x 8).
+// (kHessTabEntries x 8), whose second curve is handed out divided by -5: R in units of
+// its far form's -5 r^-7.
 extern "C" int mf_internal_near_table(int kind, double h, float *out) {
   if (!out || !(h > 0.0)) return 1;
   if (kind == 0) mf::make_field_table(h, out);
-  else if (kind == 1) mf::make_hess_table(h, out);
-  else return 1;
+  else if (kind == 1) {
+    mf::make_hess_table(h, out);
+    for (int e = 0; e < mf::kHessTabEntries; ++e)
+      for (int j = 4; j < 8; ++j) out[8 * e + j] = static_cast<float>(out[8 * e + j] / -5.0);
+  } else return 1;
   return 0;
 }

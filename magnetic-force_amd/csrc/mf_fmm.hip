@@ -3462,14 +3462,12 @@ Status apply_field_impl(mf_plan *plan, float scale, const float *px, const float
       }
       KernelTimer timer(ctx, "p2p_field", ns);
       const int grid = 8 * ((nn.nheads + 7) / 8 + (nn.ntails + 7) / 8);
-      FieldConsts fc = plan->fc;  // the plan's table holds h
-      fc.inv_h3 = fc.inv_h5 = 1.f;
       MF_TRY(once_passes_run(
           F.onceF, nn,
           [&](const OnceNear &pass) -> Status {
             MF_NEAR_LAUNCH(near_field_once_kernel, once_waves(ctx, nn.nheads + nn.ntails),
                            F.box_first.as<int32_t>(), F.box_count.as<int32_t>(),
-                           F.rec.as<SrcRec>(), n, pass, fc, F.ftab->buf.as<float4>(), near3, mask);
+                           F.rec.as<SrcRec>(), n, pass, plan->fc, F.ftab->buf.as<float4>(), near3, mask);
             MF_LAUNCH_CHECK();
             return Status::Ok();
           },
@@ -3542,14 +3540,12 @@ Status apply_force_impl(mf_plan *plan, const float *mx, const float *my, const f
       }
       KernelTimer timer(ctx, "p2p_force", ns);
       const int grid = 8 * ((nn.nheads + 7) / 8 + (nn.ntails + 7) / 8);
-      HessConsts hc = plan->hc;  // the plan's table holds h
-      hc.inv_h4 = 1.f;
       MF_TRY(once_passes_run(
           F.onceH, nn,
           [&](const OnceNear &pass) -> Status {
             MF_NEAR_LAUNCH(near_force_once_kernel, once_waves(ctx, nn.nheads + nn.ntails),
                            F.box_first.as<int32_t>(), F.box_count.as<int32_t>(),
-                           F.rec.as<SrcRec>(), n, pass, hc, F.htab->buf.as<float4>(), near3,
+                           F.rec.as<SrcRec>(), n, pass, plan->hc, F.htab->buf.as<float4>(), near3,
                            SysMask{});
             MF_LAUNCH_CHECK();
             return Status::Ok();

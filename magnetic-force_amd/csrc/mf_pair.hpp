@@ -38,9 +38,9 @@ constexpr double kMu0 = 1.25663706e-6;  // the reference's truncated value
 struct FieldConsts {
   float h;
   float near2;   // (2h)^2
-  float inv_h3;
-  float inv_h5;
   float tab_scale;  // kFieldTabN / (2h): r -> table coordinate q kFieldTabN / 2
+  float tab_high;   // how far tab_scale is rounded up, relative
+  float2 tab_a, tab_b;  // h^-5 and h^-3, each as its FP32 value and what that leaves
 };
 
 // Near-field coefficient table.  Interval k of
@@ -53,8 +53,8 @@ struct FieldConsts {
 // u that rounds up to kFieldTabN at q -> 2 reads a finite value with no
 // clamp.  At FP32 inputs q in [0, 2) the error is at most 1.5e-7 of
 // max(|alpha|, (2h)^-5) and of max(|beta|, (2h)^-3); an FP32 evaluation of the
-// closed forms stays within 7e-7 and 1.6e-6.  The all-pairs kernels read the
-// table at h = 1 (a constant of the code object) and scale by h^-5, h^-3; the
+// closed forms stays within 7e-7 and 1.6e-6.  The all-pairs kernels take the
+// table at h = 1 (a constant of the code object) times h^-5, h^-3 into LDS; the
 // FMM's tables hold h.
 //
 // Device copies of both tables (split_near_table) hold the first curve's
@@ -67,8 +67,9 @@ constexpr int kFieldTabEntries = kFieldTabN + 1;
 struct HessConsts {
   float h;
   float near2;       // (4h)^2
-  float inv_h4;
   float tab_scale;   // kHessTabN / (4h): r -> table coordinate q kHessTabN / 4
+  float tab_high;    // how far tab_scale is rounded up, relative
+  float2 tab_a, tab_b;  // h^-4 (both curves), as its FP32 value and what that leaves
 };
 
 // Force-curve table: kHessTabN intervals over q in
@@ -76,7 +77,7 @@ struct HessConsts {
 // (piece p covers (p, p + 1], so an integer q stays with the lower piece).
 // Entry e = ceil(u), u = q kHessTabN / 4, covers u in (e - 1, e] and holds two
 // cubics in t = u - e, in (-1, 0]: [0..3] C1 / (s h^4), [4..7]
-// -(C2 - 3 C1) / (5 s h^4), the R / -5 the force pair uses.  Entries
+// (C2 - 3 C1) / (s h^4), from which R follows with no further factor.  Entries
 // 1 .. kHessTabN interpolate at their interval's four Chebyshev points;
 // entry 0 (u = 0, a pair at d = 0) continues entry 1's cubics and entry
 // kHessTabN + 1 (u rounded above kHessTabN at q -> 4) entry kHessTabN's, so
@@ -112,7 +113,7 @@ __device__ __forceinline__ void field_near_coeffs_tab(const float4 *tab, float t
 }
 
 // The two curves of a force pair within 4h (r2 <= near2) from the table
-// (LDS): P = c1 irc and R / -5 = dq irc^3.  The caller clamps the inverse
+// (LDS): P = c1 irc and R = dq irc^3.  The caller clamps the inverse
 // distance irc to a finite value, so a pair at d = 0 (a particle and itself,
 // or two coincident ones) gets finite coefficients, whose terms all vanish
 // with d.

@@ -109,8 +109,6 @@ struct FieldSelf {
           if constexpr (MIXED) {
             if (p.r2[i] < fc.near2) {
               field_near_coeffs_tab(tab, fc.tab_scale, p.r2[i], p.ir[i], alpha, beta);
-              alpha *= fc.inv_h5;
-              beta *= fc.inv_h3;
             }
           }
           const float dm = fmaf(p.dx[i], v.x, fmaf(p.dy[i], v.y, p.dz[i] * v.z));
@@ -189,15 +187,15 @@ struct ForceSelf {
             // the clamp keeps a pair at d = 0 finite
             const float ir = __builtin_amdgcn_fmed3f(p.ir[i], 0.f, 1e12f);
             const float ir2 = ir * ir;
-            float c1 = ir2 * ir2, dq = c1;  // far curves
+            float c1 = ir2 * ir2, dq = -5.f * c1;  // far curves
             if (!(p.r2[i] > hc.near2)) {
               hess_near_curves_tab(tab, hc.tab_scale, p.r2[i], ir, c1, dq);
-              const float w = p.r2[i] > 0.f ? hc.inv_h4 : 0.f;  // nothing at d = 0
-              c1 *= w;
-              dq *= w;
+              const bool apart = p.r2[i] > 0.f;  // nothing at d = 0
+              c1 = apart ? c1 : 0.f;
+              dq = apart ? dq : 0.f;
             }
             P = c1 * ir;
-            e = fmaf(-5.f * dq * (ir2 * ir), dm * dn, P * mn);
+            e = fmaf(dq * (ir2 * ir), dm * dn, P * mn);
           } else {
             const float ir2 = p.ir[i] * p.ir[i];
             P = ir2 * ir2 * p.ir[i];
