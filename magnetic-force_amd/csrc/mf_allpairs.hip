@@ -818,7 +818,10 @@ __global__ __launch_bounds__(64) void force_allpairs_kernel(
 // chip enough workgroups; the chunk reduction adds the slots in a fixed order.
 
 constexpr int kSelfTPT = 4;      // 64 targets a wave, 64 = kTile
-constexpr int kSelfFlush = 4;    // units between FP64 accumulations
+// Units between FP64 accumulations: the FP32 chains are 16 terms a unit.  The force's terms
+// cancel: with four units it was 13 % further from FP64 than the directed kernels' on 12,000
+// nearly equal moments, with one it is level (262,144 particles: 29.2 -> 29.8 ms).
+constexpr int kFieldSelfFlush = 4, kForceSelfFlush = 1;
 
 struct SelfWalk {
   int ntiles;   // tiles of the record set
@@ -828,7 +831,7 @@ struct SelfWalk {
   int nchunk;
 };
 
-template <class Pairs, class Consts, int W, int NTAB>
+template <class Pairs, class Consts, int W, int NTAB, int FLUSH>
 __device__ __forceinline__ void self_walk(const SrcRec *__restrict__ rec,
                                           const float4 *__restrict__ boxes, int64_t n,
                                           const SelfWalk &w, const Consts &consts,
@@ -915,14 +918,14 @@ __device__ __forceinline__ void self_walk(const SrcRec *__restrict__ rec,
         else
           prs.template tile<true, false>(st[buf], c, q, jc);
       }
-      if (++since == kSelfFlush) {
+      if (++since == FLUSH) {
         flush();
         since = 0;
       }
     }
     if (both) {
 #pragma unroll
-      for (int a = 0; a < 3; ++a) jp[buf][wave][a][lane] = row_next(jc[a]);
+      for (int a = 0; a < 3; ++a) jp[buf][wave][a][lane] = jc[a];
     }
     wait_vm<0>();
     __syncthreads();
@@ -960,7 +963,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
                                                             int64_t n, SelfWalk w, FieldConsts fc,
                                                             double *__restrict__ partial, Skip skip) {
   if (skipped(skip)) return;
-  self_walk<FieldSelf<kSelfTPT>, FieldConsts, W, kFieldTabEntries>(
+  self_walk<FieldSelf<kSelfTPT>, FieldConsts, W, kFieldTabEntries, kFieldSelfFlush>(
       rec, boxes, n, w, fc, d_field_tab, kFieldTabMid, 1.0 / (4.0 * kPi), partial);
 }
 
@@ -969,7 +972,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
                                                             const float4 *__restrict__ boxes,
                                                             int64_t n, SelfWalk w, HessConsts hc,
                                                             double *__restrict__ partial) {
-  self_walk<ForceSelf<kSelfTPT>, HessConsts, W, kHessTabEntries>(
+  self_walk<ForceSelf<kSelfTPT>, HessConsts, W, kHessTabEntries, kForceSelfFlush>(
       rec, boxes, n, w, hc, d_hess_tab, kHessTabMid, 3.0 * kMu0 / (4.0 * kPi), partial);
 }
 

@@ -1745,7 +1745,7 @@ __device__ __forceinline__ void once_pass(Pairs &prs, const float4 *__restrict__
         prs.template tile<false, true>(st[buf], c, q, jc);
 #pragma unroll
       for (int a = 0; a < 3; ++a) {
-        float v = row_next(jc[a]);
+        float v = jc[a];
         if (p < tot) {
           float *o = sums + a * len + p;
           if (again) v += *o;  // an earlier pass of this block, by this wave

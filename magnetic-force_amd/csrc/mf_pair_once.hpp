@@ -7,7 +7,8 @@
 // tile of 64 records in LDS, 16 for each row: at step s lane c takes record
 // (s + c) mod 16 of its row's sixteen, and the sums for that record move one lane
 // down the row with it, so after 16 steps lane l holds the sums of record l over
-// the wave's targets.  64 evaluated far pairs cost 96 (field) and 121 (force) cycles
+// the wave's targets.  Sums of either side that are combined in the end (the field's two,
+// the force's term along the particle's own moment) are kept apart until then.  64 evaluated far pairs cost 96 (field) and 121 (force) cycles
 // at TPT = 4, where two directed ones cost 130 and 182.
 #pragma once
 
@@ -89,8 +90,10 @@ struct FieldSelf {
   __device__ __forceinline__ double sum(int k, int a) const {
     return 3.0 * static_cast<double>(a1[k][a]) - static_cast<double>(a2[k][a]);
   }
+  // jc (BOTH): the sums of the lane's record
   template <bool MIXED, bool BOTH>
   __device__ __forceinline__ void tile(const SelfTile &st, int c, int q, float (&jc)[3]) {
+    float j1[3] = {0.f, 0.f, 0.f}, j2[3] = {0.f, 0.f, 0.f};
 #pragma unroll 1
     for (int s = 0; s < 16; ++s) {
       const int r = 16 * q + ((s + c) & 15);
@@ -133,8 +136,17 @@ struct FieldSelf {
       }
       if constexpr (BOTH) {
 #pragma unroll
-        for (int a = 0; a < 3; ++a) jc[a] = row_next(jc[a]) + fmaf(3.f, b1[a], -b2[a]);
+        for (int a = 0; a < 3; ++a) {
+          j1[a] = row_next(j1[a]) + b1[a];
+          j2[a] = row_next(j2[a]) + b2[a];
+        }
       }
+    }
+    if constexpr (BOTH) {
+#pragma unroll
+      for (int a = 0; a < 3; ++a)
+        jc[a] = static_cast<float>(3.0 * static_cast<double>(row_next(j1[a])) -
+                                   static_cast<double>(row_next(j2[a])));
     }
   }
 };
@@ -165,8 +177,10 @@ struct ForceSelf {
     return (static_cast<double>(ad[k][a]) + static_cast<double>(am[k][a])) +
            static_cast<double>(n) * static_cast<double>(an[k]);
   }
+  // jc (BOTH): the sums of the lane's record
   template <bool MIXED, bool BOTH>
   __device__ __forceinline__ void tile(const SelfTile &st, int c, int q, float (&jc)[3]) {
+    float j[3] = {0.f, 0.f, 0.f}, jf = 0.f;
 #pragma unroll 1
     for (int s = 0; s < 16; ++s) {
       const int r = 16 * q + ((s + c) & 15);
@@ -218,10 +232,17 @@ struct ForceSelf {
         }
       }
       if constexpr (BOTH) {
-        jc[0] = row_next(jc[0]) - fmaf(v.x, bf, b[0]);
-        jc[1] = row_next(jc[1]) - fmaf(v.y, bf, b[1]);
-        jc[2] = row_next(jc[2]) - fmaf(v.z, bf, b[2]);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) j[a] = row_next(j[a]) + b[a];
+        jf = row_next(jf) + bf;
       }
+    }
+    if constexpr (BOTH) {
+      const float4 v = st.mom[16 * q + c];
+      const double f = static_cast<double>(row_next(jf));
+      jc[0] = static_cast<float>(-(static_cast<double>(v.x) * f + static_cast<double>(row_next(j[0]))));
+      jc[1] = static_cast<float>(-(static_cast<double>(v.y) * f + static_cast<double>(row_next(j[1]))));
+      jc[2] = static_cast<float>(-(static_cast<double>(v.z) * f + static_cast<double>(row_next(j[2]))));
     }
   }
 };
