@@ -373,13 +373,13 @@ int mf_set_alloc_hook(mf_alloc_hook hook, void *user);
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory (code under hipGraph stream capture, tight serving loops, harnesses
  * that forbid hipMalloc): the same product as mf_field_allpairs, with every
- * scratch buffer (packed source and target records, tile boxes, source-chunk
- * partials) in one static device array of mf_noalloc_scratch_bytes() bytes
- * (32 MiB) per GPU, held from library load until the process ends.  The call
+ * scratch buffer (packed source records, tile boxes, source-chunk partials) in
+ * one static device array of mf_noalloc_scratch_bytes() bytes (32 MiB) per GPU,
+ * held from library load until the process ends.  The call
  * itself allocates nothing; the context must exist already (mf_ctx_create
  * looks up the array's address on its device).  Limit: n_t and n_s such that
  * 32 (pad64(n_s) + 1) + 32 (pad64(n_s) / 64 + 1) + 32 (pad64(n_t) + 1)
- * + 24 n_t bytes (each term rounded up to 256) fit in the array, e.g.
+ * + 24 n_t bytes (each term rounded up to 256) are at most the array's, e.g.
  * n_t = n_s = 262144; larger sizes return MF_ERR_INVALID_ARG.  Every call on
  * one GPU shares the array: calls that overlap on one GPU race. */
 int mf_field_allpairs_noalloc(mf_ctx *ctx, int64_t n_t, const float *tx, const float *ty,

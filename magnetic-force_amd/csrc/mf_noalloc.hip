@@ -1,8 +1,8 @@
 // mf_noalloc.hip -- the all-pairs field product without any allocation.
 //
 // mf_field_allpairs_noalloc runs the same kernels as mf_field_allpairs (pack
-// the sources and targets into records, tile boxes, the chunked field kernel,
-// the fixed-order chunk reduction), but every scratch buffer lives in one
+// the sources into records, tile boxes, the chunked field kernel, the fixed-order
+// chunk reduction), but every scratch buffer lives in one
 // file-scope device array, `scratch`, instead of the context's workspaces.
 // It is for callers that cannot call hipMalloc: code under stream capture,
 // tight serving loops, harnesses that forbid allocation.
@@ -62,20 +62,22 @@ void *scratch_addr(int device) {
   return g_scratch_addr[device];
 }
 
-// Byte layout of one call inside the scratch array.
+// Byte layout of one call inside the scratch array.  `limit` is what the sizes are held
+// to (mf_capi.h): it counts a record per target, which the call no longer needs, since it
+// reads targets where they lie; the room goes to the chunk partials.
 struct NoallocLayout {
-  size_t src, boxes, tgt, partial, end;
+  size_t src, boxes, partial, limit;
 };
 
-NoallocLayout noalloc_layout(int64_t n_t, int64_t n_s, int64_t nchunk) {
+NoallocLayout noalloc_layout(int64_t n_t, int64_t n_s) {
   NoallocLayout l{};
   const size_t ns_pad = static_cast<size_t>(padded_sources(n_s));
   const size_t nt_pad = static_cast<size_t>(padded_sources(n_t));
   l.src = 0;
   l.boxes = align256(l.src + sizeof(SrcRec) * (ns_pad + 1));
-  l.tgt = align256(l.boxes + sizeof(float4) * 2 * (ns_pad / kTile + 1));
-  l.partial = align256(l.tgt + sizeof(SrcRec) * (nt_pad + 1));
-  l.end = l.partial + sizeof(double) * static_cast<size_t>(field_partial_doubles(n_t, nchunk));
+  l.partial = align256(l.boxes + sizeof(float4) * 2 * (ns_pad / kTile + 1));
+  l.limit = align256(l.partial + sizeof(SrcRec) * (nt_pad + 1)) +
+            sizeof(double) * static_cast<size_t>(field_partial_doubles(n_t, 1));
   return l;
 }
 
@@ -102,12 +104,12 @@ extern "C" int mf_field_allpairs_noalloc(mf_ctx *ctx, int64_t n_t, const float *
     MF_ARG(n_t == 0 || (tx && ty && tz && ox && oy && oz), "target/output pointers are null");
     MF_ARG(n_s == 0 || (sx && sy && sz && mx && my && mz), "source pointers are null");
     if (n_t == 0) return Status::Ok();
-    const mf::NoallocLayout need = mf::noalloc_layout(n_t, n_s, 1);
-    if (need.end > kScratchBytes)
+    const mf::NoallocLayout need = mf::noalloc_layout(n_t, n_s);
+    if (need.limit > kScratchBytes)
       return Status::Err(MF_ERR_INVALID_ARG,
                          "mf_field_allpairs_noalloc: n_t = " + std::to_string(n_t) +
                              ", n_s = " + std::to_string(n_s) + " need " +
-                             std::to_string(need.end) + " bytes of scratch; the maximum is " +
+                             std::to_string(need.limit) + " bytes of scratch; the maximum is " +
                              std::to_string(kScratchBytes));
     MF_HIP(hipSetDevice(ctx->device));
     unsigned char *base = static_cast<unsigned char *>(mf::scratch_addr(ctx->device));
