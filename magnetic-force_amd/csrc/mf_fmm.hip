@@ -2404,7 +2404,9 @@ Status build_field_table(mf_ctx *ctx, double h, bool hess, std::shared_ptr<Field
 //  * where the tiles fill the chip's resident workgroups, the ones left for a last, partly
 //    filled round (the shortest) share it: 1,153,433
 //    particles' 729 tiles over 512 resident workgroups 1.42 -> 1.35 ms, 1.36 with at most
-//    two parts; with every tile in two parts 1.71.
+//    two parts; with every tile in two parts 1.71.  At p = 6 and 8 it gains up to 14 %
+//    (FP32, p = 6, 90,000 leaves 4.78 -> 4.16 ms; p = 8, 70,000 8.74 -> 7.49) and loses 12 at
+//    worst (BF16x3, p = 6, 120,000 leaves 2.08 -> 2.34).
 constexpr int kM2LFill = 4, kM2LPartsMax = 16, kM2LTailMax = 4;
 struct M2LSplit {
   int whole, parts;
@@ -3147,7 +3149,10 @@ Status fmm_info(mf_plan *plan, mf_plan_info *info) {
 
 namespace {
 
-// Waves per SIMD that an M2L kernel's registers admit (p = 10).
+// Waves per SIMD that an M2L kernel's registers admit at p = 10.  At p = 6 and 8 the one-part
+// kernel has four instead of three and the split kernel of p = 6 three instead of two; with
+// these numbers the launches of 20,000 to 220,000 leaves were within 2 % in the mean, one
+// 20 % slower (one part, p = 8, 90,000 leaves), so one rule serves all orders.
 int m2l_resident(int prec) {
   return prec == MF_M2L_BF16X1_CUT ? 4 : prec == MF_M2L_BF16X3 || prec == MF_M2L_BF16X6 ? 2 : 3;
 }
