@@ -2195,7 +2195,7 @@ struct FmmState {
   DeviceBuffer tilesM, tilesL, tlistM, tnM, tlistL, tnL;
   std::vector<int> tileM_start, tileL_start;  // [level], size D + 2
   DeviceBuffer Mt, Lt;
-  DeviceBuffer Lp;  // the parts' locals [parts][nbox][KP] where the M2L splits its tiles
+  int64_t part_floats = 0;  // the parts' expansions where an M2L or M2M splits its tiles
   DeviceBuffer Mb;  // BF16 parts of Mt [nbox][3][KP], for the BF16-split M2L
   int64_t p2p_field_pairs = 0;  // sum over leaves of targets x near sources
   int64_t p2p_force_pairs = 0;
@@ -2540,6 +2540,17 @@ Status once_buffers(mf_ctx *ctx, FmmState::Once &o, int64_t n, OnceNear &nn, dou
     (void)hipGetLastError();  // a smaller buffer may be had
   }
   nn.sums = static_cast<float *>(p);
+  return Status::Ok();
+}
+
+// The parts' expansions of a product's split launches (null: none is split).  The context's,
+// not the plan's: at 253,555 particles it is a fifth of what a plan allocates.
+Status parts_buffer(mf_ctx *ctx, const FmmState &F, float **parts) {
+  *parts = nullptr;
+  if (F.part_floats == 0) return Status::Ok();
+  void *p = nullptr;
+  MF_TRY(workspace(ctx, "fmm_parts", sizeof(float) * static_cast<size_t>(F.part_floats), &p));
+  *parts = static_cast<float *>(p);
   return Status::Ok();
 }
 
@@ -3037,7 +3048,9 @@ Status fmm_build_at(mf_plan *plan, double s_leaf, int *wider = nullptr) {
       const int mp = nt > 0 ? m2m_parts(ctx, F.KP, nt) : 1;
       if (mp > 1) boxes = std::max(boxes, static_cast<int64_t>(cnt[l]) * mp);
     }
-    if (boxes > 0) MF_TRY(need<float>(F.Lp, boxes * F.KP));
+    F.part_floats = boxes * F.KP;
+    float *parts_mem = nullptr;
+    MF_TRY(parts_buffer(ctx, F, &parts_mem));
   }
   MF_TRY(need<uint16_t>(F.Mb, static_cast<int64_t>(F.nbox) * 3 * F.KP));
   {
@@ -3160,7 +3173,7 @@ int m2l_resident(int prec) {
 template <int P, int KP>
 Status launch_m2l(mf_ctx *ctx, FmmState &F, const FmmTables &tab, int prec, const M2LTile *tiles,
                   int ntiles, const int32_t *src, int src_rows, int nslot, const int32_t *tlist,
-                  const int32_t *tn, SysMask mask, bool fence,
+                  const int32_t *tn, SysMask mask, bool fence, float *parts_mem,
                   M2LSrc2 src2 = M2LSrc2{nullptr, 0, 0, INT_MAX, nullptr}) {
   if (ntiles <= 0) return Status::Ok();
   const M2LSplit split = m2l_split(ctx, KP, ntiles, m2l_resident(prec));
@@ -3169,7 +3182,7 @@ Status launch_m2l(mf_ctx *ctx, FmmState &F, const FmmTables &tab, int prec, cons
     src2.whole = split.whole;
     src2.parts = split.parts;
     src2.part_stride = static_cast<int64_t>(F.nbox) * KP;
-    src2.Lp = F.Lp.as<float>();
+    src2.Lp = parts_mem;
   }
   const int per = (ntiles + 7) / 8, nsplit = std::max(per - split.whole, 0);
   const dim3 grid(8 * (per - nsplit + nsplit * split.parts)), block(2 * KP);
@@ -3246,6 +3259,8 @@ Status upward_and_m2l(mf_plan *plan, bool hess, const std::function<Status()> &l
   MF_TRY(launch_near());
   if (D < 2) return Status::Ok();
   const int prec = plan->m2l_precision();
+  float *parts_mem = nullptr;
+  MF_TRY(parts_buffer(ctx, F, &parts_mem));
   {
     KernelTimer timer(ctx, "p2m");
     hipLaunchKernelGGL((p2m_kernel<P, KP>), dim3(nleaf), dim3(64), 0, ctx->stream, nleaf,
@@ -3312,7 +3327,7 @@ Status upward_and_m2l(mf_plan *plan, bool hess, const std::function<Status()> &l
       const int64_t first = static_cast<int64_t>(F.base[l]) * KP,
                     ne = static_cast<int64_t>(F.count[l]) * KP;
       // the parts of a level's boxes lie from the buffer's start on
-      float *lp = parts > 1 ? F.Lp.as<float>() - first : nullptr;
+      float *lp = parts > 1 ? parts_mem - first : nullptr;
       MF_TRY(octant_pass(npart ? F.Mb.get() : F.Mt.get(), F.Mt.as<float>(),
                          npart ? tab.W_m2m_b.get() : tab.W_m2m.get(),
                          F.tilesM.as<M2LTile>() + t0, nt, F.box_ids.as<int32_t>(),
@@ -3342,7 +3357,7 @@ Status upward_and_m2l(mf_plan *plan, bool hess, const std::function<Status()> &l
     if (!hess) {
       MF_TRY((launch_m2l<P, KP>(ctx, F, tab, prec, F.tilesF.as<M2LTile>(), F.ntilesF, F.srcF.as<int32_t>(),
                             F.nbox, tab.nslotF, F.tlistF.as<int32_t>(), F.tnF.as<int32_t>(), mask,
-                            false, M2LSrc2{nullptr, 0, 0, INT_MAX, F.orderF.as<int32_t>()})));
+                            false, parts_mem, M2LSrc2{nullptr, 0, 0, INT_MAX, F.orderF.as<int32_t>()})));
     } else {
       // Tiles are in level order: the leaf level's (trailing) tiles read the
       // force lists srcH (indexed by leaf = global index), the others srcF;
@@ -3350,7 +3365,7 @@ Status upward_and_m2l(mf_plan *plan, bool hess, const std::function<Status()> &l
       const int lt = F.leaf_tile_start;
       MF_TRY((launch_m2l<P, KP>(ctx, F, tab, prec, F.tilesH.as<M2LTile>(), F.ntilesH,
                             F.srcF.as<int32_t>(), F.nbox, tab.nslotF, F.tlistH.as<int32_t>(),
-                            F.tnH.as<int32_t>(), mask, true,
+                            F.tnH.as<int32_t>(), mask, true, parts_mem,
                             M2LSrc2{F.srcH.as<int32_t>(), tab.nslotH, F.count[D], lt,
                                     F.orderH.as<int32_t>()})));
     }
