@@ -24,8 +24,8 @@ namespace mf {
 namespace {
 
 // Device scalars of a CG solve: the residual norms r.r of the even and the odd
-// iterations (an iteration reads one and writes the other), and b.b.
-enum { S_RR0 = 0, S_RR1 = 1, S_BB = 2, S_COUNT = 8 };
+// iterations (an iteration reads one and writes the other).
+enum { S_RR0 = 0, S_RR1 = 1, S_COUNT = 2 };
 
 __device__ __forceinline__ double block_sum(double v, double *sh) {
 #pragma unroll
@@ -139,7 +139,6 @@ __global__ __launch_bounds__(kRedBlock) void cg_start_sum_kernel(const double *_
   const double rr = sum_of(partials, nb, sh), bb = sum_of(partials + nb, nb, sh);
   if (threadIdx.x == 0) {
     sc[S_RR0] = rr;
-    sc[S_BB] = bb;
     host[0] = rr;
     host[1] = bb;
   }
@@ -958,8 +957,8 @@ __global__ void fill_i32_kernel(int n, int32_t v, int32_t *__restrict__ a) {
   if (i < n) a[i] = v;
 }
 
-// An iteration's vector work is four launches, one workgroup per chunk or one
-// thread per system: ap = p - g with the chunk's part of p . ap; the systems' sums
+// An iteration's vector work is five launches, one workgroup per chunk, one
+// thread per system or one per particle: ap = p - g with the chunk's part of p . ap; the systems' sums
 // and alpha; x, r with the part of r . r; sums, beta and the largest residual, which
 // goes to pinned host memory; then p.  As nine launches over chunks of 16,384 (a dot
 // product 21 us on 96 droplets) and a copy per iteration the batch took 0.6 ms longer.
