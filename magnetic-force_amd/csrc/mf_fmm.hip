@@ -1850,7 +1850,9 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
 // Where the other blocks leave the sums of a leaf's particles: places[leaf][..] =
 // {off of the source block, stream position of the leaf's particle 0}, first the nw
 // blocks that meet the whole leaf, then the nt that meet its tail only, both in slot order;
-// np[leaf] = {nw, nt}.  One thread per slot.
+// np[leaf] = {nw, nt}.  One thread per slot.  The last workgroup leaves the build's figures in
+// pinned host memory: off and units of the last block, then the counters (longest stream,
+// and with nc = 3 the list sizes); copies of single words took the host 10 us each.
 template <int NS>
 constexpr int kPlaces = (NS - 1) / 2 + NS;  // heads at NS - 1 offsets and their own, tails at half
 template <int NS>
@@ -1859,10 +1861,18 @@ __global__ __launch_bounds__(256) void near_places_kernel(const int32_t *__restr
                                                           const int32_t *__restrict__ count,
                                                           const int32_t *__restrict__ pre,
                                                           const int32_t *__restrict__ off,
+                                                          const int32_t *__restrict__ units,
+                                                          const int32_t *__restrict__ counters,
+                                                          int nc, int32_t *__restrict__ host,
                                                           int2 *__restrict__ places,
                                                           int2 *__restrict__ np) {
   static_assert(NS <= 256, "one thread per slot");
   const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  if (b == static_cast<int>(gridDim.x) - 1 && tid == 0) {
+    host[0] = off[2 * b + 1];
+    host[1] = units[2 * b + 1];
+    for (int k = 0; k < nc; ++k) host[2 + k] = counters[k];
+  }
   const int h = head_count(count[b]);
   __shared__ int s_n[4][2];
   bool whole = false, found[2] = {false, false};
@@ -1992,7 +2002,11 @@ __global__ __launch_bounds__(256) void near_gather_kernel(
   }
 }
 
-__global__ void set_record_kernel(SrcRec *r, SrcRec v) { *r = v; }
+// The padding record, and zeros for the counters of a plan build.
+__global__ void begin_once_kernel(SrcRec *r, SrcRec v, int32_t *__restrict__ counters, int n) {
+  if (threadIdx.x == 0) *r = v;
+  if (static_cast<int>(threadIdx.x) < n) counters[threadIdx.x] = 0;
+}
 
 // Moments into the sorted records: rec[i].m = scale * weight[perm[i]] * m[perm[i]]
 // (weight: optional per-particle factor in caller order, e.g. kappa per system).
@@ -2461,20 +2475,29 @@ inline int once_waves(const mf_ctx *ctx, int nblock) {
   return w;
 }
 
-// Streams of the leaf blocks; once[field, force] receives, after a synchronize, the last
-// block's offset and units and the longest stream.
-Status build_once(mf_ctx *ctx, FmmState &F, const FmmTables &tab, int nleaf, int64_t n,
-                  int32_t (*once)[3], const int32_t **block_units) {
+// Streams, places and lists of the leaf blocks: the near-field kernels' tables.  Waits for
+// the stream.
+Status build_once(mf_ctx *ctx, FmmState &F, const FmmTables &tab, int nleaf, int64_t n) {
   const int64_t nblock = 2 * static_cast<int64_t>(nleaf);
-  void *pu = nullptr;
-  MF_TRY(workspace(ctx, "fmm_once_units", sizeof(int32_t) * static_cast<size_t>(nblock + 1), &pu));
-  int32_t *units = static_cast<int32_t *>(pu), *longest = units + nblock;
-  *block_units = units;  // the force's, once both are built
+  // counters: the field's longest stream, the force's, and the sizes of the leaf lists
+  constexpr int kCounters = 2 + kLeafLists;
+  void *pu = nullptr, *pk = nullptr;
+  MF_TRY(workspace(ctx, "fmm_once_units", sizeof(int32_t) * static_cast<size_t>(nblock + kCounters), &pu));
+  int32_t *units = static_cast<int32_t *>(pu), *counters = units + nblock;
+  MF_TRY(need<int32_t>(F.leaf_lists, nblock));
+  MF_TRY(workspace(ctx, "fmm_leaf_keys", (sizeof(uint64_t) * 2 + sizeof(int32_t)) * static_cast<size_t>(nblock), &pk));
+  uint64_t *k_in = static_cast<uint64_t *>(pk), *k_out = k_in + nblock;
+  int32_t *v_in = reinterpret_cast<int32_t *>(k_out + nblock);
+  const bool ordered = once_waves(ctx, nleaf) >= kOrderWaves;
+  int32_t *host = reinterpret_cast<int32_t *>(ctx->host_scalars),
+          *host_dev = reinterpret_cast<int32_t *>(ctx->host_scalars_dev);
+  constexpr int kHostStride = 2 + 1 + kLeafLists;
   const SrcRec pad{kPadCoord, kPadCoord, kPadCoord, 0.f, 0.f, 0.f, 0.f, 0.f};
-  hipLaunchKernelGGL(set_record_kernel, dim3(1), dim3(1), 0, ctx->stream, F.rec.as<SrcRec>() + n, pad);
+  hipLaunchKernelGGL(begin_once_kernel, dim3(1), dim3(64), 0, ctx->stream, F.rec.as<SrcRec>() + n, pad,
+                     counters, kCounters);
   MF_LAUNCH_CHECK();
   auto build = [&](auto nslot, const DeviceBuffer &near, const DeviceBuffer &sym,
-                   FmmState::Once &o, int32_t *last) -> Status {
+                   FmmState::Once &o, int which) -> Status {
     constexpr int NS = decltype(nslot)::value;
     const int64_t npl = static_cast<int64_t>(nleaf) * kPlaces<NS>, npre = nblock * (NS + 1);
     MF_TRY(o.mem.reserve(sizeof(int2) * static_cast<size_t>(npl + nleaf) +
@@ -2484,25 +2507,37 @@ Status build_once(mf_ctx *ctx, FmmState &F, const FmmTables &tab, int nleaf, int
     o.np = o.places + npl;
     o.pre = reinterpret_cast<int32_t *>(o.np + nleaf);
     o.off = o.pre + npre;
-    MF_HIP(hipMemsetAsync(longest, 0, sizeof(int32_t), ctx->stream));
     hipLaunchKernelGGL(once_stream_kernel<NS>, dim3(grid_for(nblock, 4)), dim3(256), 0, ctx->stream,
                        nleaf, near.as<int32_t>(), sym.as<int2>(), F.box_count.as<int32_t>(),
-                       o.pre, units, longest);
+                       o.pre, units, counters + which);
     MF_LAUNCH_CHECK();
     MF_TRY(exclusive_scan_i32(ctx, units, o.off, nblock));
+    if (which == 1) {
+      // heads and tails, by the force's streams
+      hipLaunchKernelGGL(classify_leaves_kernel, dim3(grid_for(nleaf, 256)), dim3(256), 0,
+                         ctx->stream, nleaf, F.box_count.as<int32_t>(), ordered ? units : nullptr,
+                         k_in, v_in, counters + 2);
+      MF_LAUNCH_CHECK();
+      MF_TRY(sort_pairs_u64_i32(ctx, k_in, k_out, v_in, F.leaf_lists.as<int32_t>(), nblock, 0,
+                                ordered ? 13 : 2));
+    }
     hipLaunchKernelGGL(near_places_kernel<NS>, dim3(nleaf), dim3(256), 0, ctx->stream,
-                       near.as<int32_t>(), sym.as<int2>(), F.box_count.as<int32_t>(),
-                       o.pre, o.off, o.places, o.np);
+                       near.as<int32_t>(), sym.as<int2>(), F.box_count.as<int32_t>(), o.pre, o.off,
+                       units, counters + which, which == 1 ? 1 + kLeafLists : 1,
+                       host_dev + which * kHostStride, o.places, o.np);
     MF_LAUNCH_CHECK();
-    MF_HIP(hipMemcpyAsync(last, o.off + nblock - 1, sizeof(int32_t),
-                          hipMemcpyDeviceToHost, ctx->stream));
-    // the last block's units and the longest stream lie side by side
-    MF_HIP(hipMemcpyAsync(last + 1, units + nblock - 1, 2 * sizeof(int32_t), hipMemcpyDeviceToHost,
-                          ctx->stream));
     return Status::Ok();
   };
-  MF_TRY(build(std::integral_constant<int, kNearF>{}, F.nearF, tab.symF, F.onceF, once[0]));
-  return build(std::integral_constant<int, kNearH>{}, F.nearH, tab.symH, F.onceH, once[1]);
+  MF_TRY(build(std::integral_constant<int, kNearF>{}, F.nearF, tab.symF, F.onceF, 0));
+  MF_TRY(build(std::integral_constant<int, kNearH>{}, F.nearH, tab.symH, F.onceH, 1));
+  MF_HIP(hipStreamSynchronize(ctx->stream));
+  FmmState::Once *once[2] = {&F.onceF, &F.onceH};
+  for (int k = 0; k < 2; ++k) {
+    once[k]->units = host[k * kHostStride] + host[k * kHostStride + 1];
+    once[k]->longest = host[k * kHostStride + 2];
+  }
+  for (int k = 0; k < kLeafLists; ++k) F.leaf_list_n[k] = host[kHostStride + 3 + k];
+  return Status::Ok();
 }
 
 // A near-field product's passes over its places: window units of 16 places each.  A block
@@ -2800,33 +2835,7 @@ Status fmm_build_at(mf_plan *plan, double s_leaf, int *wider = nullptr) {
                      dim3(256), 0, ctx->stream, nleaf, F.box_keys.as<uint64_t>(), cells, 3 * D,
                      tab.nearH.as<int3>(), kNearH, leaf_grid, F.nearH.as<int32_t>());
   MF_LAUNCH_CHECK();
-  {
-    // streams of the near-field kernels' blocks, heads and tails
-    int32_t once[2][3] = {};
-    const int32_t *units = nullptr;
-    MF_TRY(build_once(ctx, F, tab, nleaf, n, once, &units));
-    const int64_t ne = 2 * static_cast<int64_t>(nleaf);
-    const bool ordered = once_waves(ctx, nleaf) >= kOrderWaves;
-    MF_TRY(need<int32_t>(F.leaf_lists, ne));
-    void *pk = nullptr, *pz = nullptr;
-    MF_TRY(workspace(ctx, "fmm_leaf_keys", (sizeof(uint64_t) * 2 + sizeof(int32_t)) * ne, &pk));
-    MF_TRY(workspace(ctx, "fmm_leaf_sizes", sizeof(int32_t) * kLeafLists, &pz));
-    uint64_t *k_in = static_cast<uint64_t *>(pk), *k_out = k_in + ne;
-    int32_t *v_in = reinterpret_cast<int32_t *>(k_out + ne);
-    MF_HIP(hipMemsetAsync(pz, 0, sizeof(int32_t) * kLeafLists, ctx->stream));
-    hipLaunchKernelGGL(classify_leaves_kernel, dim3(grid_for(nleaf, 256)), dim3(256), 0,
-                       ctx->stream, nleaf, F.box_count.as<int32_t>(),
-                       ordered ? units : nullptr, k_in, v_in, static_cast<int32_t *>(pz));
-    MF_LAUNCH_CHECK();
-    MF_TRY(sort_pairs_u64_i32(ctx, k_in, k_out, v_in, F.leaf_lists.as<int32_t>(), ne, 0,
-                              ordered ? 13 : 2));
-    MF_HIP(hipMemcpyAsync(F.leaf_list_n, pz, sizeof(int32_t) * kLeafLists, hipMemcpyDeviceToHost, ctx->stream));
-    MF_HIP(hipStreamSynchronize(ctx->stream));
-    F.onceF.units = once[0][0] + once[0][1];
-    F.onceF.longest = once[0][2];
-    F.onceH.units = once[1][0] + once[1][1];
-    F.onceH.longest = once[1][2];
-  }
+  MF_TRY(build_once(ctx, F, tab, nleaf, n));
   // 5. M2L source slots (levels >= 2) and the class-sorted tile lists
   // one row past the last box of each slot array holds -1 throughout: the
   // M2L kernel's "no source" row
