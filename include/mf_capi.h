@@ -191,7 +191,13 @@ typedef struct mf_plan_opts {
 
 /* Replaces the construction of fmm_field_evaluator / fmm_hessian_evaluator
  * (magnetic_force.cu:650-672, 838-860) and, for the all-pairs mode, the
- * position upload of the constructor (:633).  Positions are copied. */
+ * position upload of the constructor (:633).  Positions are copied.
+ * Scratch is the context's and is kept until it is destroyed: for FMM plans the
+ * near field's pair sums, up to 12 GiB (+ 1/8), taken here and in
+ * mf_plan_update_positions as far as memory allows (256 MiB suffice); for
+ * all-pairs work on 4,096 particles or more up to 2 GiB (+ 1/8) at the first
+ * field product and as much at the first force product (less where less can be
+ * had).  Callers that need the memory allocate theirs first. */
 int mf_plan_create(mf_ctx *ctx, int64_t n, const float *x, const float *y, const float *z,
                    float h, const mf_plan_opts *opts, mf_plan **out);
 /* New positions (same or different n): setTargetpos, magnetic_force.cu:806-871. */

@@ -23,8 +23,8 @@
 //    box-to-box distance exceeds the smoothing support runs a branch-free
 //    far-field loop (pure dipole, one v_rsq_f32 per pair).  Other tiles run
 //    the mixed loop, which reads the smoothed coefficients from a table in LDS.
-//  * Sums of up to four tiles (64 terms a lane) are FP32; they are accumulated
-//    in FP64, so the summation error does not grow with N.
+//  * Sums of up to four tiles (64 terms a lane; of one for the force of a set on itself) are
+//    FP32; they are accumulated in FP64, so the summation error does not grow with N.
 //  * The source range is split into chunks of whole 16-record groups along
 //    grid.y to give the 256 CUs enough waves; chunk partials (FP64) are summed
 //    in a fixed order by a separate reduction kernel, so results are
@@ -34,7 +34,7 @@
 //  Measured per launch, at first (scalar sources, closed-form coefficients, chunks
 //  of whole tiles), directed kernels now, pairs once: field 22.6 / 8.4 us at 512
 //  particles, 65.0 / 52.8 / 41.8 us at 8,192, 33.8 / 28.3 / 22.6 ms at 262,144; force
-//  36.9 / 9.8 us, 91.9 / 76.2 / 57.0 us, 49.7 / 40.0 / 27.8 ms.  Field and tensor of
+//  36.9 / 9.8 us, 91.9 / 76.2 / 57.0 us, 49.7 / 40.0 / 29.1 ms.  Field and tensor of
 //  4,096 records on 65,520 targets 0.43 / 0.33 ms.  The VALU bounds the large sizes: a
 //  directed far field pair is 19 plain instructions at 2.3 cycles and one v_rsq_f32 at 16.
 #include <hip/hip_runtime.h>

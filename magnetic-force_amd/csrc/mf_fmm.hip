@@ -2418,7 +2418,8 @@ Status build_field_table(mf_ctx *ctx, double h, bool hess, std::shared_ptr<Field
 //  * where the tiles fill the chip's resident workgroups, the ones left for a last, partly
 //    filled round (the shortest) share it: 1,153,433
 //    particles' 729 tiles over 512 resident workgroups 1.42 -> 1.35 ms, 1.36 with at most
-//    two parts; with every tile in two parts 1.71.  At p = 6 and 8 it gains up to 14 %
+//    two parts; with every tile in two parts 1.71 (it reads 2.9 GB past L2 instead of 1.8: the
+//    parts' gathers share less).  At p = 6 and 8 it gains up to 14 %
 //    (FP32, p = 6, 90,000 leaves 4.78 -> 4.16 ms; p = 8, 70,000 8.74 -> 7.49) and loses 12 at
 //    worst (BF16x3, p = 6, 120,000 leaves 2.08 -> 2.34).
 constexpr int kM2LFill = 4, kM2LPartsMax = 16, kM2LTailMax = 4;
